@@ -105,7 +105,7 @@ int enqueue_step(brt_batch* b, const brt_steer_params* steer, float feature_rate
     if (!clean)
         BRT_HIP(brt::launch_prepare(b->meta, b->meta_words, buf->cell_start, buf->cell_end, b->total_cells, s),
                 "k_prepare");
-    brt::BatchView view{b->d_flocks, b->d_wave_flock, b->waves, b->d_step};
+    brt::BatchView view{b->d_flocks, b->d_wave_flock, b->waves, b->d_step, b->total_cells};
     uint2* A = reinterpret_cast<uint2*>(buf->hash);
     uint2* B = reinterpret_cast<uint2*>(b->tmp);
     uint2* first = (plan.passes & 1u) ? B : A;

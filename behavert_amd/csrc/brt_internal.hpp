@@ -198,6 +198,7 @@ struct BatchView {
     const uint32_t* wave_flock;  // flock of each wave
     uint32_t waves;              // total waves
     const uint32_t* step;        // device step counter (wander), may be NULL
+    uint32_t cells;              // total cells
 };
 
 // per-axis cell-box rounding margins (see the neighbour kernels)

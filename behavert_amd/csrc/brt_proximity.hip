@@ -29,7 +29,9 @@
 //     own cell index, eight (dense waves) or four (sparse waves) candidates
 //     per round, their accept bits logged per round;
 //   * vector mode (register-chunk lists): each lane walks its own stream, the
-//     wave in step cell by cell.
+//     wave in step cell by cell;
+//   * row scan (sparse waves): the cells of a row as one run, nine runs (see
+//     scan_rows).
 // Every mode skips a cell whose box lies farther than r from the agent (with
 // rounding margins so no candidate that passes the exact test is ever skipped),
 // only for interior cells: boundary cells can hold clamped out-of-grid or NaN
@@ -98,6 +100,23 @@
 #ifndef BRT_PROX_DENSE_LANES
 #define BRT_PROX_DENSE_LANES 32
 #endif
+// A wave takes the row scan (scan_rows) unless BRT_PROX_ROW_LANES of its lanes
+// have more than BRT_PROX_ROW_OCC agents in their own row's three cells: beyond
+// that some run is mostly too long for it, and the lists fill before their last
+// cells.  One step of 400,000 uniform agents, per-cell scan -> row scan, at 1 /
+// 4 / 6 agents per cell: K 32 152 -> 132 / 185 -> 166 / 204 -> 188 us, K 64
+// 190 -> 161 / 268 -> 216 / 307 -> 283 us; with the limit at 15: 4 per cell
+// 172 and 247 us; at 8 per cell no wave qualifies (208 us either way).
+#ifndef BRT_PROX_ROW_OCC
+#define BRT_PROX_ROW_OCC 23
+#endif
+// Launches of at most this many agents use the wide row scan.
+#ifndef BRT_PROX_WIDE_MAX
+#define BRT_PROX_WIDE_MAX (1u << 17)
+#endif
+#ifndef BRT_PROX_ROW_LANES
+#define BRT_PROX_ROW_LANES 32
+#endif
 #if BRT_PROX_ROLLED
 #define BRT_CELL_LOOP _Pragma("nounroll")
 #else
@@ -134,6 +153,7 @@ struct ProxArgs {
     uint32_t uniform_max_cells;
     uint32_t xcd_remap;
     uint32_t log_rounds;  // LDS lists through the round log (n < 2^24)
+    uint32_t cells;       // cells of the launch for the row scan's bounded loads; 0: no row scan
     const float4* spos;
     const float* pxyz;  // optional: the sorted positions packed as x,y,z (12 bytes each)
     const float4* sfwd;
@@ -264,17 +284,30 @@ __device__ __forceinline__ void append(Lane& L, uint32_t c, bool take) {
     L.cnt += take ? 1u : 0u;
 }
 
-// Count and padding (LDS lists), or the chunks not yet stored (register-chunk
-// lists: the pending partial chunk, then chunk 0).  Register-chunk lists
-// return the row's first all-padding chunk: those chunks are stored by the
-// whole wave together (pad_rows).
-template <bool LDSL>
-__device__ __forceinline__ uint32_t finish_list(Lane& L, uint32_t W) {
-    if (LDSL) {
-        L.row[0] = L.cnt;
-        for (uint32_t q = L.cnt + 1; q < W; ++q) L.row[q] = BRT_LIST_PAD;
-        return W / 4u;
+// Walks the 16-byte chunks of consecutive rows of W4 chunks, 64 apart: the row
+// and chunk of lane + 64 k without a division per step.
+struct ChunkWalk {
+    uint32_t row, chunk, drow, dchunk, w4;
+    __device__ __forceinline__ ChunkWalk(uint32_t lane, uint32_t W4) : w4(W4) {
+        row = lane / W4;
+        chunk = lane - row * W4;
+        drow = 64u / W4;
+        dchunk = 64u - drow * W4;
     }
+    __device__ __forceinline__ void next() {
+        row += drow;
+        chunk += dchunk;
+        if (chunk >= w4) {
+            chunk -= w4;
+            ++row;
+        }
+    }
+};
+
+// Register-chunk lists: the chunks not yet stored (the pending partial chunk,
+// then chunk 0).  Returns the row's first all-padding chunk: those chunks are
+// stored by the whole wave together (pad_rows).
+__device__ __forceinline__ uint32_t finish_list(Lane& L, uint32_t W) {
     const uint32_t P = BRT_LIST_PAD, k = L.cnt;
     uint4* row = reinterpret_cast<uint4*>(L.row);
     uint32_t q = (k > 3u ? (k - 3u) / 4u : 0u) + 1u;
@@ -297,11 +330,39 @@ __device__ __forceinline__ void pad_rows(uint32_t* lists, uint32_t row0, uint32_
     const uint32_t W4 = W / 4u, total = rows * W4;
     const uint32_t P = BRT_LIST_PAD;
     uint4* dst = reinterpret_cast<uint4*>(lists + (size_t)row0 * W);
-    for (uint32_t base = 0; base < total; base += 64u) {
+    ChunkWalk cw(lane, W4);
+    for (uint32_t base = 0; base < total; base += 64u, cw.next()) {
         const uint32_t w = base + lane;
-        const uint32_t r = w / W4;
-        const uint32_t first = (uint32_t)__shfl((int)pad_from, (int)(r < 64u ? r : 63u));
-        if (w < total && w - r * W4 >= first) dst[w] = make_uint4(P, P, P, P);
+        const uint32_t first = (uint32_t)__shfl((int)pad_from, (int)(cw.row < 64u ? cw.row : 63u));
+        if (w < total && cw.chunk >= first) dst[w] = make_uint4(P, P, P, P);
+    }
+}
+
+// Stores the wave's rows (consecutive, from sorted index row0) out of LDS with
+// consecutive 16-byte chunks per store: src holds one row of `stride` words per
+// lane, count first; words past the count are padding.  HEADS: src holds only
+// the rows' first `stride` words; of the later chunks those that hold entries
+// were stored by the row's own lane, the others are padding.
+template <bool HEADS>
+__device__ __forceinline__ void store_rows(uint32_t* lists, uint32_t row0, uint32_t rows, uint32_t W,
+                                           const uint32_t* src, uint32_t stride, uint32_t lane) {
+    const uint32_t W4 = W / 4u, total = rows * W4;
+    const uint32_t P = BRT_LIST_PAD;
+    uint4* dst = reinterpret_cast<uint4*>(lists + (size_t)row0 * W);
+    ChunkWalk cw(lane, W4);
+    for (uint32_t w = lane; w < total; w += 64u, cw.next()) {
+        const uint32_t* row = src + cw.row * stride;
+        const uint32_t cnt = row[0], e = 4u * cw.chunk;
+        if (!HEADS || e < stride) {
+            uint4 v = reinterpret_cast<const uint4*>(row)[cw.chunk];
+            v.x = e > cnt ? P : v.x;  // word 0 is the count itself
+            v.y = e + 1u > cnt ? P : v.y;
+            v.z = e + 2u > cnt ? P : v.z;
+            v.w = e + 3u > cnt ? P : v.w;
+            dst[w] = v;
+        } else if (e > cnt) {
+            dst[w] = make_uint4(P, P, P, P);
+        }
     }
 }
 
@@ -696,9 +757,243 @@ __device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane
     }
 }
 
-template <bool FUSE, bool BATCH, bool LDSL>
+// Row scan (sparse waves).  What bounds these waves is the VALU work and the
+// memory latency spent per cell, 27 cells holding one agent each or none.  x is
+// the fastest axis of the cell key, so the cells
+// x-1, x, x+1 of one (y, z) row are one contiguous run of sorted agents: nine
+// runs replace the 27 cells, and every range of a lane (18 12-byte loads) is in
+// flight at once.  The accept bits of a run are kept in a register, candidate c
+// in bit 31 - c; the lists want x outermost, so the runs' bits are split at the
+// ends of their cells x-1 and x and emitted x offset by x offset.  Runs longer
+// than kRowMax candidates do not fit (the wave takes another mode), nor does a
+// maxBodiesPerCell limit (it would cut holes into the runs).  Measured: the list
+// kernel of 4,194,304 uniform agents (one per cell, K 64) 664 -> 469 us (4,387
+// -> 2,795 VALU instructions per wave), the fused kernel of 100,003 32.2 ->
+// 25.8 us and of 4,096 (K 16) 23.4 -> 16.0 us.
+constexpr uint32_t kRowMax = 31;
+struct RowRange {
+    uint32_t start;  // the run's first sorted index
+    uint32_t ends;   // candidates before the end of cell x-1, of cell x, of cell x+1: 8 bits each
+    __device__ __forceinline__ uint32_t len() const { return ends >> 16; }
+};
+
+typedef uint32_t vuint3 __attribute__((ext_vector_type(3)));
+
+// mask of the first k (0..31) candidates
+__device__ __forceinline__ uint32_t first_bits(uint32_t k) { return ~(0xFFFFFFFFu >> k); }
+
+// Where a lane's rows are read: the three cells of a row from x = from (always
+// inside the row), shift = how far the wanted x-1 lies beyond from (not zero at
+// the grid's faces), and whether any wanted cell exists at all (the test also
+// guards the saturated coordinates of far-away agents).  Needs gx >= 3.
+struct RowX {
+    int from, shift;
+    bool any;
+};
+__device__ __forceinline__ RowX row_x(int x, int gx, bool alive) {
+    RowX r;
+    r.any = alive && x >= -1 && x <= gx;
+    const int want = (r.any ? x : 1) - 1;
+    r.from = want < 0 ? 0 : (want > gx - 3 ? gx - 3 : want);
+    r.shift = want - r.from;
+    return r;
+}
+
+// the wanted cells of a row from the three read, absent ones empty
+__device__ __forceinline__ vuint3 row_shift(vuint3 v, int shift) {
+    const uint32_t none = BRT_EMPTY_CELL;
+    vuint3 r;
+    r.x = shift == 0 ? v.x : shift == 1 ? v.y : shift == 2 ? v.z : none;
+    r.y = shift == 0 ? v.y : shift == 1 ? v.z : shift == -1 ? v.x : none;
+    r.z = shift == 0 ? v.z : shift == -1 ? v.y : shift == -2 ? v.x : none;
+    return r;
+}
+
+__device__ __forceinline__ void load_row(const Seg& sg, I3 gp, RowX x, int dy, int dz, __amdgpu_buffer_rsrc_t rs,
+                                         __amdgpu_buffer_rsrc_t re, vuint3& s, vuint3& e) {
+    const int gy = (int)sg.g.grid_size[1], gz = (int)sg.g.grid_size[2];
+    const bool ok = x.any && gp.y >= -dy && gp.y < gy - dy && gp.z >= -dz && gp.z < gz - dz;
+    const uint32_t key = sg.cell_base + (ok ? cellKey(x.from, gp.y + dy, gp.z + dz, sg.g) : 0u);
+    s = __builtin_amdgcn_raw_buffer_load_b96(rs, (int)(key * 4u), 0, 0);
+    e = __builtin_amdgcn_raw_buffer_load_b96(re, (int)(key * 4u), 0, 0);
+    const uint32_t none = ok ? 0u : BRT_EMPTY_CELL;
+    s |= none;
+    e |= none;
+}
+
+// empty cells have start = end = 0xFFFFFFFF: the least start is the run's first
+// index, and end + 1 is 0 for an empty cell, so the greatest is the run's end
+__device__ __forceinline__ RowRange row_range(vuint3 s, vuint3 e, uint32_t n, uint32_t& len) {
+    RowRange r;
+    uint32_t m = s.x < s.y ? s.x : s.y;
+    r.start = m < s.z ? m : s.z;
+    const uint32_t first = r.start + 1u;  // 0: the run is empty
+    const uint32_t top = n + 1u;
+    uint32_t ea = e.x + 1u, eb = e.y + 1u, ec = e.z + 1u;
+    eb = ea > eb ? ea : eb;
+    ec = eb > ec ? eb : ec;
+    ec = ec < top ? ec : top;
+    ea = ea < ec ? ea : ec;
+    eb = eb < ec ? eb : ec;
+    ea = ea > first ? ea : first;
+    eb = eb > first ? eb : first;
+    len = ec > first ? ec - first : 0u;
+    r.start = len != 0u ? r.start : 0u;
+    r.ends = (ea - first) | (eb - first) << 8 | len << 16;  // meant only for len <= kRowMax
+    return r;
+}
+
+// Words of a list's head (count first) that the row scan of a kernel without
+// LDS lists stages in LDS; later entries go straight to the row.
+constexpr uint32_t kHeadWords = 20u;
+
+// Scans the nine runs of the wave's sparse lanes and writes the entries to
+// head[1..] (LDS); false (nothing done) when some run of some lane is too long.
+// own: the range of the cell the agent lies in, for the other modes.
+// Every lane of the wave takes part.  WIDE: all of a lane's ranges, then all of
+// its first rounds, are in flight together (small launches, where the wave's
+// chain of memory latencies is the time and registers are not short).
+template <bool LDSL, bool PACKED, bool WIDE>
+__device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, bool alive,
+                                          uint32_t* head, uint2& own) {
+    constexpr int NL = WIDE ? 9 : 4;  // rows whose ranges load together
+    // runs whose rounds load together (with LDS lists a third would cost the
+    // fourth wave per SIMD: 129 registers)
+    constexpr int NR = WIDE ? 9 : (LDSL ? 2 : 3);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.cell_start), (short)0,
+                                                                        (int)(a.cells * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.cell_end), (short)0,
+                                                                        (int)(a.cells * 4u), 0x00020000);
+    const RowX x = row_x(gp.x, (int)sg.g.grid_size[0], alive);
+    const bool any_shift = __ballot(x.shift != 0) != 0;
+    vuint3 s[9], e[9];
+    RowRange R[9];
+    uint32_t most = 0u;
+    if (!WIDE) {
+        // the agent's own row first: it tells a crowded wave for two loads
+        load_row(sg, gp, x, 0, 0, rs, re, s[4], e[4]);
+        if (any_shift) {
+            s[4] = row_shift(s[4], x.shift);
+            e[4] = row_shift(e[4], x.shift);
+        }
+        own = make_uint2(s[4].y, e[4].y);
+        R[4] = row_range(s[4], e[4], a.n, most);
+        if (__popcll(__ballot(most > BRT_PROX_ROW_OCC)) >= BRT_PROX_ROW_LANES) return false;
+    }
+    // four rows at a time, to hold no more than their 24 registers
+#pragma unroll
+    for (int r0 = 0; r0 < 9; r0 += NL + 1) {
+#pragma unroll
+        for (int r = r0; r < (WIDE ? 9 : r0 + NL); ++r)
+            load_row(sg, gp, x, r / 3 - 1, r % 3 - 1, rs, re, s[r], e[r]);
+        if (any_shift) {
+#pragma unroll
+            for (int r = r0; r < (WIDE ? 9 : r0 + NL); ++r) {
+                s[r] = row_shift(s[r], x.shift);
+                e[r] = row_shift(e[r], x.shift);
+            }
+        }
+#pragma unroll
+        for (int r = r0; r < (WIDE ? 9 : r0 + NL); ++r) {
+            uint32_t len;
+            R[r] = row_range(s[r], e[r], a.n, len);
+            most = most > len ? most : len;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (WIDE) own = make_uint2(s[4].y, e[4].y);
+    if (WIDE && __popcll(__ballot(R[4].len() > BRT_PROX_ROW_OCC)) >= BRT_PROX_ROW_LANES) return false;
+    if (__ballot(most > kRowMax) != 0) return false;
+
+    const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
+    const __amdgpu_buffer_rsrc_t rxyz = xyz_rsrc(PACKED ? a.pxyz : nullptr, PACKED ? a.n : 0u);
+    // an agent outside the grid is stored in a cell that any of its runs may hold
+    const bool any_out = __ballot(alive && !inGrid(gp.x, gp.y, gp.z, sg.g)) != 0;
+    uint32_t M[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) M[r] = 0u;
+    // rounds of four candidates, the loads of NR runs in flight together; a run
+    // that no lane has so many candidates in is passed over
+    BRT_CELL_LOOP
+    for (uint32_t t0 = 0u; __ballot(most > t0) != 0; t0 += 4u) {
+#pragma unroll
+        for (int r0 = 0; r0 < 9; r0 += NR) {
+            float4 q[NR][4];
+            bool on[NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                if (r0 + k >= 9) continue;
+                on[k] = __ballot(R[r0 + k].len() > t0) != 0;
+                if (on[k]) load_round<4, PACKED>(rpos, rxyz, R[r0 + k].start + t0, q[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                if (r0 + k >= 9 || !on[k]) continue;
+                uint32_t m = 0;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const float rx = q[k][t].x - L.px, ry = q[k][t].y - L.py, rz = q[k][t].z - L.pz;
+                    const float xx = rx * rx, yy = ry * ry, zz = rz * rz;
+                    const float d2 = (xx + yy) + zz;
+                    m = shift_in(m, !(d2 > a.T));
+                }
+                M[r0 + k] |= m << (28u - t0);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        uint32_t keep = first_bits(R[r].len());
+        if (r == 4 || any_out) {
+            const uint32_t d = L.i - R[r].start;
+            if (d < 32u) keep &= ~(0x80000000u >> d);
+        }
+        M[r] &= keep;
+    }
+    // the lists' order is x offset outermost, then y, then z: the entries of the
+    // three x offsets go to places counted up from 0, c0 and c1, run by run
+    uint32_t c0 = 0u, c1 = 0u, all = 0u;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const uint32_t ma = first_bits(R[r].ends & 0xFFu), mb = first_bits((R[r].ends >> 8) & 0xFFu);
+        c0 += __popc(M[r] & ma);
+        c1 += __popc(M[r] & mb);
+        all += __popc(M[r]);
+    }
+    uint32_t p0 = 0u, p1 = c0, p2 = c1;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        uint32_t m = M[r];
+        const uint32_t ka = R[r].ends & 0xFFu, kb = (R[r].ends >> 8) & 0xFFu;
+        while (__ballot(m != 0u) != 0) {
+            if (m != 0u) {
+                const uint32_t k = (uint32_t)__clz(m);
+                m ^= 0x80000000u >> k;
+                const bool lo = k < ka, hi = k >= kb;
+                const uint32_t p = lo ? p0 : (hi ? p2 : p1);
+                p0 += lo ? 1u : 0u;
+                p1 += (lo || hi) ? 0u : 1u;
+                p2 += hi ? 1u : 0u;
+                if (p < a.K) {
+                    // register-chunk kernels hold the head of the list in LDS
+                    if (LDSL || p < kHeadWords - 1u)
+                        head[1u + p] = R[r].start + k;
+                    else
+                        L.row[1u + p] = R[r].start + k;
+                }
+            }
+        }
+    }
+    L.cnt = all < a.K ? all : a.K;
+    return true;
+}
+
+template <bool FUSE, bool BATCH, bool LDSL, bool WIDE = false>
 __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
-    extern __shared__ uint32_t s_list[];  // blockDim.x * W with LDS lists, else unused
+    // with LDS lists blockDim.x rows of Ws words; the list-only kernel without
+    // them blockDim.x heads of kHeadWords; else unused
+    extern __shared__ uint32_t s_list[];
+    constexpr bool ROWS = LDSL || !FUSE;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -711,6 +1006,7 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
     L.cnt = 0;
     const bool alive = wave_live && L.i < sg.end;
     L.row = LDSL ? s_list + tid * a.Ws : a.lists + (size_t)(alive ? L.i : 0u) * a.W;
+    uint32_t* const head = LDSL ? L.row : s_list + tid * kHeadWords;
     L.wp = L.row + 1u;
     L.h0 = L.h1 = L.h2 = L.b0 = L.b1 = L.b2 = BRT_LIST_PAD;
     float4 P = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -720,6 +1016,22 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
     L.pz = P.z;
     I3 gp = calcGridPos(P.x, P.y, P.z, sg.g);
     cell_gaps(sg, L, gp);
+
+    // fused: the agent's own state (the smoothed acceleration by agent ID when
+    // there is no sorted copy), loaded at once in small launches, and otherwise
+    // before the list is finished, so that the loads are in flight meanwhile
+    uint32_t own_id = 0u;
+    float4 own_fwd = make_float4(0.f, 0.f, 0.f, 0.f), own_sa = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_own = [&]() {
+        if (!FUSE || !alive) return;
+        own_id = a.hash[L.i].y;
+        own_fwd = a.sfwd[L.i];
+        if (a.ssa)
+            own_sa = a.ssa[L.i];
+        else if (own_id < a.n)
+            own_sa = a.o.sa_out[own_id];
+    };
+    if (WIDE) load_own();
 
     // wave-level mode choice: can the wave's lanes be covered by a few cells?
     const uint64_t alive_mask = __ballot(alive);
@@ -733,7 +1045,10 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
         pending &= ~__ballot(alive && gp.x == ux && gp.y == uy && gp.z == uz);
         ++groups;
     }
-    if (pending == 0) {
+    const bool uniform = pending == 0;
+    bool rows = false, have_own = false;
+    uint2 own = make_uint2(0u, 0u);
+    if (uniform) {
         pending = alive_mask;
         while (pending != 0) {
             const int leader = __ffsll((unsigned long long)pending) - 1;
@@ -745,6 +1060,15 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
             if (mine) scan_uniform<LDSL>(a, sg, L, ux, uy, uz);
         }
     } else {
+        const bool can = ROWS && a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED &&
+                         sg.g.grid_size[0] >= 3u;
+        rows = can &&
+               (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, LDSL, WIDE>(a, sg, L, gp, alive, head, own)
+                                          : scan_rows<LDSL, false, WIDE>(a, sg, L, gp, alive, head, own));
+        have_own = can && __ballot(alive && !inGrid(gp.x, gp.y, gp.z, sg.g)) == 0;
+    }
+    if (!rows && !uniform) {
+        // the row scan has read the cells of agents inside the grid
         // dense waves (most lanes in cells of >= 8 agents) take rounds of
         // kGroupL candidates and skip the self test outside the agent's own
         // cell; sparse waves, dominated by per-cell overhead, take the short
@@ -752,12 +1076,12 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
         bool dense = false;
         uint32_t own_start = 0;
         if (LDSL) {
-            uint32_t occ = 0;
-            if (alive) {
+            if (!have_own && alive) {
                 const uint32_t key = a.hash[L.i].x;
-                own_start = a.cell_start[key];
-                occ = a.cell_end[key] - own_start;
+                own = make_uint2(a.cell_start[key], a.cell_end[key]);
             }
+            own_start = own.x;
+            const uint32_t occ = own.y - own.x;
             dense = __popcll(__ballot(alive && occ >= (uint32_t)BRT_PROX_DENSE_OCC)) >= BRT_PROX_DENSE_LANES;
         }
         // with the packed positions a round's loads are 3G/4 instead of G
@@ -791,37 +1115,28 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
         }
     }
 
-    // fused: the agent's own state, loaded before the list is finished so the
-    // loads (the smoothed acceleration by agent ID when there is no sorted
-    // copy) are in flight meanwhile
-    uint32_t own_id = 0u;
-    float4 own_fwd = make_float4(0.f, 0.f, 0.f, 0.f), own_sa = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (FUSE && alive) {
-        own_id = a.hash[L.i].y;
-        own_fwd = a.sfwd[L.i];
-        if (a.ssa)
-            own_sa = a.ssa[L.i];
-        else if (own_id < a.n)
-            own_sa = a.o.sa_out[own_id];
-    }
+    if (!WIDE) load_own();
 
-    if (LDSL && a.log_rounds) expand_log(L, a.K);
-    uint32_t pad_from = a.W / 4u;
-    if (LDSL || alive) pad_from = finish_list<LDSL>(L, a.W);
-    if (!LDSL && wave_live)
-        pad_rows(a.lists, sg.row0, (sg.end - sg.row0) < 64u ? (sg.end - sg.row0) : 64u, a.W, lane, pad_from);
-    if (LDSL) __syncthreads();
-    // LDS lists: each wave writes its own rows, 16 bytes per lane per store
-    if (LDSL && wave_live) {
-        const uint32_t rows = (sg.end - sg.row0) < 64u ? (sg.end - sg.row0) : 64u;
-        const uint32_t W4 = a.W / 4u, Ws4 = a.Ws / 4u;
-        const uint32_t words4 = rows * W4;
-        uint4* dst = reinterpret_cast<uint4*>(a.lists + (size_t)sg.row0 * a.W);
-        const uint4* src = reinterpret_cast<const uint4*>(s_list + (size_t)(wid * 64u) * a.Ws);
-        for (uint32_t w = lane; w < words4; w += 64u) {
-            const uint32_t r = w / W4;
-            dst[w] = src[r * Ws4 + (w - r * W4)];
-        }
+    if (LDSL && a.log_rounds && !rows) expand_log(L, a.K);
+    const uint32_t wave_rows = wave_live ? ((sg.end - sg.row0) < 64u ? (sg.end - sg.row0) : 64u) : 0u;
+    if (LDSL) {
+        L.row[0] = L.cnt;
+        __syncthreads();
+        store_rows<false>(a.lists, sg.row0, wave_rows, a.W, s_list + (size_t)(wid * 64u) * a.Ws, a.Ws, lane);
+    } else if (ROWS && rows) {
+        head[0] = L.cnt;
+        // the lane's own entries past the head: their last chunk's padding
+        if (alive && L.cnt >= kHeadWords)
+            for (uint32_t q = L.cnt + 1u; (q & 3u) != 0u; ++q) L.row[q] = BRT_LIST_PAD;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        store_rows<true>(a.lists, sg.row0, wave_rows, a.W, s_list + (size_t)(wid * 64u) * kHeadWords, kHeadWords,
+                         lane);
+    } else {
+        uint32_t pad_from = a.W / 4u;
+        if (alive) pad_from = finish_list(L, a.W);
+        if (wave_live) pad_rows(a.lists, sg.row0, wave_rows, a.W, lane, pad_from);
     }
 
     // fused steering: walk the finished list (from LDS, or the row this lane
@@ -945,10 +1260,16 @@ uint32_t prox_block(uint32_t W, uint32_t n) {
     return B;
 }
 
+// Launches whose waves do not fill the SIMDs twice: their time is one wave's
+// chain of memory latencies, so the row scan holds all of a lane's loads in
+// flight, at two waves per SIMD.
+bool wide_launch(uint32_t n) { return n <= BRT_PROX_WIDE_MAX; }
+
 ProxArgs make_args(const brt_grid_params& g, const brt_prox_params& p, float threshold, const float4* spos,
                    const uint2* hash, const uint32_t* cell_start, const uint32_t* cell_end, uint32_t n,
-                   uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap) {
+                   uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t cells) {
     ProxArgs a{};
+    a.cells = cells < (1u << 30) ? cells : 0u;  // 32-bit byte offsets
     a.g = g;
     a.K = p.max_neighbors;
     a.W = list_stride(p.max_neighbors);
@@ -987,13 +1308,16 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
                            cell_start, cell_end, n, lists);
         return hipGetLastError();
     }
-    ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap);
+    ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
+                           g.num_cells);
     a.pxyz = pxyz;
     const uint32_t B = prox_block(a.Ws, n);
-    if (lds_lists)
+    if (lds_lists && wide_launch(n))
+        BRT_LAUNCH((k_prox<false, false, true, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
+    else if (lds_lists)
         BRT_LAUNCH((k_prox<false, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else
-        BRT_LAUNCH((k_prox<false, false, false>), dim3((n + 255) / 256), dim3(256), 0, s, a);
+        BRT_LAUNCH((k_prox<false, false, false>), dim3((n + 255) / 256), dim3(256), 256u * kHeadWords * 4u, s, a);
     return hipGetLastError();
 }
 
@@ -1004,7 +1328,8 @@ hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_param
                                   float2* wander, float4* pos_out, float4* fwd_out, float4* sa_out,
                                   uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s,
                                   const float* pxyz) {
-    ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap);
+    ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
+                           g.num_cells);
     a.pxyz = pxyz;
     a.sfwd = sfwd;
     a.ssa = ssa;
@@ -1014,7 +1339,9 @@ hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_param
     a.step = step;
     a.o = AgentOut{pos_out, fwd_out, sa_out, nullptr, wander};
     const uint32_t B = prox_block(a.Ws, n);
-    if (lds_lists)
+    if (lds_lists && wide_launch(n))
+        BRT_LAUNCH((k_prox<true, false, true, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
+    else if (lds_lists)
         BRT_LAUNCH((k_prox<true, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else
         BRT_LAUNCH((k_prox<true, false, false>), dim3((n + 255) / 256), dim3(256), 0, s, a);
@@ -1028,7 +1355,8 @@ hipError_t launch_batch_neighbors_steer(const BatchView& b, uint32_t n, const br
                                         float4* fwd_out, float4* sa_out, uint32_t block, uint32_t uniform_max_cells,
                                         uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s, const float* pxyz) {
     brt_grid_params g0{};
-    ProxArgs a = make_args(g0, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap);
+    ProxArgs a = make_args(g0, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
+                           b.cells);
     a.pxyz = pxyz;
     a.sfwd = sfwd;
     a.ssa = ssa;
