@@ -98,25 +98,32 @@ int enqueue_step(brt_batch* b, const brt_steer_params* steer, float feature_rate
     brt_context* ctx = b->ctx;
     const uint32_t n = b->total_n;
     brt::SortPlan plan = brt::make_sort_plan(n, b->total_cells, b->cfg.sort_items);
-    // the clearing launch only when the metadata is not known to be zero; the
-    // hash kernel fills the empty cells otherwise
-    const bool clean = b->meta_clean;
-    b->meta_clean = false;
-    if (!clean)
-        BRT_HIP(brt::launch_prepare(b->meta, b->meta_words, buf->cell_start, buf->cell_end, b->total_cells, s),
-                "k_prepare");
     brt::BatchView view{b->d_flocks, b->d_wave_flock, b->waves, b->d_step, b->total_cells};
-    uint2* A = reinterpret_cast<uint2*>(buf->hash);
-    uint2* B = reinterpret_cast<uint2*>(b->tmp);
-    uint2* first = (plan.passes & 1u) ? B : A;
-    BRT_HIP(brt::launch_batch_hash_hist(view, reinterpret_cast<const float4*>(buf->pos), first, b->meta, plan, s,
-                                        clean ? buf->cell_start : nullptr, buf->cell_end, b->total_cells),
-            "k_batch_hash_hist");
-    uint2* src = first;
-    uint2* dst = first == A ? B : A;
-    for (uint32_t q = 0; q < plan.passes; ++q) {
-        BRT_HIP(brt::launch_onesweep(src, dst, n, q, plan, b->meta, ctx->dev_flags, s), "k_onesweep");
-        std::swap(src, dst);
+    const bool cell_sort = brt::cell_sort_cells(n, b->total_cells) != 0u;
+    uint32_t* keys = reinterpret_cast<uint32_t*>(b->tmp);
+    if (cell_sort) {
+        BRT_HIP(brt::launch_batch_hash_keys(view, reinterpret_cast<const float4*>(buf->pos), keys, s),
+                "k_batch_hash_keys");
+    } else {
+        // the clearing launch only when the metadata is not known to be zero;
+        // the hash kernel fills the empty cells otherwise
+        const bool clean = b->meta_clean;
+        b->meta_clean = false;
+        if (!clean)
+            BRT_HIP(brt::launch_prepare(b->meta, b->meta_words, buf->cell_start, buf->cell_end, b->total_cells, s),
+                    "k_prepare");
+        uint2* A = reinterpret_cast<uint2*>(buf->hash);
+        uint2* B = reinterpret_cast<uint2*>(b->tmp);
+        uint2* first = (plan.passes & 1u) ? B : A;
+        BRT_HIP(brt::launch_batch_hash_hist(view, reinterpret_cast<const float4*>(buf->pos), first, b->meta, plan, s,
+                                            clean ? buf->cell_start : nullptr, buf->cell_end, b->total_cells),
+                "k_batch_hash_hist");
+        uint2* src = first;
+        uint2* dst = first == A ? B : A;
+        for (uint32_t q = 0; q < plan.passes; ++q) {
+            BRT_HIP(brt::launch_onesweep(src, dst, n, q, plan, b->meta, ctx->dev_flags, s), "k_onesweep");
+            std::swap(src, dst);
+        }
     }
     brt::ReorderArgs f{};
     f.count = 2;
@@ -133,11 +140,17 @@ int enqueue_step(brt_batch* b, const brt_steer_params* steer, float feature_rate
     // the LDS-list scan reads candidates from the packed x,y,z copy
     float* xyz = b->cfg.lds_lists ? b->xyz : nullptr;
     f.xyz0 = xyz;
-    const brt::SortCleanup cleanup = brt::sort_cleanup(b->meta, plan);
-    BRT_HIP(brt::launch_reorder_ranges(reinterpret_cast<const uint2*>(buf->hash), n, f, b->total_cells,
-                                       buf->cell_start, buf->cell_end, s, &cleanup),
-            "k_reorder_ranges");
-    b->meta_clean = true;
+    if (cell_sort) {
+        BRT_HIP(brt::launch_cell_sort(keys, n, b->total_cells, reinterpret_cast<uint2*>(buf->hash), f,
+                                      buf->cell_start, buf->cell_end, s),
+                "k_cell_sort");
+    } else {
+        const brt::SortCleanup cleanup = brt::sort_cleanup(b->meta, plan);
+        BRT_HIP(brt::launch_reorder_ranges(reinterpret_cast<const uint2*>(buf->hash), n, f, b->total_cells,
+                                           buf->cell_start, buf->cell_end, s, &cleanup),
+                "k_reorder_ranges");
+        b->meta_clean = true;
+    }
     BRT_HIP(brt::launch_batch_neighbors_steer(
                 view, n, b->prox, brt_radius_threshold(b->prox.search_radius), *steer, dt,
                 reinterpret_cast<const float4*>(buf->sorted_pos), reinterpret_cast<const float4*>(buf->sorted_forward),

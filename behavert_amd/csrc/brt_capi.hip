@@ -441,6 +441,16 @@ int brt_envgrid_hash_sort(brt_context* ctx, const brt_grid_params* grid, const f
     if (n == 0) return BRT_OK;
     BRT_REQUIRE(pos && hash && aligned16(pos) && ((uintptr_t)hash & 7u) == 0, "bad pos/hash pointer");
     if ((rc = use_device(ctx))) return rc;
+    if (brt::cell_sort_cells(n, grid->num_cells)) {
+        if ((rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells)))) return rc;
+        uint32_t* keys = reinterpret_cast<uint32_t*>(ctx->tmp);
+        BRT_HIP(brt::launch_hash_keys(*grid, reinterpret_cast<const float4*>(pos), n, keys, (hipStream_t)stream),
+                "k_hash_keys");
+        BRT_HIP(brt::launch_cell_sort(keys, n, grid->num_cells, reinterpret_cast<uint2*>(hash), brt::ReorderArgs{},
+                                      nullptr, nullptr, (hipStream_t)stream),
+                "k_cell_sort");
+        return BRT_OK;
+    }
     return run_hash_sort(ctx, grid, pos, n, hash, nullptr, nullptr, (hipStream_t)stream);
 }
 
@@ -958,6 +968,11 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // steering pass reads the neighbours' features by sorted index
     const bool two_pass = !(resolve_fused(ctx, prox) && !prox->use_knn);
     const bool sorted_features = do_features && two_pass;
+    // small flocks: the keys lie in the lists, which the neighbour search writes
+    // later; the context's scratch grows as for the radix sort, which a later
+    // call of the same size may take (another grid), under capture too
+    const bool cell_sort = brt::cell_sort_cells(n, grid->num_cells) != 0u;
+    if (!given && cell_sort && (rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells)))) return rc;
     if (!given && sorted_features && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
     // with LDS lists the neighbour scan reads candidate positions from a
     // packed x,y,z copy written by the reorder (three 16-byte loads per four
@@ -967,7 +982,12 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     if (!given && pack && (rc = ensure_xyz(ctx, n))) return rc;
     float* xyz = pack ? (given ? given->xyz : ctx->xyz) : nullptr;
     void* tmp = nullptr;
-    if (given) {
+    if (cell_sort) {
+        // phase 0 is the hash alone: the sort runs with the reorder, in phase 1
+        tmp = given ? given->tmp : ctx->tmp;
+        mark_phase(0);
+        BRT_HIP(brt::launch_hash_keys(*grid, reinterpret_cast<const float4*>(b->pos), n, b->lists, s), "k_hash_keys");
+    } else if (given) {
         tmp = given->tmp;
         if ((rc = run_hash_sort(ctx, grid, b->pos, n, b->hash, b->cell_start, b->cell_end, s, given->meta, tmp)))
             return rc;
@@ -1000,12 +1020,18 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     f.count = nf;
     f.xyz0 = xyz;
     mark_phase(1);
-    uint32_t* sort_meta = given ? given->meta : ctx->meta;
-    const brt::SortCleanup cleanup = brt::sort_cleanup(sort_meta, brt::make_sort_plan(n, grid->num_cells));
-    BRT_HIP(brt::launch_reorder_ranges(reinterpret_cast<const uint2*>(b->hash), n, f, grid->num_cells, b->cell_start,
-                                       b->cell_end, s, &cleanup),
-            "k_reorder_ranges");
-    if (!given) ctx->meta_clean = true;
+    if (cell_sort) {
+        BRT_HIP(brt::launch_cell_sort(b->lists, n, grid->num_cells, reinterpret_cast<uint2*>(b->hash), f,
+                                      b->cell_start, b->cell_end, s),
+                "k_cell_sort");
+    } else {
+        uint32_t* sort_meta = given ? given->meta : ctx->meta;
+        const brt::SortCleanup cleanup = brt::sort_cleanup(sort_meta, brt::make_sort_plan(n, grid->num_cells));
+        BRT_HIP(brt::launch_reorder_ranges(reinterpret_cast<const uint2*>(b->hash), n, f, grid->num_cells,
+                                           b->cell_start, b->cell_end, s, &cleanup),
+                "k_reorder_ranges");
+        if (!given) ctx->meta_clean = true;
+    }
     const float T = brt_radius_threshold(prox->search_radius);
     if (!two_pass) {
         // phase 2: neighbour lists + steering + integration in one pass

@@ -361,6 +361,366 @@ __global__ void __launch_bounds__(kSortThreads) k_onesweep(const uint2* __restri
     }
 }
 
+// ------------------------------------------------------------------ small flocks
+// A sort of up to 2^17 agents is not bound by its bytes but by its chain of
+// launches and latencies: a onesweep pass takes 8.3 us for one tile and 11 us
+// for 25, and a flock of 100,003 needs three besides the hash and the reorder.
+// Here the cells are split over up to 256 workgroups instead of the agents over
+// tiles: each workgroup reads every key (4 bytes each, from its L2), takes the
+// agents of its own cells into LDS, sorts them there by (cell, ID) and writes
+// its part of the sorted pairs, the gathered state and the cell ranges, empty
+// ones included.  Nothing passes between workgroups.  Hash + sort + reorder of
+// 4,096 / 65,536 / 100,003 agents: 24.3 -> 9.6 / 31.8 -> 18.2 / 45 -> 21.8 us.
+// The LDS stays below 64 KB: with 83 KB (twice the list) the kernel took 13 us
+// more at every size.
+constexpr uint32_t kCellThreads = 1024;
+constexpr uint32_t kCellGroups = 256;   // workgroups at most, one per CU
+constexpr uint32_t kCellIdBits = 17;    // agents below 2^17
+constexpr uint32_t kCellsPerGroup = 4096;
+constexpr uint32_t kCellCap = 4096;     // agents a workgroup sorts at a time
+constexpr uint32_t kCellRankMax = 512;  // agents ranked by counting up to here, else bitonic
+constexpr uint32_t kNoKey = 0x7FFFFFFFu;  // beside every key (below 2^20)
+constexpr uint32_t kCellDense = 64;     // agents of a cell ranked within it up to here
+constexpr uint32_t kCellGather = 4;     // float4 arrays gathered (position, heading, acceleration, features)
+
+__global__ void __launch_bounds__(256) k_hash_keys(brt_grid_params g, const float4* __restrict__ pos, uint32_t n,
+                                                   uint32_t* __restrict__ keys) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 p = pos[i];
+    keys[i] = calcGridHash(calcGridPos(p.x, p.y, p.z, g), g);
+}
+
+__global__ void __launch_bounds__(256) k_batch_hash_keys(BatchView b, const float4* __restrict__ pos,
+                                                         uint32_t* __restrict__ keys) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t gw = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (gw >= b.waves) return;
+    const uint32_t f = __builtin_amdgcn_readfirstlane(b.wave_flock[gw]);
+    const FlockDev& fd = b.flocks[f];
+    const uint32_t i = fd.offset + (gw - fd.wave_base) * 64u + lane;
+    if (i >= fd.offset + fd.n) return;
+    const float4 p = pos[i];
+    keys[i] = fd.cell_base + calcGridHash(calcGridPos(p.x, p.y, p.z, fd.g), fd.g);
+}
+
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Exclusive scan of one value per thread over the workgroup; total to all.
+__device__ __forceinline__ uint32_t cell_group_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    __syncthreads();  // the previous use of s_wave is over
+    if (lane == 63u) s_wave[wave] = x;
+    __syncthreads();
+    uint32_t before = 0u, all = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < kCellThreads / 64u; ++w) {
+        const uint32_t c = s_wave[w];
+        before += w < wave ? c : 0u;
+        all += c;
+    }
+    total = all;
+    return before + x - v;
+}
+
+// Sorts s_list[0..m), whose values are all different, ascending (m <= kCellCap).
+// Up to kCellRankMax by counting the smaller ones, the list split between
+// 1024 / m threads per value; above by a bitonic network, in which the steps
+// of distance <= 64 stay within a wave and need no barrier.
+__device__ __forceinline__ void cell_group_sort(uint32_t* s_list, uint32_t* s_rank, uint32_t m) {
+    const uint32_t tid = threadIdx.x;
+    if (m <= kCellRankMax) {
+        const uint32_t m64 = (m + 63u) / 64u * 64u, parts = kCellThreads / m64;
+        const uint32_t m4 = (m + 3u) / 4u, seg = (m4 + parts - 1u) / parts;
+        if (tid < 4u * m4 - m) s_list[m + tid] = 0xFFFFFFFFu;
+        if (tid < m64) s_rank[tid] = 0u;
+        __syncthreads();
+        const uint32_t part = tid / m64, e = tid - part * m64;
+        if (part < parts && e < m) {
+            const uint32_t mine = s_list[e];
+            const uint32_t to = (part + 1u) * seg < m4 ? (part + 1u) * seg : m4;
+            uint32_t c = 0u;
+#pragma unroll 4
+            for (uint32_t j = part * seg; j < to; ++j) {
+                const uint4 v = reinterpret_cast<const uint4*>(s_list)[j];
+                c += (v.x < mine ? 1u : 0u) + (v.y < mine ? 1u : 0u) + (v.z < mine ? 1u : 0u) +
+                     (v.w < mine ? 1u : 0u);
+            }
+            if (c) atomicAdd(&s_rank[e], c);
+        }
+        __syncthreads();
+        uint32_t v = 0u, r = 0u;
+        if (tid < m) {
+            v = s_list[tid];
+            r = s_rank[tid];
+        }
+        __syncthreads();
+        if (tid < m) s_list[r] = v;
+        __syncthreads();
+        return;
+    }
+    uint32_t P = 2u * kCellRankMax;
+    while (P < m) P *= 2u;
+    for (uint32_t t = m + tid; t < P; t += kCellThreads) s_list[t] = 0xFFFFFFFFu;
+    __syncthreads();
+    for (uint32_t k = 2u; k <= P; k *= 2u) {
+        for (uint32_t j = k / 2u; j > 0u; j /= 2u) {
+            for (uint32_t t = tid; t < P / 2u; t += kCellThreads) {
+                const uint32_t i = 2u * t - (t & (j - 1u));
+                const uint32_t a = s_list[i], b = s_list[i + j];
+                if ((a > b) == ((i & k) == 0u)) {
+                    s_list[i] = b;
+                    s_list[i + j] = a;
+                }
+            }
+            // the next step's pairs are this wave's own while its distance is <= 64
+            if (j > 64u || j == 1u)
+                __syncthreads();
+            else
+                wave_sync();
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __restrict__ keys, uint32_t n,
+                                                            uint32_t num_cells, uint32_t cells_per_group,
+                                                            uint2* __restrict__ hash, ReorderArgs f,
+                                                            uint32_t* __restrict__ cell_start,
+                                                            uint32_t* __restrict__ cell_end) {
+    __shared__ uint32_t s_list[kCellCap];
+    __shared__ uint32_t s_off[kCellsPerGroup + 1];
+    __shared__ uint32_t s_rank[kCellRankMax];
+    __shared__ uint32_t s_wave[kCellThreads / 64];
+    __shared__ uint32_t s_slot[kCellCap];
+    __shared__ uint32_t s_count, s_agents, s_below, s_most;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t c0 = blockIdx.x * cells_per_group;
+    const uint32_t nc = num_cells - c0 < cells_per_group ? num_cells - c0 : cells_per_group;
+
+    // agent id of cell c0 + rel to sorted index g; the gathers in flight together
+    auto emit = [&](uint32_t g, uint32_t rel, uint32_t id) {
+        float4 v[kCellGather];
+#pragma unroll
+        for (uint32_t q = 0; q < kCellGather; ++q)
+            if (q < f.count) v[q] = f.in[q][id];
+        hash[g] = make_uint2(c0 + rel, id);
+#pragma unroll
+        for (uint32_t q = 0; q < kCellGather; ++q)
+            if (q < f.count) f.out[q][g] = v[q];
+        if (f.xyz0) {
+            float* d = f.xyz0 + 3u * (size_t)g;
+            d[0] = v[0].x;
+            d[1] = v[0].y;
+            d[2] = v[0].z;
+        }
+    };
+    for (uint32_t c = tid; c < nc; c += kCellThreads) s_off[c] = 0u;
+    if (tid == 0u) {
+        s_count = 0u;
+        s_agents = 0u;
+        s_below = 0u;
+        s_most = 0u;
+    }
+    __syncthreads();
+
+    // Every key: the number below c0, and the quads of keys that hold one of
+    // this workgroup's cells (about one in n / (4 m)) into s_list, in any order.
+    // Bound by the VALU work per key, so a quad's hits are sorted out later; a
+    // lane has two quads loading while it tests two.
+    {
+        constexpr int U = 2;
+        constexpr uint32_t kStep = kCellThreads * 4u * U;
+        int32_t above = 0;  // minus the number of keys below c0
+        auto load = [&](uint32_t i0, uint4 (&k)[U]) {
+            if (i0 + 256u * U <= n) {  // the same for the whole wave
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    k[u] = *reinterpret_cast<const uint4*>(keys + i0 + 256u * u + 4u * lane);
+                return;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t i = i0 + 256u * u + 4u * lane;
+                k[u].x = i < n ? keys[i] : kNoKey;
+                k[u].y = i + 1u < n ? keys[i + 1u] : kNoKey;
+                k[u].z = i + 2u < n ? keys[i + 2u] : kNoKey;
+                k[u].w = i + 3u < n ? keys[i + 3u] : kNoKey;
+            }
+        };
+        auto test = [&](uint32_t i0, const uint4 (&k)[U]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int32_t r[4] = {(int32_t)(k[u].x - c0), (int32_t)(k[u].y - c0), (int32_t)(k[u].z - c0),
+                                      (int32_t)(k[u].w - c0)};
+                uint32_t least = 0xFFFFFFFFu;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int32_t below = r[c] < -1 ? -1 : (r[c] > 0 ? 0 : r[c]);
+                    above += below;
+                    least = least < (uint32_t)r[c] ? least : (uint32_t)r[c];
+                }
+                if (least < nc) {
+                    const uint32_t at = atomicAdd(&s_count, 1u);
+                    if (at < kCellCap) s_list[at] = i0 / 4u + 64u * u + lane;
+                }
+            }
+        };
+        uint4 k0[U], k1[U];
+        uint32_t i0 = wave * (256u * U);
+        load(i0, k0);
+        while (i0 < n) {
+            load(i0 + kStep, k1);
+            test(i0, k0);
+            i0 += kStep;
+            if (i0 >= n) break;
+            load(i0 + kStep, k0);
+            test(i0, k1);
+            i0 += kStep;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) above += __shfl_down(above, o);
+        if (lane == 0u) atomicAdd(&s_below, (uint32_t)-above);
+    }
+    __syncthreads();
+
+    // the quads' agents into s_slot, as cell | ID, and their number per cell (all
+    // keys again when the quads did not fit: then the agents do not either)
+    const uint32_t quads = s_count;
+    if (quads <= kCellCap) {
+        for (uint32_t t = tid; t < quads; t += kCellThreads) {
+            const uint32_t i = 4u * s_list[t];
+#pragma unroll
+            for (uint32_t c = 0; c < 4u; ++c) {
+                const uint32_t rel = (i + c < n ? keys[i + c] : kNoKey) - c0;
+                if (rel < nc) {
+                    atomicAdd(&s_off[rel], 1u);
+                    const uint32_t at = atomicAdd(&s_agents, 1u);
+                    if (at < kCellCap) s_slot[at] = rel << kCellIdBits | (i + c);
+                }
+            }
+        }
+    } else {
+        for (uint32_t i = tid; i < n; i += kCellThreads) {
+            const uint32_t rel = keys[i] - c0;
+            if (rel < nc) {
+                atomicAdd(&s_off[rel], 1u);
+                atomicAdd(&s_agents, 1u);
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t m = s_agents, base = s_below;
+
+    // cell offsets and ranges, four consecutive cells per thread at most
+    constexpr uint32_t E = kCellsPerGroup / kCellThreads;
+    uint32_t cnt[E], sum = 0u, total, most = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < E; ++k) {
+        const uint32_t c = tid * E + k;
+        cnt[k] = c < nc ? s_off[c] : 0u;
+        sum += cnt[k];
+        most = most > cnt[k] ? most : cnt[k];
+    }
+    if (most > kCellDense) s_most = 1u;  // some cell is crowded
+    uint32_t off = cell_group_scan(sum, s_wave, total);
+#pragma unroll
+    for (uint32_t k = 0; k < E; ++k) {
+        const uint32_t c = tid * E + k;
+        if (c < nc) {
+            s_off[c] = off;
+            if (cell_start) {
+                cell_start[c0 + c] = cnt[k] ? base + off : BRT_EMPTY_CELL;
+                cell_end[c0 + c] = cnt[k] ? base + off + cnt[k] : BRT_EMPTY_CELL;
+            }
+        }
+        off += cnt[k];
+    }
+    if (tid == 0u) s_off[nc] = m;
+    __syncthreads();
+
+    if (m <= kCellCap) {
+        if (m == 0u) return;
+        if (s_most == 0u) {
+            // no crowded cell: each agent to a place of its cell, then ranked among
+            // the cell's agents; s_off[c] becomes the end of cell c
+            for (uint32_t i = tid; i < m; i += kCellThreads) {
+                const uint32_t v = s_slot[i];
+                s_list[atomicAdd(&s_off[v >> kCellIdBits], 1u)] = v;
+            }
+            __syncthreads();
+            for (uint32_t i = tid; i < m; i += kCellThreads) {
+                const uint32_t v = s_list[i], rel = v >> kCellIdBits;
+                const uint32_t from = rel ? s_off[rel - 1u] : 0u, to = s_off[rel];
+                uint32_t r = from;
+                for (uint32_t j = from; j < to; ++j) r += s_list[j] < v ? 1u : 0u;
+                emit(base + r, rel, v & ((1u << kCellIdBits) - 1u));
+            }
+            return;
+        }
+        cell_group_sort(s_slot, s_rank, m);
+        for (uint32_t i = tid; i < m; i += kCellThreads) {
+            const uint32_t v = s_slot[i];
+            emit(base + i, v >> kCellIdBits, v & ((1u << kCellIdBits) - 1u));
+        }
+        return;
+    }
+    // more agents than fit: cell ranges of at most kCellCap agents in turn, each
+    // collected by reading the keys again; a cell of more is written in ID order
+    // as the keys are read
+    uint32_t c = 0u;
+    while (c < nc) {
+        const uint32_t from = s_off[c];
+        if (s_off[c + 1u] - from > kCellCap) {
+            uint32_t g = base + from;
+            for (uint32_t i0 = 0; i0 < n; i0 += kCellThreads) {
+                const uint32_t i = i0 + tid;
+                const bool hit = i < n && keys[i] == c0 + c;
+                uint32_t all;
+                const uint32_t at = cell_group_scan(hit ? 1u : 0u, s_wave, all);
+                if (hit) emit(g + at, c, i);
+                g += all;
+            }
+            ++c;
+            continue;
+        }
+        uint32_t lo = c + 1u, hi = nc;  // the last cell end with at most kCellCap agents from c
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1u) / 2u;
+            if (s_off[mid] - from <= kCellCap)
+                lo = mid;
+            else
+                hi = mid - 1u;
+        }
+        const uint32_t mm = s_off[lo] - from;
+        if (mm != 0u) {
+            __syncthreads();
+            if (tid == 0u) s_count = 0u;
+            __syncthreads();
+            for (uint32_t i = tid; i < n; i += kCellThreads) {
+                const uint32_t rel = keys[i] - c0;
+                if (rel - c < lo - c) s_list[atomicAdd(&s_count, 1u)] = rel << kCellIdBits | i;
+            }
+            __syncthreads();
+            cell_group_sort(s_list, s_rank, mm);
+            for (uint32_t i = tid; i < mm; i += kCellThreads) {
+                const uint32_t v = s_list[i];
+                emit(base + from + i, v >> kCellIdBits, v & ((1u << kCellIdBits) - 1u));
+            }
+        }
+        c = lo;
+    }
+}
+
 // reorderDataFloat4 for every feature + cell start/end of the sorted keys.
 // With cleanup, the sort's last pass's metadata goes back to zero as well.
 __global__ void __launch_bounds__(256) k_reorder_ranges(const uint2* __restrict__ hash, uint32_t n, ReorderArgs f,
@@ -482,6 +842,35 @@ hipError_t launch_hist(const uint2* in, uint2* copy_out, uint32_t n, uint32_t* m
                        hipStream_t s) {
     uint32_t grid = grid_for(n, 256, hist_blocks(n));
     hipLaunchKernelGGL(k_hist, dim3(grid), dim3(256), 0, s, in, copy_out, n, meta + kMetaHist, plan);
+    return hipGetLastError();
+}
+
+// Cells per workgroup of the small-flock sort; 0: the radix sort takes the flock.
+// The limits: IDs of 17 bits beside the cell, 4,096 cells per workgroup, and an
+// average of at most 1,024 agents per workgroup (few cells leave few workgroups).
+uint32_t cell_sort_cells(uint32_t n, uint32_t num_cells) {
+    if (n == 0u || n > (1u << kCellIdBits) || num_cells > kCellGroups * kCellsPerGroup) return 0u;
+    const uint32_t per = (num_cells + kCellGroups - 1u) / kCellGroups;
+    const uint32_t groups = (num_cells + per - 1u) / per;
+    return n <= 1024u * groups ? per : 0u;
+}
+
+hipError_t launch_hash_keys(const brt_grid_params& g, const float4* pos, uint32_t n, uint32_t* keys, hipStream_t s) {
+    BRT_LAUNCH(k_hash_keys, dim3((n + 255) / 256), dim3(256), 0, s, g, pos, n, keys);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_hash_keys(const BatchView& b, const float4* pos, uint32_t* keys, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_hash_keys, dim3((b.waves + 3) / 4), dim3(256), 0, s, b, pos, keys);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell_sort(const uint32_t* keys, uint32_t n, uint32_t num_cells, uint2* hash, const ReorderArgs& f,
+                            uint32_t* cell_start, uint32_t* cell_end, hipStream_t s) {
+    const uint32_t per = cell_sort_cells(n, num_cells);
+    if (per == 0u || f.count > kCellGather || (f.xyz0 && f.count == 0u)) return hipErrorInvalidValue;
+    BRT_LAUNCH(k_cell_sort, dim3((num_cells + per - 1u) / per), dim3(kCellThreads), 0, s, keys, n, num_cells, per,
+               hash, f, cell_start, cell_end);
     return hipGetLastError();
 }
 

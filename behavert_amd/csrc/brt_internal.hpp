@@ -99,6 +99,15 @@ hipError_t launch_reorder_ranges(const uint2* hash, uint32_t n, const ReorderArg
                                  uint32_t* cell_start, uint32_t* cell_end, hipStream_t s,
                                  const SortCleanup* cleanup = nullptr);
 
+// Hash + sort + reorder + ranges of a small flock in two launches: the keys (4
+// bytes per agent), then the sort by workgroups that each own a range of cells.
+// cell_sort_cells: 0 when n or num_cells lies outside that sort's range.
+uint32_t cell_sort_cells(uint32_t n, uint32_t num_cells);
+hipError_t launch_hash_keys(const brt_grid_params& g, const float4* pos, uint32_t n, uint32_t* keys, hipStream_t s);
+// f.count may be 0 and the cell arrays NULL (the sorted pairs alone)
+hipError_t launch_cell_sort(const uint32_t* keys, uint32_t n, uint32_t num_cells, uint2* hash, const ReorderArgs& f,
+                            uint32_t* cell_start, uint32_t* cell_end, hipStream_t s);
+
 // proximity
 hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                             const float4* spos, const uint2* hash, const uint32_t* cell_start,
@@ -210,6 +219,7 @@ inline void cell_slack(const brt_grid_params& g, float out[3]) {
 hipError_t launch_batch_hash_hist(const BatchView& b, const float4* pos, uint2* out, uint32_t* meta,
                                   const SortPlan& plan, hipStream_t s, uint32_t* cell_start = nullptr,
                                   uint32_t* cell_end = nullptr, uint32_t num_cells = 0);
+hipError_t launch_batch_hash_keys(const BatchView& b, const float4* pos, uint32_t* keys, hipStream_t s);
 hipError_t launch_set_word(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_batch_neighbors_steer(const BatchView& b, uint32_t n, const brt_prox_params& p, float threshold,
                                         const brt_steer_params& sp, float dt, const float4* spos, const float4* sfwd,

@@ -520,7 +520,9 @@ int brt_snapshot_load(brt_context* ctx, const char* path, uint32_t flags,
  * so a phase's time is the span of its own kernels, with no marker packets
  * between the phases (the gaps between phases are in no phase).
  * Phases: 0 hash+sort, 1 reorder+ranges, 2 neighbours, 3 steering+integration,
- * 4 feature update.  With BRT_OPT_FUSED_STEP, phase 2 holds the fused
+ * 4 feature update.  Flocks small enough that the sort and the reorder are one
+ * kernel (up to 2^17 agents) have the hash alone in phase 0 and the sort in
+ * phase 1.  With BRT_OPT_FUSED_STEP, phase 2 holds the fused
  * neighbours+steering kernel and phase 3 is empty; a phase that launched no
  * kernel reads 0.  Steps enqueued while their stream is being captured into a
  * graph are not timed (and not counted).  brt_phase_times() synchronises the
