@@ -847,19 +847,18 @@ __device__ __forceinline__ RowRange row_range(vuint3 s, vuint3 e, uint32_t n, ui
 // LDS lists stages in LDS; later entries go straight to the row.
 constexpr uint32_t kHeadWords = 20u;
 
-// Scans the nine runs of the wave's sparse lanes and writes the entries to
-// head[1..] (LDS); false (nothing done) when some run of some lane is too long.
-// own: the range of the cell the agent lies in, for the other modes.
-// Every lane of the wave takes part.  WIDE: all of a lane's ranges, then all of
-// its first rounds, are in flight together (small launches, where the wave's
-// chain of memory latencies is the time and registers are not short).
-template <bool LDSL, bool PACKED, bool WIDE>
-__device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, bool alive,
-                                          uint32_t* head, uint2& own) {
+// Scans the nine runs of the wave's sparse lanes; put(p, j) gets every accepted
+// index j with its place p in visiting order (not in order of p), and their
+// number is returned in all; false (nothing done) when some run of some lane is
+// too long.  own: the range of the cell the agent lies in, for the other modes.
+// Every lane of the wave takes part.  NR: runs whose rounds load together; at 9
+// all of a lane's ranges are in flight together too (small launches, where the
+// wave's chain of memory latencies is the time and registers are not short).
+template <bool PACKED, int NR, class Put>
+__device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, const Lane& L, I3 gp, bool alive,
+                                          uint2& own, uint32_t& all, Put&& put) {
+    constexpr bool WIDE = NR == 9;
     constexpr int NL = WIDE ? 9 : 4;  // rows whose ranges load together
-    // runs whose rounds load together (with LDS lists a third would cost the
-    // fourth wave per SIMD: 129 registers)
-    constexpr int NR = WIDE ? 9 : (LDSL ? 2 : 3);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.cell_start), (short)0,
                                                                         (int)(a.cells * 4u), 0x00020000);
     const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.cell_end), (short)0,
@@ -952,7 +951,8 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, Lane
     }
     // the lists' order is x offset outermost, then y, then z: the entries of the
     // three x offsets go to places counted up from 0, c0 and c1, run by run
-    uint32_t c0 = 0u, c1 = 0u, all = 0u;
+    uint32_t c0 = 0u, c1 = 0u;
+    all = 0u;
 #pragma unroll
     for (int r = 0; r < 9; ++r) {
         const uint32_t ma = first_bits(R[r].ends & 0xFFu), mb = first_bits((R[r].ends >> 8) & 0xFFu);
@@ -974,17 +974,10 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, Lane
                 p0 += lo ? 1u : 0u;
                 p1 += (lo || hi) ? 0u : 1u;
                 p2 += hi ? 1u : 0u;
-                if (p < a.K) {
-                    // register-chunk kernels hold the head of the list in LDS
-                    if (LDSL || p < kHeadWords - 1u)
-                        head[1u + p] = R[r].start + k;
-                    else
-                        L.row[1u + p] = R[r].start + k;
-                }
+                put(p, R[r].start + k);
             }
         }
     }
-    L.cnt = all < a.K ? all : a.K;
     return true;
 }
 
@@ -1062,9 +1055,20 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
     } else {
         const bool can = ROWS && a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED &&
                          sg.g.grid_size[0] >= 3u;
-        rows = can &&
-               (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, LDSL, WIDE>(a, sg, L, gp, alive, head, own)
-                                          : scan_rows<LDSL, false, WIDE>(a, sg, L, gp, alive, head, own));
+        auto put = [&](uint32_t p, uint32_t j) {
+            if (p >= a.K) return;
+            // register-chunk kernels hold the head of the list in LDS
+            if (LDSL || p < kHeadWords - 1u)
+                head[1u + p] = j;
+            else
+                L.row[1u + p] = j;
+        };
+        // with LDS lists a third run would cost the fourth wave per SIMD (129 registers)
+        constexpr int NR = WIDE ? 9 : (LDSL ? 2 : 3);
+        uint32_t all = 0u;
+        rows = can && (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, NR>(a, sg, L, gp, alive, own, all, put)
+                                                 : scan_rows<false, NR>(a, sg, L, gp, alive, own, all, put));
+        if (rows) L.cnt = all < a.K ? all : a.K;
         have_own = can && __ballot(alive && !inGrid(gp.x, gp.y, gp.z, sg.g)) == 0;
     }
     if (!rows && !uniform) {
@@ -1181,72 +1185,264 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
     }
 }
 
-// KNN mode (useKnn): the replacement depends on every candidate in order, so a
-// plain per-lane scan with the distance list staged in LDS.
-__global__ void k_neighbors_knn(brt_grid_params g, uint32_t K, uint32_t W, float T, const float4* __restrict__ spos,
-                                const uint32_t* __restrict__ cell_start, const uint32_t* __restrict__ cell_end,
-                                uint32_t n, uint32_t* __restrict__ lists) {
-    extern __shared__ uint32_t s_mem[];
-    const uint32_t B = blockDim.x;
-    uint32_t* s_list = s_mem;
-    float* s_dist = reinterpret_cast<float*>(s_mem + B * W);
-    const uint32_t tid = threadIdx.x;
-    const uint32_t i = blockIdx.x * B + tid;
-    uint32_t* my = s_list + tid * W;
-    float* md = s_dist + tid * K;
-    uint32_t cnt = 0;
-    if (i < n) {
-        const float4 p = spos[i];
-        const I3 gp = calcGridPos(p.x, p.y, p.z, g);
-        const uint32_t maxBodies = g.max_bodies_per_cell;
-        float maxDist = 0.0f;
-        for (int dx = -1; dx <= 1; ++dx)
-            for (int dy = -1; dy <= 1; ++dy)
-                for (int dz = -1; dz <= 1; ++dz) {
-                    const int cx = gp.x + dx, cy = gp.y + dy, cz = gp.z + dz;
-                    if (!inGrid(cx, cy, cz, g)) continue;
-                    const uint32_t key = cellKey(cx, cy, cz, g);
-                    const uint32_t s = cell_start[key];
-                    if (s == BRT_EMPTY_CELL) continue;
-                    const uint32_t e = cell_end[key];
-                    uint32_t lim = (e - s) > maxBodies ? s + maxBodies : e;
-                    lim = lim < n ? lim : n;
-                    for (uint32_t j = s; j < lim; ++j) {
-                        if (j == i) continue;
-                        const float4 q = spos[j];
-                        const float rx = q.x - p.x, ry = q.y - p.y, rz = q.z - p.z;
-                        const float xx = rx * rx, yy = ry * ry, zz = rz * rz;
-                        const float d2 = (xx + yy) + zz;
-                        if (d2 > T) continue;
-                        const float dist = sqrtf(d2);
-                        if (cnt < K) {
-                            my[1 + cnt] = j;
-                            md[cnt] = dist;
-                            maxDist = fmaxf(maxDist, dist);
-                            ++cnt;
-                        } else if (dist < maxDist) {
-                            maxDist = md[0];
-                            uint32_t mi = 0;
-                            for (uint32_t q2 = 1; q2 < cnt; ++q2)
-                                if (maxDist < md[q2]) {
-                                    maxDist = md[q2];
-                                    mi = q2;
-                                }
-                            my[1 + mi] = j;
-                            md[mi] = dist;
-                        }
-                    }
-                }
+// KNN mode (useKnn): what a candidate does depends on every accepted one before
+// it, so the accepted candidates are taken one by one, in visiting order.  Taken
+// as they are found, the search for the farthest entry (K reads) ran for every
+// candidate for which some lane needed it, behind one load in flight.  Here the
+// accepted indices are gathered first and each lane goes through its own, the
+// e-th of every lane at a time, the next one's position loading meanwhile:
+//   * sparse waves: the row scan puts them in order (knn_rows), if no lane has
+//     more than K + kKnnLog;
+//   * else the flat scan logs accept bits, and when some lane's log is full all
+//     lanes work theirs off (knn_scan); a full list's greatest distance then
+//     bounds what is logged further.
+// The lists, the log and the distances lie in LDS word by word across the lanes
+// (no bank conflicts).  K 16, one kernel: 200,003 agents at 2 / 4 / 8 per cell
+// (100,003, 200,003, 400,007) 56 -> 29 / 120 -> 73 / 430 -> 225 us, 200,003 in
+// 12 blobs (up to hundreds per cell) 1.70 -> 1.03 ms.  A log of 16 or 32 words:
+// 79 or 74 us at 4 per cell (below K + 24 too few waves take the rows).
+// Agents per cell from which a KNN wave's rounds take 8 candidates instead of 4
+// (200,003 agents at 4 per cell without the row scan: 81 -> 87 us at 8).
+#ifndef BRT_KNN_DENSE_OCC
+#define BRT_KNN_DENSE_OCC 3
+#endif
+constexpr uint32_t kKnnLog = 24u;
+
+// What an accepted candidate does to agent L's list (k words and distances
+// apart by B): appended while there is room, else it takes the place of the
+// farthest entry if it is nearer than the farthest was at the last replacement.
+struct KnnList {
+    uint32_t* list;
+    float* md;
+    uint32_t B, K, cnt;
+    float mx;
+    // all lanes of the wave; have: this lane has candidate j at q
+    __device__ __forceinline__ void add(const Lane& L, bool have, uint32_t j, float4 q) {
+        const float rx = q.x - L.px, ry = q.y - L.py, rz = q.z - L.pz;
+        const float xx = rx * rx, yy = ry * ry, zz = rz * rz;
+        const float dist = sqrtf((xx + yy) + zz);
+        bool replace = false;
+        if (have) {
+            if (cnt < K) {
+                list[cnt * B] = j;
+                md[cnt * B] = dist;
+                mx = fmaxf(mx, dist);
+                ++cnt;
+            } else {
+                replace = dist < mx;
+            }
+        }
+        if (__ballot(replace) != 0 && replace) {
+            float far = md[0];
+            uint32_t at = 0u;
+#pragma unroll 4
+            for (uint32_t t = 1u; t < K; ++t) {
+                const float d = md[t * B];
+                at = far < d ? t : at;
+                far = far < d ? d : far;
+            }
+            list[at * B] = j;
+            md[at * B] = dist;
+            mx = far;
+        }
     }
-    my[0] = cnt;
-    for (uint32_t q = cnt + 1; q < W; ++q) my[q] = BRT_LIST_PAD;
+};
+
+// Sparse waves: the row scan puts the accepted indices into list[0..room) in
+// visiting order, and each lane goes through its own, two loads ahead.  The
+// first K stay where they are.  false: some run or some lane's candidates are
+// too many.
+__device__ __forceinline__ bool knn_rows(const ProxArgs& a, const Seg& sg, const Lane& L, I3 gp, bool alive,
+                                         uint32_t room, KnnList& kl) {
+    uint2 own;
+    uint32_t all = 0u;
+    const uint32_t B = kl.B;
+    const bool can = a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED && sg.g.grid_size[0] >= 3u;
+    if (!can || !scan_rows<false, 3>(a, sg, L, gp, alive, own, all, [&](uint32_t p, uint32_t j) {
+            if (p < room) kl.list[p * B] = j;
+        }))
+        return false;
+    if (__ballot(all > room) != 0) return false;
+    const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
+    auto index = [&](uint32_t e) { return e < all ? kl.list[e * B] : L.i; };
+    uint32_t j = index(0u), jn = index(1u);
+    float4 q = bload(rpos, j * 16u);
+    for (uint32_t e = 0u; __ballot(e < all) != 0; ++e) {
+        const float4 qn = bload(rpos, jn * 16u);
+        const uint32_t jnn = index(e + 2u);
+        kl.add(L, e < all, j, q);
+        j = jn;
+        jn = jnn;
+        q = qn;
+    }
+    return true;
+}
+
+template <int G>
+__device__ __forceinline__ void knn_scan(const ProxArgs& a, const Seg& sg, const Lane& L, I3 gp, bool alive,
+                                         uint32_t* log, KnnList& kl) {
+    const uint32_t B = kl.B;
+    const uint32_t maxBodies = sg.g.max_bodies_per_cell;
+    const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
+    uint32_t nw = 0u;
+    float cut = a.T;  // squared distance beyond which candidates are left out
+    // words of the log: first index << 8 | accept bits, or (2^24 agents and
+    // more) one index each
+    const bool packed = a.log_rounds != 0u;
+    const uint32_t room = packed ? kKnnLog : kKnnLog - (uint32_t)G + 1u;
+
+    auto work_off = [&]() {
+        uint32_t e = 0u, m = 0u, jb = 0u;
+        auto next = [&](uint32_t& j) {
+            if (m == 0u && e < nw) {
+                const uint32_t w = log[e * B];
+                ++e;
+                jb = packed ? w >> 8 : w;
+                m = packed ? w & 0xFFu : 0x80u;
+            }
+            const bool any = m != 0u;
+            const uint32_t b = 31u - __clz(any ? m : 1u);
+            m = any ? m ^ (1u << b) : 0u;
+            j = any ? jb + 7u - b : L.i;
+            return any;
+        };
+        uint32_t j;
+        bool have = next(j);
+        float4 q = bload(rpos, j * 16u);
+        while (__ballot(have) != 0) {
+            uint32_t jn;
+            const bool have_n = next(jn);
+            const float4 qn = bload(rpos, jn * 16u);
+            kl.add(L, have, j, q);
+            j = jn;
+            have = have_n;
+            q = qn;
+        }
+        nw = 0u;
+        // Once the list is full, an entry is only ever replaced by a nearer
+        // candidate than mx, and mx is then set to one of the distances, so none
+        // of these values exceeds the greatest of them now: a candidate that is
+        // farther away can do nothing any more and is not logged (the margin is
+        // far above the rounding of sqrtf and of the square).
+        if (__ballot(kl.cnt == a.K) != 0 && kl.cnt == a.K) {
+            float far = kl.mx;
+#pragma unroll 4
+            for (uint32_t t = 0u; t < a.K; ++t) far = fmaxf(far, kl.md[t * B]);
+            cut = fminf(a.T, far * far * 1.00001f);
+        }
+    };
+
+    uint32_t todo = alive ? visit_mask(sg, L, gp, a.Tskip) : 0u;
+    uint32_t nc = 27u, ns = BRT_EMPTY_CELL, ne = 0u;
+    flat_fetch(a, sg, gp, todo, nc, ns, ne);
+    uint32_t j = 0u, lim = 0u;
+    bool live = alive;
+    while (true) {
+        if (live && j >= lim) {
+            if (nc == 27u) {
+                live = false;
+            } else {
+                if (ns == BRT_EMPTY_CELL) {
+                    j = 0u;
+                    lim = 0u;
+                } else {
+                    lim = (ne - ns) > maxBodies ? ns + maxBodies : ne;
+                    lim = lim < a.n ? lim : a.n;
+                    j = ns;
+                }
+                __builtin_amdgcn_sched_barrier(0);  // as in scan_flat
+                flat_fetch(a, sg, gp, todo, nc, ns, ne);
+            }
+        }
+        if (__ballot(live) == 0) break;
+        if (live && j < lim) {
+            float4 q[G];
+            load_round<G, false>(rpos, rpos, j, q);
+            uint32_t m = 0u;
+#pragma unroll
+            for (int t = 0; t < G; ++t) {
+                const float rx = q[t].x - L.px, ry = q[t].y - L.py, rz = q[t].z - L.pz;
+                const float xx = rx * rx, yy = ry * ry, zz = rz * rz;
+                const float d2 = (xx + yy) + zz;
+                m = shift_in(m, !(d2 > cut));
+            }
+            const uint32_t rem = lim - j, r = rem < (uint32_t)G ? rem : (uint32_t)G, di = L.i - j;
+            m &= ~((1u << ((uint32_t)G - r)) - 1u);
+            if (di < (uint32_t)G) m &= ~(1u << ((uint32_t)G - 1u - di));
+            m <<= 8 - G;
+            if (packed) {
+                if (m != 0u) {
+                    log[nw * B] = (j << 8) | m;
+                    ++nw;
+                }
+            } else {
+                while (m != 0u) {
+                    const uint32_t b = 31u - __clz(m);
+                    m ^= 1u << b;
+                    log[nw * B] = j + 7u - b;
+                    ++nw;
+                }
+            }
+            j += (uint32_t)G;
+        }
+        if (__ballot(nw >= room) != 0) work_off();
+    }
+    work_off();
+}
+
+__global__ void __launch_bounds__(64) k_neighbors_knn(ProxArgs a) {
+    extern __shared__ uint32_t s_mem[];
+    const uint32_t B = blockDim.x, lane = threadIdx.x;
+    const uint32_t blk = xcd_block(a.xcd_remap != 0);
+    Seg sg;
+    sg.g = a.g;
+    sg.slack[0] = a.slack[0];
+    sg.slack[1] = a.slack[1];
+    sg.slack[2] = a.slack[2];
+    sg.cell_base = 0;
+    sg.row0 = blk * B;
+    sg.end = a.n;
+    uint32_t* s_log = s_mem + a.K * B;
+    Lane L;
+    L.i = sg.row0 + lane;
+    const bool alive = L.i < a.n;
+    const float4 P = a.spos[alive ? L.i : a.n - 1u];
+    L.px = P.x;
+    L.py = P.y;
+    L.pz = P.z;
+    const I3 gp = calcGridPos(P.x, P.y, P.z, sg.g);
+    cell_gaps(sg, L, gp);
+    KnnList kl{s_mem + lane, reinterpret_cast<float*>(s_mem + (a.K + kKnnLog) * B) + lane, B, a.K, 0u, 0.0f};
+    // the row scan's indices run on from the list into the log
+    if (!knn_rows(a, sg, L, gp, alive, a.K + kKnnLog, kl)) {
+        // rounds of 8 candidates in crowded waves, else of 4
+        uint32_t occ = 0u;
+        if (alive && inGrid(gp.x, gp.y, gp.z, sg.g)) {
+            const uint32_t key = cellKey(gp.x, gp.y, gp.z, sg.g);
+            occ = a.cell_end[key] - a.cell_start[key];
+        }
+        if (2 * __popcll(__ballot(occ >= (uint32_t)BRT_KNN_DENSE_OCC)) >= (int)B)
+            knn_scan<8>(a, sg, L, gp, alive, s_log + lane, kl);
+        else
+            knn_scan<4>(a, sg, L, gp, alive, s_log + lane, kl);
+    }
+    const uint32_t cnt = kl.cnt;
     __syncthreads();
-    const uint32_t row0 = blockIdx.x * B;
-    const uint32_t rows = (n - row0) < B ? (n - row0) : B;
-    const uint32_t words4 = rows * W / 4u;
-    uint4* dst = reinterpret_cast<uint4*>(lists + (size_t)row0 * W);
-    const uint4* src = reinterpret_cast<const uint4*>(s_list);
-    for (uint32_t w = tid; w < words4; w += B) dst[w] = src[w];
+    s_log[lane] = cnt;
+    __syncthreads();
+    // 16 bytes per lane per store, consecutive across the lanes
+    const uint32_t W4 = a.W / 4u, rows = (a.n - sg.row0) < B ? (a.n - sg.row0) : B;
+    uint4* dst = reinterpret_cast<uint4*>(a.lists + (size_t)sg.row0 * a.W);
+    for (uint32_t w = lane; w < rows * W4; w += B) {
+        const uint32_t r = w / W4, c = w - r * W4, k = s_log[r];
+        uint32_t v[4];
+#pragma unroll
+        for (uint32_t x = 0; x < 4u; ++x) {
+            const uint32_t e = 4u * c + x;  // word e: entry e - 1; word 0: the count
+            v[x] = e == 0u ? k : e <= k ? s_mem[(e - 1u) * B + r] : BRT_LIST_PAD;
+        }
+        dst[w] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
 }
 
 // Workgroup of the single-grid LDS-list neighbour kernels: one wave for large
@@ -1299,17 +1495,15 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
                             const uint32_t* cell_end, uint32_t n, uint32_t* lists, uint32_t uniform_max_cells,
                             uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s, const float* pxyz) {
     const uint32_t K = p.max_neighbors;
-    const uint32_t W = list_stride(K);
-    if (p.use_knn) {
-        uint32_t B = 64;
-        while (B > 8 && (size_t)B * (W + K) * 4u > 60u * 1024u) B /= 2;
-        const size_t lds = (size_t)B * (W + K) * 4u;
-        BRT_LAUNCH(k_neighbors_knn, dim3((n + B - 1) / B), dim3(B), lds, s, g, K, W, threshold, spos,
-                           cell_start, cell_end, n, lists);
-        return hipGetLastError();
-    }
     ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
                            g.num_cells);
+    if (p.use_knn) {
+        // one wave per workgroup, fewer lanes of it where the lists need the LDS
+        uint32_t B = 64;
+        while (B > 8 && (size_t)B * (2u * K + kKnnLog) * 4u > 40u * 1024u) B /= 2;
+        BRT_LAUNCH(k_neighbors_knn, dim3((n + B - 1) / B), dim3(B), (size_t)B * (2u * K + kKnnLog) * 4u, s, a);
+        return hipGetLastError();
+    }
     a.pxyz = pxyz;
     const uint32_t B = prox_block(a.Ws, n);
     if (lds_lists && wide_launch(n))
