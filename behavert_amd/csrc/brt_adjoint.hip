@@ -9,13 +9,15 @@
 //   s1 = |v|, p1 = p + v dt, f1 = normalize(v).
 // Given dL/d(p1, f1, s1, a1) by agent ID, two kernels produce dL/d(p, f, s, a)
 // by agent ID, with no atomics, so the same inputs always give the same bits:
-//   k_adjoint_own (one lane per sorted agent i) recomputes agent i's forward
-//     values with the forward kernels' arithmetic, back-propagates through the
-//     integrator and its own behaviour sums, and stores by sorted index its own
-//     terms and the three vectors its neighbours' terms are made of (the
-//     separation, cohesion and alignment sums' adjoints, with flags);
+//   k_adjoint_own (one or four lanes per sorted agent i) recomputes agent i's
+//     forward values with the forward kernels' arithmetic, back-propagates
+//     through the integrator and its own behaviour sums, and stores by sorted
+//     index its own terms and a record of what its neighbours' terms are made
+//     of (position, heading, the separation, cohesion and alignment sums'
+//     adjoints, flags);
 //   k_adjoint_gather (several lanes per sorted agent j) finds every agent i
-//     whose list holds j -- j's own list when that list can stand in for them,
+//     whose list holds j -- j's own list when that list can stand in for them
+//     (and the cells where agents below the grid are kept, for j on a low face),
 //     else the agents of the 27 cells around j's cell -- by repeating the list
 //     test (radius, cell range, and, for a full list, j's place in i's
 //     visiting order against i's last entry), adds i's terms for p_j and f_j
@@ -67,14 +69,13 @@ struct AdjArgs {
     const float4* gfwd_out;
     const float4* gsa_out;
     // by sorted index: 3 float4 of own terms (dL/dp, (dL/df, dL/ds), dL/da) and
-    // 3 float4 of neighbour-term vectors (S.xyz C.x | C.yz A.xy | A.z flags)
+    // the record of 4 float4, 64 bytes, that the neighbours' terms are made of:
+    // (p.xyz f.x | f.yz S.xy | S.z C.xyz | A.xyz flags)
     float4* own;
-    float4* bars;
+    float4* rec;
     float* partials;  // per workgroup: 3 floats
     uint32_t xcd_remap;
 };
-
-__device__ __forceinline__ uint32_t list_entry(const uint32_t* row, uint32_t t) { return row[1 + t]; }
 
 // Sums the per-workgroup partials in a fixed order (strided per-thread sums,
 // then a fixed LDS tree) and adds the result to weight_grad; the same inputs
@@ -130,43 +131,116 @@ __device__ __forceinline__ V3 pair_terms(const brt_steer_params& sp, uint32_t fl
     return offbar;
 }
 
+// The value that lane k of this lane's quad holds (NL == 4: four lanes of one
+// agent, all active), or the lane's own (NL == 1).
+template <int NL>
+__device__ __forceinline__ float quad_get(float v, int k) {
+    if (NL == 1) return v;
+    const int x = __float_as_int(v);
+    int r;
+    switch (k) {
+        case 0: r = __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, true); break;
+        case 1: r = __builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, true); break;
+        case 2: r = __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, true); break;
+        default: r = __builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, true); break;
+    }
+    return __int_as_float(r);
+}
+
+// s + v of the quad's lanes in order: entry by entry as one lane would add them.
+template <int NL>
+__device__ __forceinline__ V3 quad_add(V3 s, V3 v) {
+#pragma unroll
+    for (int k = 0; k < NL; ++k) s = s + v3(quad_get<NL>(v.x, k), quad_get<NL>(v.y, k), quad_get<NL>(v.z, k));
+    return s;
+}
+
+template <int NL>
+__device__ __forceinline__ uint32_t quad_count(uint32_t v) {
+    if (NL == 1) return v;
+    v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);  // lanes 1,0,3,2
+    v += (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);  // lanes 2,3,0,1
+    return v;
+}
+
+__device__ __forceinline__ float pick(uint32_t l, float v0, float v1, float v2, float v3) {
+    return l == 0u ? v0 : (l == 1u ? v1 : (l == 2u ? v2 : v3));
+}
+
+__device__ __forceinline__ V3 keep(V3 v, bool on) { return on ? v : v3(0.f, 0.f, 0.f); }
+
+// NL lanes per agent: with four, lane l takes the list entries l, l + 4, ..., the
+// sums add the four lanes' terms in list order (the same bits as one lane), and
+// every lane carries the integrator.  Small flocks are bound by one wave's chain
+// of list and neighbour loads (65,536 agents are one wave per SIMD with one lane
+// each), which four lanes shorten; larger ones by the arithmetic.
+template <int NL>
 __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
+    constexpr int U = NL == 1 ? 4 : 2;  // entries of a lane in flight
+    constexpr uint32_t T = (uint32_t)(NL * U);
     __shared__ float s_red[3][4];
-    const uint32_t i = xcd_block(a.xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t t0 = xcd_block(a.xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = t0 / (uint32_t)NL, l = t0 % (uint32_t)NL;
     float wg[3] = {0.f, 0.f, 0.f};
     const brt_steer_params& sp = a.sp;
     if (i < a.n && a.hash[i].y < a.n) {
         const uint32_t id = a.hash[i].y;
         const float4 P = a.spos[i], Fw = a.sfwd[i], SA = a.ssa[i];
+        const float4 gP = a.gpos_out[id], gF = a.gfwd_out[id], gA = a.gsa_out[id];
         const V3 p = xyz(P), f = xyz(Fw), sa = xyz(SA);
         const float s = Fw.w;
         const uint32_t* row = a.lists + (size_t)i * a.W;
         const uint32_t count = row[0] < a.W - 1u ? row[0] : a.W - 1u;
         const bool behaviours = sp.separation[0] != 0.0f || sp.alignment[0] != 0.0f || sp.cohesion[0] != 0.0f;
 
+        // this lane's entries of the trip from entry t on, a.n where there is none
+        auto load_entries = [&](uint32_t t, uint32_t (&jj)[U], float4 (&q)[U]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t e = t + (uint32_t)(NL * u) + l;
+                const uint32_t j = row[e < a.W - 1u ? 1u + e : 0u];
+                jj[u] = e < count && j < a.n ? j : a.n;
+                q[u] = a.spos[jj[u] < a.n ? jj[u] : i];
+            }
+        };
+
         // ---- forward recompute: behaviour sums (list order) -------------------
+        // the first trip's entries and positions stay for the backward sums
+        uint32_t jf[U];
+        float4 qf[U];
         SteerAccum acc;
         acc.init();
-        if (behaviours)
-            for (uint32_t t = 0; t < count; t += 4) {
-                // four neighbours' gathers in flight
-                uint32_t jj[4];
-                float4 q[4], fq[4];
+        if (behaviours) {
+            load_entries(0u, jf, qf);
+            for (uint32_t t = 0; t < count; t += T) {
+                uint32_t jj[U];
+                float4 q[U], fq[U];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint32_t j = (t + u < count) ? list_entry(row, t + u) : a.n;
-                    jj[u] = j;
-                    const uint32_t js = j < a.n ? j : i;
-                    q[u] = a.spos[js];
-                    fq[u] = a.sfwd[js];
+                for (int u = 0; u < U; ++u) {
+                    jj[u] = jf[u];
+                    q[u] = qf[u];
                 }
+                if (t != 0u) load_entries(t, jj, q);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (jj[u] >= a.n) continue;
+                for (int u = 0; u < U; ++u) fq[u] = a.sfwd[jj[u] < a.n ? jj[u] : i];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    SteerAccum one;
+                    one.init();
                     const V3 off = xyz(q[u]) - p;
-                    acc.add(sp, weights_of(sp), f, off, dot(off, off), xyz(fq[u]));
+                    if (jj[u] < a.n) one.add(sp, weights_of(sp), f, off, dot(off, off), xyz(fq[u]));
+                    acc.sSep = quad_add<NL>(acc.sSep, one.sSep);
+                    acc.sAli = quad_add<NL>(acc.sAli, one.sAli);
+                    acc.sCoh = quad_add<NL>(acc.sCoh, one.sCoh);
+                    acc.nSep += one.nSep;
+                    acc.nAli += one.nAli;
+                    acc.nCoh += one.nCoh;
                 }
             }
+            acc.nSep = quad_count<NL>(acc.nSep);
+            acc.nAli = quad_count<NL>(acc.nAli);
+            acc.nCoh = quad_count<NL>(acc.nCoh);
+        }
         V3 xs = v3(0.f, 0.f, 0.f), xa = xs, xc = xs, us = xs, ua = xs, uc = xs;
         V3 F = v3(0.f, 0.f, 0.f);
         if (sp.separation[0] != 0.0f) {
@@ -228,7 +302,6 @@ __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
         const V3 v = truncateLength(v0, sp.max_speed);
 
         // ---- backward: integrator -------------------------------------------
-        const float4 gP = a.gpos_out[id], gF = a.gfwd_out[id], gA = a.gsa_out[id];
         const V3 gp1 = xyz(gP), gf1 = xyz(gF), ga1 = xyz(gA);
         const float gs1 = gF.w;
         const float vlen = length(v);
@@ -324,39 +397,49 @@ __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
         // this agent's share of the neighbour terms: p_i appears in every
         // offset p_j - p_i of its own sums (the same per-pair terms
         // k_adjoint_gather adds to p_j)
-        if (behaviours)
-            for (uint32_t t = 0; t < count; t += 4) {
-                uint32_t jj[4];
-                float4 q[4];
+        if (behaviours) {
+            for (uint32_t t = 0; t < count; t += T) {
+                if (t != 0u) load_entries(t, jf, qf);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint32_t j = (t + u < count) ? list_entry(row, t + u) : a.n;
-                    jj[u] = j;
-                    const uint32_t js = j < a.n ? j : i;
-                    q[u] = a.spos[js];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (jj[u] >= a.n) continue;
-                    const V3 off = xyz(q[u]) - p;
-                    bool anyP, ali;
-                    const V3 offbar = pair_terms(sp, flags, f, off, Sbar, Cbar, anyP, ali);
-                    if (anyP) pbar = pbar - offbar;
+                for (int u = 0; u < U; ++u) {
+                    const V3 off = xyz(qf[u]) - p;
+                    bool anyP = false, ali;
+                    V3 offbar = v3(0.f, 0.f, 0.f);
+                    if (jf[u] < a.n) offbar = pair_terms(sp, flags, f, off, Sbar, Cbar, anyP, ali);
+                    pbar = quad_add<NL>(pbar, keep(v3(-offbar.x, -offbar.y, -offbar.z), anyP));
                 }
             }
-        a.own[3u * i + 0u] = make_float4(pbar.x, pbar.y, pbar.z, 0.0f);
-        a.own[3u * i + 1u] = make_float4(fbar.x, fbar.y, fbar.z, sbar);
-        a.own[3u * i + 2u] = make_float4(abar.x, abar.y, abar.z, 0.0f);
-        a.bars[3u * i + 0u] = make_float4(Sbar.x, Sbar.y, Sbar.z, Cbar.x);
-        a.bars[3u * i + 1u] = make_float4(Cbar.y, Cbar.z, Abar.x, Abar.y);
-        a.bars[3u * i + 2u] = make_float4(Abar.z, __uint_as_float(flags), 0.0f, 0.0f);
-    } else if (i < a.n) {
+        }
+        float4* const own = a.own + 3u * (size_t)i;
+        float4* const rec = a.rec + 4u * (size_t)i;
+        const float fl = __uint_as_float(flags);
+        if (NL == 1) {
+            own[0] = make_float4(pbar.x, pbar.y, pbar.z, 0.0f);
+            own[1] = make_float4(fbar.x, fbar.y, fbar.z, sbar);
+            own[2] = make_float4(abar.x, abar.y, abar.z, 0.0f);
+            rec[0] = make_float4(p.x, p.y, p.z, f.x);
+            rec[1] = make_float4(f.y, f.z, Sbar.x, Sbar.y);
+            rec[2] = make_float4(Sbar.z, Cbar.x, Cbar.y, Cbar.z);
+            rec[3] = make_float4(Abar.x, Abar.y, Abar.z, fl);
+        } else {
+            // lane l stores the l-th float4 of each
+            if (l < 3u)
+                own[l] = make_float4(pick(l, pbar.x, fbar.x, abar.x, 0.0f), pick(l, pbar.y, fbar.y, abar.y, 0.0f),
+                                     pick(l, pbar.z, fbar.z, abar.z, 0.0f), l == 1u ? sbar : 0.0f);
+            rec[l] = make_float4(pick(l, p.x, f.y, Sbar.z, Abar.x), pick(l, p.y, f.z, Cbar.x, Abar.y),
+                                 pick(l, p.z, Sbar.x, Cbar.y, Abar.z), pick(l, f.x, Sbar.y, Cbar.z, fl));
+            // one lane's weight terms stand for the agent
+            wg[0] = l == 0u ? wg[0] : 0.0f;
+            wg[1] = l == 0u ? wg[1] : 0.0f;
+            wg[2] = l == 0u ? wg[2] : 0.0f;
+        }
+    } else if (i < a.n && l == 0u) {
         // a hash entry without a valid ID: no terms
         const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t k = 0; k < 3u; ++k) {
-            a.own[3u * i + k] = z;
-            a.bars[3u * i + k] = z;
-        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3u; ++k) a.own[3u * (size_t)i + k] = z;
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) a.rec[4u * (size_t)i + k] = z;
     }
     // workgroup reduction of dL/dw in a fixed order
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -382,7 +465,7 @@ __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
 #define BRT_ADJ_GATHER_LANES 4
 #endif
 constexpr uint32_t kGatherLanes = BRT_ADJ_GATHER_LANES;
-static_assert(kGatherLanes <= 64 && (kGatherLanes & (kGatherLanes - 1)) == 0, "lanes per agent: a power of 2");
+static_assert(kGatherLanes >= 4 && kGatherLanes <= 64 && (kGatherLanes & (kGatherLanes - 1)) == 0, "lanes per agent: a power of 2, at least the three output vectors");
 
 struct GatherArgs {
     brt_grid_params g;
@@ -391,13 +474,12 @@ struct GatherArgs {
     float T;        // the list test's squared-radius threshold
     uint32_t knn;   // lists built by replacement (useKnn)
     const float4* spos;
-    const float4* sfwd;
     const uint2* hash;
     const uint32_t* lists;
     const uint32_t* cell_start;
     const uint32_t* cell_end;
     const float4* own;
-    const float4* bars;
+    const float4* rec;
     float4* gpos_in;
     float4* gfwd_in;
     float4* gsa_in;
@@ -448,15 +530,23 @@ __device__ __forceinline__ bool in_list(const GatherArgs& a, uint32_t i, uint32_
     return oj < ol || (oj == ol && j <= last);
 }
 
-// Adds the terms agent i's list holds for p_j and f_j (off = p_j - p_i).
-__device__ __forceinline__ void add_pair(const GatherArgs& a, uint32_t i, float4 B2, V3 off, V3& accP, V3& accF) {
-    const float4 B0 = a.bars[3u * i + 0u], B1 = a.bars[3u * i + 1u];
-    bool anyP, ali;
-    const V3 offbar = pair_terms(a.sp, __float_as_uint(B2.y), xyz(a.sfwd[i]), off, v3(B0.x, B0.y, B0.z),
-                                 v3(B0.w, B1.x, B1.y), anyP, ali);
-    if (anyP) accP = accP + offbar;
-    if (ali) accF = accF + v3(B1.z, B1.w, B2.x);
-}
+// The record k_adjoint_own left for an agent.
+struct Rec {
+    float4 r[4];
+    __device__ __forceinline__ void load(const float4* rec, uint32_t i) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = rec[4u * (size_t)i + k];
+    }
+    __device__ __forceinline__ uint32_t flags() const { return __float_as_uint(r[3].w); }
+    // adds the terms the agent's list holds for p_j and f_j (off = p_j - p_i)
+    __device__ __forceinline__ void add_pair(const brt_steer_params& sp, V3 off, V3& accP, V3& accF) const {
+        bool anyP, ali;
+        const V3 offbar = pair_terms(sp, flags(), v3(r[0].w, r[1].x, r[1].y), off, v3(r[1].z, r[1].w, r[2].x),
+                                     v3(r[2].y, r[2].z, r[2].w), anyP, ali);
+        if (anyP) accP = accP + offbar;
+        if (ali) accF = accF + xyz(r[3]);
+    }
+};
 
 // The key coordinate, on one axis, of the cells whose agents can hold in their
 // lists an agent of key coordinate c: c + d for d = -1, 0, 1 inside the grid,
@@ -470,16 +560,23 @@ __device__ __forceinline__ int gather_axis(int c, int d, uint32_t G) {
 }
 
 // dL/d(p_j, f_j, s_j, a_j) by agent ID: agent j's own terms plus the terms of
-// every agent i whose list holds j.  When j lies in the grid off its low faces,
-// its list is not full and maxBodiesPerCell cuts no cell, those agents are all
-// in j's own list (the radius test is symmetric: d2 has the same bits both
-// ways), so the lanes walk that list; otherwise they scan the 27 cells around
-// j's cell.  Each lane
-// sums its part in order and the lanes' sums are combined by a fixed
-// butterfly.  Workgroup 0 first adds the weight-gradient partials of
-// k_adjoint_own in a fixed order.
+// every agent i whose list holds j.  When j lies in the grid, its list is not
+// full and maxBodiesPerCell cuts no cell, those agents are all in j's own list
+// (the radius test is symmetric: d2 has the same bits both ways), so the lanes
+// walk that list; for j on a low face of the grid they also scan the far
+// face's cells in which agents below the grid are kept (j's list does not reach
+// those).  Otherwise they scan the 27 cells around j's cell.
+// Each lane sums its part in order and the lanes' sums are combined by a fixed
+// butterfly.  Bound by the slowest lane's chain of loads, so all of an agent's own
+// are in flight together, then two entries' 64-byte records, and agents on a low
+// face (7 % of a 40^3 grid's, nearly every wave has one) walk their list too
+// instead of 27 cells: 65,536 agents, one per cell, 33.0 -> 16.0 us.  The last workgroup adds the weight-gradient partials of
+// k_adjoint_own in a fixed order and does nothing else.
 __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
-    if (blockIdx.x == 0) reduce_partials(a.partials, a.partial_blocks, a.weight_grad);
+    if (blockIdx.x == gridDim.x - 1u) {
+        reduce_partials(a.partials, a.partial_blocks, a.weight_grad);
+        return;
+    }
     constexpr uint32_t L = kGatherLanes;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t j = t / L, l = t % L;
@@ -487,8 +584,19 @@ __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
     const brt_grid_params& g = a.g;
     V3 accP = v3(0.f, 0.f, 0.f), accF = accP;
     uint32_t id = a.n;
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
     if (j < a.n) {
+        // all of the agent's own loads in flight together
         const uint2 hj = a.hash[j];
+        const float4 Pj = a.spos[j];
+        const uint32_t fj = __float_as_uint(a.rec[4u * (size_t)j + 3u].w);
+        const uint32_t* row = a.lists + (size_t)j * a.W;
+        const uint32_t cnt = row[0] < a.W - 1u ? row[0] : a.W - 1u;
+        constexpr uint32_t kAhead = 2u;  // entries of a lane in flight
+        uint32_t ii[kAhead];
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) ii[u] = row[l + u * L < a.W - 1u ? 1u + l + u * L : 0u];
+        own = a.own[3u * (size_t)j + (l < 3u ? l : 0u)];
         id = hj.y;
         const uint32_t key = hj.x;
         const bool behaviours = sp.separation[0] != 0.0f || sp.alignment[0] != 0.0f || sp.cohesion[0] != 0.0f;
@@ -497,28 +605,40 @@ __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
         // every list test
         const bool visible = key < g.num_cells && (unlimited || j - a.cell_start[key] < g.max_bodies_per_cell);
         if (behaviours && id < a.n && visible) {
-            const float4 Pj = a.spos[j];
             const V3 pj = xyz(Pj);
-            const uint32_t fj = __float_as_uint(a.bars[3u * j + 2u].y);
-            if (unlimited && (fj & kAdjInGrid) && !(fj & (kAdjFull | kAdjLowFace))) {
-                const uint32_t* row = a.lists + (size_t)j * a.W;
-                const uint32_t cnt = row[0];
-                for (uint32_t e = l; e < cnt; e += L) {
-                    const uint32_t i = row[1u + e];
-                    if (i >= a.n) continue;
-                    const float4 Pi = a.spos[i];
-                    const float4 B2 = a.bars[3u * i + 2u];
-                    if (!in_list(a, i, __float_as_uint(B2.y), Pi, j, I3{0, 0, 0}, true, Pj, true)) continue;
-                    add_pair(a, i, B2, pj - xyz(Pi), accP, accF);
+            const bool by_list = unlimited && (fj & kAdjInGrid) && !(fj & kAdjFull);
+            if (by_list) {
+                for (uint32_t e = l; e < cnt; e += kAhead * L) {
+                    if (e != l) {
+#pragma unroll
+                        for (uint32_t u = 0; u < kAhead; ++u)
+                            ii[u] = row[e + u * L < a.W - 1u ? 1u + e + u * L : 0u];
+                    }
+                    Rec R[kAhead];
+#pragma unroll
+                    for (uint32_t u = 0; u < kAhead; ++u) {
+                        if (e + u * L >= cnt || ii[u] >= a.n) ii[u] = a.n;
+                        R[u].load(a.rec, ii[u] < a.n ? ii[u] : j);
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < kAhead; ++u) {
+                        const uint32_t i = ii[u];
+                        if (i >= a.n) continue;
+                        if (!in_list(a, i, R[u].flags(), R[u].r[0], j, I3{0, 0, 0}, true, Pj, true)) continue;
+                        R[u].add_pair(sp, pj - xyz(R[u].r[0]), accP, accF);
+                    }
                 }
-            } else {
+            }
+            if (!by_list || (fj & kAdjLowFace)) {
                 const I3 cj = key_cell(key, g);
                 for (uint32_t c = l; c < 27u; c += L) {
-                    const int nx = gather_axis(cj.x, (int)(c / 9u) - 1, g.grid_size[0]);
-                    const int ny = gather_axis(cj.y, (int)((c / 3u) % 3u) - 1, g.grid_size[1]);
-                    const int nz = gather_axis(cj.z, (int)(c % 3u) - 1, g.grid_size[2]);
+                    const int dx = (int)(c / 9u) - 1, dy = (int)((c / 3u) % 3u) - 1, dz = (int)(c % 3u) - 1;
+                    const int nx = gather_axis(cj.x, dx, g.grid_size[0]);
+                    const int ny = gather_axis(cj.y, dy, g.grid_size[1]);
+                    const int nz = gather_axis(cj.z, dz, g.grid_size[2]);
                     if (nx < 0 || ny < 0 || nz < 0) continue;
-                    const bool near = abs(nx - cj.x) <= 1 && abs(ny - cj.y) <= 1 && abs(nz - cj.z) <= 1;
+                    const bool near = nx == cj.x + dx && ny == cj.y + dy && nz == cj.z + dz;
+                    if (by_list && near) continue;
                     const uint32_t nk = cellKey(nx, ny, nz, g);
                     const uint32_t s = a.cell_start[nk];
                     if (s == BRT_EMPTY_CELL) continue;
@@ -529,9 +649,10 @@ __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
                         // the list test of agent i for candidate j (d2 as k_prox forms it)
                         const V3 off = pj - xyz(Pi);
                         if (dot(off, off) > a.T) continue;
-                        const float4 B2 = a.bars[3u * i + 2u];
-                        if (!in_list(a, i, __float_as_uint(B2.y), Pi, j, cj, false, Pj, near)) continue;
-                        add_pair(a, i, B2, off, accP, accF);
+                        Rec R;
+                        R.load(a.rec, i);
+                        if (!in_list(a, i, R.flags(), Pi, j, cj, false, Pj, near)) continue;
+                        R.add_pair(sp, off, accP, accF);
                     }
                 }
             }
@@ -546,15 +667,22 @@ __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
         accF.y += __shfl_xor(accF.y, (int)o);
         accF.z += __shfl_xor(accF.z, (int)o);
     }
-    if (j < a.n && l == 0u && id < a.n) {
-        const float4 op = a.own[3u * j + 0u], of = a.own[3u * j + 1u], oa = a.own[3u * j + 2u];
-        a.gpos_in[id] = make_float4(op.x + accP.x, op.y + accP.y, op.z + accP.z, 0.0f);
-        a.gfwd_in[id] = make_float4(of.x + accF.x, of.y + accF.y, of.z + accF.z, of.w);
-        a.gsa_in[id] = oa;
+    // lane 0 stores dL/dp, lane 1 dL/d(f, s), lane 2 dL/da
+    if (j < a.n && l < 3u && id < a.n) {
+        const V3 more = l == 0u ? accP : accF;
+        float4 r = own;
+        if (l < 2u) r = make_float4(own.x + more.x, own.y + more.y, own.z + more.z, l == 0u ? 0.0f : own.w);
+        float4* const out = l == 0u ? a.gpos_in : (l == 1u ? a.gfwd_in : a.gsa_in);
+        out[id] = r;
     }
 }
 
+// Agents up to which k_adjoint_own takes four lanes per agent.
+constexpr uint32_t kOwnQuadMax = 1u << 17;
+
 }  // namespace
+
+uint32_t adjoint_own_blocks(uint32_t n) { return n <= kOwnQuadMax ? (n + 63u) / 64u : (n + 255u) / 256u; }
 
 hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                           const brt_steer_params& sp, float dt, uint32_t n, const float4* spos, const float4* sfwd,
@@ -562,7 +690,6 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
                           const uint32_t* cell_end, const float4* gpos_out, const float4* gfwd_out,
                           const float4* gsa_out, float4* gpos_in, float4* gfwd_in, float4* gsa_in, float4* scratch,
                           float* partials, float* weight_grad, uint32_t xcd_remap, hipStream_t s) {
-    const uint32_t blocks = (n + 255) / 256;
     AdjArgs a{};
     a.g = g;
     a.sp = sp;
@@ -578,11 +705,16 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
     a.gpos_out = gpos_out;
     a.gfwd_out = gfwd_out;
     a.gsa_out = gsa_out;
-    a.own = scratch;
-    a.bars = scratch + 3u * (size_t)n;
+    a.rec = scratch;  // 64-byte aligned
+    a.own = scratch + 4u * (size_t)n;
     a.partials = partials;
     a.xcd_remap = xcd_remap;
-    hipLaunchKernelGGL(k_adjoint_own, dim3(blocks), dim3(256), 0, s, a);
+    const bool quads = n <= kOwnQuadMax;
+    const uint32_t blocks = adjoint_own_blocks(n);
+    if (quads)
+        hipLaunchKernelGGL(k_adjoint_own<4>, dim3(blocks), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(k_adjoint_own<1>, dim3(blocks), dim3(256), 0, s, a);
     GatherArgs b{};
     b.g = g;
     b.sp = sp;
@@ -592,13 +724,12 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
     b.T = threshold;
     b.knn = p.use_knn ? 1u : 0u;
     b.spos = spos;
-    b.sfwd = sfwd;
     b.hash = hash;
     b.lists = lists;
     b.cell_start = cell_start;
     b.cell_end = cell_end;
     b.own = a.own;
-    b.bars = a.bars;
+    b.rec = a.rec;
     b.gpos_in = gpos_in;
     b.gfwd_in = gfwd_in;
     b.gsa_in = gsa_in;
@@ -606,7 +737,7 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
     b.partial_blocks = blocks;
     b.weight_grad = weight_grad;
     const size_t threads = (size_t)n * kGatherLanes;
-    hipLaunchKernelGGL(k_adjoint_gather, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(k_adjoint_gather, dim3((unsigned)((threads + 255) / 256) + 1u), dim3(256), 0, s, b);
     return hipGetLastError();
 }
 

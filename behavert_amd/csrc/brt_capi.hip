@@ -587,7 +587,7 @@ int brt_osw_adjoint_step(brt_context* ctx, const brt_grid_params* grid, const br
                 "adjoint input and output arrays must differ");
     if ((rc = use_device(ctx))) return rc;
     // per-workgroup weight-gradient partials
-    const size_t need = ((size_t)(n + 255) / 256) * 3 * sizeof(float) + 256;
+    const size_t need = (size_t)brt::adjoint_own_blocks(n) * 3 * sizeof(float) + 256;
     if (need > ctx->partials_bytes) {
         if (ctx->partials) BRT_HIP(hipFree(ctx->partials), "hipFree(partials)");
         ctx->partials = nullptr;
@@ -595,9 +595,8 @@ int brt_osw_adjoint_step(brt_context* ctx, const brt_grid_params* grid, const br
         BRT_HIP(hipMalloc((void**)&ctx->partials, need), "hipMalloc(partials)");
         ctx->partials_bytes = need;
     }
-    // each agent's own terms and neighbour-term vectors (6 x n float4) in the
-    // context's scratch
-    if ((rc = ensure_tmp(ctx, (size_t)n * 96u))) return rc;
+    // each agent's own terms and record in the context's scratch
+    if ((rc = ensure_tmp(ctx, brt::adjoint_scratch_bytes(n)))) return rc;
     BRT_HIP(brt::launch_adjoint(*grid, *prox, brt_radius_threshold(prox->search_radius), *steer, dt, n,
                                 reinterpret_cast<const float4*>(sorted_pos),
                                 reinterpret_cast<const float4*>(sorted_forward),
