@@ -520,7 +520,7 @@ int brt_prox_neighbors(brt_context* ctx, const brt_grid_params* grid, const brt_
     BRT_HIP(brt::launch_neighbors(*grid, *prox, brt_radius_threshold(prox->search_radius),
                                   reinterpret_cast<const float4*>(sorted_pos), reinterpret_cast<const uint2*>(hash),
                                   cell_start, cell_end, n, lists, ctx->uniform_max_cells, ctx->xcd_remap,
-                                  resolve_lds_lists(ctx, prox), (hipStream_t)stream),
+                                  resolve_lds_lists(ctx, prox), ctx->lds_lists < 0, (hipStream_t)stream),
             "k_neighbors");
     return BRT_OK;
 }
@@ -965,7 +965,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // the two-pass path gathers the features into sorted order with the state
     // (into the sort's ping-pong buffer, free once the sort is done), so the
     // steering pass reads the neighbours' features by sorted index
-    const bool two_pass = !(resolve_fused(ctx, prox) && !prox->use_knn);
+    const bool two_pass = !resolve_step_fused(ctx, prox, n, do_features);
     const bool sorted_features = do_features && two_pass;
     // small flocks: the keys lie in the lists, which the neighbour search writes
     // later; the context's scratch grows as for the radix sort, which a later
@@ -977,7 +977,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // packed x,y,z copy written by the reorder (three 16-byte loads per four
     // candidates; the register-list scan measured no gain from it)
     const uint32_t lds = resolve_lds_lists(ctx, prox);
-    const bool pack = !prox->use_knn && lds != 0u;
+    const bool pack = !prox->use_knn && (lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
     if (!given && pack && (rc = ensure_xyz(ctx, n))) return rc;
     float* xyz = pack ? (given ? given->xyz : ctx->xyz) : nullptr;
     void* tmp = nullptr;
@@ -1043,14 +1043,14 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
                                             b->lists, reinterpret_cast<float2*>(b->wander),
                                             reinterpret_cast<float4*>(b->pos), reinterpret_cast<float4*>(b->forward),
                                             reinterpret_cast<float4*>(b->smooth_accel), ctx->uniform_max_cells,
-                                            ctx->xcd_remap, lds, s, xyz),
+                                            ctx->xcd_remap, lds, ctx->lds_lists < 0, s, xyz),
                 "k_prox<fused>");
     } else {
         // phase 2: neighbour lists
         mark_phase(2);
         BRT_HIP(brt::launch_neighbors(*grid, *prox, T, reinterpret_cast<const float4*>(b->sorted_pos),
                                       reinterpret_cast<const uint2*>(b->hash), b->cell_start, b->cell_end, n,
-                                      b->lists, ctx->uniform_max_cells, ctx->xcd_remap, lds, s, xyz),
+                                      b->lists, ctx->uniform_max_cells, ctx->xcd_remap, lds, ctx->lds_lists < 0, s, xyz),
                 "k_neighbors");
         // phase 3: fused steering + integration, scattered back to agent-ID order,
         // with the feature update in the same pass over the lists
@@ -1125,8 +1125,9 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
                  const brt_step_buffers* b, std::vector<unsigned char>&& key) {
     const uint32_t n = b->n;
     const bool do_features = b->features && b->features_out && feature_rate != 0.0f;
-    const bool two_pass = !(resolve_fused(ctx, prox) && !prox->use_knn);
-    const bool pack = !prox->use_knn && resolve_lds_lists(ctx, prox) != 0u;
+    const bool two_pass = !resolve_step_fused(ctx, prox, n, do_features);
+    const bool pack =
+        !prox->use_knn && (resolve_lds_lists(ctx, prox) != 0u || resolve_quads(ctx, prox, n, !two_pass));
     int rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells));
     if (rc) return rc;
     if (do_features && two_pass && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;

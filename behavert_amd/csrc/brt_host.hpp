@@ -64,6 +64,19 @@ struct brt_context {
 inline bool resolve_fused(const brt_context* ctx, const brt_prox_params* p) {
     return ctx->fused_step >= 0 ? ctx->fused_step != 0 : p->max_neighbors <= 32u;
 }
+// Whether the neighbour search of n agents takes four lanes per agent (lists
+// automatic), and so packs their positions.
+inline bool resolve_quads(const brt_context* ctx, const brt_prox_params* p, uint32_t n, bool fused) {
+    return ctx->lds_lists < 0 && !p->use_knn && brt::prox_quad_fits(p->max_neighbors, n, fused);
+}
+// The shape of a step of n agents: fused also beyond K = 32 where the quads take
+// the whole step in one launch (K 64, one per cell, 1,000 / 65,536 agents: 26 / 44
+// us in two passes, 21 / 36 in one); with the feature update the two-pass path, whose steering pass does it.
+inline bool resolve_step_fused(const brt_context* ctx, const brt_prox_params* p, uint32_t n, bool features) {
+    if (p->use_knn) return false;
+    if (ctx->fused_step < 0 && !features && resolve_quads(ctx, p, n, true)) return true;
+    return resolve_fused(ctx, p);
+}
 inline uint32_t resolve_lds_lists(const brt_context* ctx, const brt_prox_params* p) {
     return ctx->lds_lists >= 0 ? (uint32_t)(ctx->lds_lists != 0) : (p->max_neighbors <= 32u ? 1u : 0u);
 }

@@ -109,18 +109,30 @@ hipError_t launch_cell_sort(const uint32_t* keys, uint32_t n, uint32_t num_cells
                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t s);
 
 // proximity
+// Launches of at most this many agents take four lanes per agent: about where
+// the chip is full with one lane each.  A step (K 32) with one lane -> four, us,
+// at 1 / 8 per cell / in blobs: 4,096 agents 33 / 67 / 92 -> 21 / 35 / 51;
+// 65,536 43 / 74 / 211 -> 36 / 56 / 117; 131,072 52 / 92 / 215 -> 52 / 89 / 145;
+// 262,144 94 / 149 / 230 -> 108 / 174 / 209; 1,048,576 255 / 462 / 525 -> 296 /
+// 590 / 620.
+#ifndef BRT_PROX_QUAD_MAX
+#define BRT_PROX_QUAD_MAX (1u << 17)
+#endif
+constexpr uint32_t kProxQuadMax = BRT_PROX_QUAD_MAX;
 hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                             const float4* spos, const uint2* hash, const uint32_t* cell_start,
                             const uint32_t* cell_end, uint32_t n, uint32_t* lists, uint32_t uniform_max_cells,
-                            uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s, const float* pxyz = nullptr);
+                            uint32_t xcd_remap, uint32_t lds_lists, bool quads, hipStream_t s,
+                            const float* pxyz = nullptr);
 // neighbour lists + steering + integration in one pass (non-KNN lists only)
 hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                                   const brt_steer_params& sp, float dt, uint32_t step, const float4* spos,
                                   const float4* sfwd, const float4* ssa, const uint2* hash,
                                   const uint32_t* cell_start, const uint32_t* cell_end, uint32_t n, uint32_t* lists,
                                   float2* wander, float4* pos_out, float4* fwd_out, float4* sa_out,
-                                  uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s,
-                                  const float* pxyz = nullptr);
+                                  uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t lds_lists, bool quads,
+                                  hipStream_t s, const float* pxyz = nullptr);
+// quads: launches of up to kProxQuadMax agents may take four lanes per agent (lists staged in LDS).
 // pxyz (optional, single-grid launches): the sorted positions packed as x,y,z,
 // 12 bytes per agent (ReorderArgs::xyz0)
 
@@ -182,6 +194,16 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
                           float* partials, float* weight_grad, uint32_t xcd_remap, hipStream_t s);
 
 inline uint32_t list_stride(uint32_t K) { return 4u * (K / 4u + 1u); }
+// LDS of a workgroup of the four-lane neighbour kernels (64 list rows and, when
+// the steering is fused, an agent's three sums and their counts: an odd number
+// of words), and whether a launch may take them.
+constexpr uint32_t kQuadSumWords = 11u;
+inline uint32_t prox_quad_lds(uint32_t K, bool fused) {
+    return 64u * (list_stride(K) + (fused ? kQuadSumWords : 0u)) * 4u;
+}
+inline bool prox_quad_fits(uint32_t K, uint32_t n, bool fused) {
+    return n <= kProxQuadMax && prox_quad_lds(K, fused) <= 64u * 1024u;
+}
 // Row stride of the LDS list tile of the neighbour kernels: the list stride,
 // widened so a round of 8 candidates can append past K without a per-candidate
 // count check (rows of W >= K + 8 words, a multiple of 4), unless a 64-lane

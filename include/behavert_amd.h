@@ -148,7 +148,10 @@ const char* brt_version(void);
 int brt_context_set_option(brt_context* ctx, int option, int value);
 int brt_context_get_option(const brt_context* ctx, int option, int* value);
 /* The launch shape brt_step and brt_prox_neighbors use for these proximity
- * parameters once automatic options are resolved: fused (0/1), lds_lists (0/1). */
+ * parameters once automatic options are resolved: fused (0/1), lds_lists (0/1).
+ * With lds_lists automatic, launches of up to 131,072 agents take four lanes per
+ * agent and stage their lists in LDS for every K, and steps without the feature
+ * update are fused there. */
 int brt_context_step_shape(const brt_context* ctx, const brt_prox_params* prox, int* fused, int* lds_lists);
 
 /* Failures the kernels record on the device instead of hanging or faulting:
