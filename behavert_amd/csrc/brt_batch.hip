@@ -163,7 +163,7 @@ int enqueue_step(brt_batch* b, const brt_steer_params* steer, float feature_rate
     if (buf->features && buf->features_out && feature_rate != 0.0f)
         BRT_HIP(brt::launch_features(b->prox.max_neighbors, feature_rate, n, reinterpret_cast<const uint2*>(buf->hash),
                                      buf->lists, reinterpret_cast<const float4*>(buf->features),
-                                     reinterpret_cast<float4*>(buf->features_out), s),
+                                     reinterpret_cast<float4*>(buf->features_out), b->cfg.xcd_remap, s),
                 "k_features");
     return BRT_OK;
 }

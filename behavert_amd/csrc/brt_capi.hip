@@ -111,7 +111,9 @@ int ensure_xyz(brt_context* ctx, uint32_t n) {
 }
 
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan) {
-    int rc = ensure_tmp(ctx, (size_t)n * 8u);
+    // 8 bytes per agent for the sort; 16 so that the passes over its lists (sorted
+    // features, labels) find their scratch there
+    int rc = ensure_tmp(ctx, (size_t)n * 16u);
     if (rc) return rc;
     size_t need_meta = brt::sort_meta_words(plan) * 4u;
     if (need_meta > ctx->meta_bytes) {
@@ -693,7 +695,7 @@ int brt_bc_neigh_similarities(brt_context* ctx, const brt_prox_params* prox, con
     BRT_HIP(brt::launch_bc_similarities(prox->max_neighbors, *bc, n, reinterpret_cast<const uint2*>(hash), lists,
                                         features, reinterpret_cast<const float4*>(stats_in),
                                         reinterpret_cast<float4*>(stats_out), similarities, ctx->tmp, nullptr,
-                                        nullptr, nullptr, nullptr, nullptr, (hipStream_t)stream),
+                                        nullptr, nullptr, nullptr, nullptr, ctx->xcd_remap, (hipStream_t)stream),
             "k_bc_similarities");
     return BRT_OK;
 }
@@ -726,7 +728,7 @@ int brt_bc_similarities_steer(brt_context* ctx, const brt_prox_params* prox, con
                                         reinterpret_cast<const float4*>(sorted_pos),
                                         reinterpret_cast<const float4*>(sorted_forward),
                                         reinterpret_cast<const float4*>(force_in),
-                                        reinterpret_cast<float4*>(force_out), (hipStream_t)stream),
+                                        reinterpret_cast<float4*>(force_out), ctx->xcd_remap, (hipStream_t)stream),
             "k_bc_similarities<steer>");
     return BRT_OK;
 }
@@ -750,7 +752,7 @@ int brt_bc_steer_for_clustering(brt_context* ctx, const brt_prox_params* prox, c
                                          reinterpret_cast<const float4*>(sorted_pos),
                                          reinterpret_cast<const float4*>(sorted_forward), lists, similarities,
                                          reinterpret_cast<const float4*>(force_in),
-                                         reinterpret_cast<float4*>(force_out), (hipStream_t)stream),
+                                         reinterpret_cast<float4*>(force_out), ctx->xcd_remap, (hipStream_t)stream),
             "k_bc_cluster_steer");
     return BRT_OK;
 }
@@ -776,7 +778,7 @@ int brt_bc_cluster_membership(brt_context* ctx, const brt_prox_params* prox, uin
     BRT_HIP(brt::launch_cluster_membership(prox->max_neighbors, n, iterations, reinterpret_cast<const uint2*>(hash),
                                            lists, reinterpret_cast<const float4*>(sorted_pos), membership_in,
                                            membership_out, reinterpret_cast<float4*>(connector), lbl,
-                                           lbl ? lbl + n : nullptr, (hipStream_t)stream),
+                                           lbl ? lbl + n : nullptr, ctx->xcd_remap, (hipStream_t)stream),
             "k_lp_iterate");
     return BRT_OK;
 }
@@ -795,10 +797,10 @@ int brt_bc_cluster_hit_rate(brt_context* ctx, const brt_prox_params* prox, float
     BRT_REQUIRE(((uintptr_t)membership_in & 3u) == 0 && ((uintptr_t)membership_out & 3u) == 0,
                 "membership arrays misaligned");
     if ((rc = use_device(ctx))) return rc;
-    if ((rc = ensure_tmp(ctx, (size_t)n * 4u))) return rc;
+    if ((rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
     BRT_HIP(brt::launch_hit_rate(prox->max_neighbors, same_cluster_max_radius, n, reinterpret_cast<const uint2*>(hash),
                                  lists, reinterpret_cast<const float4*>(sorted_pos), membership_in, membership_out,
-                                 reinterpret_cast<float*>(ctx->tmp), (hipStream_t)stream),
+                                 reinterpret_cast<float4*>(ctx->tmp), ctx->xcd_remap, (hipStream_t)stream),
             "k_hit_rate");
     return BRT_OK;
 }
@@ -822,7 +824,7 @@ int brt_osw_steer_and_slow_to_avoid_neighbors(brt_context* ctx, const brt_prox_p
     BRT_HIP(brt::launch_slow_avoid(prox->max_neighbors, *steer, n, reinterpret_cast<const float4*>(sorted_pos),
                                    reinterpret_cast<const float4*>(sorted_forward), lists,
                                    reinterpret_cast<float4*>(forward_out), reinterpret_cast<const float4*>(force_in),
-                                   reinterpret_cast<float4*>(force_out), (hipStream_t)stream),
+                                   reinterpret_cast<float4*>(force_out), ctx->xcd_remap, (hipStream_t)stream),
             "k_slow_avoid");
     return BRT_OK;
 }
@@ -883,7 +885,7 @@ int brt_bc_feature_update(brt_context* ctx, const brt_prox_params* prox, float r
     if ((rc = use_device(ctx))) return rc;
     BRT_HIP(brt::launch_features(prox->max_neighbors, rate, n, reinterpret_cast<const uint2*>(hash), lists,
                                  reinterpret_cast<const float4*>(features_in),
-                                 reinterpret_cast<float4*>(features_out), (hipStream_t)stream),
+                                 reinterpret_cast<float4*>(features_out), ctx->xcd_remap, (hipStream_t)stream),
             "k_features");
     return BRT_OK;
 }
@@ -1074,7 +1076,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
         mark_phase(4);
         BRT_HIP(brt::launch_features(prox->max_neighbors, feature_rate, n, reinterpret_cast<const uint2*>(b->hash),
                                      b->lists, reinterpret_cast<const float4*>(b->features),
-                                     reinterpret_cast<float4*>(b->features_out), s),
+                                     reinterpret_cast<float4*>(b->features_out), ctx->xcd_remap, s),
                 "k_features");
     }
     return BRT_OK;

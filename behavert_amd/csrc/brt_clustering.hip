@@ -34,9 +34,11 @@ __device__ __forceinline__ float linear_interp(float x, float xa, float ya, floa
     return ya * ((x - xb) / (xa - xb)) + yb * ((x - xa) / (xb - xa));
 }
 
+// the line through (avg, 0.5) and (mx, 1) above avg, through (mn, 0) and (avg,
+// 0.5) below, evaluated once on selected operands
 __device__ __forceinline__ float interpolate_similarity(float v, float mn, float avg, float mx) {
-    if (v > avg) return cclamp(linear_interp(v, avg, 0.5f, mx, 1.0f), 0.0f, 1.0f);
-    return cclamp(linear_interp(v, mn, 0.0f, avg, 0.5f), 0.0f, 1.0f);
+    const bool up = v > avg;
+    return cclamp(linear_interp(v, up ? avg : mn, up ? 0.5f : 0.0f, up ? mx : avg, up ? 1.0f : 0.5f), 0.0f, 1.0f);
 }
 
 __device__ __forceinline__ float4 update_similarity_stats(float sim, float4 st, const brt_bc_params& bc) {
@@ -154,24 +156,20 @@ struct ClusterAccum {
 };
 
 // computeNeighNaiveSimilarities (+ computeAdaptiveSimilarities) over sorted
-// features; with STEER also steerForClusterCohesion + Alignment on the fly
-// (the whole of BehaviorClusteringPlugIn::steerForClustering in one pass).
-// One lane per sorted agent; neighbours in groups of G (8 gathers of FQ float4
-// in flight at FQ <= 2).  Each lane writes its similarity row into LDS (dynamic,
-// blockDim * (K+1) floats); the rows of a wave's 64 agents are contiguous in
-// `sims` too, so the wave then stores them with coalesced (float4 when `vec`)
-// writes.
+// features.  One lane per sorted agent; neighbours in groups of G (8 gathers of
+// FQ float4 in flight at FQ <= 2).  Each lane writes its similarity row into LDS
+// (dynamic, blockDim * (K+1) floats); the rows of a wave's 64 agents are
+// contiguous in `sims` too, so the wave then stores them with coalesced (float4
+// when `vec`) writes.
 extern __shared__ float bc_rows[];
 
-template <bool ADAPTIVE, bool STEER, int FQ>
+template <bool ADAPTIVE, int FQ>
 __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_t W, const brt_bc_params& bc,
                                                  uint32_t n, const uint2* __restrict__ hash,
                                                  const uint32_t* __restrict__ lists,
                                                  const float4* __restrict__ sfeat, const float* __restrict__ norms,
                                                  const float4* __restrict__ stats_in, float4* __restrict__ stats_out,
-                                                 float* out, const brt_steer_params& sp,
-                                                 const float4* __restrict__ spos, const float4* __restrict__ sfwd,
-                                                 const float4* force_in, float4* force_out) {
+                                                 float* out) {
     constexpr int G = FQ <= 2 ? 8 : (FQ <= 4 ? 4 : 2);
     const uint32_t F = bc.feature_count;
     const uint32_t id = hash[i].y;
@@ -181,31 +179,17 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
     const float n1 = norms[i];
     const bool valid = id < n;
     float4 st = ADAPTIVE && valid ? stats_in[id] : make_float4(0.f, 0.f, 0.f, 0.f);
-    V3 myPos = v3(0.f, 0.f, 0.f), myFwd = myPos, vel = myPos;
-    if (STEER) {
-        const float4 P = spos[i], Fw = sfwd[i];
-        myPos = xyz(P);
-        myFwd = xyz(Fw);
-        vel = myFwd * Fw.w;
-    }
-    ClusterAccum acc;
-    acc.init();
-    const uint32_t count = for_list_octets<STEER ? kRowPrefetch : kRowWhole>(lists, W, K, i, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
+    const uint32_t count = for_list_octets(lists, W, K, i, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
 #pragma unroll
         for (int g0 = 0; g0 < 8; g0 += G) {
             float4 other[G][FQ];
             float n2[G];
-            float4 op[G], of[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const uint32_t j = jj[g0 + g];
 #pragma unroll
                 for (int q = 0; q < FQ; ++q) other[g][q] = sfeat[(size_t)j * FQ + q];
                 n2[g] = norms[j];
-                if (STEER) {
-                    op[g] = spos[j];
-                    of[g] = sfwd[j];
-                }
             }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -220,16 +204,14 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
                     }
                 }
                 out[base + k - 1u] = sim;
-                if (STEER) acc.add(myPos, vel, sp.max_speed, xyz(op[g]), xyz(of[g]), sim);
             }
         }
     });
     for (uint32_t t = count; t <= K; ++t) out[t] = 0.0f;
     if (ADAPTIVE && valid) stats_out[id] = st;
-    if (STEER) force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
 }
 
-template <bool ADAPTIVE, bool STEER, int FQ>
+template <bool ADAPTIVE, int FQ>
 __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W, brt_bc_params bc, uint32_t n,
                                                          const uint2* __restrict__ hash,
                                                          const uint32_t* __restrict__ lists,
@@ -237,16 +219,14 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
                                                          const float* __restrict__ norms,
                                                          const float4* __restrict__ stats_in,
                                                          float4* __restrict__ stats_out, float* __restrict__ sims,
-                                                         brt_steer_params sp, const float4* __restrict__ spos,
-                                                         const float4* __restrict__ sfwd, const float4* force_in,
-                                                         float4* force_out, uint32_t vec) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) similarity_agent<ADAPTIVE, STEER, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out,
-                                                      bc_rows + (size_t)threadIdx.x * (K + 1u), sp, spos, sfwd,
-                                                      force_in, force_out);
+                                                         uint32_t vec, uint32_t xcd_remap) {
+    const uint32_t blk = xcd_block(xcd_remap != 0);
+    const uint32_t i = blk * blockDim.x + threadIdx.x;
+    if (i < n) similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out,
+                                              bc_rows + (size_t)threadIdx.x * (K + 1u));
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint32_t i0 = blockIdx.x * blockDim.x + wv * 64u;
+    const uint32_t i0 = blk * blockDim.x + wv * 64u;
     if (i0 >= n) return;
     const uint32_t total = (n - i0 < 64u ? n - i0 : 64u) * (K + 1u);
     const float* src = bc_rows + (size_t)wv * 64u * (K + 1u);
@@ -260,6 +240,214 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
     for (; x < total; x += 64u) dst[x] = src[x];
 }
 
+// ---- similarities and cluster steering in one pass
+// (the whole of BehaviorClusteringPlugIn::steerForClustering).  The pass reads
+// position, heading, norm and features of every listed neighbour: five gathers
+// per entry, each touching up to 64 cache lines of which the L1 takes about one
+// a clock (10,032 per wave at K 32 and 8 features: 267 of the kernel's 357 us).
+// So a neighbour's values are one record of 64 bytes (a multiple, with more
+// features) in sorted order, and the four lanes of a quad load it together, one
+// line instead of four; the parts change lanes through LDS.  2,854 accesses per
+// wave and 237 us: bound by the arithmetic (6,890 VALU instructions per wave).
+// Record parts: (pos, norm), (heading, 0), the features; 4 * kRounds float4.
+typedef float vfloat4 __attribute__((ext_vector_type(4)));
+
+template <int FQ>
+constexpr int record_rounds() {
+    return (2 + FQ + 3) / 4;
+}
+
+template <int FQ>
+__global__ void __launch_bounds__(256) k_bc_records(uint32_t F, uint32_t n, uint32_t vec,
+                                                    const uint2* __restrict__ hash,
+                                                    const float* __restrict__ features,
+                                                    const float4* __restrict__ spos,
+                                                    const float4* __restrict__ sfwd, float4* __restrict__ rec) {
+    constexpr uint32_t RP = 4u * record_rounds<FQ>();
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = t / RP, p = t % RP;  // one lane per part
+    if (i >= n) return;
+    const uint32_t id = hash[i].y;
+    const float* f = features + (size_t)(id < n ? id : 0u) * F;
+    auto part = [&](uint32_t q) {
+        float v[4];
+        if (vec) {
+            const float4 x = reinterpret_cast<const float4*>(f)[q];
+            v[0] = x.x;
+            v[1] = x.y;
+            v[2] = x.z;
+            v[3] = x.w;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = 4u * q + c < F ? f[4u * q + c] : 0.0f;
+        }
+        return make_float4(v[0], v[1], v[2], v[3]);
+    };
+    float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (p == 0u) {
+        const float4 P = spos[i];
+        float acc = 0.0f;
+        if (id < n) {
+#pragma unroll
+            for (uint32_t q = 0; q < (uint32_t)FQ; ++q) {
+                const float4 x = part(q);
+                const float v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4u * q + c < F) acc = acc + v[c] * v[c];
+            }
+        }
+        r = make_float4(P.x, P.y, P.z, sqrtf(acc));
+    } else if (p == 1u) {
+        const float4 Fw = sfwd[i];
+        r = make_float4(Fw.x, Fw.y, Fw.z, 0.0f);
+    } else if (p < 2u + (uint32_t)FQ && id < n) {
+        r = part(p - 2u);
+    }
+    rec[t] = r;
+}
+
+// LDS of a wave: the list rows, overwritten in place by the similarities (slot t
+// at word t, entry t + 1's word once it is read), for rows of up to kStageWords
+// words, else only the similarities; and the tile that the parts change lanes in.
+constexpr uint32_t kTileChunks = 4u * 65u;  // float4; the 65: no bank conflicts
+inline __host__ __device__ uint32_t similarity_row_words(uint32_t K, uint32_t W) { return W <= kStageWords ? W : K + 1u; }
+inline uint32_t similarity_wave_bytes(uint32_t K, uint32_t W) {
+    return ((64u * similarity_row_words(K, W) * 4u + 15u) / 16u + kTileChunks) * 16u;
+}
+
+template <bool ADAPTIVE, int FQ>
+__global__ void __launch_bounds__(256) k_bc_similarities_steer(
+    uint32_t K, uint32_t W, brt_bc_params bc, uint32_t n, const uint2* __restrict__ hash,
+    const uint32_t* __restrict__ lists, const float4* __restrict__ rec, const float4* __restrict__ stats_in,
+    float4* __restrict__ stats_out, float* __restrict__ sims, brt_steer_params sp, const float4* __restrict__ sfwd,
+    const float4* force_in, float4* force_out, uint32_t wave_bytes, uint32_t xcd_remap) {
+    constexpr int NR = record_rounds<FQ>();
+    constexpr uint32_t RP = 4u * NR;
+    constexpr int G = NR == 1 ? 4 : (NR == 2 ? 2 : 1);  // entries in flight
+    const uint32_t lane = threadIdx.x & 63u, l = lane & 3u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row0 = xcd_block(xcd_remap != 0) * blockDim.x + wave * 64u;
+    if (row0 >= n) return;
+    const uint32_t i = row0 + lane, at = i < n ? i : n - 1u;
+    char* const mem = reinterpret_cast<char*>(bc_rows) + (size_t)wave * wave_bytes;
+    const uint32_t RW = similarity_row_words(K, W);
+    uint32_t* const row = reinterpret_cast<uint32_t*>(mem) + lane * RW;
+    vfloat4* const tile = reinterpret_cast<vfloat4*>(mem + wave_bytes - kTileChunks * 16u);
+    const bool staged = W <= kStageWords;
+    if (staged) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
+    const uint4* const L = reinterpret_cast<const uint4*>(lists + (size_t)at * W);
+    auto word = [&](uint32_t q) {
+        uint4 v;
+        if (staged)
+            v = reinterpret_cast<const uint4*>(row)[q];
+        else
+            v = L[q];
+        return v;
+    };
+
+    const uint32_t F = bc.feature_count;
+    const uint32_t id = hash[at].y;
+    const bool valid = id < n && i < n;
+    float4 own[RP];
+#pragma unroll
+    for (uint32_t p = 0; p < RP; ++p)
+        if (p != 1u && p < 2u + (uint32_t)FQ) own[p] = rec[(size_t)at * RP + p];
+    float4 mine[FQ];
+#pragma unroll
+    for (int q = 0; q < FQ; ++q) mine[q] = own[2 + q];
+    const float n1 = own[0].w;
+    const float4 Fw = sfwd[at];
+    const V3 myPos = xyz(own[0]), myFwd = xyz(Fw), vel = myFwd * Fw.w;
+    float4 st = ADAPTIVE && valid ? stats_in[id] : make_float4(0.f, 0.f, 0.f, 0.f);
+    ClusterAccum acc;
+    acc.init();
+
+    uint4 a = word(0);
+    const uint32_t count = i < n ? (a.x < K ? a.x : K) : 0u;
+    float* const out = reinterpret_cast<float*>(row);
+    // all lanes of the wave stay in step: those past their list load their own record
+    for (uint32_t q = 0; __ballot(4u * q <= count) != 0; q += 2) {
+        const uint32_t last = count / 4u;
+        if (q != 0u) a = word(q < last ? q : last);
+        const uint4 b = word(q + 1u < last ? q + 1u : last);
+        uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const uint32_t mask = octet_mask(jj, q, count, at, n);
+#pragma unroll
+        for (int g0 = 0; g0 < 8; g0 += G) {
+            if (__ballot((mask >> g0 & ((1u << G) - 1u)) != 0u) == 0) continue;
+            // part 4 r + l of the quad's lane k's record
+            vfloat4 in[G][NR][4];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int x = (int)jj[g0 + g];
+                    const uint32_t j = (uint32_t)(k == 0   ? __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, true)
+                                                  : k == 1 ? __builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, true)
+                                                  : k == 2 ? __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, true)
+                                                           : __builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, true));
+                    const vfloat4* const src = reinterpret_cast<const vfloat4*>(rec) + (size_t)j * RP + l;
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) in[g][r][k] = src[4 * r];
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int k = g0 + g;
+                vfloat4 got[RP];
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    // LDS operations of a wave take effect in order
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) tile[65 * c + lane] = in[g][r][c];
+                    wave_lds_sync();
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) got[4 * r + c] = tile[65u * l + (lane - l) + c];
+                    wave_lds_sync();
+                }
+                if (!(mask & (1u << k))) continue;
+                float4 other[FQ];
+#pragma unroll
+                for (int f = 0; f < FQ; ++f)
+                    other[f] = make_float4(got[2 + f].x, got[2 + f].y, got[2 + f].z, got[2 + f].w);
+                float sim = 0.0f;
+                if (valid) {
+                    sim = naive_similarity<FQ>(mine, other, F, n1, got[0].w);
+                    if (ADAPTIVE) {
+                        st = update_similarity_stats(sim, st, bc);
+                        sim = interpolate_similarity(sim, st.x, st.y, st.z);
+                    }
+                }
+                out[4u * q + (uint32_t)k - 1u] = sim;
+                acc.add(myPos, vel, sp.max_speed, v3(got[0].x, got[0].y, got[0].z), v3(got[1].x, got[1].y, got[1].z),
+                        sim);
+            }
+        }
+    }
+    if (i < n) {
+        for (uint32_t t = count; t <= K; ++t) out[t] = 0.0f;
+        if (ADAPTIVE && valid) stats_out[id] = st;
+        force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
+    }
+    wave_lds_sync();
+    // the rows, K + 1 of RW words each, are contiguous in sims
+    const uint32_t S = K + 1u, total = (n - row0 < 64u ? n - row0 : 64u) * S;
+    const float* const src = reinterpret_cast<const float*>(mem);
+    float* const dst = sims + (size_t)row0 * S;
+    const uint32_t dr = 64u / S, dc = 64u - dr * S;
+    uint32_t r = lane / S, c = lane - r * S;
+    for (uint32_t x = lane; x < total; x += 64u) {
+        dst[x] = src[r * RW + c];
+        r += dr;
+        c += dc;
+        if (c >= S) {
+            c -= S;
+            ++r;
+        }
+    }
+}
+
 // steerForClusterCohesion + Alignment from stored similarities.
 __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W, brt_steer_params sp,
                                                           brt_bc_params bc, uint32_t n,
@@ -267,16 +455,19 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
                                                           const float4* __restrict__ sfwd,
                                                           const uint32_t* __restrict__ lists,
                                                           const float* __restrict__ sims,
-                                                          const float4* force_in, float4* force_out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 P = spos[i], Fw = sfwd[i];
+                                                          const float4* force_in, float4* force_out,
+                                                          uint32_t xcd_remap) {
+    __shared__ uint4 s_stage[4][kStageChunks];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t at = i < n ? i : n - 1u;
+    const float4 P = spos[at], Fw = sfwd[at];
     const V3 myPos = xyz(P), myFwd = xyz(Fw);
     const V3 vel = myFwd * Fw.w;
-    const float* s = sims + (size_t)i * (K + 1u);
+    const float* s = sims + (size_t)at * (K + 1u);
     ClusterAccum acc;
     acc.init();
-    const uint32_t count = for_list_octets(lists, W, K, i, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
+    const uint32_t count = wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
         float4 op[8], of[8];
         float sv[8];
 #pragma unroll
@@ -289,7 +480,7 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
         for (int k = 0; k < 8; ++k)
             if (mask & (1u << k)) acc.add(myPos, vel, sp.max_speed, xyz(op[k]), xyz(of[k]), sv[k]);
     });
-    force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
+    if (i < n) force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
 }
 
 // ---------------------------------------------------------------- cluster membership
@@ -311,12 +502,26 @@ __global__ void __launch_bounds__(256) k_lp_iterate(uint32_t K, uint32_t W, uint
                                                     const uint32_t* __restrict__ lists,
                                                     const float* __restrict__ lbl_in, float* __restrict__ lbl_out,
                                                     const float* m_in, float* m_out,
-                                                    const float4* __restrict__ spos, float4* __restrict__ conn) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float mn = FIRST ? (float)i : lbl_in[i];
+                                                    const float4* __restrict__ spos, float4* __restrict__ conn,
+                                                    uint32_t xcd_remap) {
+    __shared__ uint4 s_stage[SCAN ? 4 : 1][SCAN ? kStageChunks : 1];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x, at = i < n ? i : n - 1u;
+    float mn = FIRST ? (float)i : lbl_in[at];
+    // the last iteration's reads by ID load during the walk
+    uint32_t id = n;
+    float y = 0.0f, z = 0.0f;
+    float4 P = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (LAST) {
+        id = hash[at].y;
+        if (id < n) {
+            y = m_in[(size_t)id * 3u + 1u];
+            z = m_in[(size_t)id * 3u + 2u];
+        }
+        if (conn) P = spos[at];
+    }
     if (SCAN) {
-        for_list_octets(lists, W, K, i, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+        wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
             float v[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] = FIRST ? (float)jj[k] : lbl_in[jj[k]];
@@ -325,66 +530,68 @@ __global__ void __launch_bounds__(256) k_lp_iterate(uint32_t K, uint32_t W, uint
                 if ((mask & (1u << k)) && mn > v[k]) mn = v[k];
         });
     }
+    if (i >= n) return;
     if (!LAST) {
         lbl_out[i] = mn;
         return;
     }
-    const uint32_t id = hash[i].y;
     if (id >= n) return;
     const size_t o = (size_t)id * 3u;
-    const float y = m_in[o + 1], z = m_in[o + 2];
     m_out[o] = mn;
     m_out[o + 1] = y;
     m_out[o + 2] = z;
     if (conn) {
-        conn[2u * (size_t)id] = spos[i];
+        conn[2u * (size_t)id] = P;
         conn[2u * (size_t)id + 1u] = spos[(uint32_t)mn];
     }
 }
 
-// Labels from float3 by agent ID into sorted order (one gather per agent), so
-// the hit-rate pass reads its neighbours' labels next to each other.
+// Labels from float3 by agent ID into sorted order beside the position (one
+// gather per agent), so the hit-rate pass reads a neighbour's both in one load.
 __global__ void __launch_bounds__(256) k_gather_labels(uint32_t n, const uint2* __restrict__ hash,
-                                                       const float* __restrict__ m_in, float* __restrict__ lbl) {
+                                                       const float* __restrict__ m_in,
+                                                       const float4* __restrict__ spos, float4* __restrict__ lbl) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t id = hash[i].y;
-    lbl[i] = id < n ? m_in[(size_t)id * 3u] : 0.0f;
+    const float4 p = spos[i];
+    lbl[i] = make_float4(p.x, p.y, p.z, id < n ? m_in[(size_t)id * 3u] : 0.0f);
 }
 
 // analyzeClusterHitRate's kernel (BehaviorClustering_kernel.cu:502-578): among
 // the listed neighbours within sameClusterMaxRadius, the fraction sharing the
 // agent's label and the mean of their labels (-1 with none); float3 by ID.
-__global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float radius, uint32_t n,
+// T: the greatest squared length within the radius (length(o) > radius exactly
+// when dot(o, o) > T, the square root being correctly rounded).  1M blobs, K 32,
+// with the labels gathered beside the positions: 114.8 -> 65 us.
+__global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float T, uint32_t n,
                                                   const uint2* __restrict__ hash, const uint32_t* __restrict__ lists,
-                                                  const float4* __restrict__ spos, const float* __restrict__ lbl,
-                                                  float* __restrict__ m_out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = hash[i].y;
-    if (id >= n) return;
-    const float my = lbl[i];
-    const V3 myPos = xyz(spos[i]);
+                                                  const float4* __restrict__ lbl, float* __restrict__ m_out,
+                                                  uint32_t xcd_remap) {
+    __shared__ uint4 s_stage[4][kStageChunks];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t id = i < n ? hash[i].y : n;
+    const float4 own = lbl[i < n ? i : n - 1u];
+    const float my = own.w;
+    const V3 myPos = xyz(own);
     int close = 0;
     float real = 0.0f, hit = 0.0f;
-    for_list_octets(lists, W, K, i, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+    wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
         float4 op[8];
-        float v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            op[k] = spos[jj[k]];
-            v[k] = lbl[jj[k]];
-        }
+        for (int k = 0; k < 8; ++k) op[k] = lbl[jj[k]];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             if (!(mask & (1u << k))) continue;
             const V3 offset = xyz(op[k]) - myPos;
-            if (length(offset) > radius) continue;
+            if (dot(offset, offset) > T) continue;
             ++close;
-            real = real + v[k];
-            if (my == v[k]) hit = hit + 1.0f;
+            real = real + op[k].w;
+            if (my == op[k].w) hit = hit + 1.0f;
         }
     });
+    if (id >= n) return;
     if (close > 0) {
         hit = hit / (float)close;
         real = real / (float)close;
@@ -401,62 +608,116 @@ __global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float 
 
 hipError_t launch_cluster_membership(uint32_t K, uint32_t n, uint32_t iterations, const uint2* hash,
                                      const uint32_t* lists, const float4* spos, const float* m_in, float* m_out,
-                                     float4* conn, float* lbl_a, float* lbl_b, hipStream_t s) {
+                                     float4* conn, float* lbl_a, float* lbl_b, uint32_t xcd_remap, hipStream_t s) {
     const uint32_t W = list_stride(K);
     const dim3 grid((n + 255) / 256), block(256);
     if (iterations == 0) {
         hipLaunchKernelGGL((k_lp_iterate<true, true, false>), grid, block, 0, s, K, W, n, hash, lists, nullptr,
-                           nullptr, m_in, m_out, spos, conn);
+                           nullptr, m_in, m_out, spos, conn, xcd_remap);
         return hipGetLastError();
     }
     if (iterations == 1) {
         hipLaunchKernelGGL((k_lp_iterate<true, true, true>), grid, block, 0, s, K, W, n, hash, lists, nullptr,
-                           nullptr, m_in, m_out, spos, conn);
+                           nullptr, m_in, m_out, spos, conn, xcd_remap);
         return hipGetLastError();
     }
     hipLaunchKernelGGL((k_lp_iterate<true, false, true>), grid, block, 0, s, K, W, n, hash, lists, nullptr, lbl_a,
-                       m_in, m_out, spos, conn);
+                       m_in, m_out, spos, conn, xcd_remap);
     float* src = lbl_a;
     float* dst = lbl_b;
     for (uint32_t t = 1; t + 1 < iterations; ++t) {
         hipLaunchKernelGGL((k_lp_iterate<false, false, true>), grid, block, 0, s, K, W, n, hash, lists, src, dst,
-                           m_in, m_out, spos, conn);
+                           m_in, m_out, spos, conn, xcd_remap);
         float* x = src;
         src = dst;
         dst = x;
     }
     hipLaunchKernelGGL((k_lp_iterate<false, true, true>), grid, block, 0, s, K, W, n, hash, lists, src, nullptr,
-                       m_in, m_out, spos, conn);
+                       m_in, m_out, spos, conn, xcd_remap);
     return hipGetLastError();
 }
 
 hipError_t launch_hit_rate(uint32_t K, float radius, uint32_t n, const uint2* hash, const uint32_t* lists,
-                           const float4* spos, const float* m_in, float* m_out, float* lbl, hipStream_t s) {
+                           const float4* spos, const float* m_in, float* m_out, float4* lbl, uint32_t xcd_remap,
+                           hipStream_t s) {
     const dim3 grid((n + 255) / 256), block(256);
-    hipLaunchKernelGGL(k_gather_labels, grid, block, 0, s, n, hash, m_in, lbl);
-    hipLaunchKernelGGL(k_hit_rate, grid, block, 0, s, K, list_stride(K), radius, n, hash, lists, spos, lbl, m_out);
+    hipLaunchKernelGGL(k_gather_labels, grid, block, 0, s, n, hash, m_in, spos, lbl);
+    hipLaunchKernelGGL(k_hit_rate, grid, block, 0, s, K, list_stride(K), brt_radius_threshold(radius), n, hash, lists, lbl, m_out,
+                       xcd_remap);
     return hipGetLastError();
 }
 
 namespace {
 
-template <bool ADAPTIVE, bool STEER>
-hipError_t launch_sims_fq(uint32_t FQ, uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash,
-                          const uint32_t* lists, const float4* sfeat, const float* norms, const float4* stats_in,
-                          float4* stats_out, float* sims, const brt_steer_params& sp, const float4* spos,
-                          const float4* sfwd, const float4* force_in, float4* force_out, hipStream_t s) {
-    const uint32_t W = list_stride(K);
+template <int FQ>
+hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash, const uint32_t* lists,
+                       const float* features, uint32_t vec, const float4* stats_in, float4* stats_out, float* sims,
+                       void* scratch, const brt_steer_params* sp, const float4* spos, const float4* sfwd,
+                       const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
+    const uint32_t F = bc.feature_count, W = list_stride(K);
+    if (sp) {
+        constexpr uint32_t RP = 4u * record_rounds<FQ>();
+        float4* rec = reinterpret_cast<float4*>(scratch);
+        hipLaunchKernelGGL((k_bc_records<FQ>), dim3((unsigned)(((size_t)n * RP + 255u) / 256u)), dim3(256), 0, s, F, n,
+                           vec, hash, features, spos, sfwd, rec);
+        // four waves per workgroup while three workgroups fit a CU's LDS, else one
+        const uint32_t bytes = similarity_wave_bytes(K, W), B = 4u * bytes <= 160u * 1024u / 3u ? 256u : 64u;
+        const dim3 grid((n + B - 1) / B), block(B);
+        if (bc.adaptive)
+            hipLaunchKernelGGL((k_bc_similarities_steer<true, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n, hash,
+                               lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
+                               xcd_remap);
+        else
+            hipLaunchKernelGGL((k_bc_similarities_steer<false, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n,
+                               hash, lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
+                               xcd_remap);
+        return hipGetLastError();
+    }
+    float4* sfeat = reinterpret_cast<float4*>(scratch);
+    float* norms = reinterpret_cast<float*>(sfeat + (size_t)n * FQ);
+    hipLaunchKernelGGL(k_bc_sort_features, dim3((n + 255) / 256), dim3(256), 0, s, F, (uint32_t)FQ, n, vec, hash,
+                       features, sfeat, norms);
     // the LDS row tile: 256 agents while it stays within 40 KB, else one wave
     const uint32_t B = (size_t)256u * (K + 1u) * 4u <= 40u * 1024u ? 256u : 64u;
     const size_t lds = (size_t)B * (K + 1u) * 4u;
-    const uint32_t vec = ((uintptr_t)sims & 15u) == 0 ? 1u : 0u;
+    const uint32_t vec_out = ((uintptr_t)sims & 15u) == 0 ? 1u : 0u;
     const dim3 grid((n + B - 1) / B), block(B);
-#define BRT_SIMS_CASE(Q)                                                                                            \
-    case Q:                                                                                                         \
-        hipLaunchKernelGGL((k_bc_similarities<ADAPTIVE, STEER, Q>), grid, block, lds, s, K, W, bc, n, hash, lists, \
-                           sfeat, norms, stats_in, stats_out, sims, sp, spos, sfwd, force_in, force_out, vec);     \
-        break;
-    switch (FQ) {
+    if (bc.adaptive)
+        hipLaunchKernelGGL((k_bc_similarities<true, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
+                           stats_in, stats_out, sims, vec_out, xcd_remap);
+    else
+        hipLaunchKernelGGL((k_bc_similarities<false, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
+                           stats_in, stats_out, sims, vec_out, xcd_remap);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+size_t bc_scratch_bytes(uint32_t feature_count, uint32_t n) {
+    const size_t FQ = (feature_count + 3u) / 4u;
+    return (size_t)n * ((FQ + 5u) / 4u) * 64u;  // the records; features and norms take less
+}
+
+hipError_t launch_bc_similarities(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash,
+                                  const uint32_t* lists, const float* features, const float4* stats_in,
+                                  float4* stats_out, float* sims, void* scratch, const brt_steer_params* sp,
+                                  const float4* spos, const float4* sfwd, const float4* force_in, float4* force_out,
+                                  uint32_t xcd_remap, hipStream_t s) {
+    // lists whose similarities and tile exceed the LDS of a workgroup (K 239 and
+    // more): the same sums from the stored similarities
+    if (sp && similarity_wave_bytes(K, list_stride(K)) > 64u * 1024u) {
+        const hipError_t e = launch_bc_similarities(K, bc, n, hash, lists, features, stats_in, stats_out, sims, scratch,
+                                                    nullptr, nullptr, nullptr, nullptr, nullptr, xcd_remap, s);
+        if (e != hipSuccess) return e;
+        return launch_bc_cluster_steer(K, *sp, bc, n, spos, sfwd, lists, sims, force_in, force_out, xcd_remap, s);
+    }
+    const uint32_t F = bc.feature_count;
+    const uint32_t vec = (F % 4u == 0 && ((uintptr_t)features & 15u) == 0) ? 1u : 0u;
+#define BRT_SIMS_CASE(Q)                                                                                             \
+    case Q:                                                                                                          \
+        return launch_sims<Q>(K, bc, n, hash, lists, features, vec, stats_in, stats_out, sims, scratch, sp, spos,    \
+                              sfwd, force_in, force_out, xcd_remap, s);
+    switch ((F + 3u) / 4u) {
         BRT_SIMS_CASE(1)
         BRT_SIMS_CASE(2)
         BRT_SIMS_CASE(3)
@@ -469,47 +730,13 @@ hipError_t launch_sims_fq(uint32_t FQ, uint32_t K, const brt_bc_params& bc, uint
             return hipErrorInvalidValue;
     }
 #undef BRT_SIMS_CASE
-    return hipGetLastError();
-}
-
-}  // namespace
-
-size_t bc_scratch_bytes(uint32_t feature_count, uint32_t n) {
-    const size_t FQ = (feature_count + 3u) / 4u;
-    return (size_t)n * FQ * 16u + ((size_t)n * 4u + 15u) / 16u * 16u;
-}
-
-hipError_t launch_bc_similarities(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash,
-                                  const uint32_t* lists, const float* features, const float4* stats_in,
-                                  float4* stats_out, float* sims, void* scratch, const brt_steer_params* sp,
-                                  const float4* spos, const float4* sfwd, const float4* force_in, float4* force_out,
-                                  hipStream_t s) {
-    const uint32_t F = bc.feature_count, FQ = (F + 3u) / 4u;
-    float4* sfeat = reinterpret_cast<float4*>(scratch);
-    float* norms = reinterpret_cast<float*>(sfeat + (size_t)n * FQ);
-    const uint32_t vec = (F % 4u == 0 && ((uintptr_t)features & 15u) == 0) ? 1u : 0u;
-    hipLaunchKernelGGL(k_bc_sort_features, dim3((n + 255) / 256), dim3(256), 0, s, F, FQ, n, vec, hash, features,
-                       sfeat, norms);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const brt_steer_params none{};
-    const brt_steer_params& p = sp ? *sp : none;
-    if (bc.adaptive)
-        return sp ? launch_sims_fq<true, true>(FQ, K, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, sims, p,
-                                               spos, sfwd, force_in, force_out, s)
-                  : launch_sims_fq<true, false>(FQ, K, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, sims,
-                                                p, spos, sfwd, force_in, force_out, s);
-    return sp ? launch_sims_fq<false, true>(FQ, K, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, sims, p,
-                                            spos, sfwd, force_in, force_out, s)
-              : launch_sims_fq<false, false>(FQ, K, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, sims, p,
-                                             spos, sfwd, force_in, force_out, s);
 }
 
 hipError_t launch_bc_cluster_steer(uint32_t K, const brt_steer_params& sp, const brt_bc_params& bc, uint32_t n,
                                    const float4* spos, const float4* sfwd, const uint32_t* lists, const float* sims,
-                                   const float4* force_in, float4* force_out, hipStream_t s) {
+                                   const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
     hipLaunchKernelGGL(k_bc_cluster_steer, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, bc, n, spos,
-                       sfwd, lists, sims, force_in, force_out);
+                       sfwd, lists, sims, force_in, force_out, xcd_remap);
     return hipGetLastError();
 }
 

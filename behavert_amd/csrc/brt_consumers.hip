@@ -22,20 +22,25 @@ namespace {
 // Separation (calcSeparation, OpenSteerWrapper_resources.cu:166-211) scaled by
 // its weight, amplified when the list holds more than 16 agents; the agent's
 // speed drops by 10 % when that steering opposes its heading (cos < -0.8) and
-// rises by 2 % when it agrees (> 0.5).  forward_out (sorted) keeps the heading;
+// rises by 2 % when it agrees (> 0.5).  Bound by the arithmetic per entry, so the
+// neighbourhood test is decided by the cuts.  forward_out (sorted) keeps the heading;
 // force_out = steering + force_in (blendIntoSteeringForce).
-__global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_steer_params sp, uint32_t n,
+__global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_steer_params sp, SteerCuts cuts, uint32_t n,
                                                     const float4* __restrict__ spos, const float4* sfwd,
                                                     const uint32_t* __restrict__ lists, float4* fwd_out,
-                                                    const float4* force_in, float4* force_out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float4 P = spos[i], Fw = sfwd[i];
+                                                    const float4* force_in, float4* force_out,
+                                                    uint32_t xcd_remap) {
+    __shared__ uint4 s_stage[4][kStageChunks];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t at = i < n ? i : n - 1u;
+    const float4 P = spos[at], Fw = sfwd[at];
     const V3 myPos = xyz(P), myFwd = xyz(Fw);
     const Weights sepOnly{1.0f, 0.0f, 0.0f};
+    const float margin = cut_margin(myFwd);
     SteerAccum acc;
     acc.init();
-    const uint32_t count = for_list_octets(lists, W, K, i, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+    const uint32_t count = wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
         float4 qp[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) qp[k] = spos[jj[k]];
@@ -43,9 +48,10 @@ __global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_
         for (int k = 0; k < 8; ++k) {
             if (!(mask & (1u << k))) continue;
             const V3 offset = xyz(qp[k]) - myPos;
-            acc.add(sp, sepOnly, myFwd, offset, dot(offset, offset), myFwd);
+            acc.add_cut(sp, cuts, sepOnly, myFwd, margin, offset, dot(offset, offset), myFwd);
         }
     });
+    if (i >= n) return;
     V3 steering = (acc.nSep > 0 ? normalize(acc.sSep / (float)acc.nSep) : acc.sSep) * sp.separation[0];
     if (count > 16u) steering = steering * ((float)(count - 16u) * 0.5f);
     float mySpeed = Fw.w;
@@ -103,13 +109,25 @@ __global__ void __launch_bounds__(256) k_move_towards_target(int shift, float bx
     force_out[i] = make_float4(f.x + f0.x, f.y + f0.y, f.z + f0.z, 0.0f);
 }
 
+// The cuts with the separation's radius and angle for every behaviour: only the
+// separation is summed, so one test serves.
+SteerCuts separation_cuts(const brt_steer_params& sp) {
+    SteerCuts c = steer_cuts(sp);
+    for (int k = 1; k < 3; ++k) {
+        c.tmax[k] = c.tmax[0];
+        c.cmax[k] = c.cmax[0];
+    }
+    c.same = 1u;
+    return c;
+}
+
 }  // namespace
 
 hipError_t launch_slow_avoid(uint32_t K, const brt_steer_params& sp, uint32_t n, const float4* spos,
                              const float4* sfwd, const uint32_t* lists, float4* fwd_out, const float4* force_in,
-                             float4* force_out, hipStream_t s) {
-    hipLaunchKernelGGL(k_slow_avoid, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, n, spos, sfwd,
-                       lists, fwd_out, force_in, force_out);
+                             float4* force_out, uint32_t xcd_remap, hipStream_t s) {
+    hipLaunchKernelGGL(k_slow_avoid, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, separation_cuts(sp),
+                       n, spos, sfwd, lists, fwd_out, force_in, force_out, xcd_remap);
     return hipGetLastError();
 }
 

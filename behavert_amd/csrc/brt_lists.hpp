@@ -8,6 +8,15 @@
 
 namespace brt {
 
+typedef uint32_t vuint4 __attribute__((ext_vector_type(4)));
+
+// What every lane of the wave wrote to LDS is seen by the others.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Bit k set for the valid entries e = 4q + k of an octet (1 <= e <= count and
 // a sorted index below n); invalid lanes of jj are set to i.  Word entry 0 of
 // word 0 is the count; the slot of word entry k is e - 1 = 4q + k - 1.
@@ -24,69 +33,114 @@ __device__ __forceinline__ uint32_t octet_mask(uint32_t (&jj)[8], uint32_t q, ui
     return mask;
 }
 
-// How a list walk reads its row.
-enum ListRows : int {
-    kRowPairs = 0,     // two 16-byte words per octet, after the previous octet's work
-    kRowPrefetch = 1,  // two words per octet, the next octet's pair loading with this one
-    kRowWhole = 2,     // rows of W = 36 words (K 32..35) whole, else kRowPrefetch
-};
-
 // Visits the entries e = 1..count (count capped at K) of agent i's list in
 // order, eight at a time: f(base, jj, mask) gets word entries base..base+7
 // (list slot base + k - 1), with bit k of mask set for the valid ones.
 // Invalid lanes of jj hold i, so gathers through them stay in bounds.
-// kRowWhole loads a K 32 row as nine 16-byte words in flight together (1M-boid
-// blobs, K 32: label propagation 97 -> 51 us per iteration,
-// steer-and-slow-to-avoid 166 -> 84 us, cluster steering 427 -> 319 us).  A
-// kernel holding much else in registers reads pairs: the one-pass
-// similarities + cluster steering measured 4 % slower with whole rows and 4 %
-// faster with prefetched pairs (384 -> 367 us); the steering pass with the
-// feature update (K 64) 3 % slower with prefetched pairs than without.
-template <int ROWS = kRowWhole, class Fn>
+// Each lane reads its own row, the next two 16-byte words loading (AHEAD) while
+// the current octet's gathers are in flight.  (A word past the count is not
+// left out by a select with a constant: that becomes a select of addresses, one
+// of them on the stack, and flat loads.)
+template <bool AHEAD = true, class Fn>
 __device__ __forceinline__ uint32_t for_list_octets(const uint32_t* __restrict__ lists, uint32_t W, uint32_t K,
                                                     uint32_t i, uint32_t n, Fn&& f) {
     const uint4* L = reinterpret_cast<const uint4*>(lists + (size_t)i * W);
-    if (ROWS == kRowWhole && W == 36u) {
-        uint4 c[10];
+    uint4 a = L[0];
+    const uint32_t count = a.x < K ? a.x : K;
+    const uint32_t last = count / 4u;  // the word that holds the last entry
+    uint4 b = L[last < 1u ? last : 1u];
+    for (uint32_t q = 0; q <= last; q += 2) {
+        uint4 na, nb;
+        if (AHEAD) {
+            na = L[q + 2u < last ? q + 2u : last];
+            nb = L[q + 3u < last ? q + 3u : last];
+        } else if (q != 0u) {
+            a = L[q];
+            b = L[q + 1u < last ? q + 1u : last];
+        }
+        uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const uint32_t mask = octet_mask(jj, q, count, i, n);
+        f(4u * q, jj, mask);
+        if (AHEAD) {
+            a = na;
+            b = nb;
+        }
+    }
+    return count;
+}
+
+// The same with the rows of a wave's 64 agents loaded by the wave together.
+// What bounds most list walks is the number of 64-byte accesses that their loads
+// make (about one a clock per CU): a 16-byte word of every lane's own row is 64
+// of them, the same bytes in order 16.  Rows of up to kStageWords words (K 35) go
+// through LDS at once, longer ones in blocks of 32 words.  Every lane of the wave
+// takes part: row0 is the wave's first agent, i = row0 + lane, and lanes beyond
+// n visit nothing.  stage: the wave's kStageChunks of LDS.  1M blobs, K 32, whole
+// rows by their own lanes -> staged: a label iteration 45.3 -> 37.5 us; with the
+// XCD slices, behaviour forces + features of 300,007 agents 57 + 70 -> 46 + 49.
+constexpr uint32_t kStageWords = 36u;
+constexpr uint32_t kStageChunks = 64u * kStageWords / 4u;  // 16-byte words per wave
+
+// Loads a wave's rows (W <= kStageWords) into LDS, 64 rows of W words.
+__device__ __forceinline__ void stage_rows(uint4* stage, const uint32_t* __restrict__ lists, uint32_t W,
+                                           uint32_t row0, uint32_t lane, uint32_t n) {
+    const uint32_t W4 = W / 4u, rows = row0 < n ? (n - row0 < 64u ? n - row0 : 64u) : 0u, total = rows * W4;
+    const vuint4* src = reinterpret_cast<const vuint4*>(lists + (size_t)(rows ? row0 : 0u) * W);
+    vuint4* const to = reinterpret_cast<vuint4*>(stage);
+    const uint32_t top = total ? total - 1u : 0u;
+    if (W4 == 9u) {
+        vuint4 c[9];
 #pragma unroll
-        for (int k = 0; k < 9; ++k) c[k] = L[k];
-        c[9] = make_uint4(0u, 0u, 0u, 0u);
-        const uint32_t count = c[0].x < K ? c[0].x : K;
+        for (uint32_t k = 0; k < 9u; ++k) c[k] = src[lane + 64u * k < total ? lane + 64u * k : top];
 #pragma unroll
-        for (uint32_t q = 0; q < 10u; q += 2) {
-            if (4u * q <= count) {
-                const uint4 a = c[q];
-                const uint4 b = (4u * (q + 1) <= count) ? c[q + 1] : make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t k = 0; k < 9u; ++k) to[lane + 64u * k] = c[k];
+    } else {
+#pragma unroll 4
+        for (uint32_t k = 0; k < W4; ++k) to[lane + 64u * k] = src[lane + 64u * k < total ? lane + 64u * k : top];
+    }
+    wave_lds_sync();
+}
+
+template <class Fn>
+__device__ __forceinline__ uint32_t wave_list_octets(uint4* stage, const uint32_t* __restrict__ lists, uint32_t W,
+                                                     uint32_t K, uint32_t row0, uint32_t lane, uint32_t n, Fn&& f) {
+    const uint32_t i = row0 + lane;
+    if (W > kStageWords) {
+        const uint32_t W4 = W / 4u;
+        uint32_t count = i < n ? 1u : 0u;  // until the first block is there
+        for (uint32_t q0 = 0; __ballot(4u * q0 <= count) != 0; q0 += 8u) {
+            // 8 chunks of every row; those past it and rows past n repeat others
+            vuint4 c[8];
+            const uint32_t at = q0 + (lane & 7u) < W4 ? q0 + (lane & 7u) : W4 - 1u;
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const uint32_t r = row0 + 8u * k + (lane >> 3);
+                c[k] = reinterpret_cast<const vuint4*>(lists + (size_t)(r < n ? r : n - 1u) * W)[at];
+            }
+            wave_lds_sync();  // the previous block has been read
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) reinterpret_cast<vuint4*>(stage)[(8u * k + (lane >> 3)) * 9u + (lane & 7u)] = c[k];
+            wave_lds_sync();
+            const uint4* L = stage + lane * 9u;
+            if (q0 == 0u && i < n) count = L[0].x < K ? L[0].x : K;
+            for (uint32_t q = q0; i < n && q < q0 + 8u && 4u * q <= count; q += 2) {
+                const uint4 a = L[q - q0], b = L[4u * (q + 1u) <= count ? q + 1u - q0 : q - q0];
                 uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
                 const uint32_t mask = octet_mask(jj, q, count, i, n);
                 f(4u * q, jj, mask);
             }
         }
-        return count;
+        return i < n ? count : 0u;
     }
-    const uint4 w0 = L[0];
-    const uint32_t count = w0.x < K ? w0.x : K;
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    if (ROWS == kRowPairs) {
-        for (uint32_t q = 0; 4u * q <= count; q += 2) {
-            const uint4 a = q == 0 ? w0 : L[q];
-            const uint4 b = (4u * (q + 1) <= count) ? L[q + 1] : z;
-            uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-            const uint32_t mask = octet_mask(jj, q, count, i, n);
-            f(4u * q, jj, mask);
-        }
-        return count;
-    }
-    uint4 a = w0, b = 4u <= count ? L[1] : z;
+    stage_rows(stage, lists, W, row0, lane, n);
+    if (i >= n) return 0u;
+    const uint4* L = stage + lane * (W / 4u);
+    const uint32_t head = L[0].x, count = head < K ? head : K;
     for (uint32_t q = 0; 4u * q <= count; q += 2) {
-        // the next pair of words loads while this octet's gathers are in flight
-        const uint4 na = 4u * (q + 2) <= count ? L[q + 2] : z;
-        const uint4 nb = 4u * (q + 3) <= count ? L[q + 3] : z;
+        const uint4 a = L[q], b = L[4u * (q + 1u) <= count ? q + 1u : q];
         uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         const uint32_t mask = octet_mask(jj, q, count, i, n);
         f(4u * q, jj, mask);
-        a = na;
-        b = nb;
     }
     return count;
 }

@@ -32,28 +32,28 @@ namespace {
 // f + (mean of the listed neighbours' features - f) * rate, the mean over the
 // list's count; the entries are visited eight at a time with their ID and
 // feature gathers in flight together and summed in list order.
-__device__ __forceinline__ float4 feature_update(uint32_t W, float rate, uint32_t n, const uint2* __restrict__ hash,
-                                                 const uint32_t* __restrict__ lists, const float4* __restrict__ fin,
-                                                 uint32_t i, uint32_t id) {
+// walk(fn) visits the agent's list.
+template <class Walk>
+__device__ __forceinline__ float4 feature_update(float rate, uint32_t n, const uint2* __restrict__ hash,
+                                                 const float4* __restrict__ fin, uint32_t id, Walk&& walk) {
     const float4 f = fin[id];
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t count =
-        for_list_octets(lists, W, W - 1u, i, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
-            uint32_t jid[8];
+    const uint32_t count = walk([&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+        uint32_t jid[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) jid[k] = hash[jj[k]].y;
-            float4 q[8];
+        for (int k = 0; k < 8; ++k) jid[k] = hash[jj[k]].y;
+        float4 q[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) q[k] = fin[jid[k] < n ? jid[k] : id];
+        for (int k = 0; k < 8; ++k) q[k] = fin[jid[k] < n ? jid[k] : id];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (((mask >> k) & 1u) == 0u || jid[k] >= n) continue;
-                s.x = s.x + q[k].x;
-                s.y = s.y + q[k].y;
-                s.z = s.z + q[k].z;
-                s.w = s.w + q[k].w;
-            }
-        });
+        for (int k = 0; k < 8; ++k) {
+            if (((mask >> k) & 1u) == 0u || jid[k] >= n) continue;
+            s.x = s.x + q[k].x;
+            s.y = s.y + q[k].y;
+            s.z = s.z + q[k].z;
+            s.w = s.w + q[k].w;
+        }
+    });
     if (count == 0) return f;
     const float inv = 1.0f / (float)count;  // cutil float4 / float
     float4 r;
@@ -66,12 +66,16 @@ __device__ __forceinline__ float4 feature_update(uint32_t W, float rate, uint32_
 
 __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32_t n, const uint2* __restrict__ hash,
                                                   const uint32_t* __restrict__ lists,
-                                                  const float4* __restrict__ fin, float4* __restrict__ fout) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = hash[i].y;
-    if (id >= n) return;
-    fout[id] = feature_update(W, rate, n, hash, lists, fin, i, id);
+                                                  const float4* __restrict__ fin, float4* __restrict__ fout,
+                                                  uint32_t xcd_remap) {
+    __shared__ uint4 s_stage[4][kStageChunks];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t id = i < n ? hash[i].y : n;
+    const float4 f = feature_update(rate, n, hash, fin, id < n ? id : 0u, [&](auto&& fn) {
+        return wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, fn);
+    });
+    if (id < n) fout[id] = f;
 }
 
 // FEAT: the same pass also writes the agent's feature update (the result of
@@ -90,14 +94,17 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
                                                float feature_rate = 0.0f, const float4* __restrict__ fin = nullptr,
                                                float4* __restrict__ fout = nullptr,
                                                const float4* __restrict__ sfeat = nullptr) {
+    __shared__ uint4 s_stage[FEAT ? 1 : 4][FEAT ? 1 : kStageChunks];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t id = hash[i].y;
-    if (id >= n) return;
-    const float4 P = spos[i];
-    const float4 Fw = sfwd[i];
+    const uint32_t at = i < n ? i : n - 1u;
+    const uint32_t id = i < n ? hash[i].y : n;
+    if (FEAT && id >= n) return;
+    const float4 P = spos[at];
+    const float4 Fw = sfwd[at];
     // no sorted copy of the smoothed acceleration: the agent's own, by ID
-    const float4 SA = ssa ? ssa[i] : (APPLY ? o.sa_out[id] : make_float4(0.f, 0.f, 0.f, 0.f));
+    float4 SA = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (APPLY && id < n) SA = ssa ? ssa[at] : o.sa_out[id];
     const V3 myPos = xyz(P);
     const V3 myFwd = xyz(Fw);
 
@@ -113,10 +120,9 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
     uint32_t count = 0;
     if (any) {
         // the list in order, eight entries at a time with their gathers in flight;
-        // the feature variants hold four more gathers per entry and read the
-        // row in pairs (whole K 32 rows: 213 -> 162 us for the two-kernel
-        // step's steering on 1M blobs, 185 -> 117 us for the behaviour forces)
-        count = for_list_octets<FEAT ? kRowPairs : kRowWhole>(lists, W, W - 1u, i, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+        // the feature variants hold four more gathers per entry and load the
+        // next words after them (K 64: 3 % faster than ahead)
+        auto visit = [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
             float4 qp[8], qf[8], fq[8];
             uint32_t jid[8];
 #pragma unroll
@@ -147,11 +153,16 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
                     fsum.w = fsum.w + fq[t].w;
                 }
             }
-        });
+        };
+        if (FEAT)
+            count = for_list_octets<false>(lists, W, W - 1u, i, n, visit);
+        else
+            count = wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, visit);
     }
     if (FEAT) {
         if (!any) {
-            fout[id] = feature_update(W, feature_rate, n, hash, lists, fin, i, id);
+            fout[id] = feature_update(feature_rate, n, hash, fin, id,
+                                      [&](auto&& fn) { return for_list_octets(lists, W, W - 1u, i, n, fn); });
         } else {
             const float4 f = SFEAT ? sfeat[i] : fin[id];
             float4 r = f;
@@ -165,6 +176,7 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
             fout[id] = r;
         }
     }
+    if (id >= n) return;
     if (APPLY) {
         finish_agent(g, sp, wts, dt, step, i, id, id, myPos, myFwd, Fw.w, xyz(SA), SA.w, acc, o);
     } else {
@@ -264,9 +276,9 @@ hipError_t launch_apply(const brt_grid_params& g, const brt_steer_params& sp, fl
 }
 
 hipError_t launch_features(uint32_t K, float rate, uint32_t n, const uint2* hash, const uint32_t* lists,
-                           const float4* fin, float4* fout, hipStream_t s) {
+                           const float4* fin, float4* fout, uint32_t xcd_remap, hipStream_t s) {
     BRT_LAUNCH(k_features, dim3((n + 255) / 256), dim3(256), 0, s, list_stride(K), rate, n, hash, lists, fin,
-                       fout);
+                       fout, xcd_remap);
     return hipGetLastError();
 }
 
