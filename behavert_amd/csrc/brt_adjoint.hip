@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
     constexpr int U = NL == 1 ? 4 : 2;  // entries of a lane in flight
     constexpr uint32_t T = (uint32_t)(NL * U);
     __shared__ float s_red[3][4];
-    const uint32_t t0 = xcd_block(a.xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t t0 = xcd_block(a.xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t i = t0 / (uint32_t)NL, l = t0 % (uint32_t)NL;
     float wg[3] = {0.f, 0.f, 0.f};
     const brt_steer_params& sp = a.sp;

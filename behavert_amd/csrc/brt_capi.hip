@@ -904,7 +904,40 @@ struct StepScratch {
     uint32_t* meta;
     void* tmp;
     float* xyz;
+    size_t tmp_bytes;
 };
+
+// Two-pass steps of this many agents or more, with the feature update, wander or
+// the sorted smoothed acceleration, move the state by ID as 64-byte records: an
+// access by ID costs the same for 16 bytes as for 64 (about 45 G a second reach
+// memory), and with these options a step makes eight or more per agent.  K 64, one
+// agent per cell, arrays -> records, us a step with features, targets and wander:
+// 262,144 agents 136 -> 137, 524,288 219 -> 209, 1,048,576 468 -> 414, 4,194,304
+// 1799 -> 1539; with none of them 524,288 181 -> 191, 4,194,304 1473 -> 1480.
+#ifndef BRT_STEP_RECORDS_MIN
+#define BRT_STEP_RECORDS_MIN (1u << 19)
+#endif
+
+// What a two-pass step keeps in its tmp scratch after the sort.
+struct StepTmp {
+    size_t features = 0, records = 0, ssa = 0, bytes = 0;  // byte offsets, and the whole
+    bool use_records = false;
+};
+StepTmp step_tmp(uint32_t n, bool two_pass, bool features, bool own_ssa, bool wander) {
+    StepTmp t;
+    if (!two_pass) return t;
+    if (features) t.bytes = (size_t)n * 16u;
+    t.use_records = n >= BRT_STEP_RECORDS_MIN && (features || own_ssa || wander);
+    if (t.use_records) {
+        t.records = (t.bytes + 63u) / 64u * 64u;
+        t.bytes = t.records + (size_t)n * 64u;
+        if (!own_ssa) {
+            t.ssa = t.bytes;
+            t.bytes += (size_t)n * 16u;
+        }
+    }
+    return t;
+}
 
 int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_params* prox,
               const brt_steer_params* steer, float feature_rate, float dt, uint32_t step,
@@ -974,7 +1007,9 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // call of the same size may take (another grid), under capture too
     const bool cell_sort = brt::cell_sort_cells(n, grid->num_cells) != 0u;
     if (!given && cell_sort && (rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells)))) return rc;
-    if (!given && sorted_features && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    StepTmp st = step_tmp(n, two_pass, sorted_features, b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f);
+    if (given && given->tmp_bytes < st.bytes) st.use_records = false;
+    if (!given && (rc = ensure_tmp(ctx, st.bytes))) return rc;
     // with LDS lists the neighbour scan reads candidate positions from a
     // packed x,y,z copy written by the reorder (three 16-byte loads per four
     // candidates; the register-list scan measured no gain from it)
@@ -1010,9 +1045,13 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     f.out[nf++] = reinterpret_cast<float4*>(b->sorted_pos);
     f.in[nf] = reinterpret_cast<const float4*>(b->forward);
     f.out[nf++] = reinterpret_cast<float4*>(b->sorted_forward);
-    if (b->sorted_smooth_accel) {
+    // with records the smoothed acceleration comes with the rest of the record
+    float* const ssa = b->sorted_smooth_accel
+                           ? b->sorted_smooth_accel
+                           : (st.use_records ? reinterpret_cast<float*>((char*)tmp + st.ssa) : nullptr);
+    if (ssa) {
         f.in[nf] = reinterpret_cast<const float4*>(b->smooth_accel);
-        f.out[nf++] = reinterpret_cast<float4*>(b->sorted_smooth_accel);
+        f.out[nf++] = reinterpret_cast<float4*>(ssa);
     }
     if (sorted_features) {
         f.in[nf] = reinterpret_cast<const float4*>(b->features);
@@ -1021,6 +1060,14 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     f.count = nf;
     f.xyz0 = xyz;
     mark_phase(1);
+    float4* const rec = st.use_records ? reinterpret_cast<float4*>((char*)tmp + st.records) : nullptr;
+    if (rec && !cell_sort) {
+        const hipEvent_t stop = brt::launch_mark().stop;
+        brt::launch_mark().stop = nullptr;
+        BRT_HIP(brt::launch_pack(n, f.in[0], f.in[1], f.in[2], nf > 3u ? f.in[3] : nullptr, rec, s), "k_pack");
+        brt::launch_mark().stop = stop;
+        f.records = rec;
+    }
     if (cell_sort) {
         BRT_HIP(brt::launch_cell_sort(b->lists, n, grid->num_cells, reinterpret_cast<uint2*>(b->hash), f,
                                       b->cell_start, b->cell_end, s),
@@ -1060,14 +1107,14 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
         BRT_HIP(brt::launch_steer(*grid, prox->max_neighbors, *steer, dt, step, n,
                                   reinterpret_cast<const float4*>(b->sorted_pos),
                                   reinterpret_cast<const float4*>(b->sorted_forward),
-                                  reinterpret_cast<const float4*>(b->sorted_smooth_accel),
+                                  reinterpret_cast<const float4*>(ssa),
                                   reinterpret_cast<const uint2*>(b->hash), b->lists,
                                   reinterpret_cast<float2*>(b->wander), reinterpret_cast<float4*>(b->pos),
                                   reinterpret_cast<float4*>(b->forward), reinterpret_cast<float4*>(b->smooth_accel),
                                   nullptr, ctx->xcd_remap, s, feature_rate,
                                   do_features ? reinterpret_cast<const float4*>(b->features) : nullptr,
                                   do_features ? reinterpret_cast<float4*>(b->features_out) : nullptr,
-                                  sorted_features ? reinterpret_cast<const float4*>(tmp) : nullptr),
+                                  sorted_features ? reinterpret_cast<const float4*>(tmp) : nullptr, rec),
                 "k_steer");
         do_features = false;
     }
@@ -1132,7 +1179,10 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
         !prox->use_knn && (resolve_lds_lists(ctx, prox) != 0u || resolve_quads(ctx, prox, n, !two_pass));
     int rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells));
     if (rc) return rc;
-    if (do_features && two_pass && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    if ((rc = ensure_tmp(ctx, step_tmp(n, two_pass, do_features && two_pass,
+                                       b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f)
+                                  .bytes)))
+        return rc;
     if (pack && (rc = ensure_xyz(ctx, n))) return rc;
     if (!ctx->cap_stream)
         BRT_HIP(hipStreamCreateWithFlags(&ctx->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
@@ -1140,7 +1190,7 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
         destroy_step_graph(ctx->graphs.front());
         ctx->graphs.erase(ctx->graphs.begin());
     }
-    StepScratch sc{ctx->meta, ctx->tmp, ctx->xyz};
+    StepScratch sc{ctx->meta, ctx->tmp, ctx->xyz, ctx->tmp_bytes};
     BRT_HIP(hipStreamBeginCapture(ctx->cap_stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     rc = step_core(ctx, grid, prox, steer, feature_rate, dt, step, b, ctx->cap_stream, &sc);
     hipGraph_t g = nullptr;
@@ -1221,6 +1271,7 @@ int brt_step_noalloc(brt_context* ctx, const brt_grid_params* grid, const brt_pr
     sc.meta = reinterpret_cast<uint32_t*>(base + kNoAllocMetaOffset);
     sc.tmp = base + kNoAllocTmpOffset;
     sc.xyz = reinterpret_cast<float*>(base + kNoAllocXyzOffset);
+    sc.tmp_bytes = (size_t)BRT_NOALLOC_MAX_AGENTS * 16u;
     return step_core(ctx, grid, prox, steer, feature_rate, dt, step, b, stream, &sc);
 }
 

@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
                                                          const float4* __restrict__ stats_in,
                                                          float4* __restrict__ stats_out, float* __restrict__ sims,
                                                          uint32_t vec, uint32_t xcd_remap) {
-    const uint32_t blk = xcd_block(xcd_remap != 0);
+    const uint32_t blk = xcd_block(xcd_remap);
     const uint32_t i = blk * blockDim.x + threadIdx.x;
     if (i < n) similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out,
                                               bc_rows + (size_t)threadIdx.x * (K + 1u));
@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     constexpr int G = NR == 1 ? 4 : (NR == 2 ? 2 : 1);  // entries in flight
     const uint32_t lane = threadIdx.x & 63u, l = lane & 3u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t row0 = xcd_block(xcd_remap != 0) * blockDim.x + wave * 64u;
+    const uint32_t row0 = xcd_block(xcd_remap) * blockDim.x + wave * 64u;
     if (row0 >= n) return;
     const uint32_t i = row0 + lane, at = i < n ? i : n - 1u;
     char* const mem = reinterpret_cast<char*>(bc_rows) + (size_t)wave * wave_bytes;
@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
                                                           uint32_t xcd_remap) {
     __shared__ uint4 s_stage[4][kStageChunks];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
     const float4 P = spos[at], Fw = sfwd[at];
     const V3 myPos = xyz(P), myFwd = xyz(Fw);
@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(256) k_lp_iterate(uint32_t K, uint32_t W, uint
                                                     uint32_t xcd_remap) {
     __shared__ uint4 s_stage[SCAN ? 4 : 1][SCAN ? kStageChunks : 1];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x, at = i < n ? i : n - 1u;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x, at = i < n ? i : n - 1u;
     float mn = FIRST ? (float)i : lbl_in[at];
     // the last iteration's reads by ID load during the walk
     uint32_t id = n;
@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float 
                                                   uint32_t xcd_remap) {
     __shared__ uint4 s_stage[4][kStageChunks];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t id = i < n ? hash[i].y : n;
     const float4 own = lbl[i < n ? i : n - 1u];
     const float my = own.w;

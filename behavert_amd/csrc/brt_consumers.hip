@@ -32,7 +32,7 @@ __global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_
                                                     uint32_t xcd_remap) {
     __shared__ uint4 s_stage[4][kStageChunks];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
     const float4 P = spos[at], Fw = sfwd[at];
     const V3 myPos = xyz(P), myFwd = xyz(Fw);

@@ -754,6 +754,39 @@ __global__ void __launch_bounds__(256) k_reorder_ranges(const uint2* __restrict_
     }
 }
 
+// k_reorder_ranges from records of four float4 by ID (k_pack's), one lane per
+// part: the four lanes of an agent read its 64 bytes together.
+__global__ void __launch_bounds__(256) k_reorder_records(const uint2* __restrict__ hash, uint32_t n,
+                                                         const float4* __restrict__ rec, ReorderArgs f,
+                                                         uint32_t num_cells, uint32_t* __restrict__ cell_start,
+                                                         uint32_t* __restrict__ cell_end, SortCleanup cleanup) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t >> 2, p = t & 3u;
+    if (cleanup.hist) {
+        const uint32_t stride = gridDim.x * blockDim.x;
+        for (uint32_t w = t; w < cleanup.status_words; w += stride) cleanup.status[w] = 0u;
+        for (uint32_t w = t; w < kHistCopies * kRadix; w += stride)
+            cleanup.hist[(w / kRadix) * kHistWords + (w % kRadix)] = 0u;
+        if (t == 0) *cleanup.counter = 0u;
+    }
+    if (i >= n) return;
+    const uint2 h = hash[i];
+    if (p < f.count && h.y < n) {
+        const float4 v = rec[4u * (size_t)h.y + p];
+        float4* const out = p == 0u ? f.out[0] : (p == 1u ? f.out[1] : (p == 2u ? f.out[2] : f.out[3]));
+        out[i] = v;
+        if (p == 0u && f.xyz0) {
+            float* d = f.xyz0 + 3u * (size_t)i;
+            d[0] = v.x;
+            d[1] = v.y;
+            d[2] = v.z;
+        }
+    }
+    if (p == 3u && h.x < num_cells) {
+        if (i == 0 || hash[i - 1].x != h.x) cell_start[h.x] = i;
+        if (i == n - 1 || hash[i + 1].x != h.x) cell_end[h.x] = i + 1;
+    }
+}
+
 // Workgroups of the histogram kernels: each adds its per-workgroup histograms
 // of every pass into one of the kHistCopies global copies, one atomic per
 // nonzero bin.  With a single copy the contended atomics set the kernel's time
@@ -899,6 +932,11 @@ hipError_t launch_reorder_ranges(const uint2* hash, uint32_t n, const ReorderArg
     if (c.hist && work < kHistCopies * kRadix) work = kHistCopies * kRadix;
     uint32_t grid = (work + 255) / 256;
     if (grid == 0) return hipSuccess;
+    if (f.records) {
+        BRT_LAUNCH(k_reorder_records, dim3((unsigned)(((size_t)n * 4u + 255u) / 256u)), dim3(256), 0, s, hash, n,
+                   f.records, f, num_cells, cell_start, cell_end, c);
+        return hipGetLastError();
+    }
     BRT_LAUNCH(k_reorder_ranges, dim3(grid), dim3(256), 0, s, hash, n, f, num_cells, cell_start, cell_end, c);
     return hipGetLastError();
 }

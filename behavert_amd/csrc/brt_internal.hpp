@@ -83,6 +83,9 @@ struct ReorderArgs {
     float4* out[kMaxReorderFeatures];
     uint32_t count;
     float* xyz0;  // optional: feature 0's x,y,z packed, 12 bytes per agent
+    // optional (launch_reorder_ranges with cell arrays): records of four float4 by ID
+    // in the place of in[]
+    const float4* records = nullptr;
 };
 // The sort metadata a finished sort leaves nonzero: the last pass's histogram
 // slice (every copy), tile counter and status words.  A reorder launched right
@@ -142,7 +145,12 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
                         const uint32_t* lists, float2* wander, float4* pos_out, float4* fwd_out, float4* sa_out,
                         float4* force_out, uint32_t xcd_remap, hipStream_t s, float feature_rate = 0.0f,
                         const float4* features_in = nullptr, float4* features_out = nullptr,
-                        const float4* sorted_features = nullptr);
+                        const float4* sorted_features = nullptr, float4* records = nullptr);
+// records (optional, 4 float4 per agent, with features_in only where sorted_features
+// are there): scratch through which the new state goes to the arrays; ssa != NULL.
+// launch_pack: up to four float4 arrays (NULL: left out) into such records.
+hipError_t launch_pack(uint32_t n, const float4* a, const float4* b, const float4* c, const float4* d, float4* rec,
+                       hipStream_t s);
 hipError_t launch_features(uint32_t K, float rate, uint32_t n, const uint2* hash, const uint32_t* lists,
                            const float4* fin, float4* fout, uint32_t xcd_remap, hipStream_t s);
 // the decomposed steering sequence: behaviour forces only, then the integrator
@@ -195,6 +203,8 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
                           const float4* gsa_out, float4* gpos_in, float4* gfwd_in, float4* gsa_in, float4* scratch,
                           float* partials, float* weight_grad, uint32_t xcd_remap, hipStream_t s);
 
+// Agents from which the passes with long rows map runs of workgroups to the XCDs.
+constexpr uint32_t kXcdRunMin = 1u << 21;
 inline uint32_t list_stride(uint32_t K) { return 4u * (K / 4u + 1u); }
 // LDS of a workgroup of the four-lane neighbour kernels (64 list rows and, when
 // the steering is fused, an agent's three sums and their counts: an odd number

@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32
                                                   uint32_t xcd_remap) {
     __shared__ uint4 s_stage[4][kStageChunks];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t id = i < n ? hash[i].y : n;
     const float4 f = feature_update(rate, n, hash, fin, id < n ? id : 0u, [&](auto&& fn) {
         return wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, fn);
@@ -84,7 +84,10 @@ __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32
 // SFEAT: the neighbours' features are read from sfeat, the features in sorted
 // order (sfeat[j] = fin[hash[j].y], gathered with the state), so the walk reads
 // them next to their positions instead of at random agent IDs.
-template <bool APPLY, bool FEAT = false, bool SFEAT = false>
+// REC: the new state (and feature) goes to one 64-byte record by ID instead of
+// to the arrays: a write to a random ID costs the same whatever its size (about
+// 45 G a second), and k_unpack moves the records to the arrays in order.
+template <bool APPLY, bool FEAT = false, bool SFEAT = false, bool REC = false>
 __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, brt_steer_params sp, SteerCuts cuts,
                                                float dt,
                                                uint32_t step, uint32_t n, const float4* __restrict__ spos,
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
                                                const float4* __restrict__ sfeat = nullptr) {
     __shared__ uint4 s_stage[FEAT ? 1 : 4][FEAT ? 1 : kStageChunks];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap != 0) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
     const uint32_t id = i < n ? hash[i].y : n;
     if (FEAT && id >= n) return;
@@ -159,9 +162,10 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
         else
             count = wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, visit);
     }
+    float4 feature = make_float4(0.f, 0.f, 0.f, 0.f);
     if (FEAT) {
         if (!any) {
-            fout[id] = feature_update(feature_rate, n, hash, fin, id,
+            feature = feature_update(feature_rate, n, hash, fin, id,
                                       [&](auto&& fn) { return for_list_octets(lists, W, W - 1u, i, n, fn); });
         } else {
             const float4 f = SFEAT ? sfeat[i] : fin[id];
@@ -173,16 +177,55 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
                 r.z = f.z + (fsum.z * inv - f.z) * feature_rate;
                 r.w = f.w + (fsum.w * inv - f.w) * feature_rate;
             }
-            fout[id] = r;
+            feature = r;
         }
+        if (!REC) fout[id] = feature;
     }
     if (id >= n) return;
+    if (APPLY && REC) {
+        float2 wander = make_float2(0.f, 0.f);
+        const V3 f = behaviour_force(sp, wts, dt, step, id, id, myPos, myFwd, Fw.w, acc, o.wander, &wander);
+        const NewState s = integrate(g, sp, dt, i, f, myPos, myFwd, Fw.w, xyz(SA), nullptr);
+        float4* const rec = o.rec + 4u * (size_t)id;
+        rec[0] = make_float4(s.pos.x, s.pos.y, s.pos.z, wander.x);
+        rec[1] = make_float4(s.fwd.x, s.fwd.y, s.fwd.z, s.speed);
+        rec[2] = make_float4(s.sa.x, s.sa.y, s.sa.z, wander.y);
+        rec[3] = feature;  // without features too: whole 64 bytes
+        return;
+    }
     if (APPLY) {
         finish_agent(g, sp, wts, dt, step, i, id, id, myPos, myFwd, Fw.w, xyz(SA), SA.w, acc, o);
     } else {
-        const V3 f = behaviour_force(sp, wts, dt, step, id, id, myPos, myFwd, Fw.w, acc, o.wander);
+        const V3 f = behaviour_force(sp, wts, dt, step, id, id, myPos, myFwd, Fw.w, acc, o.wander, o.wander + id);
         o.force_out[i] = make_float4(f.x, f.y, f.z, 0.0f);
     }
+}
+
+// Four state arrays (float4 by ID) into one 64-byte record per agent, so that a
+// gather by ID reads one of them: one lane per part.
+__global__ void __launch_bounds__(256) k_pack(uint32_t n, const float4* __restrict__ a, const float4* __restrict__ b,
+                                              const float4* __restrict__ c, const float4* __restrict__ d,
+                                              float4* __restrict__ rec) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t >> 2, p = t & 3u;
+    if (i >= n) return;
+    const float4* const src = p == 0u ? a : (p == 1u ? b : (p == 2u ? c : d));
+    if (src) rec[t] = src[i];
+}
+
+// k_steer's records to the arrays (feature and wander optional; the smoothed
+// acceleration keeps its fourth component).
+__global__ void __launch_bounds__(256) k_unpack(uint32_t n, const float4* __restrict__ rec, AgentOut o,
+                                                float4* __restrict__ feature) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t >> 2, p = t & 3u;
+    if (i >= n) return;
+    if (p == 3u && !feature) return;
+    float4 v = rec[t];
+    const float extra = v.w;
+    if (p == 0u) v.w = 1.0f;
+    if (p == 2u) v.w = o.sa_out[i].w;
+    float4* const dst = p == 0u ? o.pos_out : (p == 1u ? o.fwd_out : (p == 2u ? o.sa_out : feature));
+    dst[i] = v;
+    if (o.wander && (p & 1u) == 0u) reinterpret_cast<float*>(o.wander)[2u * (size_t)i + (p >> 1)] = extra;
 }
 
 // applySteeringForces from an accumulated force (sorted float4): the world-centre
@@ -237,9 +280,30 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
                         uint32_t n, const float4* spos, const float4* sfwd, const float4* ssa, const uint2* hash,
                         const uint32_t* lists, float2* wander, float4* pos_out, float4* fwd_out, float4* sa_out,
                         float4* force_out, uint32_t xcd_remap, hipStream_t s, float feature_rate,
-                        const float4* features_in, float4* features_out, const float4* sorted_features) {
+                        const float4* features_in, float4* features_out, const float4* sorted_features,
+                        float4* records) {
     AgentOut o{pos_out, fwd_out, sa_out, force_out, wander};
     const SteerCuts cuts = steer_cuts(sp);
+    if (K > 32u && n >= kXcdRunMin && xcd_remap) xcd_remap = 2u;  // as the list pass before it
+    if (records) {
+        o.rec = records;
+        // the phase's events: the first kernel's start, the second's end
+        const hipEvent_t stop = launch_mark().stop;
+        launch_mark().stop = nullptr;
+        if (features_in)
+            BRT_LAUNCH((k_steer<true, true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
+                       sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
+                       features_out, sorted_features);
+        else
+            BRT_LAUNCH((k_steer<true, false, false, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
+                       sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr,
+                       nullptr);
+        o.wander = sp.wander_weight != 0.0f ? wander : nullptr;
+        launch_mark().stop = stop;
+        BRT_LAUNCH(k_unpack, dim3((unsigned)(((size_t)n * 4u + 255u) / 256u)), dim3(256), 0, s, n, records, o,
+                   features_in ? features_out : nullptr);
+        return hipGetLastError();
+    }
     if (features_in && sorted_features)
         BRT_LAUNCH((k_steer<true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp,
                            cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
@@ -252,6 +316,12 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
         BRT_LAUNCH((k_steer<true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt,
                            step,
                            n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack(uint32_t n, const float4* a, const float4* b, const float4* c, const float4* d, float4* rec,
+                       hipStream_t s) {
+    BRT_LAUNCH(k_pack, dim3((unsigned)(((size_t)n * 4u + 255u) / 256u)), dim3(256), 0, s, n, a, b, c, d, rec);
     return hipGetLastError();
 }
 

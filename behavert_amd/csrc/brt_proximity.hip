@@ -979,7 +979,7 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t blk = xcd_block(a.xcd_remap != 0);
+    const uint32_t blk = xcd_block(a.xcd_remap);
     const uint32_t gw = blk * (blockDim.x >> 6) + wid;
     Seg sg;
     const bool wave_live = wave_segment<BATCH>(a, gw, sg);
@@ -1382,7 +1382,7 @@ __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l = tid & 3u;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     Seg sg;
-    wave_segment<false>(a, xcd_block(a.xcd_remap != 0), sg);
+    wave_segment<false>(a, xcd_block(a.xcd_remap), sg);
     const uint32_t base = sg.row0;  // the workgroup's first agent
     sg.row0 += 16u * wid;
     Lane L;
@@ -1700,7 +1700,7 @@ __device__ __forceinline__ void knn_scan(const ProxArgs& a, const Seg& sg, const
 __global__ void __launch_bounds__(64) k_neighbors_knn(ProxArgs a) {
     extern __shared__ uint32_t s_mem[];
     const uint32_t B = blockDim.x, lane = threadIdx.x;
-    const uint32_t blk = xcd_block(a.xcd_remap != 0);
+    const uint32_t blk = xcd_block(a.xcd_remap);
     Seg sg;
     sg.g = a.g;
     sg.slack[0] = a.slack[0];
@@ -1818,8 +1818,10 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
     if (quads && launch_quad<false>(a, s)) return hipGetLastError();
     if (lds_lists)
         BRT_LAUNCH((k_prox<false, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
-    else
+    else {
+        if (n >= kXcdRunMin && a.xcd_remap) a.xcd_remap = 2u;
         BRT_LAUNCH((k_prox<false, false, false>), dim3((n + 255) / 256), dim3(256), 256u * kHeadWords * 4u, s, a);
+    }
     return hipGetLastError();
 }
 

@@ -141,6 +141,7 @@ struct AgentOut {
     float4* sa_out;
     float4* force_out;  // sorted, optional
     float2* wander;     // by ID, in/out, optional
+    float4* rec = nullptr;  // k_steer with records: the new state as one record per ID (see k_unpack)
 };
 
 // The behaviour forces in the reference's accumulation order (each term added
@@ -150,7 +151,7 @@ struct AgentOut {
 // to id outside batches) picks the seek target and keys the wander stream.
 __device__ __forceinline__ V3 behaviour_force(const brt_steer_params& sp, Weights w, float dt, uint32_t step,
                                               uint32_t id, uint32_t lid, V3 myPos, V3 myFwd, float mySpeed,
-                                              const SteerAccum& acc, float2* wander) {
+                                              const SteerAccum& acc, const float2* wander, float2* wander_out) {
     V3 force = v3(0.f, 0.f, 0.f);
     if (w.s != 0.0f) {
         V3 s = acc.nSep > 0 ? normalize(acc.sSep / (float)acc.nSep) : acc.sSep;
@@ -179,7 +180,7 @@ __device__ __forceinline__ V3 behaviour_force(const brt_steer_params& sp, Weight
         ws = ws < -1.0f ? -1.0f : (ws > 1.0f ? 1.0f : ws);
         float wu = wsu.y + ((u1 * 2.0f - 1.0f) * walk);
         wu = wu < -1.0f ? -1.0f : (wu > 1.0f ? 1.0f : wu);
-        wander[id] = make_float2(ws, wu);
+        *wander_out = make_float2(ws, wu);
         // OpenSteer's right-handed local space (LocalSpace.h:277-305) with the
         // world up (0,1,0) as the previous up: side = normalize(forward x up),
         // up = side x forward.  A heading along the world up has no such side;
@@ -193,12 +194,17 @@ __device__ __forceinline__ V3 behaviour_force(const brt_steer_params& sp, Weight
     return force;
 }
 
-// computeSeekingsWorldCenter (added last), then applySteeringForceSingle, then
-// the scatter of the new state to agent-ID order.  force_out (sorted, optional)
-// receives the summed force before the integrator.
-__device__ __forceinline__ void apply_force(const brt_grid_params& g, const brt_steer_params& sp, float dt,
-                                            uint32_t i, uint32_t id, V3 force, V3 myPos, V3 myFwd, float mySpeed,
-                                            V3 mySa, float saW, const AgentOut& o) {
+// An agent's state after the integrator.
+struct NewState {
+    V3 pos, fwd, sa;
+    float speed;
+};
+
+// computeSeekingsWorldCenter (added last), then applySteeringForceSingle.
+// force_out (sorted, optional) receives the summed force before the integrator.
+__device__ __forceinline__ NewState integrate(const brt_grid_params& g, const brt_steer_params& sp, float dt,
+                                              uint32_t i, V3 force, V3 myPos, V3 myFwd, float mySpeed, V3 mySa,
+                                              float4* force_out) {
     if (sp.seek_world_center) {
         const float cx = g.world_center[0], cy = g.world_center[1], cz = g.world_center[2];
         const float rx = g.world_radius[0], ry = g.world_radius[1], rz = g.world_radius[2];
@@ -207,7 +213,7 @@ __device__ __forceinline__ void apply_force(const brt_grid_params& g, const brt_
         V3 s = inside ? v3(0.f, 0.f, 0.f) : steerForSeek(myPos, mySpeed, myFwd, v3(cx, cy, cz), sp.max_speed);
         force = s + force;
     }
-    if (o.force_out) o.force_out[i] = make_float4(force.x, force.y, force.z, 0.0f);
+    if (force_out) force_out[i] = make_float4(force.x, force.y, force.z, 0.0f);
 
     if (sp.use_2d_projection) force.y = 0.0f;
     const V3 adjusted = adjustRawSteeringForce(force, mySpeed, myFwd, sp.max_speed);
@@ -225,10 +231,17 @@ __device__ __forceinline__ void apply_force(const brt_grid_params& g, const brt_
     if (sp.use_2d_projection) newVel.y = 0.0f;
     const V3 newFwd = normalize(newVel);
     if (sp.use_2d_projection) newPos.y = 0.5f;
+    return NewState{newPos, newFwd, mySa, mySpeed};
+}
 
-    o.pos_out[id] = make_float4(newPos.x, newPos.y, newPos.z, 1.0f);
-    o.sa_out[id] = make_float4(mySa.x, mySa.y, mySa.z, saW);
-    o.fwd_out[id] = make_float4(newFwd.x, newFwd.y, newFwd.z, mySpeed);
+// The integrator, then the scatter of the new state to agent-ID order.
+__device__ __forceinline__ void apply_force(const brt_grid_params& g, const brt_steer_params& sp, float dt,
+                                            uint32_t i, uint32_t id, V3 force, V3 myPos, V3 myFwd, float mySpeed,
+                                            V3 mySa, float saW, const AgentOut& o) {
+    const NewState s = integrate(g, sp, dt, i, force, myPos, myFwd, mySpeed, mySa, o.force_out);
+    o.pos_out[id] = make_float4(s.pos.x, s.pos.y, s.pos.z, 1.0f);
+    o.sa_out[id] = make_float4(s.sa.x, s.sa.y, s.sa.z, saW);
+    o.fwd_out[id] = make_float4(s.fwd.x, s.fwd.y, s.fwd.z, s.speed);
 }
 
 // The whole per-agent tail of the steering pass.
@@ -236,7 +249,8 @@ __device__ __forceinline__ void finish_agent(const brt_grid_params& g, const brt
                                              float dt, uint32_t step, uint32_t i, uint32_t id, uint32_t lid,
                                              V3 myPos, V3 myFwd, float mySpeed, V3 mySa, float saW,
                                              const SteerAccum& acc, const AgentOut& o) {
-    const V3 force = behaviour_force(sp, w, dt, step, id, lid, myPos, myFwd, mySpeed, acc, o.wander);
+    const V3 force =
+        behaviour_force(sp, w, dt, step, id, lid, myPos, myFwd, mySpeed, acc, o.wander, o.wander + id);
     apply_force(g, sp, dt, i, id, force, myPos, myFwd, mySpeed, mySa, saW, o);
 }
 
