@@ -9,12 +9,12 @@
 //   s1 = |v|, p1 = p + v dt, f1 = normalize(v).
 // Given dL/d(p1, f1, s1, a1) by agent ID, two kernels produce dL/d(p, f, s, a)
 // by agent ID, with no atomics, so the same inputs always give the same bits:
-//   k_adjoint_own (one or four lanes per sorted agent i) recomputes agent i's
-//     forward values with the forward kernels' arithmetic, back-propagates
-//     through the integrator and its own behaviour sums, and stores by sorted
-//     index its own terms and a record of what its neighbours' terms are made
-//     of (position, heading, the separation, cohesion and alignment sums'
-//     adjoints, flags);
+//   k_adjoint_own (one lane per sorted agent i) or k_adjoint_own_quad (four)
+//     recomputes agent i's forward values with the forward kernels' arithmetic,
+//     back-propagates through the integrator and its own behaviour sums, and
+//     stores by sorted index its own terms and a record of what its neighbours'
+//     terms are made of (position, heading, the separation, cohesion and
+//     alignment sums' adjoints, flags);
 //   k_adjoint_gather (several lanes per sorted agent j) finds every agent i
 //     whose list holds j -- j's own list when that list can stand in for them
 //     (and the cells where agents below the grid are kept, for j on a low face),
@@ -163,290 +163,323 @@ __device__ __forceinline__ uint32_t quad_count(uint32_t v) {
     return v;
 }
 
-__device__ __forceinline__ float pick(uint32_t l, float v0, float v1, float v2, float v3) {
-    return l == 0u ? v0 : (l == 1u ? v1 : (l == 2u ? v2 : v3));
-}
-
 __device__ __forceinline__ V3 keep(V3 v, bool on) { return on ? v : v3(0.f, 0.f, 0.f); }
 
-// NL lanes per agent: with four, lane l takes the list entries l, l + 4, ..., the
-// sums add the four lanes' terms in list order (the same bits as one lane), and
-// every lane carries the integrator.  Small flocks are bound by one wave's chain
-// of list and neighbour loads (65,536 agents are one wave per SIMD with one lane
-// each), which four lanes shorten; larger ones by the arithmetic.
-template <int NL>
-__global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
-    constexpr int U = NL == 1 ? 4 : 2;  // entries of a lane in flight
-    constexpr uint32_t T = (uint32_t)(NL * U);
-    __shared__ float s_red[3][4];
-    const uint32_t t0 = xcd_block(a.xcd_remap) * blockDim.x + threadIdx.x;
-    const uint32_t i = t0 / (uint32_t)NL, l = t0 % (uint32_t)NL;
-    float wg[3] = {0.f, 0.f, 0.f};
+// An agent's adjoints before its neighbours' share, and the record's vectors.
+struct OwnBack {
+    V3 p, f, a, S, A, C;
+    float s;
+    uint32_t flags;
+    float wg[3];
+};
+
+// From the behaviour sums through the integrator and back to them; full: the
+// agent's list is full.
+__device__ __forceinline__ OwnBack own_backward(const AdjArgs& a, uint32_t id, float4 P, float4 Fw, float4 SA,
+                                                float4 gP, float4 gF, float4 gA, const SteerAccum& acc, bool full) {
     const brt_steer_params& sp = a.sp;
+    const V3 p = xyz(P), f = xyz(Fw), sa = xyz(SA);
+    const float s = Fw.w;
+    OwnBack r;
+    r.wg[0] = r.wg[1] = r.wg[2] = 0.0f;
+    V3 xs = v3(0.f, 0.f, 0.f), xa = xs, xc = xs, us = xs, ua = xs, uc = xs;
+    V3 F = v3(0.f, 0.f, 0.f);
+    if (sp.separation[0] != 0.0f) {
+        if (acc.nSep > 0) {
+            xs = acc.sSep / (float)acc.nSep;
+            us = normalize(xs);
+        }
+        F = us * sp.separation[0] + F;
+    }
+    if (sp.alignment[0] != 0.0f) {
+        if (acc.nAli > 0) {
+            xa = acc.sAli / (float)acc.nAli - f;
+            ua = normalize(xa);
+        }
+        F = ua * sp.alignment[0] + F;
+    }
+    if (sp.cohesion[0] != 0.0f) {
+        if (acc.nCoh > 0) {
+            xc = acc.sCoh / (float)acc.nCoh;
+            uc = normalize(xc);
+        }
+        F = uc * sp.cohesion[0] + F;
+    }
+    V3 tgt = v3(0.f, 0.f, 0.f), seekOff = tgt;
+    const bool doTarget = sp.num_targets > 0 && sp.target_weight != 0.0f;
+    if (doTarget) {
+        const float* t = sp.targets[id % sp.num_targets];
+        tgt = v3(t[0], t[1], t[2]);
+        seekOff = tgt - p;
+        F = steerForSeek(p, s, f, tgt, sp.max_speed) * sp.target_weight + F;
+    }
+    bool doCenter = false;
+    V3 centerOff = v3(0.f, 0.f, 0.f);
+    if (sp.seek_world_center) {
+        const brt_grid_params& g = a.g;
+        const bool inside = (p.x > g.world_center[0] - g.world_radius[0]) &&
+                            (p.x < g.world_center[0] + g.world_radius[0]) &&
+                            (p.y > g.world_center[1] - g.world_radius[1]) &&
+                            (p.y < g.world_center[1] + g.world_radius[1]) &&
+                            (p.z > g.world_center[2] - g.world_radius[2]) &&
+                            (p.z < g.world_center[2] + g.world_radius[2]);
+        const V3 c = v3(g.world_center[0], g.world_center[1], g.world_center[2]);
+        doCenter = !inside;
+        centerOff = c - p;
+        F = (inside ? v3(0.f, 0.f, 0.f) : steerForSeek(p, s, f, c, sp.max_speed)) + F;
+    }
+
+    // ---- forward recompute: integrator ------------------------------------
+    const V3 adjF = adjustRawSteeringForce(F, s, f, sp.max_speed);
+    const V3 clipped = truncateLength(adjF, sp.max_force);
+    const V3 accel = clipped / sp.mass;
+    float rate = 0.0f;
+    V3 a1 = sa;
+    if (a.dt > 0.0f) {
+        rate = clampf(clampf(9.0f * a.dt, 0.15f, 0.4f), 0.0f, 1.0f);
+        a1 = sa + (accel - sa) * rate;
+    }
+    const V3 v0 = f * s + a1 * a.dt;
+    const V3 v = truncateLength(v0, sp.max_speed);
+
+    // ---- backward: integrator -------------------------------------------
+    const V3 gp1 = xyz(gP), gf1 = xyz(gF), ga1 = xyz(gA);
+    const float gs1 = gF.w;
+    const float vlen = length(v);
+    const V3 f1 = v * (1.0f / vlen);
+    V3 vbar = gp1 * a.dt + normalize_bwd(v, gf1) + f1 * gs1;
+    const V3 v0bar = truncate_bwd(v0, sp.max_speed, vbar);
+    V3 pbar = gp1;
+    V3 fbar = v0bar * s;
+    float sbar = dot(v0bar, f);
+    V3 a1bar = ga1 + v0bar * a.dt;
+    V3 abar = a1bar;
+    V3 accbar = v3(0.f, 0.f, 0.f);
+    if (a.dt > 0.0f) {
+        abar = a1bar * (1.0f - rate);
+        accbar = a1bar * rate;
+    }
+    const V3 clipbar = accbar / sp.mass;
+    V3 Fbar = truncate_bwd(adjF, sp.max_force, clipbar);
+    // adjustRawSteeringForce: identity unless slow and F != 0 and outside the cone
+    const float maxAdj = 0.2f * sp.max_speed;
+    const bool zeroF = F.x == 0.0f && F.y == 0.0f && F.z == 0.0f;
+    if (!(s > maxAdj || zeroF)) {
+        const float range = s / maxAdj;
+        const float c = 1.0f + (-2.0f * pow20(range));
+        const float L = length(F);
+        const V3 d = F / L;
+        if (dot(d, f) < c) {
+            const V3 o = Fbar;  // dL/d(output of the cone limit)
+            const float proj = dot(F, f);
+            const V3 perp = F - f * proj;
+            const float pl = length(perp);
+            const V3 u = perp * (1.0f / pl);
+            const float pd = sqrtf(1.0f - c * c);
+            const V3 inner = f * c + u * pd;
+            const float Lbar = dot(o, inner);
+            const V3 gi = o * L;
+            fbar = fbar + gi * c;
+            const V3 ubar = gi * pd;
+            const V3 perpbar = (ubar - u * dot(u, ubar)) * (1.0f / pl);
+            Fbar = perpbar - f * dot(f, perpbar) + F * (Lbar / L);
+            fbar = fbar - perpbar * proj - F * dot(f, perpbar);
+            // c = 1 - 2x, x = (s/maxAdj)^20, and pd = sqrt(1 - c^2) = 2 r^10 sqrt(1 - x):
+            // dc/ds = -40 r^19 / maxAdj and dpd/ds = 20 c r^9 / (maxAdj sqrt(1 - x)), finite
+            // where the FP32 pd itself rounds to 0 (c rounds to 1 for small r)
+            float r9 = 1.0f;
+            for (int k = 0; k < 9; ++k) r9 = r9 * range;
+            const float r10 = r9 * range;
+            const float r19 = r9 * r10;
+            const float om = 1.0f - r10 * r10;
+            const float dc_ds = -40.0f * r19 / maxAdj;
+            const float dpd_ds = om > 0.0f ? 20.0f * c * r9 / (maxAdj * sqrtf(om)) : 0.0f;
+            sbar = sbar + dot(gi, f) * dc_ds + dot(gi, u) * dpd_ds;
+        }
+    }
+    // seeks: d/d(p, f, s) of truncate(target - p, maxS) - f s
+    if (doTarget) {
+        const V3 g = Fbar * sp.target_weight;
+        pbar = pbar - truncate_bwd(seekOff, sp.max_speed, g);
+        fbar = fbar - g * s;
+        sbar = sbar - dot(g, f);
+    }
+    if (doCenter) {
+        pbar = pbar - truncate_bwd(centerOff, sp.max_speed, Fbar);
+        fbar = fbar - Fbar * s;
+        sbar = sbar - dot(Fbar, f);
+    }
+
+    // ---- backward: behaviour sums -------------------------------------------
+    V3 Sbar = v3(0.f, 0.f, 0.f), Abar = Sbar, Cbar = Sbar;
+    uint32_t flags = full ? kAdjFull : 0u;
+    {
+        const I3 gpi = calcGridPos(p.x, p.y, p.z, a.g);
+        if (inGrid(gpi.x, gpi.y, gpi.z, a.g)) flags |= kAdjInGrid;
+        if (gpi.x == 0 || gpi.y == 0 || gpi.z == 0) flags |= kAdjLowFace;
+    }
+    if (sp.separation[0] != 0.0f && acc.nSep > 0) {
+        flags |= kAdjSep;
+        r.wg[0] = dot(Fbar, us);
+        Sbar = normalize_bwd(xs, Fbar * sp.separation[0]) * (1.0f / (float)acc.nSep);
+    }
+    if (sp.alignment[0] != 0.0f && acc.nAli > 0) {
+        flags |= kAdjAli;
+        r.wg[1] = dot(Fbar, ua);
+        const V3 xbar = normalize_bwd(xa, Fbar * sp.alignment[0]);
+        fbar = fbar - xbar;
+        Abar = xbar * (1.0f / (float)acc.nAli);
+    }
+    if (sp.cohesion[0] != 0.0f && acc.nCoh > 0) {
+        flags |= kAdjCoh;
+        r.wg[2] = dot(Fbar, uc);
+        Cbar = normalize_bwd(xc, Fbar * sp.cohesion[0]) * (1.0f / (float)acc.nCoh);
+    }
+    r.p = pbar;
+    r.f = fbar;
+    r.a = abar;
+    r.S = Sbar;
+    r.A = Abar;
+    r.C = Cbar;
+    r.s = sbar;
+    r.flags = flags;
+    return r;
+}
+
+// The list entries one lane takes of an agent's list, NL lanes to the agent:
+// U of them from entry t on, a.n where there is none, with their positions.
+template <int NL, int U>
+__device__ __forceinline__ void load_entries(const AdjArgs& a, uint32_t i, uint32_t l, const uint32_t* row,
+                                             uint32_t count, uint32_t t, uint32_t (&jj)[U], float4 (&q)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t e = t + (uint32_t)(NL * u) + l;
+        const uint32_t j = row[e < a.W - 1u ? 1u + e : 0u];
+        jj[u] = e < count && j < a.n ? j : a.n;
+        q[u] = a.spos[jj[u] < a.n ? jj[u] : i];
+    }
+}
+
+// The agent's behaviour sums, in list order; jf, qf: the first trip's entries and
+// positions, kept for own_share.
+template <int NL, int U>
+__device__ __forceinline__ SteerAccum own_sums(const AdjArgs& a, uint32_t i, uint32_t l, const uint32_t* row,
+                                               uint32_t count, V3 p, V3 f, uint32_t (&jf)[U], float4 (&qf)[U]) {
+    const brt_steer_params& sp = a.sp;
+    SteerAccum acc;
+    acc.init();
+    load_entries<NL, U>(a, i, l, row, count, 0u, jf, qf);
+    for (uint32_t t = 0; t < count; t += (uint32_t)(NL * U)) {
+        uint32_t jj[U];
+        float4 q[U], fq[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            jj[u] = jf[u];
+            q[u] = qf[u];
+        }
+        if (t != 0u) load_entries<NL, U>(a, i, l, row, count, t, jj, q);
+#pragma unroll
+        for (int u = 0; u < U; ++u) fq[u] = a.sfwd[jj[u] < a.n ? jj[u] : i];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            SteerAccum one;
+            one.init();
+            const V3 off = xyz(q[u]) - p;
+            if (jj[u] < a.n) one.add(sp, weights_of(sp), f, off, dot(off, off), xyz(fq[u]));
+            acc.sSep = quad_add<NL>(acc.sSep, one.sSep);
+            acc.sAli = quad_add<NL>(acc.sAli, one.sAli);
+            acc.sCoh = quad_add<NL>(acc.sCoh, one.sCoh);
+            acc.nSep += one.nSep;
+            acc.nAli += one.nAli;
+            acc.nCoh += one.nCoh;
+        }
+    }
+    acc.nSep = quad_count<NL>(acc.nSep);
+    acc.nAli = quad_count<NL>(acc.nAli);
+    acc.nCoh = quad_count<NL>(acc.nCoh);
+    return acc;
+}
+
+// The agent's share of the neighbour terms: p_i appears in every offset p_j - p_i
+// of its own sums (the same per-pair terms k_adjoint_gather adds to p_j).
+template <int NL, int U>
+__device__ __forceinline__ V3 own_share(const AdjArgs& a, uint32_t i, uint32_t l, const uint32_t* row, uint32_t count,
+                                        V3 p, V3 f, uint32_t flags, V3 S, V3 C, V3 pbar, uint32_t (&jf)[U],
+                                        float4 (&qf)[U]) {
+    for (uint32_t t = 0; t < count; t += (uint32_t)(NL * U)) {
+        if (t != 0u) load_entries<NL, U>(a, i, l, row, count, t, jf, qf);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const V3 off = xyz(qf[u]) - p;
+            bool anyP = false, ali;
+            V3 o = v3(0.f, 0.f, 0.f);
+            if (jf[u] < a.n) o = pair_terms(a.sp, flags, f, off, S, C, anyP, ali);
+            pbar = quad_add<NL>(pbar, keep(v3(-o.x, -o.y, -o.z), anyP));
+        }
+    }
+    return pbar;
+}
+
+__device__ __forceinline__ void store_record(const AdjArgs& a, uint32_t i, V3 p, V3 f, const OwnBack& r) {
+    float4* const rec = a.rec + 4u * (size_t)i;
+    rec[0] = make_float4(p.x, p.y, p.z, f.x);
+    rec[1] = make_float4(f.y, f.z, r.S.x, r.S.y);
+    rec[2] = make_float4(r.S.z, r.C.x, r.C.y, r.C.z);
+    rec[3] = make_float4(r.A.x, r.A.y, r.A.z, __uint_as_float(r.flags));
+}
+
+// a hash entry without a valid ID: no terms
+__device__ __forceinline__ void store_nothing(const AdjArgs& a, uint32_t i) {
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (uint32_t k = 0; k < 3u; ++k) a.own[3u * (size_t)i + k] = z;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) a.rec[4u * (size_t)i + k] = z;
+}
+
+// sum over the wave in a fixed order, to lane 0
+__device__ __forceinline__ float wave_sum(float v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+    return v;
+}
+
+__device__ __forceinline__ bool has_behaviours(const brt_steer_params& sp) {
+    return sp.separation[0] != 0.0f || sp.alignment[0] != 0.0f || sp.cohesion[0] != 0.0f;
+}
+
+// One lane per agent.
+__global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
+    constexpr int U = 4;
+    __shared__ float s_red[3][4];
+    const uint32_t i = xcd_block(a.xcd_remap) * blockDim.x + threadIdx.x;
+    float wg[3] = {0.f, 0.f, 0.f};
     if (i < a.n && a.hash[i].y < a.n) {
         const uint32_t id = a.hash[i].y;
         const float4 P = a.spos[i], Fw = a.sfwd[i], SA = a.ssa[i];
         const float4 gP = a.gpos_out[id], gF = a.gfwd_out[id], gA = a.gsa_out[id];
-        const V3 p = xyz(P), f = xyz(Fw), sa = xyz(SA);
-        const float s = Fw.w;
+        const V3 p = xyz(P), f = xyz(Fw);
         const uint32_t* row = a.lists + (size_t)i * a.W;
-        const uint32_t count = row[0] < a.W - 1u ? row[0] : a.W - 1u;
-        const bool behaviours = sp.separation[0] != 0.0f || sp.alignment[0] != 0.0f || sp.cohesion[0] != 0.0f;
-
-        // this lane's entries of the trip from entry t on, a.n where there is none
-        auto load_entries = [&](uint32_t t, uint32_t (&jj)[U], float4 (&q)[U]) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t e = t + (uint32_t)(NL * u) + l;
-                const uint32_t j = row[e < a.W - 1u ? 1u + e : 0u];
-                jj[u] = e < count && j < a.n ? j : a.n;
-                q[u] = a.spos[jj[u] < a.n ? jj[u] : i];
-            }
-        };
-
-        // ---- forward recompute: behaviour sums (list order) -------------------
-        // the first trip's entries and positions stay for the backward sums
+        const uint32_t count = has_behaviours(a.sp) ? (row[0] < a.W - 1u ? row[0] : a.W - 1u) : 0u;
         uint32_t jf[U];
         float4 qf[U];
-        SteerAccum acc;
-        acc.init();
-        if (behaviours) {
-            load_entries(0u, jf, qf);
-            for (uint32_t t = 0; t < count; t += T) {
-                uint32_t jj[U];
-                float4 q[U], fq[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    jj[u] = jf[u];
-                    q[u] = qf[u];
-                }
-                if (t != 0u) load_entries(t, jj, q);
-#pragma unroll
-                for (int u = 0; u < U; ++u) fq[u] = a.sfwd[jj[u] < a.n ? jj[u] : i];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    SteerAccum one;
-                    one.init();
-                    const V3 off = xyz(q[u]) - p;
-                    if (jj[u] < a.n) one.add(sp, weights_of(sp), f, off, dot(off, off), xyz(fq[u]));
-                    acc.sSep = quad_add<NL>(acc.sSep, one.sSep);
-                    acc.sAli = quad_add<NL>(acc.sAli, one.sAli);
-                    acc.sCoh = quad_add<NL>(acc.sCoh, one.sCoh);
-                    acc.nSep += one.nSep;
-                    acc.nAli += one.nAli;
-                    acc.nCoh += one.nCoh;
-                }
-            }
-            acc.nSep = quad_count<NL>(acc.nSep);
-            acc.nAli = quad_count<NL>(acc.nAli);
-            acc.nCoh = quad_count<NL>(acc.nCoh);
-        }
-        V3 xs = v3(0.f, 0.f, 0.f), xa = xs, xc = xs, us = xs, ua = xs, uc = xs;
-        V3 F = v3(0.f, 0.f, 0.f);
-        if (sp.separation[0] != 0.0f) {
-            if (acc.nSep > 0) {
-                xs = acc.sSep / (float)acc.nSep;
-                us = normalize(xs);
-            }
-            F = us * sp.separation[0] + F;
-        }
-        if (sp.alignment[0] != 0.0f) {
-            if (acc.nAli > 0) {
-                xa = acc.sAli / (float)acc.nAli - f;
-                ua = normalize(xa);
-            }
-            F = ua * sp.alignment[0] + F;
-        }
-        if (sp.cohesion[0] != 0.0f) {
-            if (acc.nCoh > 0) {
-                xc = acc.sCoh / (float)acc.nCoh;
-                uc = normalize(xc);
-            }
-            F = uc * sp.cohesion[0] + F;
-        }
-        V3 tgt = v3(0.f, 0.f, 0.f), seekOff = tgt;
-        const bool doTarget = sp.num_targets > 0 && sp.target_weight != 0.0f;
-        if (doTarget) {
-            const float* t = sp.targets[id % sp.num_targets];
-            tgt = v3(t[0], t[1], t[2]);
-            seekOff = tgt - p;
-            F = steerForSeek(p, s, f, tgt, sp.max_speed) * sp.target_weight + F;
-        }
-        bool doCenter = false;
-        V3 centerOff = v3(0.f, 0.f, 0.f);
-        if (sp.seek_world_center) {
-            const brt_grid_params& g = a.g;
-            const bool inside = (p.x > g.world_center[0] - g.world_radius[0]) &&
-                                (p.x < g.world_center[0] + g.world_radius[0]) &&
-                                (p.y > g.world_center[1] - g.world_radius[1]) &&
-                                (p.y < g.world_center[1] + g.world_radius[1]) &&
-                                (p.z > g.world_center[2] - g.world_radius[2]) &&
-                                (p.z < g.world_center[2] + g.world_radius[2]);
-            const V3 c = v3(g.world_center[0], g.world_center[1], g.world_center[2]);
-            doCenter = !inside;
-            centerOff = c - p;
-            F = (inside ? v3(0.f, 0.f, 0.f) : steerForSeek(p, s, f, c, sp.max_speed)) + F;
-        }
-
-        // ---- forward recompute: integrator ------------------------------------
-        const V3 adjF = adjustRawSteeringForce(F, s, f, sp.max_speed);
-        const V3 clipped = truncateLength(adjF, sp.max_force);
-        const V3 accel = clipped / sp.mass;
-        float rate = 0.0f;
-        V3 a1 = sa;
-        if (a.dt > 0.0f) {
-            rate = clampf(clampf(9.0f * a.dt, 0.15f, 0.4f), 0.0f, 1.0f);
-            a1 = sa + (accel - sa) * rate;
-        }
-        const V3 v0 = f * s + a1 * a.dt;
-        const V3 v = truncateLength(v0, sp.max_speed);
-
-        // ---- backward: integrator -------------------------------------------
-        const V3 gp1 = xyz(gP), gf1 = xyz(gF), ga1 = xyz(gA);
-        const float gs1 = gF.w;
-        const float vlen = length(v);
-        const V3 f1 = v * (1.0f / vlen);
-        V3 vbar = gp1 * a.dt + normalize_bwd(v, gf1) + f1 * gs1;
-        const V3 v0bar = truncate_bwd(v0, sp.max_speed, vbar);
-        V3 pbar = gp1;
-        V3 fbar = v0bar * s;
-        float sbar = dot(v0bar, f);
-        V3 a1bar = ga1 + v0bar * a.dt;
-        V3 abar = a1bar;
-        V3 accbar = v3(0.f, 0.f, 0.f);
-        if (a.dt > 0.0f) {
-            abar = a1bar * (1.0f - rate);
-            accbar = a1bar * rate;
-        }
-        const V3 clipbar = accbar / sp.mass;
-        V3 Fbar = truncate_bwd(adjF, sp.max_force, clipbar);
-        // adjustRawSteeringForce: identity unless slow and F != 0 and outside the cone
-        const float maxAdj = 0.2f * sp.max_speed;
-        const bool zeroF = F.x == 0.0f && F.y == 0.0f && F.z == 0.0f;
-        if (!(s > maxAdj || zeroF)) {
-            const float range = s / maxAdj;
-            const float c = 1.0f + (-2.0f * pow20(range));
-            const float L = length(F);
-            const V3 d = F / L;
-            if (dot(d, f) < c) {
-                const V3 o = Fbar;  // dL/d(output of the cone limit)
-                const float proj = dot(F, f);
-                const V3 perp = F - f * proj;
-                const float pl = length(perp);
-                const V3 u = perp * (1.0f / pl);
-                const float pd = sqrtf(1.0f - c * c);
-                const V3 inner = f * c + u * pd;
-                const float Lbar = dot(o, inner);
-                const V3 gi = o * L;
-                fbar = fbar + gi * c;
-                const V3 ubar = gi * pd;
-                const V3 perpbar = (ubar - u * dot(u, ubar)) * (1.0f / pl);
-                Fbar = perpbar - f * dot(f, perpbar) + F * (Lbar / L);
-                fbar = fbar - perpbar * proj - F * dot(f, perpbar);
-                // c = 1 - 2x, x = (s/maxAdj)^20, and pd = sqrt(1 - c^2) = 2 r^10 sqrt(1 - x):
-                // dc/ds = -40 r^19 / maxAdj and dpd/ds = 20 c r^9 / (maxAdj sqrt(1 - x)), finite
-                // where the FP32 pd itself rounds to 0 (c rounds to 1 for small r)
-                float r9 = 1.0f;
-                for (int k = 0; k < 9; ++k) r9 = r9 * range;
-                const float r10 = r9 * range;
-                const float r19 = r9 * r10;
-                const float om = 1.0f - r10 * r10;
-                const float dc_ds = -40.0f * r19 / maxAdj;
-                const float dpd_ds = om > 0.0f ? 20.0f * c * r9 / (maxAdj * sqrtf(om)) : 0.0f;
-                sbar = sbar + dot(gi, f) * dc_ds + dot(gi, u) * dpd_ds;
-            }
-        }
-        // seeks: d/d(p, f, s) of truncate(target - p, maxS) - f s
-        if (doTarget) {
-            const V3 g = Fbar * sp.target_weight;
-            pbar = pbar - truncate_bwd(seekOff, sp.max_speed, g);
-            fbar = fbar - g * s;
-            sbar = sbar - dot(g, f);
-        }
-        if (doCenter) {
-            pbar = pbar - truncate_bwd(centerOff, sp.max_speed, Fbar);
-            fbar = fbar - Fbar * s;
-            sbar = sbar - dot(Fbar, f);
-        }
-
-        // ---- backward: behaviour sums -------------------------------------------
-        V3 Sbar = v3(0.f, 0.f, 0.f), Abar = Sbar, Cbar = Sbar;
-        uint32_t flags = row[0] >= a.K ? kAdjFull : 0u;
-        {
-            const I3 gpi = calcGridPos(p.x, p.y, p.z, a.g);
-            if (inGrid(gpi.x, gpi.y, gpi.z, a.g)) flags |= kAdjInGrid;
-            if (gpi.x == 0 || gpi.y == 0 || gpi.z == 0) flags |= kAdjLowFace;
-        }
-        if (sp.separation[0] != 0.0f && acc.nSep > 0) {
-            flags |= kAdjSep;
-            wg[0] = dot(Fbar, us);
-            Sbar = normalize_bwd(xs, Fbar * sp.separation[0]) * (1.0f / (float)acc.nSep);
-        }
-        if (sp.alignment[0] != 0.0f && acc.nAli > 0) {
-            flags |= kAdjAli;
-            wg[1] = dot(Fbar, ua);
-            const V3 xbar = normalize_bwd(xa, Fbar * sp.alignment[0]);
-            fbar = fbar - xbar;
-            Abar = xbar * (1.0f / (float)acc.nAli);
-        }
-        if (sp.cohesion[0] != 0.0f && acc.nCoh > 0) {
-            flags |= kAdjCoh;
-            wg[2] = dot(Fbar, uc);
-            Cbar = normalize_bwd(xc, Fbar * sp.cohesion[0]) * (1.0f / (float)acc.nCoh);
-        }
-        // this agent's share of the neighbour terms: p_i appears in every
-        // offset p_j - p_i of its own sums (the same per-pair terms
-        // k_adjoint_gather adds to p_j)
-        if (behaviours) {
-            for (uint32_t t = 0; t < count; t += T) {
-                if (t != 0u) load_entries(t, jf, qf);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const V3 off = xyz(qf[u]) - p;
-                    bool anyP = false, ali;
-                    V3 offbar = v3(0.f, 0.f, 0.f);
-                    if (jf[u] < a.n) offbar = pair_terms(sp, flags, f, off, Sbar, Cbar, anyP, ali);
-                    pbar = quad_add<NL>(pbar, keep(v3(-offbar.x, -offbar.y, -offbar.z), anyP));
-                }
-            }
-        }
-        float4* const own = a.own + 3u * (size_t)i;
-        float4* const rec = a.rec + 4u * (size_t)i;
-        const float fl = __uint_as_float(flags);
-        if (NL == 1) {
-            own[0] = make_float4(pbar.x, pbar.y, pbar.z, 0.0f);
-            own[1] = make_float4(fbar.x, fbar.y, fbar.z, sbar);
-            own[2] = make_float4(abar.x, abar.y, abar.z, 0.0f);
-            rec[0] = make_float4(p.x, p.y, p.z, f.x);
-            rec[1] = make_float4(f.y, f.z, Sbar.x, Sbar.y);
-            rec[2] = make_float4(Sbar.z, Cbar.x, Cbar.y, Cbar.z);
-            rec[3] = make_float4(Abar.x, Abar.y, Abar.z, fl);
-        } else {
-            // lane l stores the l-th float4 of each
-            if (l < 3u)
-                own[l] = make_float4(pick(l, pbar.x, fbar.x, abar.x, 0.0f), pick(l, pbar.y, fbar.y, abar.y, 0.0f),
-                                     pick(l, pbar.z, fbar.z, abar.z, 0.0f), l == 1u ? sbar : 0.0f);
-            rec[l] = make_float4(pick(l, p.x, f.y, Sbar.z, Abar.x), pick(l, p.y, f.z, Cbar.x, Abar.y),
-                                 pick(l, p.z, Sbar.x, Cbar.y, Abar.z), pick(l, f.x, Sbar.y, Cbar.z, fl));
-            // one lane's weight terms stand for the agent
-            wg[0] = l == 0u ? wg[0] : 0.0f;
-            wg[1] = l == 0u ? wg[1] : 0.0f;
-            wg[2] = l == 0u ? wg[2] : 0.0f;
-        }
-    } else if (i < a.n && l == 0u) {
-        // a hash entry without a valid ID: no terms
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (uint32_t k = 0; k < 3u; ++k) a.own[3u * (size_t)i + k] = z;
-#pragma unroll
-        for (uint32_t k = 0; k < 4u; ++k) a.rec[4u * (size_t)i + k] = z;
+        const SteerAccum acc = own_sums<1, U>(a, i, 0u, row, count, p, f, jf, qf);
+        const OwnBack r = own_backward(a, id, P, Fw, SA, gP, gF, gA, acc, row[0] >= a.K);
+        const V3 pbar = own_share<1, U>(a, i, 0u, row, count, p, f, r.flags, r.S, r.C, r.p, jf, qf);
+        a.own[3u * (size_t)i + 0u] = make_float4(pbar.x, pbar.y, pbar.z, 0.0f);
+        a.own[3u * (size_t)i + 1u] = make_float4(r.f.x, r.f.y, r.f.z, r.s);
+        a.own[3u * (size_t)i + 2u] = make_float4(r.a.x, r.a.y, r.a.z, 0.0f);
+        store_record(a, i, p, f, r);
+        wg[0] = r.wg[0];
+        wg[1] = r.wg[1];
+        wg[2] = r.wg[2];
+    } else if (i < a.n) {
+        store_nothing(a, i);
     }
     // workgroup reduction of dL/dw in a fixed order
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        float v = wg[k];
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+        const float v = wave_sum(wg[k]);
         if (lane == 0) s_red[k][wave] = v;
     }
     __syncthreads();
@@ -456,6 +489,105 @@ __global__ void __launch_bounds__(256) k_adjoint_own(AdjArgs a) {
         for (uint32_t w = 0; w < nw; ++w) v += s_red[threadIdx.x][w];
         a.partials[(size_t)blockIdx.x * 3 + threadIdx.x] = v;
     }
+}
+
+// Four lanes per agent, 64 agents per workgroup (small flocks): lane l takes the
+// list entries l, l + 4, ..., and the sums add the four lanes' terms in list
+// order (the same bits as one lane).  The integrator between the two walks, some
+// 1,500 instructions, runs on the first wave, one lane per agent.  Bound by a
+// wave's chain of list and neighbour loads, which four lanes shorten (65,536
+// agents are one wave per SIMD with one lane each): 65,536 agents 23.4 us with one
+// lane, 19.9 with the integrator on all four, 16.5 so.
+constexpr uint32_t kOwnWords = 13u;  // LDS words per agent: odd, no bank conflicts
+__global__ void __launch_bounds__(256) k_adjoint_own_quad(AdjArgs a) {
+    constexpr int U = 2;
+    __shared__ float s_own[64u * kOwnWords];
+    const uint32_t tid = threadIdx.x, l = tid & 3u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t base = xcd_block(a.xcd_remap) * 64u;
+    const uint32_t i = base + (tid >> 2), at = i < a.n ? i : a.n - 1u;
+    const bool walk = i < a.n && has_behaviours(a.sp);
+    const V3 p = xyz(a.spos[at]), f = xyz(a.sfwd[at]);
+    const uint32_t* row = a.lists + (size_t)at * a.W;
+    const uint32_t count = walk ? (row[0] < a.W - 1u ? row[0] : a.W - 1u) : 0u;
+    // the first wave's agents: their own loads start now
+    const uint32_t mi = base + tid;
+    uint32_t id = a.n;
+    float4 P, Fw, SA, gP, gF, gA;
+    bool full = false;
+    if (wave == 0u && mi < a.n) {
+        id = a.hash[mi].y;
+        P = a.spos[mi];
+        Fw = a.sfwd[mi];
+        SA = a.ssa[mi];
+        full = a.lists[(size_t)mi * a.W] >= a.K;
+        if (id < a.n) {
+            gP = a.gpos_out[id];
+            gF = a.gfwd_out[id];
+            gA = a.gsa_out[id];
+        }
+    }
+    uint32_t jf[U];
+    float4 qf[U];
+    const SteerAccum acc = own_sums<4, U>(a, at, l, row, count, p, f, jf, qf);
+    float* const d = s_own + (tid >> 2) * kOwnWords;
+    if (l == 0u) {
+        d[0] = acc.sSep.x;
+        d[1] = acc.sSep.y;
+        d[2] = acc.sSep.z;
+        d[3] = acc.sAli.x;
+        d[4] = acc.sAli.y;
+        d[5] = acc.sAli.z;
+        d[6] = acc.sCoh.x;
+        d[7] = acc.sCoh.y;
+        d[8] = acc.sCoh.z;
+        d[9] = __uint_as_float(acc.nSep | acc.nAli << 10 | acc.nCoh << 20);
+    }
+    __syncthreads();
+    if (wave == 0u) {
+        float wg[3] = {0.f, 0.f, 0.f};
+        float* const m = s_own + tid * kOwnWords;
+        if (id < a.n) {
+            SteerAccum sum;
+            sum.sSep = v3(m[0], m[1], m[2]);
+            sum.sAli = v3(m[3], m[4], m[5]);
+            sum.sCoh = v3(m[6], m[7], m[8]);
+            const uint32_t c = __float_as_uint(m[9]);
+            sum.nSep = c & 0x3FFu;
+            sum.nAli = c >> 10 & 0x3FFu;
+            sum.nCoh = c >> 20;
+            const OwnBack r = own_backward(a, id, P, Fw, SA, gP, gF, gA, sum, full);
+            m[0] = r.S.x;
+            m[1] = r.S.y;
+            m[2] = r.S.z;
+            m[3] = r.C.x;
+            m[4] = r.C.y;
+            m[5] = r.C.z;
+            m[6] = r.p.x;
+            m[7] = r.p.y;
+            m[8] = r.p.z;
+            m[9] = __uint_as_float(r.flags);
+            a.own[3u * (size_t)mi + 1u] = make_float4(r.f.x, r.f.y, r.f.z, r.s);
+            a.own[3u * (size_t)mi + 2u] = make_float4(r.a.x, r.a.y, r.a.z, 0.0f);
+            store_record(a, mi, xyz(P), xyz(Fw), r);
+            wg[0] = r.wg[0];
+            wg[1] = r.wg[1];
+            wg[2] = r.wg[2];
+        } else if (mi < a.n) {
+#pragma unroll
+            for (uint32_t k = 0; k < 10u; ++k) m[k] = 0.0f;  // no flags: no share
+            store_nothing(a, mi);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float v = wave_sum(wg[k]);
+            if (tid == 0u) a.partials[(size_t)blockIdx.x * 3 + k] = v;
+        }
+    }
+    __syncthreads();
+    const V3 pbar = own_share<4, U>(a, at, l, row, count, p, f, __float_as_uint(d[9]), v3(d[0], d[1], d[2]),
+                                    v3(d[3], d[4], d[5]), v3(d[6], d[7], d[8]), jf, qf);
+    if (l == 0u && i < a.n) a.own[3u * (size_t)i] = make_float4(pbar.x, pbar.y, pbar.z, 0.0f);
 }
 
 // Lanes per agent of k_adjoint_gather: lane l takes entries l, l+L, ... of the
@@ -630,28 +762,50 @@ __global__ void __launch_bounds__(256) k_adjoint_gather(GatherArgs a) {
                 }
             }
             if (!by_list || (fj & kAdjLowFace)) {
+                // the lane's cells: their ranges load together, then the first
+                // agent of each (a chain of three loads instead of three per cell)
+                constexpr uint32_t kCells = (27u + L - 1u) / L;
                 const I3 cj = key_cell(key, g);
-                for (uint32_t c = l; c < 27u; c += L) {
+                uint32_t cs[kCells], ce[kCells], nearby = 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < kCells; ++k) {
+                    const uint32_t c = l + k * L;
                     const int dx = (int)(c / 9u) - 1, dy = (int)((c / 3u) % 3u) - 1, dz = (int)(c % 3u) - 1;
                     const int nx = gather_axis(cj.x, dx, g.grid_size[0]);
                     const int ny = gather_axis(cj.y, dy, g.grid_size[1]);
                     const int nz = gather_axis(cj.z, dz, g.grid_size[2]);
-                    if (nx < 0 || ny < 0 || nz < 0) continue;
                     const bool near = nx == cj.x + dx && ny == cj.y + dy && nz == cj.z + dz;
-                    if (by_list && near) continue;
-                    const uint32_t nk = cellKey(nx, ny, nz, g);
-                    const uint32_t s = a.cell_start[nk];
-                    if (s == BRT_EMPTY_CELL) continue;
-                    const uint32_t e = a.cell_end[nk];
-                    for (uint32_t i = s; i < e; ++i) {
-                        if (i == j) continue;
-                        const float4 Pi = a.spos[i];
-                        // the list test of agent i for candidate j (d2 as k_prox forms it)
-                        const V3 off = pj - xyz(Pi);
+                    const bool take = c < 27u && nx >= 0 && ny >= 0 && nz >= 0 && !(by_list && near);
+                    cs[k] = BRT_EMPTY_CELL;
+                    ce[k] = 0u;
+                    if (take) {
+                        const uint32_t nk = cellKey(nx, ny, nz, g);
+                        cs[k] = a.cell_start[nk];
+                        ce[k] = a.cell_end[nk];
+                    }
+                    nearby |= near ? 1u << k : 0u;
+                }
+                float4 first[kCells];
+#pragma unroll
+                for (uint32_t k = 0; k < kCells; ++k) {
+                    first[k] = Pj;
+                    if (cs[k] != BRT_EMPTY_CELL) first[k] = a.spos[cs[k]];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kCells; ++k) {
+                    if (cs[k] == BRT_EMPTY_CELL) continue;
+                    float4 Pi = first[k];
+                    for (uint32_t i = cs[k]; i < ce[k];) {
+                        const uint32_t here = i++;
+                        const float4 Ph = Pi;
+                        if (i < ce[k]) Pi = a.spos[i];
+                        if (here == j) continue;
+                        // the list test of agent `here` for candidate j (d2 as k_prox forms it)
+                        const V3 off = pj - xyz(Ph);
                         if (dot(off, off) > a.T) continue;
                         Rec R;
-                        R.load(a.rec, i);
-                        if (!in_list(a, i, R.flags(), Pi, j, cj, false, Pj, near)) continue;
+                        R.load(a.rec, here);
+                        if (!in_list(a, here, R.flags(), Ph, j, cj, false, Pj, (nearby >> k & 1u) != 0u)) continue;
                         R.add_pair(sp, off, accP, accF);
                     }
                 }
@@ -712,9 +866,9 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
     const bool quads = n <= kOwnQuadMax;
     const uint32_t blocks = adjoint_own_blocks(n);
     if (quads)
-        hipLaunchKernelGGL(k_adjoint_own<4>, dim3(blocks), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k_adjoint_own_quad, dim3(blocks), dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL(k_adjoint_own<1>, dim3(blocks), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k_adjoint_own, dim3(blocks), dim3(256), 0, s, a);
     GatherArgs b{};
     b.g = g;
     b.sp = sp;
