@@ -9,7 +9,7 @@ import pytest
 
 from behavert_amd import workloads as W
 from behavert_amd.engine import Flock
-from behavert_amd.types import GridParams, ProxParams, SteerParams
+from behavert_amd.types import OPT_LDS_LISTS, GridParams, ProxParams, SteerParams
 
 from ._parity import dev, empty_u32, first_mismatch, oracle_grid_outputs, u32
 
@@ -100,3 +100,19 @@ def test_both_sides_of_the_limit(ctx, orc, n, side):
     got = fl.state()
     for k in ("pos", "forward", "smooth_accel"):
         assert first_mismatch(got[k].view(np.uint32), getattr(hf, k).view(np.uint32)) is None, k
+
+
+@pytest.mark.parametrize("K", [27, 28, 32])
+@pytest.mark.parametrize("per_cell,max_bodies", [(9, 0xFFFFFFFF), (30, 0xFFFFFFFF), (30, 7)])
+def test_one_lane_scans_in_step(ctx, orc, K, per_cell, max_bodies):
+    """The one-lane kernel's crowded waves, whose quads walk the same cells from
+    K 28 on where they share one: quads that span cells, a tail of three lanes,
+    agents outside the grid among them."""
+    rng = np.random.default_rng(K + per_cell)
+    grid = GridParams.direct((0.0,) * 3, (4.0,) * 3, (5, 4, 6), max_bodies=max_bodies)
+    xyz = rng.uniform(-1.0, [21.0, 17.0, 25.0], (120 * per_cell // 64 * 64 + 3, 3))
+    ctx.set_option(OPT_LDS_LISTS, 1)
+    try:
+        check(ctx, orc, grid, K, state(rng, xyz))
+    finally:
+        ctx.set_option(OPT_LDS_LISTS, -1)
