@@ -155,12 +155,40 @@ struct ClusterAccum {
     }
 };
 
+// LDS of a wave: the list rows, overwritten in place by the similarities (slot t
+// at word t, entry t + 1's word once it is read), for rows of up to kStageWords
+// words, else only the similarities; and, with the cluster steering, the tile that
+// the records' parts change lanes in.
+constexpr uint32_t kTileChunks = 4u * 65u;  // float4; the 65: no bank conflicts
+inline __host__ __device__ uint32_t similarity_row_words(uint32_t K, uint32_t W) { return W <= kStageWords ? W : K + 1u; }
+inline uint32_t similarity_wave_bytes(uint32_t K, uint32_t W) {
+    return ((64u * similarity_row_words(K, W) * 4u + 15u) / 16u + kTileChunks) * 16u;
+}
+
+// Stores the similarities of a wave's agents out of LDS: rows of RW words, K + 1
+// of them contiguous in sims.
+__device__ __forceinline__ void store_similarities(float* __restrict__ sims, uint32_t row0, uint32_t n, uint32_t K,
+                                                   uint32_t RW, const float* src, uint32_t lane) {
+    const uint32_t S = K + 1u, total = (n - row0 < 64u ? n - row0 : 64u) * S;
+    float* const dst = sims + (size_t)row0 * S;
+    const uint32_t dr = 64u / S, dc = 64u - dr * S;
+    uint32_t r = lane / S, c = lane - r * S;
+    for (uint32_t x = lane; x < total; x += 64u) {
+        dst[x] = src[r * RW + c];
+        r += dr;
+        c += dc;
+        if (c >= S) {
+            c -= S;
+            ++r;
+        }
+    }
+}
+
 // computeNeighNaiveSimilarities (+ computeAdaptiveSimilarities) over sorted
 // features.  One lane per sorted agent; neighbours in groups of G (8 gathers of
-// FQ float4 in flight at FQ <= 2).  Each lane writes its similarity row into LDS
-// (dynamic, blockDim * (K+1) floats); the rows of a wave's 64 agents are
-// contiguous in `sims` too, so the wave then stores them with coalesced (float4
-// when `vec`) writes.
+// FQ float4 in flight at FQ <= 2).  Each lane writes its similarity row into LDS,
+// in the place of its staged list row where there is one, and the wave then stores
+// the rows with coalesced writes.
 extern __shared__ float bc_rows[];
 
 template <bool ADAPTIVE, int FQ>
@@ -169,7 +197,8 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
                                                  const uint32_t* __restrict__ lists,
                                                  const float4* __restrict__ sfeat, const float* __restrict__ norms,
                                                  const float4* __restrict__ stats_in, float4* __restrict__ stats_out,
-                                                 float* out) {
+                                                 uint32_t* row, bool staged) {
+    float* const out = reinterpret_cast<float*>(row);
     constexpr int G = FQ <= 2 ? 8 : (FQ <= 4 ? 4 : 2);
     const uint32_t F = bc.feature_count;
     const uint32_t id = hash[i].y;
@@ -179,7 +208,7 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
     const float n1 = norms[i];
     const bool valid = id < n;
     float4 st = ADAPTIVE && valid ? stats_in[id] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t count = for_list_octets(lists, W, K, i, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
+    auto visit = [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
 #pragma unroll
         for (int g0 = 0; g0 < 8; g0 += G) {
             float4 other[G][FQ];
@@ -206,7 +235,14 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
                 out[base + k - 1u] = sim;
             }
         }
-    });
+    };
+    uint32_t count;
+    if (staged) {
+        count = row[0] < K ? row[0] : K;
+        visit_staged(reinterpret_cast<const uint4*>(row), count, i, n, visit);
+    } else {
+        count = for_list_octets(lists, W, K, i, n, visit);
+    }
     for (uint32_t t = count; t <= K; ++t) out[t] = 0.0f;
     if (ADAPTIVE && valid) stats_out[id] = st;
 }
@@ -219,25 +255,19 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
                                                          const float* __restrict__ norms,
                                                          const float4* __restrict__ stats_in,
                                                          float4* __restrict__ stats_out, float* __restrict__ sims,
-                                                         uint32_t vec, uint32_t xcd_remap) {
-    const uint32_t blk = xcd_block(xcd_remap);
-    const uint32_t i = blk * blockDim.x + threadIdx.x;
-    if (i < n) similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out,
-                                              bc_rows + (size_t)threadIdx.x * (K + 1u));
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint32_t i0 = blk * blockDim.x + wv * 64u;
-    if (i0 >= n) return;
-    const uint32_t total = (n - i0 < 64u ? n - i0 : 64u) * (K + 1u);
-    const float* src = bc_rows + (size_t)wv * 64u * (K + 1u);
-    float* dst = sims + (size_t)i0 * (K + 1u);
-    uint32_t x = lane;
-    if (vec) {
-        const uint32_t t4 = total / 4u;
-        for (; x < t4; x += 64u) reinterpret_cast<float4*>(dst)[x] = reinterpret_cast<const float4*>(src)[x];
-        x = 4u * t4 + lane;
-    }
-    for (; x < total; x += 64u) dst[x] = src[x];
+                                                         uint32_t xcd_remap) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t row0 = xcd_block(xcd_remap) * blockDim.x + wave * 64u, i = row0 + lane;
+    if (row0 >= n) return;
+    const uint32_t RW = similarity_row_words(K, W);
+    uint32_t* const mem = reinterpret_cast<uint32_t*>(bc_rows) + (size_t)wave * 64u * RW;
+    const bool staged = W <= kStageWords;
+    if (staged) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
+    if (i < n)
+        similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, mem + lane * RW,
+                                       staged);
+    wave_lds_sync();
+    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane);
 }
 
 // ---- similarities and cluster steering in one pass
@@ -305,15 +335,6 @@ __global__ void __launch_bounds__(256) k_bc_records(uint32_t F, uint32_t n, uint
         r = part(p - 2u);
     }
     rec[t] = r;
-}
-
-// LDS of a wave: the list rows, overwritten in place by the similarities (slot t
-// at word t, entry t + 1's word once it is read), for rows of up to kStageWords
-// words, else only the similarities; and the tile that the parts change lanes in.
-constexpr uint32_t kTileChunks = 4u * 65u;  // float4; the 65: no bank conflicts
-inline __host__ __device__ uint32_t similarity_row_words(uint32_t K, uint32_t W) { return W <= kStageWords ? W : K + 1u; }
-inline uint32_t similarity_wave_bytes(uint32_t K, uint32_t W) {
-    return ((64u * similarity_row_words(K, W) * 4u + 15u) / 16u + kTileChunks) * 16u;
 }
 
 template <bool ADAPTIVE, int FQ>
@@ -431,21 +452,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
         force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
     }
     wave_lds_sync();
-    // the rows, K + 1 of RW words each, are contiguous in sims
-    const uint32_t S = K + 1u, total = (n - row0 < 64u ? n - row0 : 64u) * S;
-    const float* const src = reinterpret_cast<const float*>(mem);
-    float* const dst = sims + (size_t)row0 * S;
-    const uint32_t dr = 64u / S, dc = 64u - dr * S;
-    uint32_t r = lane / S, c = lane - r * S;
-    for (uint32_t x = lane; x < total; x += 64u) {
-        dst[x] = src[r * RW + c];
-        r += dr;
-        c += dc;
-        if (c >= S) {
-            c -= S;
-            ++r;
-        }
-    }
+    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane);
 }
 
 // steerForClusterCohesion + Alignment from stored similarities.
@@ -677,17 +684,17 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
     float* norms = reinterpret_cast<float*>(sfeat + (size_t)n * FQ);
     hipLaunchKernelGGL(k_bc_sort_features, dim3((n + 255) / 256), dim3(256), 0, s, F, (uint32_t)FQ, n, vec, hash,
                        features, sfeat, norms);
-    // the LDS row tile: 256 agents while it stays within 40 KB, else one wave
-    const uint32_t B = (size_t)256u * (K + 1u) * 4u <= 40u * 1024u ? 256u : 64u;
-    const size_t lds = (size_t)B * (K + 1u) * 4u;
-    const uint32_t vec_out = ((uintptr_t)sims & 15u) == 0 ? 1u : 0u;
+    // the LDS rows: 256 agents while they stay within 40 KB, else one wave
+    const size_t bytes = (size_t)64u * similarity_row_words(K, W) * 4u;
+    const uint32_t B = 4u * bytes <= 40u * 1024u ? 256u : 64u;
+    const size_t lds = B / 64u * bytes;
     const dim3 grid((n + B - 1) / B), block(B);
     if (bc.adaptive)
         hipLaunchKernelGGL((k_bc_similarities<true, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, vec_out, xcd_remap);
+                           stats_in, stats_out, sims, xcd_remap);
     else
         hipLaunchKernelGGL((k_bc_similarities<false, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, vec_out, xcd_remap);
+                           stats_in, stats_out, sims, xcd_remap);
     return hipGetLastError();
 }
 

@@ -101,6 +101,18 @@ __device__ __forceinline__ void stage_rows(uint4* stage, const uint32_t* __restr
     wave_lds_sync();
 }
 
+// Visits the entries of a row in LDS.  Entry e is read before f gets entry e + 1
+// (f may overwrite word e - 1 once it has entry e).
+template <class Fn>
+__device__ __forceinline__ void visit_staged(const uint4* L, uint32_t count, uint32_t i, uint32_t n, Fn&& f) {
+    for (uint32_t q = 0; 4u * q <= count; q += 2) {
+        const uint4 a = L[q], b = L[4u * (q + 1u) <= count ? q + 1u : q];
+        uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const uint32_t mask = octet_mask(jj, q, count, i, n);
+        f(4u * q, jj, mask);
+    }
+}
+
 template <class Fn>
 __device__ __forceinline__ uint32_t wave_list_octets(uint4* stage, const uint32_t* __restrict__ lists, uint32_t W,
                                                      uint32_t K, uint32_t row0, uint32_t lane, uint32_t n, Fn&& f) {
@@ -136,12 +148,7 @@ __device__ __forceinline__ uint32_t wave_list_octets(uint4* stage, const uint32_
     if (i >= n) return 0u;
     const uint4* L = stage + lane * (W / 4u);
     const uint32_t head = L[0].x, count = head < K ? head : K;
-    for (uint32_t q = 0; 4u * q <= count; q += 2) {
-        const uint4 a = L[q], b = L[4u * (q + 1u) <= count ? q + 1u : q];
-        uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        const uint32_t mask = octet_mask(jj, q, count, i, n);
-        f(4u * q, jj, mask);
-    }
+    visit_staged(L, count, i, n, f);
     return count;
 }
 
