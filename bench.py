@@ -243,13 +243,13 @@ def adjoint_ratio(steps=None, every=None) -> dict:
     ctx.close()
     # the adjoint step's compulsory bytes per agent (K 32, W 36): k_adjoint_own
     # reads the hash 8, the sorted state 48, the list 4W and the cotangents by
-    # ID 48, and writes its own terms 48 and neighbour-term vectors 48;
+    # ID 48, and writes its own terms 48 and the record of its neighbour terms 64;
     # k_adjoint_gather reads the hash 8, the own terms 48 and the list 4W, and
     # writes the gradients by ID 48 (neighbours' data is cache-resident)
     from behavert_amd.types import list_stride
 
     Wl = list_stride(w.prox.max_neighbors)
-    adj_bpa = (200 + 4 * Wl) + (104 + 4 * Wl)
+    adj_bpa = (216 + 4 * Wl) + (104 + 4 * Wl)
     adj_gbs = adj_bpa * w.n / 1e9 / (adj_ms / 1e3)
     return {"workload": "differentiable_65k", "n": w.n, "steps": T, "checkpoint_every": K,
             "replay_overlaps_adjoint": ro.overlap,
