@@ -522,7 +522,8 @@ int brt_prox_neighbors(brt_context* ctx, const brt_grid_params* grid, const brt_
     BRT_HIP(brt::launch_neighbors(*grid, *prox, brt_radius_threshold(prox->search_radius),
                                   reinterpret_cast<const float4*>(sorted_pos), reinterpret_cast<const uint2*>(hash),
                                   cell_start, cell_end, n, lists, ctx->uniform_max_cells, ctx->xcd_remap,
-                                  resolve_lds_lists(ctx, prox), ctx->lds_lists < 0, (hipStream_t)stream),
+                                  resolve_list_lds(ctx, prox, n, grid->num_cells), ctx->lds_lists < 0,
+                                  (hipStream_t)stream),
             "k_neighbors");
     return BRT_OK;
 }
@@ -1000,7 +1001,8 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // the two-pass path gathers the features into sorted order with the state
     // (into the sort's ping-pong buffer, free once the sort is done), so the
     // steering pass reads the neighbours' features by sorted index
-    const bool two_pass = !resolve_step_fused(ctx, prox, n, do_features);
+    const StepShape shape = resolve_step(ctx, prox, n, grid->num_cells, do_features);
+    const bool two_pass = !shape.fused;
     const bool sorted_features = do_features && two_pass;
     // small flocks: the keys lie in the lists, which the neighbour search writes
     // later; the context's scratch grows as for the radix sort, which a later
@@ -1013,7 +1015,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // with LDS lists the neighbour scan reads candidate positions from a
     // packed x,y,z copy written by the reorder (three 16-byte loads per four
     // candidates; the register-list scan measured no gain from it)
-    const uint32_t lds = resolve_lds_lists(ctx, prox);
+    const uint32_t lds = shape.lds;
     const bool pack = !prox->use_knn && (lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
     if (!given && pack && (rc = ensure_xyz(ctx, n))) return rc;
     float* xyz = pack ? (given ? given->xyz : ctx->xyz) : nullptr;
@@ -1174,9 +1176,9 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
                  const brt_step_buffers* b, std::vector<unsigned char>&& key) {
     const uint32_t n = b->n;
     const bool do_features = b->features && b->features_out && feature_rate != 0.0f;
-    const bool two_pass = !resolve_step_fused(ctx, prox, n, do_features);
-    const bool pack =
-        !prox->use_knn && (resolve_lds_lists(ctx, prox) != 0u || resolve_quads(ctx, prox, n, !two_pass));
+    const StepShape shape = resolve_step(ctx, prox, n, grid->num_cells, do_features);
+    const bool two_pass = !shape.fused;
+    const bool pack = !prox->use_knn && (shape.lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
     int rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells));
     if (rc) return rc;
     if ((rc = ensure_tmp(ctx, step_tmp(n, two_pass, do_features && two_pass,

@@ -59,26 +59,55 @@ struct brt_context {
 
 // Automatic launch shapes, from the K = 32 and K = 64 workloads measured on
 // gfx950: at K = 32 the fused neighbour + steering kernel and LDS-staged lists
-// are fastest; at K = 64 the two-pass path with register-chunk lists is (the
-// fused kernel's registers and the LDS list tile cut occupancy).
+// are fastest; beyond, two passes with register-chunk lists unless the flock's
+// size and grid say otherwise (resolve_step).
 inline bool resolve_fused(const brt_context* ctx, const brt_prox_params* p) {
     return ctx->fused_step >= 0 ? ctx->fused_step != 0 : p->max_neighbors <= 32u;
+}
+inline uint32_t resolve_lds_lists(const brt_context* ctx, const brt_prox_params* p) {
+    return ctx->lds_lists >= 0 ? (uint32_t)(ctx->lds_lists != 0) : (p->max_neighbors <= 32u ? 1u : 0u);
 }
 // Whether the neighbour search of n agents takes four lanes per agent (lists
 // automatic), and so packs their positions.
 inline bool resolve_quads(const brt_context* ctx, const brt_prox_params* p, uint32_t n, bool fused) {
     return ctx->lds_lists < 0 && !p->use_knn && brt::prox_quad_fits(p->max_neighbors, n, fused);
 }
-// The shape of a step of n agents: fused also beyond K = 32 where the quads take
-// the whole step in one launch (K 64, one per cell, 1,000 / 65,536 agents: 26 / 44
-// us in two passes, 21 / 36 in one); with the feature update the two-pass path, whose steering pass does it.
-inline bool resolve_step_fused(const brt_context* ctx, const brt_prox_params* p, uint32_t n, bool features) {
-    if (p->use_knn) return false;
-    if (ctx->fused_step < 0 && !features && resolve_quads(ctx, p, n, true)) return true;
-    return resolve_fused(ctx, p);
+// Lists beyond K = 32, automatic: from K 81 on the LDS rows leave too few waves.
+inline bool wide_lists(const brt_context* ctx, const brt_prox_params* p) {
+    return ctx->lds_lists < 0 && !p->use_knn && p->max_neighbors > 32u && p->max_neighbors <= 80u;
 }
-inline uint32_t resolve_lds_lists(const brt_context* ctx, const brt_prox_params* p) {
-    return ctx->lds_lists >= 0 ? (uint32_t)(ctx->lds_lists != 0) : (p->max_neighbors <= 32u ? 1u : 0u);
+// Whether a list pass alone stages such lists in LDS: in crowded grids, whose
+// waves then scan in flat mode.  A two-pass step with features, 1,048,576 agents,
+// K 40, registers -> LDS at 1 / 4 / 16 per cell: 386 -> 402, 513 -> 536, 975 ->
+// 767 us; K 64 419 -> 460, 547 -> 612, 1271 -> 1120.
+inline uint32_t resolve_list_lds(const brt_context* ctx, const brt_prox_params* p, uint32_t n, uint32_t cells) {
+    return wide_lists(ctx, p) ? (n / 8u >= cells ? 1u : 0u) : resolve_lds_lists(ctx, p);
+}
+
+// The shape of a step of n agents in a grid of `cells`.  Beyond K = 32:
+//   * fused where the quads take the whole step in one launch (K 64, one per cell,
+//     1,000 / 65,536 agents: 26 / 44 us in two passes, 21 / 36 in one);
+//   * fused with LDS lists up to K 80, two passes with register lists -> fused at
+//     1 / 4 / 16 per cell / in blobs: 1,048,576 agents, K 48, 353 -> 320, 471 ->
+//     408, 972 -> 607, 1108 -> 701 us, K 64 377 -> 369, 494 -> 462, 1146 -> 805,
+//     1274 -> 889, K 80 402 -> 402, 513 -> 514, 1213 -> 949, 1410 -> 1083 (K 100
+//     420 -> 469, 1230 -> 1251); but from 2^21 agents only where the grid is
+//     crowded: 2,097,152 agents, K 64, 729 -> 802, 936 -> 984, 2267 -> 1651;
+//   * two passes with the feature update, whose steering pass does it (fused and
+//     the features apart: 433 us against 386 at K 40 and one per cell, 823
+//     against 767 at 16).
+struct StepShape {
+    bool fused;
+    uint32_t lds;
+};
+inline StepShape resolve_step(const brt_context* ctx, const brt_prox_params* p, uint32_t n, uint32_t cells,
+                              bool features) {
+    if (p->use_knn) return StepShape{false, resolve_lds_lists(ctx, p)};
+    bool fused = resolve_fused(ctx, p);
+    if (ctx->fused_step < 0 && !features)
+        fused = fused || resolve_quads(ctx, p, n, true) ||
+                (wide_lists(ctx, p) && (n < (1u << 21) || n / 8u >= cells));
+    return StepShape{fused, fused && wide_lists(ctx, p) ? 1u : resolve_list_lds(ctx, p, n, cells)};
 }
 
 namespace brt {

@@ -151,7 +151,9 @@ int brt_context_get_option(const brt_context* ctx, int option, int* value);
  * parameters once automatic options are resolved: fused (0/1), lds_lists (0/1).
  * With lds_lists automatic, launches of up to 131,072 agents take four lanes per
  * agent and stage their lists in LDS for every K, and steps without the feature
- * update are fused there. */
+ * update are fused there; larger ones of 32 < K <= 80 are fused with LDS lists
+ * too (without features; from 2^21 agents where the grid holds 8 per cell or
+ * more), and in such crowded grids list passes stage their lists in LDS. */
 int brt_context_step_shape(const brt_context* ctx, const brt_prox_params* prox, int* fused, int* lds_lists);
 
 /* Failures the kernels record on the device instead of hanging or faulting:
