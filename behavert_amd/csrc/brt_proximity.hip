@@ -19,7 +19,7 @@
 // sqrtf, "sqrtf(d2) > r" and "d2 > T" agree for every d2, NaN included.
 //
 // MI355X design.  One lane per sorted agent, 256 lanes per workgroup (64 for
-// LDS-list launches of 2^18 agents or more, see prox_block); lists are staged
+// LDS-list launches of more than 2^17 agents, see prox_block); lists are staged
 // in LDS and written out with 16-byte coalesced stores, or gathered in
 // registers as 16-byte chunks.  Per wave64:
 //   * uniform mode (all lanes in few cells): lanes are grouped by cell; a group
@@ -87,8 +87,8 @@
 #ifndef BRT_PROX_FLAT_SPARSE
 #define BRT_PROX_FLAT_SPARSE 1
 #endif
-// Workgroup of the single-grid LDS-list neighbour kernels for launches of 2^18
-// agents or more (see prox_block).
+// Workgroup of the single-grid LDS-list neighbour kernels for launches of more
+// than 2^17 agents (see prox_block).
 #ifndef BRT_PROX_BLOCK_LARGE
 #define BRT_PROX_BLOCK_LARGE 64
 #endif
@@ -1777,13 +1777,14 @@ __global__ void __launch_bounds__(64) k_neighbors_knn(ProxArgs a) {
     }
 }
 
-// Workgroup of the single-grid LDS-list neighbour kernels: one wave for large
-// launches, so that a wave that finishes early releases its LDS tile at once
-// instead of waiting for the slowest wave of a larger workgroup (1M-boid blob
-// flock: 64 lanes 4-5 % faster than 256); 256 lanes for small launches (65k
-// boids: 3 % faster than 64), halved while the tile exceeds 40 KB.
+// Workgroup of the single-grid LDS-list neighbour kernels: one wave for launches
+// above the four-lane kernels', so that a wave that finishes early releases its LDS
+// tile at once instead of waiting for the slowest wave of a larger workgroup
+// (1M-boid blob flock: 64 lanes 4-5 % faster than 256; a step of 200,003 agents at
+// 1 / 16 per cell / in blobs, K 20, 90 / 118 / 204 -> 87 / 109 / 199 us); 256 lanes
+// for smaller ones, halved while the tile exceeds 40 KB.
 uint32_t prox_block(uint32_t W, uint32_t n) {
-    uint32_t B = n >= (1u << 18) ? BRT_PROX_BLOCK_LARGE : 256u;
+    uint32_t B = n > kProxQuadMax ? BRT_PROX_BLOCK_LARGE : 256u;
     while (B > 64 && (size_t)B * W * 4u > 40u * 1024u) B /= 2;
     return B;
 }
