@@ -864,6 +864,9 @@ __device__ __forceinline__ RowRange row_range(vuint3 s, vuint3 e, uint32_t n, ui
     return r;
 }
 
+// whether the range of a cell (start, end; both BRT_EMPTY_CELL when empty) holds sorted index i
+__device__ __forceinline__ bool holds(uint2 cell, uint32_t i) { return cell.x <= i && i < cell.y; }
+
 // Words of a list's head (count first) that the row scan of a kernel without
 // LDS lists stages in LDS; later entries go straight to the row.
 constexpr uint32_t kHeadWords = 20u;
@@ -920,8 +923,9 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, cons
 
     const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
     const __amdgpu_buffer_rsrc_t rxyz = xyz_rsrc(PACKED ? a.pxyz : nullptr, PACKED ? a.n : 0u);
-    // an agent outside the grid is stored in a cell that any of its runs may hold
-    const bool any_out = __ballot(alive && !inGrid(gp.x, gp.y, gp.z, sg.g)) != 0;
+    // an agent that is not sorted into the cell of its position (outside the grid, or
+    // moved since the sort) is stored in a cell that any of its runs may hold
+    const bool any_out = __ballot(alive && !holds(own, L.i)) != 0;
     uint32_t M[9];
 #pragma unroll
     for (int r = 0; r < 9; ++r) M[r] = 0u;
@@ -1082,10 +1086,10 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
         rows = can && (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, NR>(a, sg, L, gp, alive, own, all, put)
                                                  : scan_rows<false, NR>(a, sg, L, gp, alive, own, all, put));
         if (rows) L.cnt = all < a.K ? all : a.K;
-        have_own = can && __ballot(alive && !inGrid(gp.x, gp.y, gp.z, sg.g)) == 0;
+        have_own = can && __ballot(alive && !holds(own, L.i)) == 0;
     }
     if (!rows && !uniform) {
-        // the row scan has read the cells of agents inside the grid
+        // the row scan has read the own cells of agents sorted into them
         // dense waves (most lanes in cells of >= 8 agents) take rounds of
         // kGroupL candidates and skip the self test outside the agent's own
         // cell; sparse waves, dominated by per-cell overhead, take the short
