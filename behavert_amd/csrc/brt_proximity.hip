@@ -667,14 +667,19 @@ __device__ __forceinline__ uint32_t cells_of(uint32_t bx, uint32_t by, uint32_t 
     return x & y & z;
 }
 
+// The cells of the 27-neighbourhood that lie in the grid.
+__device__ __forceinline__ uint32_t grid_mask(const brt_grid_params& g, I3 gp) {
+    return cells_of(offset_bits(gp.x, 0, (int)g.grid_size[0] - 1), offset_bits(gp.y, 0, (int)g.grid_size[1] - 1),
+                    offset_bits(gp.z, 0, (int)g.grid_size[2] - 1));
+}
+
 // The cells of the 27-neighbourhood a lane visits: in the grid, and not an
 // interior cell whose box lies farther than r (same tests as the cell-by-cell
 // scan, without branches).
 __device__ __forceinline__ uint32_t visit_mask(const Seg& sg, const Lane& L, I3 gp, float Tskip) {
     const brt_grid_params& g = sg.g;
     const int gx = (int)g.grid_size[0], gy = (int)g.grid_size[1], gz = (int)g.grid_size[2];
-    const uint32_t in_grid = cells_of(offset_bits(gp.x, 0, gx - 1), offset_bits(gp.y, 0, gy - 1),
-                                      offset_bits(gp.z, 0, gz - 1));
+    const uint32_t in_grid = grid_mask(g, gp);
     const uint32_t inner = cells_of(offset_bits(gp.x, 1, gx - 2), offset_bits(gp.y, 1, gy - 2),
                                     offset_bits(gp.z, 1, gz - 2));
     uint32_t far = 0;
@@ -1668,7 +1673,9 @@ __device__ __forceinline__ void knn_scan(const ProxArgs& a, const Seg& sg, const
         }
     };
 
-    uint32_t todo = alive ? visit_mask(sg, L, gp, a.Tskip) : 0u;
+    // every cell in the grid: with positions that have moved since the sort, a
+    // cell's agents can lie outside its box
+    uint32_t todo = alive ? grid_mask(sg.g, gp) : 0u;
     uint32_t nc = 27u, ns = BRT_EMPTY_CELL, ne = 0u;
     flat_fetch(a, sg, gp, todo, nc, ns, ne);
     uint32_t j = 0u, lim = 0u;
@@ -1747,7 +1754,6 @@ __global__ void __launch_bounds__(64) k_neighbors_knn(ProxArgs a) {
     L.py = P.y;
     L.pz = P.z;
     const I3 gp = calcGridPos(P.x, P.y, P.z, sg.g);
-    cell_gaps(sg, L, gp);
     KnnList kl{s_mem + lane, reinterpret_cast<float*>(s_mem + (a.K + kKnnLog) * B) + lane, B, a.K, 0u, 0.0f};
     // the row scan's indices run on from the list into the log
     if (!knn_rows(a, sg, L, gp, alive, a.K + kKnnLog, kl)) {

@@ -1,14 +1,14 @@
 """Lists of positions that have moved since the sort (the reorder gathers new
 positions through the older permutation): an agent never enters its own list,
 wherever its position lies, on both sides of 2^17 agents and with every way of
-building the lists."""
+building the lists; KNN lists are the oracle's bits."""
 import numpy as np
 import pytest
 
 from behavert_amd import workloads as W
 from behavert_amd.types import OPT_LDS_LISTS, ProxParams
 
-from ._parity import dev, empty_u32, u32
+from ._parity import dev, empty_u32, first_mismatch, u32
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +48,13 @@ def test_no_agent_in_its_own_list(ctx, orc, n, lds, knn, per_cell, far):
     held = np.arange(16)[None, :] < lists[:, :1]
     assert held.any()
     assert not (held & (lists[:, 1:17] == np.arange(n, dtype=np.uint32)[:, None])).any()
+
+
+@pytest.mark.parametrize("per_cell", [1, 5, 30])
+@pytest.mark.parametrize("K", [4, 16])
+@pytest.mark.parametrize("far", [False, True])
+def test_knn_lists(ctx, orc, per_cell, K, far):
+    grid, h, s, e, spos = moved(orc, 4099, per_cell, far, K + per_cell)
+    prox = ProxParams.make(K, 4.0, use_knn=True)
+    lists = device_lists(ctx, grid, prox, h, s, e, spos)
+    assert first_mismatch(lists, orc.neighbors(grid, prox, spos, h, s, e)) is None
