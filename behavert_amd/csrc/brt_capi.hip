@@ -110,6 +110,26 @@ int ensure_xyz(brt_context* ctx, uint32_t n) {
     return BRT_OK;
 }
 
+bool ensure_records(brt_context* ctx, size_t need, hipStream_t s) {
+    if (need <= ctx->records_bytes) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ctx->records && hipFree(ctx->records) != hipSuccess) return false;
+    ctx->records = nullptr;
+    ctx->records_bytes = 0;
+    const size_t bytes = need + need / 4 + 4096;
+    if (hipMalloc(&ctx->records, bytes) != hipSuccess) {
+        ctx->records = nullptr;
+        (void)hipGetLastError();  // the caller goes on without
+        return false;
+    }
+    ctx->records_bytes = bytes;
+    return true;
+}
+
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan) {
     // 8 bytes per agent for the sort; 16 so that the passes over its lists (sorted
     // features, labels) find their scratch there
@@ -257,6 +277,7 @@ int brt_context_destroy(brt_context* ctx) {
     if (ctx->meta) (void)hipFree(ctx->meta);
     if (ctx->partials) (void)hipFree(ctx->partials);
     if (ctx->xyz) (void)hipFree(ctx->xyz);
+    if (ctx->records) (void)hipFree(ctx->records);
     if (ctx->dev_flags) (void)hipFree(ctx->dev_flags);
     for (auto& g : ctx->graphs) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -905,7 +926,7 @@ struct StepScratch {
     uint32_t* meta;
     void* tmp;
     float* xyz;
-    size_t tmp_bytes;
+    void* records;  // NULL: the step moves its state as arrays
 };
 
 // Two-pass steps of this many agents or more, with the feature update, wander or
@@ -919,25 +940,15 @@ struct StepScratch {
 #define BRT_STEP_RECORDS_MIN (1u << 19)
 #endif
 
-// What a two-pass step keeps in its tmp scratch after the sort.
-struct StepTmp {
-    size_t features = 0, records = 0, ssa = 0, bytes = 0;  // byte offsets, and the whole
-    bool use_records = false;
-};
-StepTmp step_tmp(uint32_t n, bool two_pass, bool features, bool own_ssa, bool wander) {
-    StepTmp t;
-    if (!two_pass) return t;
-    if (features) t.bytes = (size_t)n * 16u;
-    t.use_records = n >= BRT_STEP_RECORDS_MIN && (features || own_ssa || wander);
-    if (t.use_records) {
-        t.records = (t.bytes + 63u) / 64u * 64u;
-        t.bytes = t.records + (size_t)n * 64u;
-        if (!own_ssa) {
-            t.ssa = t.bytes;
-            t.bytes += (size_t)n * 16u;
-        }
-    }
-    return t;
+// The records of a two-pass step: 64 bytes per agent by ID, then the smoothed
+// acceleration in sorted order where the caller keeps no copy of it; 0 for a step
+// that moves its state as arrays.  They have a buffer of their own, and a step that
+// cannot get it (under capture, or out of memory) moves arrays: which options a
+// step has never decides whether its scratch suffices, nor moves the scratch that
+// an earlier call was captured with.
+size_t step_record_bytes(uint32_t n, bool two_pass, bool features, bool keeps_ssa, bool wander) {
+    if (!two_pass || n < BRT_STEP_RECORDS_MIN || !(features || keeps_ssa || wander)) return 0;
+    return (size_t)n * (keeps_ssa ? 64u : 80u);
 }
 
 int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_params* prox,
@@ -1009,9 +1020,16 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // call of the same size may take (another grid), under capture too
     const bool cell_sort = brt::cell_sort_cells(n, grid->num_cells) != 0u;
     if (!given && cell_sort && (rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells)))) return rc;
-    StepTmp st = step_tmp(n, two_pass, sorted_features, b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f);
-    if (given && given->tmp_bytes < st.bytes) st.use_records = false;
-    if (!given && (rc = ensure_tmp(ctx, st.bytes))) return rc;
+    if (!given && sorted_features && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    const size_t record_bytes = step_record_bytes(n, two_pass, sorted_features, b->sorted_smooth_accel != nullptr,
+                                                  steer->wander_weight != 0.0f);
+    char* records = nullptr;
+    if (record_bytes != 0u && !cell_sort) {
+        if (given)
+            records = reinterpret_cast<char*>(given->records);
+        else if (ensure_records(ctx, record_bytes, s))
+            records = reinterpret_cast<char*>(ctx->records);
+    }
     // with LDS lists the neighbour scan reads candidate positions from a
     // packed x,y,z copy written by the reorder (three 16-byte loads per four
     // candidates; the register-list scan measured no gain from it)
@@ -1050,7 +1068,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // with records the smoothed acceleration comes with the rest of the record
     float* const ssa = b->sorted_smooth_accel
                            ? b->sorted_smooth_accel
-                           : (st.use_records ? reinterpret_cast<float*>((char*)tmp + st.ssa) : nullptr);
+                           : (records ? reinterpret_cast<float*>(records + (size_t)n * 64u) : nullptr);
     if (ssa) {
         f.in[nf] = reinterpret_cast<const float4*>(b->smooth_accel);
         f.out[nf++] = reinterpret_cast<float4*>(ssa);
@@ -1062,8 +1080,8 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     f.count = nf;
     f.xyz0 = xyz;
     mark_phase(1);
-    float4* const rec = st.use_records ? reinterpret_cast<float4*>((char*)tmp + st.records) : nullptr;
-    if (rec && !cell_sort) {
+    float4* const rec = reinterpret_cast<float4*>(records);
+    if (rec) {
         const hipEvent_t stop = brt::launch_mark().stop;
         brt::launch_mark().stop = nullptr;
         BRT_HIP(brt::launch_pack(n, f.in[0], f.in[1], f.in[2], nf > 3u ? f.in[3] : nullptr, rec, s), "k_pack");
@@ -1173,7 +1191,7 @@ std::vector<unsigned char> step_key(const brt_context* ctx, const brt_grid_param
 // context's scratch (grown first, outside the capture) and keeps it.
 int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_params* prox,
                  const brt_steer_params* steer, float feature_rate, float dt, uint32_t step,
-                 const brt_step_buffers* b, std::vector<unsigned char>&& key) {
+                 const brt_step_buffers* b, hipStream_t s, std::vector<unsigned char>&& key) {
     const uint32_t n = b->n;
     const bool do_features = b->features && b->features_out && feature_rate != 0.0f;
     const StepShape shape = resolve_step(ctx, prox, n, grid->num_cells, do_features);
@@ -1181,10 +1199,10 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
     const bool pack = !prox->use_knn && (shape.lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
     int rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells));
     if (rc) return rc;
-    if ((rc = ensure_tmp(ctx, step_tmp(n, two_pass, do_features && two_pass,
-                                       b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f)
-                                  .bytes)))
-        return rc;
+    if (do_features && two_pass && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    const size_t record_bytes = step_record_bytes(n, two_pass, do_features && two_pass,
+                                                  b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f);
+    const bool records = record_bytes != 0u && ensure_records(ctx, record_bytes, s);
     if (pack && (rc = ensure_xyz(ctx, n))) return rc;
     if (!ctx->cap_stream)
         BRT_HIP(hipStreamCreateWithFlags(&ctx->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
@@ -1192,7 +1210,7 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
         destroy_step_graph(ctx->graphs.front());
         ctx->graphs.erase(ctx->graphs.begin());
     }
-    StepScratch sc{ctx->meta, ctx->tmp, ctx->xyz, ctx->tmp_bytes};
+    StepScratch sc{ctx->meta, ctx->tmp, ctx->xyz, records ? ctx->records : nullptr};
     BRT_HIP(hipStreamBeginCapture(ctx->cap_stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     rc = step_core(ctx, grid, prox, steer, feature_rate, dt, step, b, ctx->cap_stream, &sc);
     hipGraph_t g = nullptr;
@@ -1208,6 +1226,7 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
     ng.tmp = ctx->tmp;
     ng.meta = ctx->meta;
     ng.xyz = ctx->xyz;
+    ng.records = ctx->records;
     const hipError_t ie = hipGraphInstantiate(&ng.exec, ng.graph, nullptr, nullptr, 0);
     if (ie != hipSuccess) {
         destroy_step_graph(ng);
@@ -1235,7 +1254,9 @@ int brt_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_param
     size_t hit = ctx->graphs.size();
     for (size_t k = 0; k < ctx->graphs.size(); ++k) {
         const brt_context::StepGraph& g = ctx->graphs[k];
-        if (g.key == key && g.tmp == ctx->tmp && g.meta == ctx->meta && g.xyz == ctx->xyz) hit = k;
+        if (g.key == key && g.tmp == ctx->tmp && g.meta == ctx->meta && g.xyz == ctx->xyz &&
+            g.records == ctx->records)
+            hit = k;
     }
     if (hit == ctx->graphs.size()) {
         // the first call with a key runs (and checks its arguments) directly;
@@ -1247,7 +1268,7 @@ int brt_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_param
         }
         int rc = use_device(ctx);
         if (rc) return rc;
-        if ((rc = capture_step(ctx, grid, prox, steer, feature_rate, dt, step, b, std::move(key)))) return rc;
+        if ((rc = capture_step(ctx, grid, prox, steer, feature_rate, dt, step, b, s, std::move(key)))) return rc;
     } else if (hit + 1 != ctx->graphs.size()) {
         std::swap(ctx->graphs[hit], ctx->graphs.back());
     }
@@ -1273,7 +1294,7 @@ int brt_step_noalloc(brt_context* ctx, const brt_grid_params* grid, const brt_pr
     sc.meta = reinterpret_cast<uint32_t*>(base + kNoAllocMetaOffset);
     sc.tmp = base + kNoAllocTmpOffset;
     sc.xyz = reinterpret_cast<float*>(base + kNoAllocXyzOffset);
-    sc.tmp_bytes = (size_t)BRT_NOALLOC_MAX_AGENTS * 16u;
+    sc.records = nullptr;
     return step_core(ctx, grid, prox, steer, feature_rate, dt, step, b, stream, &sc);
 }
 

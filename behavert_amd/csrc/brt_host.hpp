@@ -26,6 +26,8 @@ struct brt_context {
     size_t partials_bytes = 0;
     float* xyz = nullptr;       // brt_step: the sorted positions packed as x,y,z
     size_t xyz_bytes = 0;
+    void* records = nullptr;    // brt_step: the state by ID as records (step_record_bytes)
+    size_t records_bytes = 0;
     uint32_t* dev_flags = nullptr;  // sticky device-side failure flags (BRT_DEVFLAG_*)
     void* scratch = nullptr;        // this device's no-allocation step scratch (a static device array)
     bool timing = false;
@@ -50,6 +52,7 @@ struct brt_context {
         void* tmp = nullptr;  // the scratch the graph was captured with
         uint32_t* meta = nullptr;
         float* xyz = nullptr;
+        void* records = nullptr;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
     };
@@ -124,6 +127,8 @@ int check_prox(brt_context* ctx, const brt_prox_params* p);
 int check_steer(brt_context* ctx, const brt_steer_params* s);
 int ensure_tmp(brt_context* ctx, size_t bytes);
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan);
+// whether the context's records hold `need` bytes; they do not grow while s is being captured
+bool ensure_records(brt_context* ctx, size_t need, hipStream_t s);
 // synchronises the device, reads and clears the sticky flags; BRT_ERR_HIP with
 // a message when one was raised
 int check_dev_flags(brt_context* ctx);
