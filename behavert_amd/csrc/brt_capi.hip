@@ -97,37 +97,37 @@ int ensure_tmp(brt_context* ctx, size_t need_tmp) {
     return BRT_OK;
 }
 
-int ensure_xyz(brt_context* ctx, uint32_t n) {
-    const size_t need = (size_t)n * 12u;
-    if (need > ctx->xyz_bytes) {
-        if (ctx->xyz) BRT_HIP(hipFree(ctx->xyz), "hipFree(xyz)");
-        ctx->xyz = nullptr;
-        ctx->xyz_bytes = 0;
-        const size_t bytes = need + need / 4 + 4096;
-        BRT_HIP(hipMalloc((void**)&ctx->xyz, bytes), "hipMalloc(xyz)");
-        ctx->xyz_bytes = bytes;
-    }
-    return BRT_OK;
-}
-
-bool ensure_records(brt_context* ctx, size_t need, hipStream_t s) {
-    if (need <= ctx->records_bytes) return true;
+// Grows a buffer that its caller can do without; false: it is too small and
+// cannot grow (s is being captured, or no memory).
+static bool grow_optional(void*& p, size_t& have, size_t need, hipStream_t s) {
+    if (need <= have) return true;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return false;
     }
-    if (ctx->records && hipFree(ctx->records) != hipSuccess) return false;
-    ctx->records = nullptr;
-    ctx->records_bytes = 0;
-    const size_t bytes = need + need / 4 + 4096;
-    if (hipMalloc(&ctx->records, bytes) != hipSuccess) {
-        ctx->records = nullptr;
-        (void)hipGetLastError();  // the caller goes on without
+    if (p && hipFree(p) != hipSuccess) {
+        (void)hipGetLastError();
         return false;
     }
-    ctx->records_bytes = bytes;
+    p = nullptr;
+    have = 0;
+    const size_t bytes = need + need / 4 + 4096;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        p = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    have = bytes;
     return true;
+}
+
+bool ensure_records(brt_context* ctx, size_t need, hipStream_t s) {
+    return grow_optional(ctx->records, ctx->records_bytes, need, s);
+}
+
+float* step_xyz(brt_context* ctx, uint32_t n, hipStream_t s) {
+    return grow_optional(ctx->xyz, ctx->xyz_bytes, (size_t)n * 12u, s) ? reinterpret_cast<float*>(ctx->xyz) : nullptr;
 }
 
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan) {
@@ -1035,8 +1035,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // candidates; the register-list scan measured no gain from it)
     const uint32_t lds = shape.lds;
     const bool pack = !prox->use_knn && (lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
-    if (!given && pack && (rc = ensure_xyz(ctx, n))) return rc;
-    float* xyz = pack ? (given ? given->xyz : ctx->xyz) : nullptr;
+    float* xyz = pack ? (given ? given->xyz : step_xyz(ctx, n, s)) : nullptr;
     void* tmp = nullptr;
     if (cell_sort) {
         // phase 0 is the hash alone: the sort runs with the reorder, in phase 1
@@ -1203,14 +1202,14 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
     const size_t record_bytes = step_record_bytes(n, two_pass, do_features && two_pass,
                                                   b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f);
     const bool records = record_bytes != 0u && ensure_records(ctx, record_bytes, s);
-    if (pack && (rc = ensure_xyz(ctx, n))) return rc;
+    float* const xyz = pack ? step_xyz(ctx, n, s) : nullptr;
     if (!ctx->cap_stream)
         BRT_HIP(hipStreamCreateWithFlags(&ctx->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
     if (ctx->graphs.size() == 2) {
         destroy_step_graph(ctx->graphs.front());
         ctx->graphs.erase(ctx->graphs.begin());
     }
-    StepScratch sc{ctx->meta, ctx->tmp, ctx->xyz, records ? ctx->records : nullptr};
+    StepScratch sc{ctx->meta, ctx->tmp, xyz, records ? ctx->records : nullptr};
     BRT_HIP(hipStreamBeginCapture(ctx->cap_stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     rc = step_core(ctx, grid, prox, steer, feature_rate, dt, step, b, ctx->cap_stream, &sc);
     hipGraph_t g = nullptr;

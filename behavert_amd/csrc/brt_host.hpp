@@ -24,7 +24,7 @@ struct brt_context {
     bool meta_clean = false;
     float* partials = nullptr;  // adjoint: per-workgroup weight-gradient partials
     size_t partials_bytes = 0;
-    float* xyz = nullptr;       // brt_step: the sorted positions packed as x,y,z
+    void* xyz = nullptr;        // brt_step: the sorted positions packed as x,y,z
     size_t xyz_bytes = 0;
     void* records = nullptr;    // brt_step: the state by ID as records (step_record_bytes)
     size_t records_bytes = 0;
@@ -51,7 +51,7 @@ struct brt_context {
         std::vector<unsigned char> key;
         void* tmp = nullptr;  // the scratch the graph was captured with
         uint32_t* meta = nullptr;
-        float* xyz = nullptr;
+        void* xyz = nullptr;
         void* records = nullptr;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
@@ -127,8 +127,11 @@ int check_prox(brt_context* ctx, const brt_prox_params* p);
 int check_steer(brt_context* ctx, const brt_steer_params* s);
 int ensure_tmp(brt_context* ctx, size_t bytes);
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan);
-// whether the context's records hold `need` bytes; they do not grow while s is being captured
+// Scratch that a step can do without and that does not grow while s is being
+// captured: whether the records hold `need` bytes; the packed positions of n
+// agents, or NULL (the neighbour search then reads the float4 ones).
 bool ensure_records(brt_context* ctx, size_t need, hipStream_t s);
+float* step_xyz(brt_context* ctx, uint32_t n, hipStream_t s);
 // synchronises the device, reads and clears the sticky flags; BRT_ERR_HIP with
 // a message when one was raised
 int check_dev_flags(brt_context* ctx);

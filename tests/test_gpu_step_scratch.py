@@ -135,3 +135,21 @@ def test_step_graph_and_no_allocation_step(own, wander, features):
             fl.features, fl.features_out = fl.features_out, fl.features
         torch.cuda.synchronize()
         assert same(outputs(flocks[0]), outputs(flocks[1])) and same(outputs(flocks[0]), outputs(flocks[2]))
+
+
+@pytest.mark.parametrize("n,K", [((1 << 17) + 77, 48), (5000, 100)])
+def test_captured_without_packed_positions(own, n, K):
+    """Fused steps beyond K 32 after a warm-up whose search takes no packed
+    positions: two passes with the feature update, KNN lists."""
+    grid, prox, st = inputs(K, n)
+    want = eager(grid, prox, st, 3)
+    fl = flock(own, grid, prox, st, features=n > 1 << 17)
+    if n > 1 << 17:
+        fl.step(DT, 0, 0.1)
+        fl.features = fl.features_out = None
+    else:
+        fl.prox = ProxParams.make(K, 4.0, use_knn=True)
+        fl.step(DT, 0)
+        fl.prox = prox
+    put(fl, st)
+    replay_equals(capture(fl), fl, want)
