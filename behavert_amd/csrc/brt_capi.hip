@@ -130,10 +130,13 @@ float* step_xyz(brt_context* ctx, uint32_t n, hipStream_t s) {
     return grow_optional(ctx->xyz, ctx->xyz_bytes, (size_t)n * 12u, s) ? reinterpret_cast<float*>(ctx->xyz) : nullptr;
 }
 
+// Bytes per agent that the sort (8), the label propagation (8), the hit rate and the
+// sorted features (16) ask for alike: any one of them is a warm-up for the others
+// before a capture, and none moves the scratch that another was captured with.
+constexpr size_t kListScratch = 16u;
+
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan) {
-    // 8 bytes per agent for the sort; 16 so that the passes over its lists (sorted
-    // features, labels) find their scratch there
-    int rc = ensure_tmp(ctx, (size_t)n * 16u);
+    int rc = ensure_tmp(ctx, (size_t)n * kListScratch);
     if (rc) return rc;
     size_t need_meta = brt::sort_meta_words(plan) * 4u;
     if (need_meta > ctx->meta_bytes) {
@@ -794,7 +797,7 @@ int brt_bc_cluster_membership(brt_context* ctx, const brt_prox_params* prox, uin
     if ((rc = use_device(ctx))) return rc;
     float* lbl = nullptr;
     if (iterations >= 2) {
-        if ((rc = ensure_tmp(ctx, (size_t)n * 8u))) return rc;
+        if ((rc = ensure_tmp(ctx, (size_t)n * kListScratch))) return rc;
         lbl = reinterpret_cast<float*>(ctx->tmp);
     }
     BRT_HIP(brt::launch_cluster_membership(prox->max_neighbors, n, iterations, reinterpret_cast<const uint2*>(hash),
@@ -819,7 +822,7 @@ int brt_bc_cluster_hit_rate(brt_context* ctx, const brt_prox_params* prox, float
     BRT_REQUIRE(((uintptr_t)membership_in & 3u) == 0 && ((uintptr_t)membership_out & 3u) == 0,
                 "membership arrays misaligned");
     if ((rc = use_device(ctx))) return rc;
-    if ((rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    if ((rc = ensure_tmp(ctx, (size_t)n * kListScratch))) return rc;
     BRT_HIP(brt::launch_hit_rate(prox->max_neighbors, same_cluster_max_radius, n, reinterpret_cast<const uint2*>(hash),
                                  lists, reinterpret_cast<const float4*>(sorted_pos), membership_in, membership_out,
                                  reinterpret_cast<float4*>(ctx->tmp), ctx->xcd_remap, (hipStream_t)stream),
@@ -1020,7 +1023,7 @@ int step_core(brt_context* ctx, const brt_grid_params* grid, const brt_prox_para
     // call of the same size may take (another grid), under capture too
     const bool cell_sort = brt::cell_sort_cells(n, grid->num_cells) != 0u;
     if (!given && cell_sort && (rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells)))) return rc;
-    if (!given && sorted_features && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    if (!given && sorted_features && (rc = ensure_tmp(ctx, (size_t)n * kListScratch))) return rc;
     const size_t record_bytes = step_record_bytes(n, two_pass, sorted_features, b->sorted_smooth_accel != nullptr,
                                                   steer->wander_weight != 0.0f);
     char* records = nullptr;
@@ -1198,7 +1201,7 @@ int capture_step(brt_context* ctx, const brt_grid_params* grid, const brt_prox_p
     const bool pack = !prox->use_knn && (shape.lds != 0u || resolve_quads(ctx, prox, n, !two_pass));
     int rc = ensure_scratch(ctx, n, brt::make_sort_plan(n, grid->num_cells));
     if (rc) return rc;
-    if (do_features && two_pass && (rc = ensure_tmp(ctx, (size_t)n * 16u))) return rc;
+    if (do_features && two_pass && (rc = ensure_tmp(ctx, (size_t)n * kListScratch))) return rc;
     const size_t record_bytes = step_record_bytes(n, two_pass, do_features && two_pass,
                                                   b->sorted_smooth_accel != nullptr, steer->wander_weight != 0.0f);
     const bool records = record_bytes != 0u && ensure_records(ctx, record_bytes, s);

@@ -1,7 +1,8 @@
-"""The scratch of a step against captures and other calls on the same context: a
+"""The scratch of a context against captures and other calls on the same context: a
 step captured into a caller's graph after a warm-up with other options runs, a
 captured step keeps its scratch while eager steps with other options run, and the
-steps that move their state as records equal those that cannot."""
+steps that move their state as records equal those that cannot; so for the passes
+over the lists."""
 import ctypes as C
 
 import numpy as np
@@ -153,3 +154,26 @@ def test_captured_without_packed_positions(own, n, K):
         fl.prox = prox
     put(fl, st)
     replay_equals(capture(fl), fl, want)
+
+
+def test_hit_rate_captured_after_the_label_propagation(own):
+    n = 20003
+    grid, prox, st = inputs(16, n)
+    other = Context(0)
+    fl = flock(other, grid, prox, st)
+    fl.reorder_sim_data()
+    fl.compute_neighborhoods()
+    zero = torch.zeros(n, 3, device="cuda")
+    label, want, got = torch.empty_like(zero), torch.empty_like(zero), torch.empty_like(zero)
+    own.cluster_membership(prox, 10, fl.hash, fl.lists, fl.sorted_pos, zero, label)
+    other.cluster_hit_rate(prox, 3.0, fl.hash, fl.lists, fl.sorted_pos, label, want)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        own.cluster_hit_rate(prox, 3.0, fl.hash, fl.lists, fl.sorted_pos, label, got)
+    for _ in range(3):
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert same([got], [want])
+    other.close()
