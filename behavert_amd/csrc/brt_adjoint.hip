@@ -836,8 +836,6 @@ constexpr uint32_t kOwnQuadMax = 1u << 17;
 
 }  // namespace
 
-uint32_t adjoint_own_blocks(uint32_t n) { return n <= kOwnQuadMax ? (n + 63u) / 64u : (n + 255u) / 256u; }
-
 hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                           const brt_steer_params& sp, float dt, uint32_t n, const float4* spos, const float4* sfwd,
                           const float4* ssa, const uint2* hash, const uint32_t* lists, const uint32_t* cell_start,
@@ -864,7 +862,7 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
     a.partials = partials;
     a.xcd_remap = xcd_remap;
     const bool quads = n <= kOwnQuadMax;
-    const uint32_t blocks = adjoint_own_blocks(n);
+    const uint32_t blocks = quads ? (n + 63u) / 64u : (n + 255u) / 256u;
     if (quads)
         hipLaunchKernelGGL(k_adjoint_own_quad, dim3(blocks), dim3(256), 0, s, a);
     else

@@ -613,8 +613,9 @@ int brt_osw_adjoint_step(brt_context* ctx, const brt_grid_params* grid, const br
                     adj_smooth_accel_in != adj_smooth_accel_out,
                 "adjoint input and output arrays must differ");
     if ((rc = use_device(ctx))) return rc;
-    // per-workgroup weight-gradient partials
-    const size_t need = (size_t)brt::adjoint_own_blocks(n) * 3 * sizeof(float) + 256;
+    // per-workgroup weight-gradient partials: those of 64 agents at every size, so
+    // that a smaller flock (which has more of them) never moves a larger one's
+    const size_t need = (size_t)((n + 63u) / 64u) * 3 * sizeof(float) + 256;
     if (need > ctx->partials_bytes) {
         if (ctx->partials) BRT_HIP(hipFree(ctx->partials), "hipFree(partials)");
         ctx->partials = nullptr;

@@ -193,9 +193,8 @@ hipError_t launch_move_towards_target(int shift, const float base[3], uint32_t n
                                       float4* force_out, hipStream_t s);
 
 // adjoint
-// scratch: adjoint_scratch_bytes(n), 64-byte aligned; partials: 3 floats for each of adjoint_own_blocks(n)
+// scratch: adjoint_scratch_bytes(n), 64-byte aligned; partials: 3 floats for each 64 agents
 inline size_t adjoint_scratch_bytes(uint32_t n) { return (size_t)n * 112u; }
-uint32_t adjoint_own_blocks(uint32_t n);
 hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, float threshold,
                           const brt_steer_params& sp, float dt, uint32_t n, const float4* spos, const float4* sfwd,
                           const float4* ssa, const uint2* hash, const uint32_t* lists, const uint32_t* cell_start,

@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from behavert_amd import workloads as W
+from behavert_amd.autograd import Rollout
 from behavert_amd.engine import Context, Flock, current_stream
 from behavert_amd.types import OPT_STEP_GRAPH, ProxParams, SteerParams
 
@@ -176,4 +177,34 @@ def test_hit_rate_captured_after_the_label_propagation(own):
         g.replay()
         torch.cuda.synchronize()
         assert same([got], [want])
+    other.close()
+
+
+def adjoint(c, n):
+    """One step's records and adjoint seeds of a flock, ready for its adjoint call."""
+    grid, prox, st = inputs(8, n)
+    r = Rollout(c, grid, prox, steer_with(False), n, DT, 1, 1, overlap=False)
+    r.forward((1.0, 0.8, 0.6), *[torch.from_numpy(st[k]).cuda() for k in ("pos", "forward", "smooth_accel")])
+    r._replay(r.checkpoints[0], 0, c)
+    for k, t in enumerate(r.g[0]):
+        t.normal_(generator=torch.Generator(device="cuda").manual_seed(k))
+    return r
+
+
+def test_adjoint_captured_after_a_larger_flocks(own):
+    """A flock of the four-lane adjoint, whose workgroups are smaller."""
+    large, small, other = adjoint(own, 200003), adjoint(own, 131072), Context(0)
+    large._adjoint(0, 0, 0)
+    ref = adjoint(other, 131072)
+    ref._adjoint(0, 0, 0)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        small._adjoint(0, 0, 0)
+    for _ in range(3):
+        small.wgrad.zero_()
+        large._adjoint(0, 0, 0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert same([small.wgrad, *small.g[1]], [ref.wgrad, *ref.g[1]])
     other.close()
