@@ -166,14 +166,47 @@ inline uint32_t similarity_wave_bytes(uint32_t K, uint32_t W) {
 }
 
 // Stores the similarities of a wave's agents out of LDS: rows of RW words, K + 1
-// of them contiguous in sims.
+// of them contiguous in sims.  vec: sims is 16-byte aligned, and so is the wave's
+// first row; then 16 bytes per lane per store (similarities alone of 100,003 agents, F 8,
+// short lists: K 32 16.6 -> 15.6, K 128 38 -> 28, K 252 99 -> 57 us).
 __device__ __forceinline__ void store_similarities(float* __restrict__ sims, uint32_t row0, uint32_t n, uint32_t K,
-                                                   uint32_t RW, const float* src, uint32_t lane) {
+                                                   uint32_t RW, const float* src, uint32_t lane, uint32_t vec) {
     const uint32_t S = K + 1u, total = (n - row0 < 64u ? n - row0 : 64u) * S;
     float* const dst = sims + (size_t)row0 * S;
+    uint32_t x = 0u;  // the words stored so far
+    if (vec) {
+        const uint32_t total4 = total / 4u;
+        x = 4u * total4;
+        if (RW == S) {
+            for (uint32_t t = lane; t < total4; t += 64u)
+                reinterpret_cast<float4*>(dst)[t] = reinterpret_cast<const float4*>(src)[t];
+        } else {
+            const uint32_t dr = 256u / S, dc = 256u - dr * S;
+            uint32_t r = 4u * lane / S, c = 4u * lane - r * S;
+            for (uint32_t t = lane; t < total4; t += 64u) {
+                float v[4];
+                uint32_t at = r * RW + c, cc = c;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    v[k] = src[at];
+                    const bool wrap = ++cc == S;
+                    at += wrap ? RW - S + 1u : 1u;
+                    cc = wrap ? 0u : cc;
+                }
+                reinterpret_cast<float4*>(dst)[t] = make_float4(v[0], v[1], v[2], v[3]);
+                r += dr;
+                c += dc;
+                if (c >= S) {
+                    c -= S;
+                    ++r;
+                }
+            }
+        }
+    }
     const uint32_t dr = 64u / S, dc = 64u - dr * S;
-    uint32_t r = lane / S, c = lane - r * S;
-    for (uint32_t x = lane; x < total; x += 64u) {
+    x += lane;
+    uint32_t r = x / S, c = x - r * S;
+    for (; x < total; x += 64u) {
         dst[x] = src[r * RW + c];
         r += dr;
         c += dc;
@@ -255,7 +288,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
                                                          const float* __restrict__ norms,
                                                          const float4* __restrict__ stats_in,
                                                          float4* __restrict__ stats_out, float* __restrict__ sims,
-                                                         uint32_t xcd_remap) {
+                                                         uint32_t sims_vec, uint32_t xcd_remap) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t row0 = xcd_block(xcd_remap) * blockDim.x + wave * 64u, i = row0 + lane;
     if (row0 >= n) return;
@@ -267,7 +300,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
         similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, mem + lane * RW,
                                        staged);
     wave_lds_sync();
-    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane);
+    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane, sims_vec);
 }
 
 // ---- similarities and cluster steering in one pass
@@ -342,7 +375,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     uint32_t K, uint32_t W, brt_bc_params bc, uint32_t n, const uint2* __restrict__ hash,
     const uint32_t* __restrict__ lists, const float4* __restrict__ rec, const float4* __restrict__ stats_in,
     float4* __restrict__ stats_out, float* __restrict__ sims, brt_steer_params sp, const float4* __restrict__ sfwd,
-    const float4* force_in, float4* force_out, uint32_t wave_bytes, uint32_t xcd_remap) {
+    const float4* force_in, float4* force_out, uint32_t wave_bytes, uint32_t sims_vec, uint32_t xcd_remap) {
     constexpr int NR = record_rounds<FQ>();
     constexpr uint32_t RP = 4u * NR;
     constexpr int G = NR == 1 ? 4 : (NR == 2 ? 2 : 1);  // entries in flight
@@ -452,7 +485,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
         force_out[i] = acc.finish(count, myFwd, bc, force_in[i]);
     }
     wave_lds_sync();
-    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane);
+    store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane, sims_vec);
 }
 
 // steerForClusterCohesion + Alignment from stored similarities.
@@ -662,6 +695,7 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
                        void* scratch, const brt_steer_params* sp, const float4* spos, const float4* sfwd,
                        const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
     const uint32_t F = bc.feature_count, W = list_stride(K);
+    const uint32_t sims_vec = ((uintptr_t)sims & 15u) == 0 ? 1u : 0u;
     if (sp) {
         constexpr uint32_t RP = 4u * record_rounds<FQ>();
         float4* rec = reinterpret_cast<float4*>(scratch);
@@ -673,11 +707,11 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
         if (bc.adaptive)
             hipLaunchKernelGGL((k_bc_similarities_steer<true, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n, hash,
                                lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
-                               xcd_remap);
+                               sims_vec, xcd_remap);
         else
             hipLaunchKernelGGL((k_bc_similarities_steer<false, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n,
                                hash, lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
-                               xcd_remap);
+                               sims_vec, xcd_remap);
         return hipGetLastError();
     }
     float4* sfeat = reinterpret_cast<float4*>(scratch);
@@ -691,10 +725,10 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
     const dim3 grid((n + B - 1) / B), block(B);
     if (bc.adaptive)
         hipLaunchKernelGGL((k_bc_similarities<true, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, xcd_remap);
+                           stats_in, stats_out, sims, sims_vec, xcd_remap);
     else
         hipLaunchKernelGGL((k_bc_similarities<false, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, xcd_remap);
+                           stats_in, stats_out, sims, sims_vec, xcd_remap);
     return hipGetLastError();
 }
 
