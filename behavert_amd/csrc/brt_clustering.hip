@@ -489,6 +489,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
 }
 
 // steerForClusterCohesion + Alignment from stored similarities.
+template <ListRows ROWS>
 __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W, brt_steer_params sp,
                                                           brt_bc_params bc, uint32_t n,
                                                           const float4* __restrict__ spos,
@@ -497,9 +498,9 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
                                                           const float* __restrict__ sims,
                                                           const float4* force_in, float4* force_out,
                                                           uint32_t xcd_remap) {
-    __shared__ uint4 s_stage[4][kStageChunks];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(ROWS == kRowsOwn ? 0u : xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
     const float4 P = spos[at], Fw = sfwd[at];
     const V3 myPos = xyz(P), myFwd = xyz(Fw);
@@ -507,7 +508,7 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
     const float* s = sims + (size_t)at * (K + 1u);
     ClusterAccum acc;
     acc.init();
-    const uint32_t count = wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
+    const uint32_t count = walk_list<ROWS>(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
         float4 op[8], of[8];
         float sv[8];
 #pragma unroll
@@ -537,16 +538,17 @@ __global__ void __launch_bounds__(256) k_bc_cluster_steer(uint32_t K, uint32_t W
 // The first iteration reads no labels (they are the indices themselves) and
 // the last writes the float3 by ID and the connector.  Same values: a min of
 // the same operands, the same T, no rounding.
-template <bool FIRST, bool LAST, bool SCAN>
+// SCAN: false without iterations (the labels are the indices).
+template <bool FIRST, bool LAST, ListRows ROWS, bool SCAN = true>
 __global__ void __launch_bounds__(256) k_lp_iterate(uint32_t K, uint32_t W, uint32_t n, const uint2* __restrict__ hash,
                                                     const uint32_t* __restrict__ lists,
                                                     const float* __restrict__ lbl_in, float* __restrict__ lbl_out,
                                                     const float* m_in, float* m_out,
                                                     const float4* __restrict__ spos, float4* __restrict__ conn,
                                                     uint32_t xcd_remap) {
-    __shared__ uint4 s_stage[SCAN ? 4 : 1][SCAN ? kStageChunks : 1];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x, at = i < n ? i : n - 1u;
+    const uint32_t i = xcd_block(ROWS == kRowsOwn ? 0u : xcd_remap) * blockDim.x + threadIdx.x, at = i < n ? i : n - 1u;
     float mn = FIRST ? (float)i : lbl_in[at];
     // the last iteration's reads by ID load during the walk
     uint32_t id = n;
@@ -561,7 +563,7 @@ __global__ void __launch_bounds__(256) k_lp_iterate(uint32_t K, uint32_t W, uint
         if (conn) P = spos[at];
     }
     if (SCAN) {
-        wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+        walk_list<ROWS>(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
             float v[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] = FIRST ? (float)jj[k] : lbl_in[jj[k]];
@@ -604,20 +606,21 @@ __global__ void __launch_bounds__(256) k_gather_labels(uint32_t n, const uint2* 
 // T: the greatest squared length within the radius (length(o) > radius exactly
 // when dot(o, o) > T, the square root being correctly rounded).  1M blobs, K 32,
 // with the labels gathered beside the positions: 114.8 -> 65 us.
+template <ListRows ROWS>
 __global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float T, uint32_t n,
                                                   const uint2* __restrict__ hash, const uint32_t* __restrict__ lists,
                                                   const float4* __restrict__ lbl, float* __restrict__ m_out,
                                                   uint32_t xcd_remap) {
-    __shared__ uint4 s_stage[4][kStageChunks];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(ROWS == kRowsOwn ? 0u : xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t id = i < n ? hash[i].y : n;
     const float4 own = lbl[i < n ? i : n - 1u];
     const float my = own.w;
     const V3 myPos = xyz(own);
     int close = 0;
     float real = 0.0f, hit = 0.0f;
-    wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+    walk_list<ROWS>(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
         float4 op[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) op[k] = lbl[jj[k]];
@@ -646,35 +649,50 @@ __global__ void __launch_bounds__(256) k_hit_rate(uint32_t K, uint32_t W, float 
 
 }  // namespace
 
-hipError_t launch_cluster_membership(uint32_t K, uint32_t n, uint32_t iterations, const uint2* hash,
-                                     const uint32_t* lists, const float4* spos, const float* m_in, float* m_out,
-                                     float4* conn, float* lbl_a, float* lbl_b, uint32_t xcd_remap, hipStream_t s) {
+namespace {
+
+template <ListRows ROWS>
+hipError_t launch_label_iterations(uint32_t K, uint32_t n, uint32_t iterations, const uint2* hash,
+                                   const uint32_t* lists, const float4* spos, const float* m_in, float* m_out,
+                                   float4* conn, float* lbl_a, float* lbl_b, uint32_t xcd_remap, hipStream_t s) {
     const uint32_t W = list_stride(K);
     const dim3 grid((n + 255) / 256), block(256);
-    if (iterations == 0) {
-        hipLaunchKernelGGL((k_lp_iterate<true, true, false>), grid, block, 0, s, K, W, n, hash, lists, nullptr,
-                           nullptr, m_in, m_out, spos, conn, xcd_remap);
-        return hipGetLastError();
-    }
     if (iterations == 1) {
-        hipLaunchKernelGGL((k_lp_iterate<true, true, true>), grid, block, 0, s, K, W, n, hash, lists, nullptr,
+        hipLaunchKernelGGL((k_lp_iterate<true, true, ROWS>), grid, block, 0, s, K, W, n, hash, lists, nullptr,
                            nullptr, m_in, m_out, spos, conn, xcd_remap);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL((k_lp_iterate<true, false, true>), grid, block, 0, s, K, W, n, hash, lists, nullptr, lbl_a,
+    hipLaunchKernelGGL((k_lp_iterate<true, false, ROWS>), grid, block, 0, s, K, W, n, hash, lists, nullptr, lbl_a,
                        m_in, m_out, spos, conn, xcd_remap);
     float* src = lbl_a;
     float* dst = lbl_b;
     for (uint32_t t = 1; t + 1 < iterations; ++t) {
-        hipLaunchKernelGGL((k_lp_iterate<false, false, true>), grid, block, 0, s, K, W, n, hash, lists, src, dst,
+        hipLaunchKernelGGL((k_lp_iterate<false, false, ROWS>), grid, block, 0, s, K, W, n, hash, lists, src, dst,
                            m_in, m_out, spos, conn, xcd_remap);
         float* x = src;
         src = dst;
         dst = x;
     }
-    hipLaunchKernelGGL((k_lp_iterate<false, true, true>), grid, block, 0, s, K, W, n, hash, lists, src, nullptr,
+    hipLaunchKernelGGL((k_lp_iterate<false, true, ROWS>), grid, block, 0, s, K, W, n, hash, lists, src, nullptr,
                        m_in, m_out, spos, conn, xcd_remap);
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_cluster_membership(uint32_t K, uint32_t n, uint32_t iterations, const uint2* hash,
+                                     const uint32_t* lists, const float4* spos, const float* m_in, float* m_out,
+                                     float4* conn, float* lbl_a, float* lbl_b, uint32_t xcd_remap, hipStream_t s) {
+    if (iterations == 0) {
+        hipLaunchKernelGGL((k_lp_iterate<true, true, kRowsOwn, false>), dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), n,
+                           hash, lists, nullptr, nullptr, m_in, m_out, spos, conn, xcd_remap);
+        return hipGetLastError();
+    }
+    const ListRows rows = list_rows(list_stride(K), n);
+    const auto launch = rows == kRowsOwn     ? launch_label_iterations<kRowsOwn>
+                        : rows == kRowsWhole ? launch_label_iterations<kRowsWhole>
+                                             : launch_label_iterations<kRowsBlocks>;
+    return launch(K, n, iterations, hash, lists, spos, m_in, m_out, conn, lbl_a, lbl_b, xcd_remap, s);
 }
 
 hipError_t launch_hit_rate(uint32_t K, float radius, uint32_t n, const uint2* hash, const uint32_t* lists,
@@ -682,8 +700,9 @@ hipError_t launch_hit_rate(uint32_t K, float radius, uint32_t n, const uint2* ha
                            hipStream_t s) {
     const dim3 grid((n + 255) / 256), block(256);
     hipLaunchKernelGGL(k_gather_labels, grid, block, 0, s, n, hash, m_in, spos, lbl);
-    hipLaunchKernelGGL(k_hit_rate, grid, block, 0, s, K, list_stride(K), brt_radius_threshold(radius), n, hash, lists, lbl, m_out,
-                       xcd_remap);
+    const auto kernel = list_stride(K) <= kStageWords ? k_hit_rate<kRowsWhole> : k_hit_rate<kRowsBlocks>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, K, list_stride(K), brt_radius_threshold(radius), n, hash, lists, lbl,
+                       m_out, xcd_remap);
     return hipGetLastError();
 }
 
@@ -776,8 +795,12 @@ hipError_t launch_bc_similarities(uint32_t K, const brt_bc_params& bc, uint32_t 
 hipError_t launch_bc_cluster_steer(uint32_t K, const brt_steer_params& sp, const brt_bc_params& bc, uint32_t n,
                                    const float4* spos, const float4* sfwd, const uint32_t* lists, const float* sims,
                                    const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
-    hipLaunchKernelGGL(k_bc_cluster_steer, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, bc, n, spos,
-                       sfwd, lists, sims, force_in, force_out, xcd_remap);
+    const ListRows rows = list_rows(list_stride(K), n);
+    const auto kernel = rows == kRowsOwn     ? k_bc_cluster_steer<kRowsOwn>
+                        : rows == kRowsWhole ? k_bc_cluster_steer<kRowsWhole>
+                                             : k_bc_cluster_steer<kRowsBlocks>;
+    hipLaunchKernelGGL(kernel, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, bc, n, spos, sfwd, lists,
+                       sims, force_in, force_out, xcd_remap);
     return hipGetLastError();
 }
 

@@ -25,12 +25,13 @@ namespace {
 // rises by 2 % when it agrees (> 0.5).  Bound by the arithmetic per entry, so the
 // neighbourhood test is decided by the cuts.  forward_out (sorted) keeps the heading;
 // force_out = steering + force_in (blendIntoSteeringForce).
+template <ListRows ROWS>
 __global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_steer_params sp, SteerCuts cuts, uint32_t n,
                                                     const float4* __restrict__ spos, const float4* sfwd,
                                                     const uint32_t* __restrict__ lists, float4* fwd_out,
                                                     const float4* force_in, float4* force_out,
                                                     uint32_t xcd_remap) {
-    __shared__ uint4 s_stage[4][kStageChunks];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
@@ -40,7 +41,7 @@ __global__ void __launch_bounds__(256) k_slow_avoid(uint32_t K, uint32_t W, brt_
     const float margin = cut_margin(myFwd);
     SteerAccum acc;
     acc.init();
-    const uint32_t count = wave_list_octets(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
+    const uint32_t count = walk_list<ROWS>(s_stage[wave], lists, W, K, i - lane, lane, n, [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
         float4 qp[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) qp[k] = spos[jj[k]];
@@ -126,7 +127,8 @@ SteerCuts separation_cuts(const brt_steer_params& sp) {
 hipError_t launch_slow_avoid(uint32_t K, const brt_steer_params& sp, uint32_t n, const float4* spos,
                              const float4* sfwd, const uint32_t* lists, float4* fwd_out, const float4* force_in,
                              float4* force_out, uint32_t xcd_remap, hipStream_t s) {
-    hipLaunchKernelGGL(k_slow_avoid, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, separation_cuts(sp),
+    const auto kernel = list_stride(K) <= kStageWords ? k_slow_avoid<kRowsWhole> : k_slow_avoid<kRowsBlocks>;
+    hipLaunchKernelGGL(kernel, dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), sp, separation_cuts(sp),
                        n, spos, sfwd, lists, fwd_out, force_in, force_out, xcd_remap);
     return hipGetLastError();
 }

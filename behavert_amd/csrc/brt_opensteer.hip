@@ -64,16 +64,17 @@ __device__ __forceinline__ float4 feature_update(float rate, uint32_t n, const u
     return r;
 }
 
+template <ListRows ROWS>
 __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32_t n, const uint2* __restrict__ hash,
                                                   const uint32_t* __restrict__ lists,
                                                   const float4* __restrict__ fin, float4* __restrict__ fout,
                                                   uint32_t xcd_remap) {
-    __shared__ uint4 s_stage[4][kStageChunks];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(ROWS == kRowsOwn ? 0u : xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t id = i < n ? hash[i].y : n;
     const float4 f = feature_update(rate, n, hash, fin, id < n ? id : 0u, [&](auto&& fn) {
-        return wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, fn);
+        return walk_list<ROWS>(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, fn);
     });
     if (id < n) fout[id] = f;
 }
@@ -87,8 +88,9 @@ __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32
 // REC: the new state (and feature) goes to one 64-byte record by ID instead of
 // to the arrays: a write to a random ID costs the same whatever its size (about
 // 45 G a second), and k_unpack moves the records to the arrays in order.
-template <bool APPLY, bool FEAT = false, bool SFEAT = false, bool REC = false>
-__global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, brt_steer_params sp, SteerCuts cuts,
+// With FEAT each lane reads its own row.
+template <bool APPLY, ListRows ROWS, bool FEAT = false, bool SFEAT = false, bool REC = false>
+__global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4) k_steer(brt_grid_params g, uint32_t W, brt_steer_params sp, SteerCuts cuts,
                                                float dt,
                                                uint32_t step, uint32_t n, const float4* __restrict__ spos,
                                                const float4* __restrict__ sfwd, const float4* __restrict__ ssa,
@@ -97,9 +99,9 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
                                                float feature_rate = 0.0f, const float4* __restrict__ fin = nullptr,
                                                float4* __restrict__ fout = nullptr,
                                                const float4* __restrict__ sfeat = nullptr) {
-    __shared__ uint4 s_stage[FEAT ? 1 : 4][FEAT ? 1 : kStageChunks];
+    __shared__ uint4 s_stage[4][list_rows_chunks(ROWS)];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t i = xcd_block(xcd_remap) * blockDim.x + threadIdx.x;
+    const uint32_t i = xcd_block(ROWS == kRowsOwn ? 0u : xcd_remap) * blockDim.x + threadIdx.x;
     const uint32_t at = i < n ? i : n - 1u;
     const uint32_t id = i < n ? hash[i].y : n;
     if (FEAT && id >= n) return;
@@ -160,7 +162,7 @@ __global__ void __launch_bounds__(256) k_steer(brt_grid_params g, uint32_t W, br
         if (FEAT)
             count = for_list_octets<false>(lists, W, W - 1u, i, n, visit);
         else
-            count = wave_list_octets(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, visit);
+            count = walk_list<ROWS>(s_stage[wave], lists, W, W - 1u, i - lane, lane, n, visit);
     }
     float4 feature = make_float4(0.f, 0.f, 0.f, 0.f);
     if (FEAT) {
@@ -284,6 +286,7 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
                         float4* records) {
     AgentOut o{pos_out, fwd_out, sa_out, force_out, wander};
     const SteerCuts cuts = steer_cuts(sp);
+    const ListRows rows = list_rows(list_stride(K), n);  // records: from 2^19 agents, never kRowsOwn
     if (K > 32u && n >= kXcdRunMin && xcd_remap) xcd_remap = 2u;  // as the list pass before it
     if (records) {
         o.rec = records;
@@ -291,12 +294,13 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
         const hipEvent_t stop = launch_mark().stop;
         launch_mark().stop = nullptr;
         if (features_in)
-            BRT_LAUNCH((k_steer<true, true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
+            BRT_LAUNCH((k_steer<true, kRowsOwn, true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
                        sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
                        features_out, sorted_features);
         else
-            BRT_LAUNCH((k_steer<true, false, false, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
-                       sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr,
+            BRT_LAUNCH((rows == kRowsWhole ? k_steer<true, kRowsWhole, false, false, true>
+                                           : k_steer<true, kRowsBlocks, false, false, true>),
+                       dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr,
                        nullptr);
         o.wander = sp.wander_weight != 0.0f ? wander : nullptr;
         launch_mark().stop = stop;
@@ -305,17 +309,18 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
         return hipGetLastError();
     }
     if (features_in && sorted_features)
-        BRT_LAUNCH((k_steer<true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp,
+        BRT_LAUNCH((k_steer<true, kRowsOwn, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp,
                            cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
                            features_out, sorted_features);
     else if (features_in)
-        BRT_LAUNCH((k_steer<true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt,
+        BRT_LAUNCH((k_steer<true, kRowsOwn, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt,
                            step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
                            features_out, nullptr);
     else
-        BRT_LAUNCH((k_steer<true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt,
-                           step,
-                           n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr, nullptr);
+        BRT_LAUNCH((rows == kRowsOwn     ? k_steer<true, kRowsOwn>
+                    : rows == kRowsWhole ? k_steer<true, kRowsWhole>
+                                         : k_steer<true, kRowsBlocks>), dim3((n + 255) / 256), dim3(256),
+                   0, s, g, list_stride(K), sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 
@@ -330,9 +335,12 @@ hipError_t launch_steer_forces(uint32_t K, const brt_steer_params& sp, float dt,
                                float2* wander, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
     AgentOut o{nullptr, nullptr, nullptr, force_out, wander};
     brt_grid_params g{};
-    hipLaunchKernelGGL((k_steer<false>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp,
-                       steer_cuts(sp), dt, step, n,
-                       spos, sfwd, sfwd, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr);
+    const ListRows rows = list_rows(list_stride(K), n);
+    const auto kernel = rows == kRowsOwn     ? k_steer<false, kRowsOwn>
+                        : rows == kRowsWhole ? k_steer<false, kRowsWhole>
+                                             : k_steer<false, kRowsBlocks>;
+    hipLaunchKernelGGL(kernel, dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, steer_cuts(sp), dt, step,
+                       n, spos, sfwd, sfwd, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 
@@ -347,8 +355,11 @@ hipError_t launch_apply(const brt_grid_params& g, const brt_steer_params& sp, fl
 
 hipError_t launch_features(uint32_t K, float rate, uint32_t n, const uint2* hash, const uint32_t* lists,
                            const float4* fin, float4* fout, uint32_t xcd_remap, hipStream_t s) {
-    BRT_LAUNCH(k_features, dim3((n + 255) / 256), dim3(256), 0, s, list_stride(K), rate, n, hash, lists, fin,
-                       fout, xcd_remap);
+    const ListRows rows = list_rows(list_stride(K), n);
+    BRT_LAUNCH((rows == kRowsOwn     ? k_features<kRowsOwn>
+                : rows == kRowsWhole ? k_features<kRowsWhole>
+                                     : k_features<kRowsBlocks>), dim3((n + 255) / 256), dim3(256), 0, s,
+               list_stride(K), rate, n, hash, lists, fin, fout, xcd_remap);
     return hipGetLastError();
 }
 
