@@ -721,7 +721,7 @@ int brt_bc_neigh_similarities(brt_context* ctx, const brt_prox_params* prox, con
     BRT_HIP(brt::launch_bc_similarities(prox->max_neighbors, *bc, n, reinterpret_cast<const uint2*>(hash), lists,
                                         features, reinterpret_cast<const float4*>(stats_in),
                                         reinterpret_cast<float4*>(stats_out), similarities, ctx->tmp, nullptr,
-                                        nullptr, nullptr, nullptr, nullptr, ctx->xcd_remap, (hipStream_t)stream),
+                                        nullptr, nullptr, nullptr, nullptr, nullptr, ctx->xcd_remap, (hipStream_t)stream),
             "k_bc_similarities");
     return BRT_OK;
 }
@@ -748,9 +748,12 @@ int brt_bc_similarities_steer(brt_context* ctx, const brt_prox_params* prox, con
                 "float4 arrays must be 16-byte aligned");
     if ((rc = use_device(ctx))) return rc;
     if ((rc = ensure_tmp(ctx, brt::bc_scratch_bytes(bc->feature_count, n)))) return rc;
+    const size_t record_bytes = brt::bc_record_bytes(prox->max_neighbors, bc->feature_count, n);
+    void* const records =
+        record_bytes != 0u && ensure_records(ctx, record_bytes, (hipStream_t)stream) ? ctx->records : nullptr;
     BRT_HIP(brt::launch_bc_similarities(prox->max_neighbors, *bc, n, reinterpret_cast<const uint2*>(hash), lists,
                                         features, reinterpret_cast<const float4*>(stats_in),
-                                        reinterpret_cast<float4*>(stats_out), similarities, ctx->tmp, steer,
+                                        reinterpret_cast<float4*>(stats_out), similarities, ctx->tmp, records, steer,
                                         reinterpret_cast<const float4*>(sorted_pos),
                                         reinterpret_cast<const float4*>(sorted_forward),
                                         reinterpret_cast<const float4*>(force_in),

@@ -218,19 +218,30 @@ __device__ __forceinline__ void store_similarities(float* __restrict__ sims, uin
 }
 
 // computeNeighNaiveSimilarities (+ computeAdaptiveSimilarities) over sorted
-// features.  One lane per sorted agent; neighbours in groups of G (8 gathers of
-// FQ float4 in flight at FQ <= 2).  Each lane writes its similarity row into LDS,
-// in the place of its staged list row where there is one, and the wave then stores
-// the rows with coalesced writes.
-extern __shared__ float bc_rows[];
+// features; with STEER also steerForClusterCohesion + Alignment on the fly (the
+// whole of BehaviorClusteringPlugIn::steerForClustering).  One lane per sorted
+// agent; neighbours in groups of G (8 gathers of FQ float4 in flight at FQ <= 2).
+// Each lane writes its similarity row into LDS, in the place of its staged list row
+// where there is one (not with STEER, whose lanes read their own rows), and the
+// wave then stores the rows with coalesced writes.
+extern __shared__ float4 bc_rows[];
 
-template <bool ADAPTIVE, int FQ>
+// What the steering of STEER reads and writes.
+struct SteerIo {
+    brt_steer_params sp;
+    const float4* spos;
+    const float4* sfwd;
+    const float4* force_in;
+    float4* force_out;
+};
+
+template <bool ADAPTIVE, bool STEER, int FQ>
 __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_t W, const brt_bc_params& bc,
                                                  uint32_t n, const uint2* __restrict__ hash,
                                                  const uint32_t* __restrict__ lists,
                                                  const float4* __restrict__ sfeat, const float* __restrict__ norms,
                                                  const float4* __restrict__ stats_in, float4* __restrict__ stats_out,
-                                                 uint32_t* row, bool staged) {
+                                                 uint32_t* row, bool staged, const SteerIo& io) {
     float* const out = reinterpret_cast<float*>(row);
     constexpr int G = FQ <= 2 ? 8 : (FQ <= 4 ? 4 : 2);
     const uint32_t F = bc.feature_count;
@@ -241,10 +252,19 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
     const float n1 = norms[i];
     const bool valid = id < n;
     float4 st = ADAPTIVE && valid ? stats_in[id] : make_float4(0.f, 0.f, 0.f, 0.f);
+    V3 myPos = v3(0.f, 0.f, 0.f), myFwd = myPos, vel = myPos;
+    if (STEER) {
+        const float4 P = io.spos[i], Fw = io.sfwd[i];
+        myPos = xyz(P);
+        myFwd = xyz(Fw);
+        vel = myFwd * Fw.w;
+    }
+    ClusterAccum acc;
+    acc.init();
     auto visit = [&](uint32_t base, const uint32_t(&jj)[8], uint32_t mask) {
 #pragma unroll
         for (int g0 = 0; g0 < 8; g0 += G) {
-            float4 other[G][FQ];
+            float4 other[G][FQ], op[G], of[G];
             float n2[G];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -252,6 +272,10 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
 #pragma unroll
                 for (int q = 0; q < FQ; ++q) other[g][q] = sfeat[(size_t)j * FQ + q];
                 n2[g] = norms[j];
+                if (STEER) {
+                    op[g] = io.spos[j];
+                    of[g] = io.sfwd[j];
+                }
             }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -266,11 +290,12 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
                     }
                 }
                 out[base + k - 1u] = sim;
+                if (STEER) acc.add(myPos, vel, io.sp.max_speed, xyz(op[g]), xyz(of[g]), sim);
             }
         }
     };
     uint32_t count;
-    if (staged) {
+    if (!STEER && staged) {
         count = row[0] < K ? row[0] : K;
         visit_staged(reinterpret_cast<const uint4*>(row), count, i, n, visit);
     } else {
@@ -278,9 +303,10 @@ __device__ __forceinline__ void similarity_agent(uint32_t i, uint32_t K, uint32_
     }
     for (uint32_t t = count; t <= K; ++t) out[t] = 0.0f;
     if (ADAPTIVE && valid) stats_out[id] = st;
+    if (STEER) io.force_out[i] = acc.finish(count, myFwd, bc, io.force_in[i]);
 }
 
-template <bool ADAPTIVE, int FQ>
+template <bool ADAPTIVE, bool STEER, int FQ>
 __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W, brt_bc_params bc, uint32_t n,
                                                          const uint2* __restrict__ hash,
                                                          const uint32_t* __restrict__ lists,
@@ -288,17 +314,17 @@ __global__ void __launch_bounds__(256) k_bc_similarities(uint32_t K, uint32_t W,
                                                          const float* __restrict__ norms,
                                                          const float4* __restrict__ stats_in,
                                                          float4* __restrict__ stats_out, float* __restrict__ sims,
-                                                         uint32_t sims_vec, uint32_t xcd_remap) {
+                                                         uint32_t sims_vec, SteerIo io, uint32_t xcd_remap) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t row0 = xcd_block(xcd_remap) * blockDim.x + wave * 64u, i = row0 + lane;
     if (row0 >= n) return;
-    const uint32_t RW = similarity_row_words(K, W);
+    const bool staged = !STEER && W <= kStageWords;
+    const uint32_t RW = STEER ? K + 1u : similarity_row_words(K, W);
     uint32_t* const mem = reinterpret_cast<uint32_t*>(bc_rows) + (size_t)wave * 64u * RW;
-    const bool staged = W <= kStageWords;
     if (staged) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
     if (i < n)
-        similarity_agent<ADAPTIVE, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, mem + lane * RW,
-                                       staged);
+        similarity_agent<ADAPTIVE, STEER, FQ>(i, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out,
+                                              mem + lane * RW, staged, io);
     wave_lds_sync();
     store_similarities(sims, row0, n, K, RW, reinterpret_cast<const float*>(mem), lane, sims_vec);
 }
@@ -390,13 +416,16 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     vfloat4* const tile = reinterpret_cast<vfloat4*>(mem + wave_bytes - kTileChunks * 16u);
     const bool staged = W <= kStageWords;
     if (staged) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
-    const uint4* const L = reinterpret_cast<const uint4*>(lists + (size_t)at * W);
-    auto word = [&](uint32_t q) {
-        uint4 v;
-        if (staged)
-            v = reinterpret_cast<const uint4*>(row)[q];
-        else
-            v = L[q];
+    const vuint4* const L = reinterpret_cast<const vuint4*>(lists + (size_t)at * W);
+    // word q of the row, if it holds an entry
+    auto word = [&](uint32_t q, uint32_t last) {
+        vuint4 v = {0u, 0u, 0u, 0u};
+        if (q <= last) {
+            if (staged)
+                v = reinterpret_cast<const vuint4*>(row)[q];
+            else
+                v = L[q];
+        }
         return v;
     };
 
@@ -417,14 +446,22 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     ClusterAccum acc;
     acc.init();
 
-    uint4 a = word(0);
-    const uint32_t count = i < n ? (a.x < K ? a.x : K) : 0u;
+    vuint4 a = word(0u, 0u);
+    const uint32_t count = i < n ? (a.x < K ? a.x : K) : 0u, last = count / 4u;
     float* const out = reinterpret_cast<float*>(row);
+    vuint4 b = word(1u, last), na, nb;
     // all lanes of the wave stay in step: those past their list load their own record
-    for (uint32_t q = 0; __ballot(4u * q <= count) != 0; q += 2) {
-        const uint32_t last = count / 4u;
-        if (q != 0u) a = word(q < last ? q : last);
-        const uint4 b = word(q + 1u < last ? q + 1u : last);
+    for (uint32_t q = 0; __ballot(q <= last) != 0; q += 2) {
+        // rows in memory: the next words load during this octet's gathers; staged
+        // ones are read when they are used (this octet overwrites the row up to word
+        // 4 q + 6)
+        if (!staged) {
+            na = word(q + 2u, last);
+            nb = word(q + 3u, last);
+        } else if (q != 0u) {
+            a = word(q, last);
+            b = word(q + 1u, last);
+        }
         uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         const uint32_t mask = octet_mask(jj, q, count, at, n);
 #pragma unroll
@@ -477,6 +514,10 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
                 acc.add(myPos, vel, sp.max_speed, v3(got[0].x, got[0].y, got[0].z), v3(got[1].x, got[1].y, got[1].z),
                         sim);
             }
+        }
+        if (!staged) {
+            a = na;
+            b = nb;
         }
     }
     if (i < n) {
@@ -711,26 +752,21 @@ namespace {
 template <int FQ>
 hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash, const uint32_t* lists,
                        const float* features, uint32_t vec, const float4* stats_in, float4* stats_out, float* sims,
-                       void* scratch, const brt_steer_params* sp, const float4* spos, const float4* sfwd,
-                       const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
+                       void* scratch, void* records, const brt_steer_params* sp, const float4* spos,
+                       const float4* sfwd, const float4* force_in, float4* force_out, uint32_t xcd_remap,
+                       hipStream_t s) {
     const uint32_t F = bc.feature_count, W = list_stride(K);
     const uint32_t sims_vec = ((uintptr_t)sims & 15u) == 0 ? 1u : 0u;
-    if (sp) {
+    if (sp && records) {
         constexpr uint32_t RP = 4u * record_rounds<FQ>();
-        float4* rec = reinterpret_cast<float4*>(scratch);
+        float4* rec = reinterpret_cast<float4*>(records);
         hipLaunchKernelGGL((k_bc_records<FQ>), dim3((unsigned)(((size_t)n * RP + 255u) / 256u)), dim3(256), 0, s, F, n,
                            vec, hash, features, spos, sfwd, rec);
         // four waves per workgroup while three workgroups fit a CU's LDS, else one
         const uint32_t bytes = similarity_wave_bytes(K, W), B = 4u * bytes <= 160u * 1024u / 3u ? 256u : 64u;
-        const dim3 grid((n + B - 1) / B), block(B);
-        if (bc.adaptive)
-            hipLaunchKernelGGL((k_bc_similarities_steer<true, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n, hash,
-                               lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
-                               sims_vec, xcd_remap);
-        else
-            hipLaunchKernelGGL((k_bc_similarities_steer<false, FQ>), grid, block, B / 64u * bytes, s, K, W, bc, n,
-                               hash, lists, rec, stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes,
-                               sims_vec, xcd_remap);
+        const auto kernel = bc.adaptive ? k_bc_similarities_steer<true, FQ> : k_bc_similarities_steer<false, FQ>;
+        hipLaunchKernelGGL(kernel, dim3((n + B - 1) / B), dim3(B), B / 64u * bytes, s, K, W, bc, n, hash, lists, rec,
+                           stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes, sims_vec, xcd_remap);
         return hipGetLastError();
     }
     float4* sfeat = reinterpret_cast<float4*>(scratch);
@@ -738,16 +774,15 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
     hipLaunchKernelGGL(k_bc_sort_features, dim3((n + 255) / 256), dim3(256), 0, s, F, (uint32_t)FQ, n, vec, hash,
                        features, sfeat, norms);
     // the LDS rows: 256 agents while they stay within 40 KB, else one wave
-    const size_t bytes = (size_t)64u * similarity_row_words(K, W) * 4u;
+    const size_t bytes = (size_t)64u * (sp ? K + 1u : similarity_row_words(K, W)) * 4u;
     const uint32_t B = 4u * bytes <= 40u * 1024u ? 256u : 64u;
     const size_t lds = B / 64u * bytes;
     const dim3 grid((n + B - 1) / B), block(B);
-    if (bc.adaptive)
-        hipLaunchKernelGGL((k_bc_similarities<true, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, sims_vec, xcd_remap);
-    else
-        hipLaunchKernelGGL((k_bc_similarities<false, FQ>), grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms,
-                           stats_in, stats_out, sims, sims_vec, xcd_remap);
+    const SteerIo io = sp ? SteerIo{*sp, spos, sfwd, force_in, force_out} : SteerIo{};
+    const auto kernel = sp ? (bc.adaptive ? k_bc_similarities<true, true, FQ> : k_bc_similarities<false, true, FQ>)
+                           : (bc.adaptive ? k_bc_similarities<true, false, FQ> : k_bc_similarities<false, false, FQ>);
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, K, W, bc, n, hash, lists, sfeat, norms, stats_in, stats_out, sims,
+                       sims_vec, io, sp ? 0u : xcd_remap);
     return hipGetLastError();
 }
 
@@ -755,28 +790,37 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
 
 size_t bc_scratch_bytes(uint32_t feature_count, uint32_t n) {
     const size_t FQ = (feature_count + 3u) / 4u;
-    return (size_t)n * ((FQ + 5u) / 4u) * 64u;  // the records; features and norms take less
+    return (size_t)n * FQ * 16u + ((size_t)n * 4u + 15u) / 16u * 16u;
+}
+
+// From 147,456 agents (196,608 for up to 4 features or beyond K 48), where the
+// accesses of the gathers set the pace: below, each agent's own gathers have the
+// shorter chain and leave room for more waves (K 32, F 8: 1,000 agents 13.4 us, from
+// records 15.5; 60,000 20 and 22; 131,072 23 and 28).  Lists beyond K 64 (80 from 9
+// features on) leave the records' tile too few waves.  With up to 4 features a record
+// saves one access in four, which pays for its making only where lists are long: K
+// 24 to 48.  1,048,576 agents at 1 / 4 / 12 per cell, own gathers -> records, us: F 4,
+// K 32 150 -> 180, 244 -> 249, 390 -> 279; F 8, K 32 194 -> 187, 307 -> 255, 433 ->
+// 293, K 80 238 -> 260, 373 -> 383, 661 -> 675; F 16, K 32 289 -> 272, 462 -> 377,
+// 788 -> 429, K 80 344 -> 341, 525 -> 501, 990 -> 885.
+size_t bc_record_bytes(uint32_t K, uint32_t feature_count, uint32_t n) {
+    const size_t FQ = (feature_count + 3u) / 4u;
+    const bool pays = FQ == 1u ? K >= 24u && K <= 48u : K <= (FQ == 2u ? 64u : 80u);
+    const uint32_t least = FQ == 1u || K > 48u ? 3u << 16 : 9u << 14;
+    return n >= least && pays ? (size_t)n * ((FQ + 5u) / 4u) * 64u : 0u;
 }
 
 hipError_t launch_bc_similarities(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash,
                                   const uint32_t* lists, const float* features, const float4* stats_in,
-                                  float4* stats_out, float* sims, void* scratch, const brt_steer_params* sp,
-                                  const float4* spos, const float4* sfwd, const float4* force_in, float4* force_out,
-                                  uint32_t xcd_remap, hipStream_t s) {
-    // lists whose similarities and tile exceed the LDS of a workgroup (K 239 and
-    // more): the same sums from the stored similarities
-    if (sp && similarity_wave_bytes(K, list_stride(K)) > 64u * 1024u) {
-        const hipError_t e = launch_bc_similarities(K, bc, n, hash, lists, features, stats_in, stats_out, sims, scratch,
-                                                    nullptr, nullptr, nullptr, nullptr, nullptr, xcd_remap, s);
-        if (e != hipSuccess) return e;
-        return launch_bc_cluster_steer(K, *sp, bc, n, spos, sfwd, lists, sims, force_in, force_out, xcd_remap, s);
-    }
+                                  float4* stats_out, float* sims, void* scratch, void* records,
+                                  const brt_steer_params* sp, const float4* spos, const float4* sfwd,
+                                  const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s) {
     const uint32_t F = bc.feature_count;
     const uint32_t vec = (F % 4u == 0 && ((uintptr_t)features & 15u) == 0) ? 1u : 0u;
 #define BRT_SIMS_CASE(Q)                                                                                             \
     case Q:                                                                                                          \
-        return launch_sims<Q>(K, bc, n, hash, lists, features, vec, stats_in, stats_out, sims, scratch, sp, spos,    \
-                              sfwd, force_in, force_out, xcd_remap, s);
+        return launch_sims<Q>(K, bc, n, hash, lists, features, vec, stats_in, stats_out, sims, scratch, records, sp, \
+                              spos, sfwd, force_in, force_out, xcd_remap, s);
     switch ((F + 3u) / 4u) {
         BRT_SIMS_CASE(1)
         BRT_SIMS_CASE(2)

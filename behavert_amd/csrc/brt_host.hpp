@@ -26,7 +26,9 @@ struct brt_context {
     size_t partials_bytes = 0;
     void* xyz = nullptr;        // brt_step: the sorted positions packed as x,y,z
     size_t xyz_bytes = 0;
-    void* records = nullptr;    // brt_step: the state by ID as records (step_record_bytes)
+    // brt_step: the state by ID as records (step_record_bytes); brt_bc_similarities_steer:
+    // the neighbours' (bc_record_bytes)
+    void* records = nullptr;
     size_t records_bytes = 0;
     uint32_t* dev_flags = nullptr;  // sticky device-side failure flags (BRT_DEVFLAG_*)
     void* scratch = nullptr;        // this device's no-allocation step scratch (a static device array)
@@ -127,7 +129,7 @@ int check_prox(brt_context* ctx, const brt_prox_params* p);
 int check_steer(brt_context* ctx, const brt_steer_params* s);
 int ensure_tmp(brt_context* ctx, size_t bytes);
 int ensure_scratch(brt_context* ctx, uint32_t n, const brt::SortPlan& plan);
-// Scratch that a step can do without and that does not grow while s is being
+// Scratch that its callers can do without and that does not grow while s is being
 // captured: whether the records hold `need` bytes; the packed positions of n
 // agents, or NULL (the neighbour search then reads the float4 ones).
 bool ensure_records(brt_context* ctx, size_t need, hipStream_t s);

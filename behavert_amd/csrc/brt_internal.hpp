@@ -162,15 +162,17 @@ hipError_t launch_apply(const brt_grid_params& g, const brt_steer_params& sp, fl
                         float4* pos_out, float4* fwd_out, float4* sa_out, float4* force_out, hipStream_t s);
 
 // BehaviorClustering similarities and cluster steering
-// scratch: bc_scratch_bytes(F, n), 64-byte aligned (the agents' records, or features and
-// norms, in sorted order);
-// sp != nullptr also runs the cluster steering on the fly (force_in -> force_out)
+// scratch: bc_scratch_bytes(F, n), 16-byte aligned (features in sorted order + norms);
+// sp != nullptr also runs the cluster steering on the fly (force_in -> force_out),
+// from records (64-byte aligned) instead of the scratch where bc_record_bytes is not
+// 0 and the caller has them; each gives the same bits
 size_t bc_scratch_bytes(uint32_t feature_count, uint32_t n);
+size_t bc_record_bytes(uint32_t K, uint32_t feature_count, uint32_t n);
 hipError_t launch_bc_similarities(uint32_t K, const brt_bc_params& bc, uint32_t n, const uint2* hash,
                                   const uint32_t* lists, const float* features, const float4* stats_in,
-                                  float4* stats_out, float* sims, void* scratch, const brt_steer_params* sp,
-                                  const float4* spos, const float4* sfwd, const float4* force_in, float4* force_out,
-                                  uint32_t xcd_remap, hipStream_t s);
+                                  float4* stats_out, float* sims, void* scratch, void* records,
+                                  const brt_steer_params* sp, const float4* spos, const float4* sfwd,
+                                  const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s);
 hipError_t launch_bc_cluster_steer(uint32_t K, const brt_steer_params& sp, const brt_bc_params& bc, uint32_t n,
                                    const float4* spos, const float4* sfwd, const uint32_t* lists, const float* sims,
                                    const float4* force_in, float4* force_out, uint32_t xcd_remap, hipStream_t s);
