@@ -205,7 +205,10 @@ hipError_t launch_adjoint(const brt_grid_params& g, const brt_prox_params& p, fl
                           float* partials, float* weight_grad, uint32_t xcd_remap, hipStream_t s);
 
 // Agents from which the passes with long rows map runs of workgroups to the XCDs.
-constexpr uint32_t kXcdRunMin = 1u << 21;
+// Slices -> runs, list pass, K 64, at 1 / 6 per cell / in blobs, us: 2,100,003 agents
+// 228 -> 234, 547 -> 523, 1399 -> 1481; 3,000,001 327 -> 333, 760 -> 731, 1972 -> 1981;
+// 4,194,304 453 -> 452, 1001 -> 962, 2697 -> 2644.
+constexpr uint32_t kXcdRunMin = 3u << 20;
 inline uint32_t list_stride(uint32_t K) { return 4u * (K / 4u + 1u); }
 // LDS of a workgroup of the four-lane neighbour kernels (64 list rows and, when
 // the steering is fused, an agent's three sums and their counts: an odd number
