@@ -1005,7 +1005,7 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, cons
 }
 
 template <bool FUSE, bool BATCH, bool LDSL>
-__global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
+__global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) {
     // with LDS lists blockDim.x rows of Ws words; the list-only kernel without
     // them blockDim.x heads of kHeadWords; else unused
     extern __shared__ uint32_t s_list[];
@@ -1085,8 +1085,11 @@ __global__ void __launch_bounds__(256) k_prox(ProxArgs a) {
             else
                 L.row[1u + p] = j;
         };
-        // with LDS lists a third run would cost the fourth wave per SIMD (129 registers)
-        constexpr int NR = LDSL ? 2 : 3;
+        // with LDS lists a third run would cost the fourth wave per SIMD (129 registers),
+        // without them a second one the fifth, on which the other scans rely (300,007
+        // agents, K 48, three runs and four waves -> one and five: 12 per cell 117 -> 84
+        // us, in blobs 416 -> 340, at one per cell 38 -> 34)
+        constexpr int NR = LDSL ? 2 : 1;
         uint32_t all = 0u;
         rows = can && (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, NR>(a, sg, L, gp, alive, own, all, put)
                                                  : scan_rows<false, NR>(a, sg, L, gp, alive, own, all, put));
