@@ -151,6 +151,9 @@ struct ProxArgs {
     uint32_t xcd_remap;
     uint32_t log_rounds;  // LDS lists through the round log (n < 2^24)
     uint32_t cells;       // cells of the launch for the row scan's bounded loads; 0: no row scan
+    // agents of its own row beyond which an agent would rather not have its rows
+    // scanned, by one lane and by four (row_limit)
+    uint32_t row_occ, row_occ_quad;
     const float4* spos;
     const float* pxyz;  // optional: the sorted positions packed as x,y,z (12 bytes each)
     const float4* sfwd;
@@ -902,7 +905,7 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, cons
     }
     own = make_uint2(s[4].y, e[4].y);
     R[4] = row_range(s[4], e[4], a.n, most);
-    if (__popcll(__ballot(most > BRT_PROX_ROW_OCC)) >= BRT_PROX_ROW_LANES) return false;
+    if (__popcll(__ballot(most > a.row_occ)) >= BRT_PROX_ROW_LANES) return false;
     // four rows at a time, to hold no more than their 24 registers
 #pragma unroll
     for (int r0 = 0; r0 < 9; r0 += NL + 1) {
@@ -1278,6 +1281,7 @@ __device__ __forceinline__ bool quad_rows(const ProxArgs& a, const Seg& sg, Lane
         most = most > len ? most : len;
     }
     if (__ballot(most > kRowMax) != 0) return false;
+    if (__popcll(__ballot(l == 1u && R[1].len() > a.row_occ_quad)) >= 8) return false;
     uint32_t M[3] = {0u, 0u, 0u};
     BRT_CELL_LOOP
     for (uint32_t t0 = 0u; __ballot(most > t0) != 0; t0 += 4u) {
@@ -1802,9 +1806,25 @@ uint32_t prox_block(uint32_t W, uint32_t n) {
     return B;
 }
 
+// ProxArgs::row_occ: a list that fills in its first cells needs no row scan, which
+// tests the candidates of all 27.  Agents of the own row (three per one in a cell) at
+// which the two cost the same: 1.6 K with one lane per agent, 2 K but no fewer than
+// 14 with four.  One lane, 131,072 agents at 1 / 3 / 6 per cell, cell by cell -> row
+// scan, us: K 4 20 -> 16 / 20 -> 23 / 20 -> 32, K 8 22 -> 16 / 24 -> 23 / 26 -> 32, K
+// 16 23 -> 17 / 30 -> 24 / 36 -> 34; four lanes, a step: K 4 68 -> 48 / 65 -> 59 / 57
+// -> 71, K 8 57 -> 49 / 74 -> 60 / 63 -> 72.  KNN lists, whose row scan holds K + 24
+// accepted candidates: about half of that.
+uint32_t row_limit(const brt_prox_params& p, bool quads) {
+    const uint32_t K = p.max_neighbors;
+    if (quads) return 2u * K > 14u ? 2u * K : 14u;
+    const uint32_t k = p.use_knn ? (K + kKnnLog) / 2u : K * 8u / 5u;
+    return k < BRT_PROX_ROW_OCC ? k : BRT_PROX_ROW_OCC;
+}
+
 template <bool FUSE>
-bool launch_quad(const ProxArgs& a, hipStream_t s) {
+bool launch_quad(ProxArgs a, const brt_prox_params& p, hipStream_t s) {
     if (!prox_quad_fits(a.K, a.n, FUSE)) return false;
+    a.row_occ_quad = row_limit(p, true);
     BRT_LAUNCH((k_prox_quad<FUSE>), dim3((a.n + 63u) / 64u), dim3(256), prox_quad_lds(a.K, FUSE), s, a);
     return true;
 }
@@ -1814,6 +1834,7 @@ ProxArgs make_args(const brt_grid_params& g, const brt_prox_params& p, float thr
                    uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t cells) {
     ProxArgs a{};
     a.cells = cells < (1u << 30) ? cells : 0u;  // 32-bit byte offsets
+    a.row_occ = row_limit(p, false);
     a.g = g;
     a.K = p.max_neighbors;
     a.W = list_stride(p.max_neighbors);
@@ -1854,7 +1875,7 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
     }
     a.pxyz = pxyz;
     const uint32_t B = prox_block(a.Ws, n);
-    if (quads && launch_quad<false>(a, s)) return hipGetLastError();
+    if (quads && launch_quad<false>(a, p, s)) return hipGetLastError();
     if (lds_lists)
         BRT_LAUNCH((k_prox<false, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else {
@@ -1882,7 +1903,7 @@ hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_param
     a.step = step;
     a.o = AgentOut{pos_out, fwd_out, sa_out, nullptr, wander};
     const uint32_t B = prox_block(a.Ws, n);
-    if (quads && launch_quad<true>(a, s)) return hipGetLastError();
+    if (quads && launch_quad<true>(a, p, s)) return hipGetLastError();
     if (lds_lists)
         BRT_LAUNCH((k_prox<true, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else
