@@ -884,9 +884,10 @@ constexpr uint32_t kHeadWords = 20u;
 // number is returned in all; false (nothing done) when some run of some lane is
 // too long.  own: the range of the cell the agent lies in, for the other modes.
 // Every lane of the wave takes part.  NR: runs whose rounds load together.
-template <bool PACKED, int NR, class Put>
+// decided(ok): called once, by the whole wave, when it is known whether it scans.
+template <bool PACKED, int NR, class Put, class Decided>
 __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, const Lane& L, I3 gp, bool alive,
-                                          uint2& own, uint32_t& all, Put&& put) {
+                                          uint2& own, uint32_t& all, Put&& put, Decided&& decided) {
     constexpr int NL = 4;  // rows whose ranges load together
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.cell_start), (short)0,
                                                                         (int)(a.cells * 4u), 0x00020000);
@@ -905,7 +906,10 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, cons
     }
     own = make_uint2(s[4].y, e[4].y);
     R[4] = row_range(s[4], e[4], a.n, most);
-    if (__popcll(__ballot(most > a.row_occ)) >= BRT_PROX_ROW_LANES) return false;
+    if (__popcll(__ballot(most > a.row_occ)) >= BRT_PROX_ROW_LANES) {
+        decided(false);
+        return false;
+    }
     // four rows at a time, to hold no more than their 24 registers
 #pragma unroll
     for (int r0 = 0; r0 < 9; r0 += NL + 1) {
@@ -927,7 +931,9 @@ __device__ __forceinline__ bool scan_rows(const ProxArgs& a, const Seg& sg, cons
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (__ballot(most > kRowMax) != 0) return false;
+    const bool fits = __ballot(most > kRowMax) == 0;
+    decided(fits);
+    if (!fits) return false;
 
     const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
     const __amdgpu_buffer_rsrc_t rxyz = xyz_rsrc(PACKED ? a.pxyz : nullptr, PACKED ? a.n : 0u);
@@ -1094,8 +1100,9 @@ __global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) 
         // us, in blobs 416 -> 340, at one per cell 38 -> 34)
         constexpr int NR = LDSL ? 2 : 1;
         uint32_t all = 0u;
-        rows = can && (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, NR>(a, sg, L, gp, alive, own, all, put)
-                                                 : scan_rows<false, NR>(a, sg, L, gp, alive, own, all, put));
+        auto any = [](bool) {};
+        rows = can && (LDSL && a.pxyz != nullptr ? scan_rows<LDSL, NR>(a, sg, L, gp, alive, own, all, put, any)
+                                                 : scan_rows<false, NR>(a, sg, L, gp, alive, own, all, put, any));
         if (rows) L.cnt = all < a.K ? all : a.K;
         have_own = can && __ballot(alive && !holds(own, L.i)) == 0;
     }
@@ -1416,6 +1423,51 @@ __device__ __forceinline__ void quad_flat(const ProxArgs& a, const Seg& sg, Lane
     L.cnt = L.cnt < a.K ? L.cnt : a.K;
 }
 
+// Lists alone, above kQuadRowsMax agents: the chip has waves enough, and the row scan
+// of quads, whose fourth lane idles, takes a third more instructions than one lane
+// per agent.  So the workgroup's first wave scans the rows of all 64 agents; only
+// where it cannot do the quads go on.  True: this wave is done.  (Every wave meets
+// the two barriers, the first wave in scan_rows' decision; the second lets it reuse
+// the word that holds the decision.)
+// Not beyond K 80, whose list rows would hold a CU's LDS for one wave.
+constexpr uint32_t kQuadRowsMax = 49152u;
+constexpr uint32_t kQuadRowsMaxK = 80u;
+__device__ __forceinline__ bool one_lane_rows(const ProxArgs& a, Seg sg, uint32_t base, uint32_t lane, uint32_t wid,
+                                              uint32_t* s_list) {
+    if (wid != 0u) {
+        __syncthreads();
+        const uint32_t rows = s_list[0];
+        __syncthreads();
+        return rows != 0u;
+    }
+    sg.row0 = base;
+    Lane L;
+    L.i = base + lane;
+    L.row = s_list + (size_t)lane * a.W;
+    const bool alive = L.i < sg.end;
+    const float4 P = a.spos[alive ? L.i : a.n - 1u];
+    L.px = P.x;
+    L.py = P.y;
+    L.pz = P.z;
+    uint2 own;
+    uint32_t all = 0u;
+    const bool rows = scan_rows<false, 1>(
+        a, sg, L, calcGridPos(P.x, P.y, P.z, sg.g), alive, own, all,
+        [&](uint32_t p, uint32_t j) {
+            if (p < a.K) L.row[1u + p] = j;
+        },
+        [&](bool ok) {
+            if (lane == 0u) s_list[0] = ok ? 1u : 0u;
+            __syncthreads();
+            __syncthreads();
+        });
+    if (!rows) return false;
+    L.row[0] = all < a.K ? all : a.K;
+    wave_lds_sync();
+    store_rows<false>(a.lists, base, sg.end - base < 64u ? sg.end - base : 64u, a.W, s_list, a.W, lane);
+    return true;
+}
+
 // five waves per SIMD: 100,003 agents 46.3 -> 45.3 us a step, 131,072 in blobs 155 -> 146
 template <bool FUSE>
 __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
@@ -1454,6 +1506,7 @@ __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
     }
     const bool can = a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED && sg.g.grid_size[0] >= 3u;
     const bool packed = a.pxyz != nullptr;
+    if (!FUSE && can && a.n > kQuadRowsMax && a.K <= kQuadRowsMaxK && one_lane_rows(a, sg, base, lane, wid, s_list)) return;
     const bool rows = can && (packed ? quad_rows<true>(a, sg, L, gp, alive, l)
                                      : quad_rows<false>(a, sg, L, gp, alive, l));
     if (!rows) {
@@ -1608,7 +1661,7 @@ __device__ __forceinline__ bool knn_rows(const ProxArgs& a, const Seg& sg, const
     const bool can = a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED && sg.g.grid_size[0] >= 3u;
     if (!can || !scan_rows<false, 3>(a, sg, L, gp, alive, own, all, [&](uint32_t p, uint32_t j) {
             if (p < room) kl.list[p * B] = j;
-        }))
+        }, [](bool) {}))
         return false;
     if (__ballot(all > room) != 0) return false;
     const __amdgpu_buffer_rsrc_t rpos = float4_rsrc(a.spos, a.n);
