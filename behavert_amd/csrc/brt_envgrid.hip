@@ -497,11 +497,11 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
                                                             uint2* __restrict__ hash, ReorderArgs f,
                                                             uint32_t* __restrict__ cell_start,
                                                             uint32_t* __restrict__ cell_end) {
-    __shared__ uint32_t s_list[kCellCap];
+    __shared__ alignas(16) uint32_t s_list[kCellCap];  // the sort reads four values at once
     __shared__ uint32_t s_off[kCellsPerGroup + 1];
     __shared__ uint32_t s_rank[kCellRankMax];
     __shared__ uint32_t s_wave[kCellThreads / 64];
-    __shared__ uint32_t s_slot[kCellCap];
+    __shared__ alignas(16) uint32_t s_slot[kCellCap];
     __shared__ uint32_t s_count, s_agents, s_below, s_most;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t c0 = blockIdx.x * cells_per_group;
