@@ -1017,7 +1017,7 @@ template <bool FUSE, bool BATCH, bool LDSL>
 __global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) {
     // with LDS lists blockDim.x rows of Ws words; the list-only kernel without
     // them blockDim.x heads of kHeadWords; else unused
-    extern __shared__ alignas(16) uint32_t s_list[];
+    alignas(16) extern __shared__ uint32_t s_list[];
     constexpr bool ROWS = LDSL || !FUSE;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
@@ -1471,7 +1471,7 @@ __device__ __forceinline__ bool one_lane_rows(const ProxArgs& a, Seg sg, uint32_
 // five waves per SIMD: 100,003 agents 46.3 -> 45.3 us a step, 131,072 in blobs 155 -> 146
 template <bool FUSE>
 __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
-    extern __shared__ alignas(16) uint32_t s_list[];  // 64 rows of W words, then (fused) 64 of kQuadSumWords
+    alignas(16) extern __shared__ uint32_t s_list[];  // 64 rows of W words, then (fused) 64 of kQuadSumWords
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l = tid & 3u;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     Seg sg;
