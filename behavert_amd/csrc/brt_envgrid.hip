@@ -371,8 +371,17 @@ __global__ void __launch_bounds__(kSortThreads) k_onesweep(const uint2* __restri
 // its part of the sorted pairs, the gathered state and the cell ranges, empty
 // ones included.  Nothing passes between workgroups.  Hash + sort + reorder of
 // 4,096 / 65,536 / 100,003 agents: 24.3 -> 9.6 / 31.8 -> 18.2 / 45 -> 21.8 us.
-// The LDS stays below 64 KB: with 83 KB (twice the list) the kernel took 13 us
-// more at every size.
+// A flock gathered in few cells would fall to few workgroups.  So a range with more
+// agents than one workgroup sorts well (crowded) is cut into chunks of up to 2,047
+// agents by their IDs, and workgroups whose own range is light take chunks of it too:
+// which of them help with which range follows from a sample of the keys (CellShare),
+// the same in every workgroup.  131,072 agents in 1 / 27 / 2,197 cells of 64^3, sorted
+// pairs alone: 251 / 1170 / 192 us by the ranges' own workgroups, 61 / 72 / 80 us so
+// (the radix sort: 40); the whole step 539 / 3200 / 315 -> 99 / 1172 / 155 us, with
+// the radix sort and its separate passes 84 / 4828 / 151.  The sample costs up to
+// 0.4 us at 130,200 evenly spread agents (17.9 -> 18.2).
+// The kernel keeps no array in scratch (see emit): with 20 bytes per lane there some
+// builds of it took 13 us more at every size.
 constexpr uint32_t kCellThreads = 1024;
 constexpr uint32_t kCellGroups = 256;   // workgroups at most, one per CU
 constexpr uint32_t kCellIdBits = 17;    // agents below 2^17
@@ -381,6 +390,11 @@ constexpr uint32_t kCellCap = 4096;     // agents a workgroup sorts at a time
 constexpr uint32_t kCellRankMax = 512;  // agents ranked by counting up to here, else bitonic
 constexpr uint32_t kNoKey = 0x7FFFFFFFu;  // beside every key (below 2^20)
 constexpr uint32_t kCellDense = 64;     // agents of a cell ranked within it up to here
+constexpr uint32_t kCellAlone = 2048;   // agents that a workgroup sorts by itself, if some cell holds more than those
+constexpr uint32_t kCellBlock = 1024;   // IDs of a block; a chunk ends with the block in which it reaches as many agents
+constexpr uint32_t kCellBlocks = (1u << kCellIdBits) / kCellBlock;
+constexpr uint32_t kCellSample = 1024;  // keys from which the helpers are spread,
+constexpr uint32_t kCellRun = 8;        // in runs of so many
 constexpr uint32_t kCellGather = 4;     // float4 arrays gathered (position, heading, acceleration, features)
 
 __global__ void __launch_bounds__(256) k_hash_keys(brt_grid_params g, const float4* __restrict__ pos, uint32_t n,
@@ -492,31 +506,194 @@ __device__ __forceinline__ void cell_group_sort(uint32_t* s_list, uint32_t* s_ra
     }
 }
 
+// The quad of keys from i on, kNoKey from n on.
+__device__ __forceinline__ uint4 key_quad(const uint32_t* __restrict__ keys, uint32_t i, uint32_t n) {
+    if (i + 4u <= n) return *reinterpret_cast<const uint4*>(keys + i);
+    return make_uint4(i < n ? keys[i] : kNoKey, i + 1u < n ? keys[i + 1u] : kNoKey,
+                      i + 2u < n ? keys[i + 2u] : kNoKey, i + 3u < n ? keys[i + 3u] : kNoKey);
+}
+
+// f(i, rel) for every quad of keys from i on, [from, to): rel = key - c0, beyond every
+// cell of the workgroup for the others.  All lanes of a wave, whose 64 quads follow
+// each other; four quads of a lane load together.  from: a multiple of 4.
+template <class Fn>
+__device__ __forceinline__ void for_quads(const uint32_t* __restrict__ keys, uint32_t from, uint32_t to, uint32_t c0,
+                                          Fn&& f) {
+    for (uint32_t i0 = from + 4u * threadIdx.x; i0 - 4u * threadIdx.x < to; i0 += 16u * kCellThreads) {
+        const uint4 k0 = key_quad(keys, i0, to), k1 = key_quad(keys, i0 + 4u * kCellThreads, to);
+        const uint4 k2 = key_quad(keys, i0 + 8u * kCellThreads, to), k3 = key_quad(keys, i0 + 12u * kCellThreads, to);
+        f(i0, make_uint4(k0.x - c0, k0.y - c0, k0.z - c0, k0.w - c0));
+        f(i0 + 4u * kCellThreads, make_uint4(k1.x - c0, k1.y - c0, k1.z - c0, k1.w - c0));
+        f(i0 + 8u * kCellThreads, make_uint4(k2.x - c0, k2.y - c0, k2.z - c0, k2.w - c0));
+        f(i0 + 12u * kCellThreads, make_uint4(k3.x - c0, k3.y - c0, k3.z - c0, k3.w - c0));
+    }
+}
+
+// ++count[r] for every r < nc of the wave's rel.  Where most are the same, those in one
+// go (atomics of many lanes to one cell follow each other); the four most frequent ones
+// so, at each wave, took 120 instead of 67 us for 131,072 agents in 216 cells.
+__device__ __forceinline__ void wave_count(uint32_t* count, uint4 rel, uint32_t nc) {
+    const uint32_t r = __builtin_amdgcn_readfirstlane(rel.x);
+    if (r < nc && __popcll(__ballot(rel.x == r)) >= 32) {
+        const uint32_t hits = (uint32_t)(__popcll(__ballot(rel.x == r)) + __popcll(__ballot(rel.y == r)) +
+                                         __popcll(__ballot(rel.z == r)) + __popcll(__ballot(rel.w == r)));
+        if ((threadIdx.x & 63u) == 0u) atomicAdd(&count[r], hits);
+        rel.x = rel.x == r ? kNoKey : rel.x;
+        rel.y = rel.y == r ? kNoKey : rel.y;
+        rel.z = rel.z == r ? kNoKey : rel.z;
+        rel.w = rel.w == r ? kNoKey : rel.w;
+    }
+    if (rel.x < nc) atomicAdd(&count[rel.x], 1u);
+    if (rel.y < nc) atomicAdd(&count[rel.y], 1u);
+    if (rel.z < nc) atomicAdd(&count[rel.z], 1u);
+    if (rel.w < nc) atomicAdd(&count[rel.w], 1u);
+}
+
+// A place of *next for every lane that hits.
+__device__ __forceinline__ uint32_t wave_place(uint32_t* next, bool hit) {
+    const uint64_t m = __ballot(hit);
+    uint32_t at = 0u;
+    if (m == 0) return at;
+    const int first = __ffsll((unsigned long long)m) - 1;
+    if ((int)(threadIdx.x & 63u) == first) at = atomicAdd(next, (uint32_t)__popcll(m));
+    at = __builtin_amdgcn_readlane(at, first);
+    return at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Who helps with the crowded ranges.  s_cnt[g] of the kCellSample sampled keys lie in
+// range g; a range that seems to hold more than kCellAlone agents wants one helper per
+// kCellBlock (16 samples or more, where even spreading gives 4 or fewer).
+// The ranges that want none are light; the h-th light range's workgroup is the h-th
+// helper, if there are so many.  One wave (lane l has the ranges 4 l .. 4 l + 3); the
+// same in every workgroup.
+struct CellShare {
+    static constexpr uint32_t kOwn = kCellGroups / 64u;
+    uint32_t wants[kOwn], wanted;  // helpers, and those of the ranges before
+    uint32_t light;                // light ranges before, of 4 l on
+    uint32_t lights;               // all
+    __device__ __forceinline__ CellShare(const uint32_t* s_cnt, uint32_t n, uint32_t groups, uint32_t lane) {
+        uint32_t sum = 0u;  // wanted helpers << 16 | light ranges
+#pragma unroll
+        for (uint32_t g = 0; g < kOwn; ++g) {
+            const uint32_t agents = (uint32_t)((uint64_t)s_cnt[kOwn * lane + g] * n / kCellSample);
+            wants[g] = agents > kCellAlone ? agents / kCellBlock : 0u;
+            sum += wants[g] << 16 | (wants[g] == 0u && kOwn * lane + g < groups ? 1u : 0u);
+        }
+        uint32_t x = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        lights = __builtin_amdgcn_readlane(x, 63) & 0xFFFFu;
+        wanted = (x - sum) >> 16;
+        light = (x - sum) & 0xFFFFu;
+    }
+    // of the helpers before + 0 .. before + want, those that there are
+    __device__ __forceinline__ uint32_t have(uint32_t before, uint32_t want) const {
+        const uint32_t end = before + want < lights ? before + want : lights;
+        return end > before ? end - before : 0u;
+    }
+    // To one lane: the workgroups that share range g.
+    __device__ __forceinline__ void shared(uint32_t g, uint32_t lane, uint32_t* s_slices) const {
+        uint32_t before = wanted;
+#pragma unroll
+        for (uint32_t k = 0; k < kOwn; ++k) {
+            if (kOwn * lane + k == g) *s_slices = 1u + have(before, wants[k]);
+            before += wants[k];
+        }
+    }
+    // To one lane, if the workgroup of range b helps: with which range, as which of
+    // how many.
+    __device__ __forceinline__ void help(uint32_t b, uint32_t lane, uint32_t* s_group, uint32_t* s_slice,
+                                         uint32_t* s_slices) const {
+        uint32_t h = light;
+        bool is_light = false;
+#pragma unroll
+        for (uint32_t k = 0; k < kOwn; ++k) {
+            if (kOwn * lane + k < b && wants[k] == 0u) ++h;
+            if (kOwn * lane + k == b) is_light = wants[k] == 0u;
+        }
+        is_light = __ballot(is_light) != 0;
+        h = __builtin_amdgcn_readlane(h, b / kOwn);
+        uint32_t before = wanted;
+#pragma unroll
+        for (uint32_t k = 0; k < kOwn; ++k) {
+            if (is_light && before <= h && h < before + wants[k]) {
+                *s_group = kOwn * lane + k;
+                *s_slice = 1u + h - before;
+                *s_slices = 1u + have(before, wants[k]);
+            }
+            before += wants[k];
+        }
+    }
+};
+
+// Offsets of the cells c0 .. c0 + nc - 1 from their counts s_off, and, with cell_start,
+// their ranges, four consecutive cells per thread at most.  The largest count of the
+// thread's cells.
+__device__ __forceinline__ uint32_t cell_group_offsets(uint32_t* s_off, uint32_t* s_wave, uint32_t c0, uint32_t nc,
+                                                       uint32_t base, uint32_t* __restrict__ cell_start,
+                                                       uint32_t* __restrict__ cell_end) {
+    constexpr uint32_t E = kCellsPerGroup / kCellThreads;
+    uint32_t cnt[E], sum = 0u, total, most = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < E; ++k) {
+        const uint32_t c = threadIdx.x * E + k;
+        cnt[k] = c < nc ? s_off[c] : 0u;
+        sum += cnt[k];
+        most = most > cnt[k] ? most : cnt[k];
+    }
+    uint32_t off = cell_group_scan(sum, s_wave, total);
+#pragma unroll
+    for (uint32_t k = 0; k < E; ++k) {
+        const uint32_t c = threadIdx.x * E + k;
+        if (c < nc) {
+            s_off[c] = off;
+            if (cell_start) {
+                cell_start[c0 + c] = cnt[k] ? base + off : BRT_EMPTY_CELL;
+                cell_end[c0 + c] = cnt[k] ? base + off + cnt[k] : BRT_EMPTY_CELL;
+            }
+        }
+        off += cnt[k];
+    }
+    return most;
+}
+
 __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __restrict__ keys, uint32_t n,
                                                             uint32_t num_cells, uint32_t cells_per_group,
                                                             uint2* __restrict__ hash, ReorderArgs f,
                                                             uint32_t* __restrict__ cell_start,
                                                             uint32_t* __restrict__ cell_end) {
-    __shared__ alignas(16) uint32_t s_list[kCellCap];  // the sort reads four values at once
-    __shared__ uint32_t s_off[kCellsPerGroup + 1];
+    // 16-byte aligned: the sort reads four values at once
+    __shared__ alignas(16) uint32_t s_list[kCellCap];
+    __shared__ alignas(16) uint32_t s_slot[kCellCap];
+    __shared__ uint32_t s_off[kCellsPerGroup];
     __shared__ uint32_t s_rank[kCellRankMax];
     __shared__ uint32_t s_wave[kCellThreads / 64];
-    __shared__ alignas(16) uint32_t s_slot[kCellCap];
-    __shared__ uint32_t s_count, s_agents, s_below, s_most;
+    __shared__ uint32_t s_cnt[kCellGroups], s_block[kCellBlocks];
+    __shared__ uint32_t s_count, s_agents, s_below, s_most, s_wanted, s_group, s_slice, s_slices, s_lo, s_hi;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t c0 = blockIdx.x * cells_per_group;
-    const uint32_t nc = num_cells - c0 < cells_per_group ? num_cells - c0 : cells_per_group;
+    const bool spread = n > kCellAlone;  // some range may be crowded
+    // this thread's key of the sample: in short runs, since IDs may be in order of place
+    const uint32_t sampled = spread ? keys[tid / kCellRun * (n / (kCellSample / kCellRun)) + tid % kCellRun] : 0u;
+    static_assert(kCellSample == kCellThreads, "one sampled key per thread");
+    uint32_t c0 = blockIdx.x * cells_per_group;
+    uint32_t nc = num_cells - c0 < cells_per_group ? num_cells - c0 : cells_per_group;
 
     // agent id of cell c0 + rel to sorted index g; the gathers in flight together
+    // (of the compiler's own vector type: float4 structs that are loaded under a
+    // condition end up in memory, 16 bytes per lane in LDS and 20 in scratch)
     auto emit = [&](uint32_t g, uint32_t rel, uint32_t id) {
-        float4 v[kCellGather];
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        f32x4 v[kCellGather];
 #pragma unroll
         for (uint32_t q = 0; q < kCellGather; ++q)
-            if (q < f.count) v[q] = f.in[q][id];
+            if (q < f.count) v[q] = reinterpret_cast<const f32x4*>(f.in[q])[id];
         hash[g] = make_uint2(c0 + rel, id);
 #pragma unroll
         for (uint32_t q = 0; q < kCellGather; ++q)
-            if (q < f.count) f.out[q][g] = v[q];
+            if (q < f.count) reinterpret_cast<f32x4*>(f.out[q])[g] = v[q];
         if (f.xyz0) {
             float* d = f.xyz0 + 3u * (size_t)g;
             d[0] = v[0].x;
@@ -525,11 +702,13 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
         }
     };
     for (uint32_t c = tid; c < nc; c += kCellThreads) s_off[c] = 0u;
+    if (tid < kCellGroups) s_cnt[tid] = 0u;
     if (tid == 0u) {
         s_count = 0u;
         s_agents = 0u;
         s_below = 0u;
         s_most = 0u;
+        s_wanted = 0u;
     }
     __syncthreads();
 
@@ -541,6 +720,7 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
         constexpr int U = 2;
         constexpr uint32_t kStep = kCellThreads * 4u * U;
         int32_t above = 0;  // minus the number of keys below c0
+        bool full = false;
         auto load = [&](uint32_t i0, uint4 (&k)[U]) {
             if (i0 + 256u * U <= n) {  // the same for the whole wave
 #pragma unroll
@@ -569,9 +749,11 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
                     above += below;
                     least = least < (uint32_t)r[c] ? least : (uint32_t)r[c];
                 }
-                if (least < nc) {
+                // (the list is full: the range is crowded, and its keys are read again)
+                if (least < nc && !full) {
                     const uint32_t at = atomicAdd(&s_count, 1u);
                     if (at < kCellCap) s_list[at] = i0 / 4u + 64u * u + lane;
+                    full = at >= kCellCap;
                 }
             }
         };
@@ -591,11 +773,15 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
         for (int o = 32; o > 0; o >>= 1) above += __shfl_down(above, o);
         if (lane == 0u) atomicAdd(&s_below, (uint32_t)-above);
     }
+    if (spread) {
+        const uint32_t g = sampled / cells_per_group;
+        if (g < kCellGroups) atomicAdd(&s_cnt[g], 1u);
+    }
     __syncthreads();
 
-    // the quads' agents into s_slot, as cell | ID, and their number per cell (all
-    // keys again when the quads did not fit: then the agents do not either)
+    // the quads' agents into s_slot, as cell | ID, and their number per cell
     const uint32_t quads = s_count;
+    if (spread && tid < kCellGroups && s_cnt[tid] > kCellAlone * kCellSample / n) s_wanted = 1u;
     if (quads <= kCellCap) {
         for (uint32_t t = tid; t < quads; t += kCellThreads) {
             const uint32_t i = 4u * s_list[t];
@@ -609,47 +795,14 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
                 }
             }
         }
-    } else {
-        for (uint32_t i = tid; i < n; i += kCellThreads) {
-            const uint32_t rel = keys[i] - c0;
-            if (rel < nc) {
-                atomicAdd(&s_off[rel], 1u);
-                atomicAdd(&s_agents, 1u);
-            }
-        }
     }
     __syncthreads();
-    const uint32_t m = s_agents, base = s_below;
-
-    // cell offsets and ranges, four consecutive cells per thread at most
-    constexpr uint32_t E = kCellsPerGroup / kCellThreads;
-    uint32_t cnt[E], sum = 0u, total, most = 0u;
-#pragma unroll
-    for (uint32_t k = 0; k < E; ++k) {
-        const uint32_t c = tid * E + k;
-        cnt[k] = c < nc ? s_off[c] : 0u;
-        sum += cnt[k];
-        most = most > cnt[k] ? most : cnt[k];
-    }
-    if (most > kCellDense) s_most = 1u;  // some cell is crowded
-    uint32_t off = cell_group_scan(sum, s_wave, total);
-#pragma unroll
-    for (uint32_t k = 0; k < E; ++k) {
-        const uint32_t c = tid * E + k;
-        if (c < nc) {
-            s_off[c] = off;
-            if (cell_start) {
-                cell_start[c0 + c] = cnt[k] ? base + off : BRT_EMPTY_CELL;
-                cell_end[c0 + c] = cnt[k] ? base + off + cnt[k] : BRT_EMPTY_CELL;
-            }
-        }
-        off += cnt[k];
-    }
-    if (tid == 0u) s_off[nc] = m;
-    __syncthreads();
-
-    if (m <= kCellCap) {
-        if (m == 0u) return;
+    uint32_t m = s_agents, base = s_below;
+    bool crowded = quads > kCellCap || m > kCellCap;
+    if (!crowded) {
+        const uint32_t most = cell_group_offsets(s_off, s_wave, c0, nc, base, cell_start, cell_end);
+        if (most > kCellDense) s_most = 1u;  // some cell is crowded
+        __syncthreads();
         if (s_most == 0u) {
             // no crowded cell: each agent to a place of its cell, then ranked among
             // the cell's agents; s_off[c] becomes the end of cell c
@@ -665,59 +818,122 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
                 for (uint32_t j = from; j < to; ++j) r += s_list[j] < v ? 1u : 0u;
                 emit(base + r, rel, v & ((1u << kCellIdBits) - 1u));
             }
-            return;
+        } else if (m <= kCellAlone) {
+            cell_group_sort(s_slot, s_rank, m);
+            for (uint32_t i = tid; i < m; i += kCellThreads) {
+                const uint32_t v = s_slot[i];
+                emit(base + i, v >> kCellIdBits, v & ((1u << kCellIdBits) - 1u));
+            }
+        } else {
+            crowded = true;
         }
-        cell_group_sort(s_slot, s_rank, m);
-        for (uint32_t i = tid; i < m; i += kCellThreads) {
-            const uint32_t v = s_slot[i];
-            emit(base + i, v >> kCellIdBits, v & ((1u << kCellIdBits) - 1u));
-        }
-        return;
     }
-    // more agents than fit: cell ranges of at most kCellCap agents in turn, each
-    // collected by reading the keys again; a cell of more is written in ID order
-    // as the keys are read
-    uint32_t c = 0u;
-    while (c < nc) {
-        const uint32_t from = s_off[c];
-        if (s_off[c + 1u] - from > kCellCap) {
-            uint32_t g = base + from;
-            for (uint32_t i0 = 0; i0 < n; i0 += kCellThreads) {
-                const uint32_t i = i0 + tid;
-                const bool hit = i < n && keys[i] == c0 + c;
-                uint32_t all;
-                const uint32_t at = cell_group_scan(hit ? 1u : 0u, s_wave, all);
-                if (hit) emit(g + at, c, i);
-                g += all;
-            }
-            ++c;
-            continue;
+    if (!crowded && s_wanted == 0u) return;
+
+    // The crowded range of this workgroup, or a share of another's.
+    __syncthreads();
+    if (tid == 0u) {
+        s_group = blockIdx.x;
+        s_slice = 0u;
+        s_slices = crowded ? 1u : 0u;
+    }
+    __syncthreads();
+    if (wave == 0u && s_wanted != 0u) {
+        const CellShare share(s_cnt, n, (num_cells + cells_per_group - 1u) / cells_per_group, lane);
+        if (crowded)
+            share.shared(blockIdx.x, lane, &s_slices);
+        else
+            share.help(blockIdx.x, lane, &s_group, &s_slice, &s_slices);
+    }
+    __syncthreads();
+    const uint32_t slice = s_slice, slices = s_slices;
+    if (slices == 0u) return;
+    c0 = s_group * cells_per_group;
+    nc = num_cells - c0 < cells_per_group ? num_cells - c0 : cells_per_group;
+    for (uint32_t c = tid; c < nc; c += kCellThreads) s_off[c] = 0u;
+    if (tid < kCellBlocks) s_block[tid] = 0u;
+    if (tid == 0u) {
+        s_agents = 0u;
+        s_below = 0u;
+        s_most = 0u;
+    }
+    __syncthreads();
+    {
+        uint32_t agents = 0u, below = 0u;  // of the wave
+        for_quads(keys, 0u, n, c0, [&](uint32_t i, const uint4& rel) {
+            wave_count(s_off, rel, nc);
+            const uint32_t hits = (uint32_t)(__popcll(__ballot(rel.x < nc)) + __popcll(__ballot(rel.y < nc)) +
+                                             __popcll(__ballot(rel.z < nc)) + __popcll(__ballot(rel.w < nc)));
+            below += (uint32_t)(__popcll(__ballot((int32_t)rel.x < 0)) + __popcll(__ballot((int32_t)rel.y < 0)) +
+                                __popcll(__ballot((int32_t)rel.z < 0)) + __popcll(__ballot((int32_t)rel.w < 0)));
+            agents += hits;
+            // a wave's quads lie in one block
+            if (hits != 0u && lane == 0u) atomicAdd(&s_block[i / kCellBlock], hits);
+        });
+        if (lane == 0u) {
+            atomicAdd(&s_agents, agents);
+            atomicAdd(&s_below, below);
         }
-        uint32_t lo = c + 1u, hi = nc;  // the last cell end with at most kCellCap agents from c
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1u) / 2u;
-            if (s_off[mid] - from <= kCellCap)
-                lo = mid;
-            else
-                hi = mid - 1u;
+    }
+    __syncthreads();
+    m = s_agents;
+    base = s_below;
+    const uint32_t most =
+        cell_group_offsets(s_off, s_wave, c0, nc, base, slice == 0u ? cell_start : nullptr, cell_end);
+    if (most > kCellDense) s_most = 1u;
+    __syncthreads();
+    // (the range's own workgroup has sorted it)
+    if (m <= kCellAlone || (m <= kCellCap && s_most == 0u)) return;
+
+    // chunks of consecutive IDs, each of at most 2 kCellBlock - 1 agents, in turn by
+    // the workgroups that share the range
+    // a block's chunk: the agents of the blocks before it / kCellBlock
+    const uint32_t in_block = tid < kCellBlocks ? s_block[tid] : 0u;
+    uint32_t sum_blocks;
+    const uint32_t before_block = cell_group_scan(in_block, s_wave, sum_blocks);
+    const uint32_t my_chunk = before_block / kCellBlock, chunks = (m - 1u) / kCellBlock + 1u;
+    uint32_t* const s_before = s_slot;  // by cell: its agents before the chunk
+    static_assert(kCellCap >= kCellsPerGroup && kCellCap >= 2u * kCellBlock, "LDS of the crowded path");
+    for (uint32_t chunk = slice; chunk < chunks; chunk += slices) {
+        __syncthreads();  // the chunk before is done
+        for (uint32_t c = tid; c < nc; c += kCellThreads) s_before[c] = 0u;
+        if (tid == 0u) {
+            s_count = 0u;
+            s_lo = kCellBlocks;
+            s_hi = 0u;
         }
-        const uint32_t mm = s_off[lo] - from;
-        if (mm != 0u) {
-            __syncthreads();
-            if (tid == 0u) s_count = 0u;
-            __syncthreads();
-            for (uint32_t i = tid; i < n; i += kCellThreads) {
-                const uint32_t rel = keys[i] - c0;
-                if (rel - c < lo - c) s_list[atomicAdd(&s_count, 1u)] = rel << kCellIdBits | i;
-            }
-            __syncthreads();
-            cell_group_sort(s_list, s_rank, mm);
-            for (uint32_t i = tid; i < mm; i += kCellThreads) {
-                const uint32_t v = s_list[i];
-                emit(base + from + i, v >> kCellIdBits, v & ((1u << kCellIdBits) - 1u));
-            }
+        __syncthreads();
+        if (in_block != 0u && my_chunk == chunk) {
+            atomicMin(&s_lo, tid);
+            atomicMax(&s_hi, tid + 1u);
         }
-        c = lo;
+        __syncthreads();
+        const uint32_t lo = s_lo * kCellBlock, end = s_hi * kCellBlock, hi = end < n ? end : n;
+        if (lo >= hi) continue;  // no block ends up in this one
+        for_quads(keys, 0u, lo, c0, [&](uint32_t, const uint4& rel) { wave_count(s_before, rel, nc); });
+        auto take = [&](uint32_t i, uint32_t rel) {
+            const uint32_t at = wave_place(&s_count, rel < nc);
+            if (rel < nc) s_list[at] = rel << kCellIdBits | i;
+        };
+        for_quads(keys, lo, hi, c0, [&](uint32_t i, const uint4& rel) {
+            take(i, rel.x);
+            take(i + 1u, rel.y);
+            take(i + 2u, rel.z);
+            take(i + 3u, rel.w);
+        });
+        __syncthreads();
+        const uint32_t mm = s_count;
+        cell_group_sort(s_list, s_rank, mm);
+        // s_before[c]: the place of the chunk's first agent of cell c, less its index
+        for (uint32_t i = tid; i < mm; i += kCellThreads) {
+            const uint32_t rel = s_list[i] >> kCellIdBits;
+            if (i == 0u || s_list[i - 1u] >> kCellIdBits != rel) s_before[rel] += s_off[rel] - i;
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < mm; i += kCellThreads) {
+            const uint32_t v = s_list[i], rel = v >> kCellIdBits;
+            emit(base + s_before[rel] + i, rel, v & ((1u << kCellIdBits) - 1u));
+        }
     }
 }
 
@@ -902,8 +1118,9 @@ hipError_t launch_cell_sort(const uint32_t* keys, uint32_t n, uint32_t num_cells
                             uint32_t* cell_start, uint32_t* cell_end, hipStream_t s) {
     const uint32_t per = cell_sort_cells(n, num_cells);
     if (per == 0u || f.count > kCellGather || (f.xyz0 && f.count == 0u)) return hipErrorInvalidValue;
-    BRT_LAUNCH(k_cell_sort, dim3((num_cells + per - 1u) / per), dim3(kCellThreads), 0, s, keys, n, num_cells, per,
-               hash, f, cell_start, cell_end);
+    const uint32_t groups = (num_cells + per - 1u) / per;
+    BRT_LAUNCH(k_cell_sort, dim3(groups), dim3(kCellThreads), 0, s, keys, n, num_cells, per, hash, f, cell_start,
+               cell_end);
     return hipGetLastError();
 }
 
