@@ -32,6 +32,7 @@ SIGNATURES = {
     "brt_context_set_option": (_I, [_P, _I, _I]),
     "brt_context_get_option": (_I, [_P, _I, C.POINTER(_I)]),
     "brt_context_step_shape": (_I, [_P, _PP, C.POINTER(_I), C.POINTER(_I)]),
+    "brt_context_step_shape_for": (_I, [_P, _PP, _U32, _U32, _I, C.POINTER(_I), C.POINTER(_I), C.POINTER(_I)]),
     "brt_context_check": (_I, [_P]),
     "brt_grid_setup": (_I, [C.POINTER(_F), C.POINTER(_F), C.POINTER(_F), _U32, _GP]),
     "brt_list_stride": (_U32, [_U32]),

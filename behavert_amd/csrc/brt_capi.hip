@@ -373,6 +373,17 @@ int brt_context_step_shape(const brt_context* ctx, const brt_prox_params* prox, 
     return BRT_OK;
 }
 
+int brt_context_step_shape_for(const brt_context* ctx, const brt_prox_params* prox, uint32_t n, uint32_t num_cells,
+                               int features, int* fused, int* lds_lists, int* lanes_per_agent) {
+    if (!ctx || !prox || !fused || !lds_lists || !lanes_per_agent) return BRT_ERR_INVALID_ARGUMENT;
+    const StepShape shape = resolve_step(ctx, prox, n, num_cells, features != 0);
+    const bool quads = resolve_quads(ctx, prox, n, shape.fused);
+    *fused = shape.fused ? 1 : 0;
+    *lds_lists = shape.lds != 0u || quads ? 1 : 0;
+    *lanes_per_agent = quads ? 4 : 1;
+    return BRT_OK;
+}
+
 int brt_grid_setup(const float world_center[3], const float world_radius[3], const float cell_size[3],
                    uint32_t max_bodies_per_cell, brt_grid_params* out) {
     if (!world_center || !world_radius || !cell_size || !out) return BRT_ERR_INVALID_ARGUMENT;

@@ -183,10 +183,19 @@ class Context:
         self.check(self._lib.brt_context_set_option(self.handle, int(option), int(value)))
 
     def step_shape(self, prox) -> tuple[bool, bool]:
-        """(fused, lds_lists) that brt_step uses for these proximity parameters."""
+        """(fused, lds_lists) that the options and these proximity parameters alone
+        ask for; a step's own shape: step_shape_for."""
         f, l = C.c_int(), C.c_int()
         self.check(self._lib.brt_context_step_shape(self.handle, C.byref(prox), C.byref(f), C.byref(l)))
         return bool(f.value), bool(l.value)
+
+    def step_shape_for(self, prox, n: int, num_cells: int, features: bool = False) -> tuple[bool, bool, int]:
+        """(fused, lds_lists, lanes_per_agent) of a step of n agents in a grid of
+        num_cells cells, with the feature update or without."""
+        f, l, a = C.c_int(), C.c_int(), C.c_int()
+        self.check(self._lib.brt_context_step_shape_for(self.handle, C.byref(prox), int(n), int(num_cells),
+                                                        int(bool(features)), C.byref(f), C.byref(l), C.byref(a)))
+        return bool(f.value), bool(l.value), a.value
 
     def get_option(self, option: int) -> int:
         v = C.c_int()

@@ -25,6 +25,11 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 
 
+def has_features(w) -> bool:
+    """Whether the workload's steps update features."""
+    return w.features is not None and bool(w.feature_rate)
+
+
 def algorithmic_bytes_per_agent(w, packed=False, sorted_sa=False) -> dict:
     """Compulsory single-touch HBM bytes per agent for each phase of brt_step.
     D digit passes, W list words, C/N cells per agent, F reordered float4s
@@ -51,7 +56,7 @@ def algorithmic_bytes_per_agent(w, packed=False, sorted_sa=False) -> dict:
         "steer_integrate": 100 + 4 * W,
         "features": 0.0,
     }
-    if w.features is not None and w.feature_rate:
+    if has_features(w):
         b["features"] = 4 + 4 * W + 32  # R ID + list, R own feature 16, W 16
         # the two-pass step gathers the features into sorted order with the
         # state (R 16 by ID, W 16) and updates them in the steering pass (the
@@ -288,8 +293,8 @@ def full_stack(steps=20, warmup=3) -> dict:
     run(warmup, steps)
     torch.cuda.synchronize()
     el = time.perf_counter() - t0
-    fused, lds = ctx.step_shape(w.prox)
-    abytes = algorithmic_bytes_per_agent(w, packed=bool(lds) and not w.prox.use_knn, sorted_sa=False)
+    fused, lds, lanes = ctx.step_shape_for(w.prox, w.n, w.grid.num_cells, has_features(w))
+    abytes = algorithmic_bytes_per_agent(w, packed=lds and not w.prox.use_knn, sorted_sa=False)
     ph = phase_table(ctx, w, abytes, fused=fused)
     ctx.phase_timing(False)
     ctx.close()
@@ -300,7 +305,8 @@ def full_stack(steps=20, warmup=3) -> dict:
                 "agents_per_launch": w.n, "avg_launch_ms": ph[dom]["ms"]}
     return {**w.describe(), "sorted_smooth_accel": False, "ms_per_step": round(1e3 * el / steps, 4),
             "agent_updates_per_s": w.n * steps / el,
-            "phases": ph, "roofline": roofline, "timed_steps": steps, "step_shape": {"fused": fused, "lds_lists": lds}}
+            "phases": ph, "roofline": roofline, "timed_steps": steps,
+            "step_shape": {"fused": fused, "lds_lists": lds, "lanes_per_agent": lanes}}
 
 
 def clustering(reps=20, features=8, lp_iterations=10) -> dict:
@@ -562,8 +568,8 @@ def main():
                 fl.steer.set_targets(w.targets_at(i))
             fl.step(w.dt, i, w.feature_rate)
 
-    abytes = algorithmic_bytes_per_agent(w, packed=bool(ctx.step_shape(w.prox)[1]) and not w.prox.use_knn,
-                                         sorted_sa=False)
+    lds = ctx.step_shape_for(w.prox, w.n, w.grid.num_cells, has_features(w))[1]
+    abytes = algorithmic_bytes_per_agent(w, packed=lds and not w.prox.use_knn, sorted_sa=False)
     run(0, args.warmup)
     torch.cuda.synchronize()
     # the timed steps: nothing between them but the steps themselves

@@ -116,8 +116,8 @@ const char* brt_version(void);
 /* Context options (launch-shape and fusion choices; none changes any result bit).
  * BRT_OPT_FUSED_STEP: brt_step builds the neighbour lists and runs steering +
  *   integration in one kernel (1) or writes the lists and steers from them (0)
- *   (default -1 = automatic: fused for K <= 32, two passes above, where the
- *   fused kernel's occupancy falls; KNN lists always use two passes).
+ *   (default -1 = automatic: fused for K <= 32; above by the step's size, grid and
+ *   feature update, brt_context_step_shape_for; KNN lists always use two passes).
  * BRT_OPT_UNIFORM_MAX_CELLS: a wave64 whose agents lie in at most this many
  *   cells scans candidates with wave-uniform (scalar-cache) loads (default 1;
  *   0 = every wave scans per lane).
@@ -126,7 +126,8 @@ const char* brt_version(void);
  * BRT_OPT_LDS_LISTS: the neighbour kernels stage each workgroup's lists in LDS
  *   and write them out with coalesced 16-byte stores (1), or gather each list's
  *   16-byte chunks in registers and store them as they fill (0), which leaves
- *   LDS free and raises occupancy (default -1 = automatic: LDS for K <= 32).
+ *   LDS free and raises occupancy (default -1 = automatic: LDS for K <= 32 and in
+ *   small launches, above by the step's size and grid, brt_context_step_shape_for).
  * No counterpart in the reference (its launch shapes are fixed per kernel:
  * Proximity3DPlugIn.h:133-134, CommonResources.cpp:78-82). */
 #define BRT_OPT_FUSED_STEP 1
@@ -147,14 +148,22 @@ const char* brt_version(void);
 #define BRT_OPT_STEP_GRAPH 6
 int brt_context_set_option(brt_context* ctx, int option, int value);
 int brt_context_get_option(const brt_context* ctx, int option, int* value);
-/* The launch shape brt_step and brt_prox_neighbors use for these proximity
- * parameters once automatic options are resolved: fused (0/1), lds_lists (0/1).
- * With lds_lists automatic, launches of up to 131,072 agents take four lanes per
- * agent and stage their lists in LDS for every K, and steps without the feature
- * update are fused there; larger ones of 32 < K <= 80 are fused with LDS lists
- * too (without features; from 2^21 agents where the grid holds 8 per cell or
- * more), and in such crowded grids list passes stage their lists in LDS. */
+/* The launch shape that the options and these proximity parameters alone ask for:
+ * fused (0/1), lds_lists (0/1).  With automatic options a step's own shape follows
+ * from its size, grid and feature update too: brt_context_step_shape_for. */
 int brt_context_step_shape(const brt_context* ctx, const brt_prox_params* prox, int* fused, int* lds_lists);
+/* The launch shape that brt_step takes for n agents in a grid of num_cells cells,
+ * features: whether it updates features (a feature_rate other than 0):
+ *   fused            lists, steering and integration in one kernel (0/1)
+ *   lds_lists        the lists are built in LDS (0/1)
+ *   lanes_per_agent  lanes that search one agent's neighbours (4 or 1)
+ * With lists automatic, launches of up to 131,072 agents (fewer for some K) take four
+ * lanes per agent and build their lists in LDS, and steps without the feature update
+ * are fused there; larger ones of 32 < K <= 80 are fused with LDS lists (without
+ * features; from 2^21 agents where the grid holds 8 per cell or more), and in such
+ * crowded grids two-pass steps build their lists in LDS. */
+int brt_context_step_shape_for(const brt_context* ctx, const brt_prox_params* prox, uint32_t n, uint32_t num_cells,
+                               int features, int* fused, int* lds_lists, int* lanes_per_agent);
 
 /* Failures the kernels record on the device instead of hanging or faulting:
  * BRT_DEVFLAG_SORT_LOOKBACK - a radix-sort pass gave up a look-back wait after
