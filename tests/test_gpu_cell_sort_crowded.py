@@ -73,6 +73,18 @@ def test_blobs_beside_even_agents(ctx, orc, size, sigma):
     check_sort(ctx, orc, grid, st)
 
 
+@pytest.mark.parametrize("n,side,blobs", [(47839, 140.0, 2), (100517, 184.0, 6)])
+@pytest.mark.parametrize("seed", [16, 21, 22, 23])
+def test_ranges_on_either_side_of_the_sample(ctx, orc, n, side, blobs, seed):
+    """Ranges of about 2,048 agents, which the sampled keys show crowded or light by
+    chance: the workgroup of one that they show light is counted on as a helper."""
+    rng = np.random.default_rng(seed)
+    centres = rng.random((blobs, 3)) * side
+    of = rng.permutation(n) % blobs
+    xyz = side - np.abs(side - np.abs(centres[of] + 10.0 * rng.standard_normal((n, 3))))
+    check_sort(ctx, orc, W.cube_grid(side), flock_state(n, np.clip(xyz, 0.0, np.nextafter(np.float32(side), 0))))
+
+
 def test_two_crowded_cells_and_their_neighbours(ctx, orc):
     """Whole steps, with the gathers of the sorted state and the lists."""
     rng = np.random.default_rng(5)
