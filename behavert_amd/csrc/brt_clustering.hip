@@ -396,7 +396,10 @@ __global__ void __launch_bounds__(256) k_bc_records(uint32_t F, uint32_t n, uint
     rec[t] = r;
 }
 
-template <bool ADAPTIVE, int FQ>
+// STAGED: the list rows in LDS (W <= kStageWords); else in memory, read ahead, which
+// takes the registers of the fourth wave per SIMD with up to 8 features (staged rows
+// too, when both were one kernel: 200,003 agents, K 16, F 8 44 -> 48 us).
+template <bool ADAPTIVE, int FQ, bool STAGED>
 __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     uint32_t K, uint32_t W, brt_bc_params bc, uint32_t n, const uint2* __restrict__ hash,
     const uint32_t* __restrict__ lists, const float4* __restrict__ rec, const float4* __restrict__ stats_in,
@@ -414,18 +417,13 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     const uint32_t RW = similarity_row_words(K, W);
     uint32_t* const row = reinterpret_cast<uint32_t*>(mem) + lane * RW;
     vfloat4* const tile = reinterpret_cast<vfloat4*>(mem + wave_bytes - kTileChunks * 16u);
-    const bool staged = W <= kStageWords;
-    if (staged) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
+    if (STAGED) stage_rows(reinterpret_cast<uint4*>(mem), lists, W, row0, lane, n);
     const vuint4* const L = reinterpret_cast<const vuint4*>(lists + (size_t)at * W);
-    // word q of the row, if it holds an entry
+    // word q of the row, if it holds an entry (else any value)
     auto word = [&](uint32_t q, uint32_t last) {
+        if (STAGED) return reinterpret_cast<const vuint4*>(row)[q < last ? q : last];
         vuint4 v = {0u, 0u, 0u, 0u};
-        if (q <= last) {
-            if (staged)
-                v = reinterpret_cast<const vuint4*>(row)[q];
-            else
-                v = L[q];
-        }
+        if (q <= last) v = L[q];
         return v;
     };
 
@@ -449,17 +447,18 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
     vuint4 a = word(0u, 0u);
     const uint32_t count = i < n ? (a.x < K ? a.x : K) : 0u, last = count / 4u;
     float* const out = reinterpret_cast<float*>(row);
-    vuint4 b = word(1u, last), na, nb;
+    vuint4 b, na, nb;
+    if (!STAGED) b = word(1u, last);
     // all lanes of the wave stay in step: those past their list load their own record
     for (uint32_t q = 0; __ballot(q <= last) != 0; q += 2) {
         // rows in memory: the next words load during this octet's gathers; staged
         // ones are read when they are used (this octet overwrites the row up to word
         // 4 q + 6)
-        if (!staged) {
+        if (!STAGED) {
             na = word(q + 2u, last);
             nb = word(q + 3u, last);
-        } else if (q != 0u) {
-            a = word(q, last);
+        } else {
+            if (q != 0u) a = word(q, last);
             b = word(q + 1u, last);
         }
         uint32_t jj[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
@@ -515,7 +514,7 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
                         sim);
             }
         }
-        if (!staged) {
+        if (!STAGED) {
             a = na;
             b = nb;
         }
@@ -764,7 +763,10 @@ hipError_t launch_sims(uint32_t K, const brt_bc_params& bc, uint32_t n, const ui
                            vec, hash, features, spos, sfwd, rec);
         // four waves per workgroup while three workgroups fit a CU's LDS, else one
         const uint32_t bytes = similarity_wave_bytes(K, W), B = 4u * bytes <= 160u * 1024u / 3u ? 256u : 64u;
-        const auto kernel = bc.adaptive ? k_bc_similarities_steer<true, FQ> : k_bc_similarities_steer<false, FQ>;
+        const auto kernel = W <= kStageWords ? (bc.adaptive ? k_bc_similarities_steer<true, FQ, true>
+                                                            : k_bc_similarities_steer<false, FQ, true>)
+                                             : (bc.adaptive ? k_bc_similarities_steer<true, FQ, false>
+                                                            : k_bc_similarities_steer<false, FQ, false>);
         hipLaunchKernelGGL(kernel, dim3((n + B - 1) / B), dim3(B), B / 64u * bytes, s, K, W, bc, n, hash, lists, rec,
                            stats_in, stats_out, sims, *sp, sfwd, force_in, force_out, bytes, sims_vec, xcd_remap);
         return hipGetLastError();
@@ -793,20 +795,28 @@ size_t bc_scratch_bytes(uint32_t feature_count, uint32_t n) {
     return (size_t)n * FQ * 16u + ((size_t)n * 4u + 15u) / 16u * 16u;
 }
 
-// From 147,456 agents (196,608 for up to 4 features or beyond K 48), where the
-// accesses of the gathers set the pace: below, each agent's own gathers have the
-// shorter chain and leave room for more waves (K 32, F 8: 1,000 agents 13.4 us, from
-// records 15.5; 60,000 20 and 22; 131,072 23 and 28).  Lists beyond K 64 (80 from 9
-// features on) leave the records' tile too few waves.  With up to 4 features a record
-// saves one access in four, which pays for its making only where lists are long: K
-// 24 to 48.  1,048,576 agents at 1 / 4 / 12 per cell, own gathers -> records, us: F 4,
-// K 32 150 -> 180, 244 -> 249, 390 -> 279; F 8, K 32 194 -> 187, 307 -> 255, 433 ->
-// 293, K 80 238 -> 260, 373 -> 383, 661 -> 675; F 16, K 32 289 -> 272, 462 -> 377,
-// 788 -> 429, K 80 344 -> 341, 525 -> 501, 990 -> 885.
+// Where the accesses of the gathers set the pace: below, each agent's own gathers have
+// the shorter chain and leave room for more waves (K 32, F 8: 1,000 agents 13.4 us, from
+// records 15.5; 60,000 20 and 22).  Lists of one density or another lie on either side;
+// the lines are where the records win over flocks of 1, 4 and 12 per cell and blobs
+// taken together.  Own gathers -> records, us, at these four:
+//   * from 98,304 agents with 5 features or more, K >= 24 (from 9 on, every K): 100,003
+//     agents, K 32, F 8 27 -> 29, 42 -> 42, 51 -> 44, 49 -> 44; F 16 31 -> 37, 56 -> 54,
+//     76 -> 56, 74 -> 56; K 16, F 16 30 -> 35, 44 -> 39, 46 -> 39, 44 -> 38;
+//   * from 147,456 below K 24: 131,072 agents, K 16, F 8 27 -> 30, 31 -> 34, 32 -> 33,
+//     33 -> 34;
+//   * from 196,608 with up to 4 features, where a record saves one access in four, and
+//     from K 49 on: 131,072 agents, K 24, F 4 25 -> 29, 34 -> 39, 38 -> 39, 39 -> 39;
+//     and there for K 16 to 48 (K 16, F 4, 200,003 agents 33 -> 35, 48 -> 43, 50 -> 42,
+//     47 -> 42), up to 786,432 agents for the short ones (1,048,576 agents 132 -> 156,
+//     186 -> 190, 212 -> 190, 196 -> 185).
+// Lists beyond K 64 (80 from 9 features on) leave the records' tile too few waves:
+// 1,048,576 agents at 1 / 4 / 12 per cell, F 8, K 80 238 -> 260, 373 -> 383, 661 -> 675;
+// F 16, K 80 344 -> 341, 525 -> 501, 990 -> 885.
 size_t bc_record_bytes(uint32_t K, uint32_t feature_count, uint32_t n) {
     const size_t FQ = (feature_count + 3u) / 4u;
-    const bool pays = FQ == 1u ? K >= 24u && K <= 48u : K <= (FQ == 2u ? 64u : 80u);
-    const uint32_t least = FQ == 1u || K > 48u ? 3u << 16 : 9u << 14;
+    const bool pays = FQ == 1u ? K >= (n < (3u << 18) ? 16u : 24u) && K <= 48u : K <= (FQ == 2u ? 64u : 80u);
+    const uint32_t least = FQ == 1u || K > 48u ? 3u << 16 : FQ == 2u && K < 24u ? 9u << 14 : 3u << 15;
     return n >= least && pays ? (size_t)n * ((FQ + 5u) / 4u) * 64u : 0u;
 }
 

@@ -93,6 +93,17 @@ def test_records(ctx, orc, n, K, F, adaptive):
         assert same(st, rst)
 
 
+SOON = 3 << 15
+
+
+@pytest.mark.parametrize("n,K,F,adaptive", [(SOON - 1, 32, 8, True), (SOON, 32, 8, True), (SOON + 63, 24, 5, False),
+                                            (SOON, 23, 8, True), (SOON + 1, 36, 6, True), (SOON + 1, 4, 9, True),
+                                            (SOON, 48, 16, True), (LEAST + 1, 16, 8, True), (WIDE - 1, 16, 4, True),
+                                            (WIDE + 63, 16, 3, False), (WIDE, 15, 4, True)])
+def test_records_by_list_and_feature_length(ctx, orc, n, K, F, adaptive):
+    test_records(ctx, orc, n, K, F, adaptive)
+
+
 def test_captured_without_room_for_records(orc):
     """A warm-up with the similarities alone, then the pass with the steering captured."""
     n, K, F = LEAST + 5, 32, 8
