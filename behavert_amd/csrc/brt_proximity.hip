@@ -704,7 +704,12 @@ __device__ __forceinline__ uint32_t visit_mask(const Seg& sg, const Lane& L, I3 
 // and in blobs gains 4 / 3 / 3 % at K 32, 5 / 3 / 3 % at K 28, 3 / 1 / 0 % at K 24
 // and -0 / -1 / -1 % at K 16; of 500,009 agents 7 / 5 / 2 % at K 32, of 300,007
 // (one wave more than the chip holds at once) 0 / 1 / 0 %.
+// Fused steps of long lists lose by it where the cells hold many (the waves in flight
+// are fewer then): 1M agents at 10 / 32 per cell and in blobs +8 / -1 / -3 % at K 48,
+// +3 / -6 / -5 % at K 64 and +2 / -6 / -5 % at K 80; the list pass alone gains or stays:
+// +15 / 1 / 0 % at K 48, +13 / -3 / 0 % at K 64.
 constexpr uint32_t kTogetherK = 28u;
+constexpr uint32_t kTogetherFusedMax = 56u;
 template <int CTRL>
 __device__ __forceinline__ uint32_t visit_with(uint32_t todo, I3 gp) {
     const bool same = __builtin_amdgcn_mov_dpp(gp.x, CTRL, 0xF, 0xF, true) == gp.x &&
@@ -740,7 +745,8 @@ __device__ __forceinline__ void flat_fetch(const ProxArgs& a, const Seg& sg, I3 
 // in the round j_self = own_start + G * floor((i - own_start) / G), in slot
 // (i - own_start) mod G, and in no round of another cell.
 template <int G, bool PACKED>
-__device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, uint32_t own_start) {
+__device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, uint32_t own_start,
+                                          bool together) {
     static_assert((G & (G - 1)) == 0, "the self round is found with a mask");
     const brt_grid_params& g = sg.g;
     const uint32_t maxBodies = g.max_bodies_per_cell;
@@ -750,7 +756,7 @@ __device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane
     const uint32_t jself = L.i - ds;
     const uint32_t smask = ~(1u << ((uint32_t)G - 1u - ds));
     uint32_t todo = visit_mask(sg, L, gp, a.Tskip);
-    if (a.K >= kTogetherK) todo = visit_together(todo, gp);
+    if (together) todo = visit_together(todo, gp);
     // the fetched (next) cell: ordinal nc (27: none left) and its range
     uint32_t nc = 27u, ns = BRT_EMPTY_CELL, ne = 0u;
     flat_fetch(a, sg, gp, todo, nc, ns, ne);
@@ -1125,19 +1131,20 @@ __global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) 
         }
         // with the packed positions a round's loads are 3G/4 instead of G
         const bool packed = a.pxyz != nullptr;
+        const bool together = a.K >= kTogetherK && (!FUSE || a.K <= kTogetherFusedMax);
         if (LDSL && BRT_PROX_FLAT && dense && a.log_rounds) {
             if (alive) {
                 if (packed)
-                    scan_flat<kGroupL, true>(a, sg, L, gp, own_start);
+                    scan_flat<kGroupL, true>(a, sg, L, gp, own_start, together);
                 else
-                    scan_flat<kGroupL, false>(a, sg, L, gp, own_start);
+                    scan_flat<kGroupL, false>(a, sg, L, gp, own_start, together);
             }
         } else if (LDSL && BRT_PROX_FLAT_SPARSE && a.log_rounds) {
             if (alive) {
                 if (packed)
-                    scan_flat<kGroupR, true>(a, sg, L, gp, own_start);
+                    scan_flat<kGroupR, true>(a, sg, L, gp, own_start, together);
                 else
-                    scan_flat<kGroupR, false>(a, sg, L, gp, own_start);
+                    scan_flat<kGroupR, false>(a, sg, L, gp, own_start, together);
             }
         } else if (alive) {
             if (dense) {

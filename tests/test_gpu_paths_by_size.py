@@ -79,3 +79,20 @@ def test_four_lanes_with_nan_and_coincident_agents(ctx, orc, K, maxb):
         got, want = fl.state(), host.state()
         for k in ("pos", "forward", "smooth_accel"):
             assert np.array_equal(got[k], want[k], equal_nan=True), (step, k)
+
+
+@pytest.mark.parametrize("K", [27, 28, 56, 57, 80])
+def test_crowded_fused_steps(ctx, orc, K):
+    """About 20 agents per cell: quads of lanes visit their cells together or not, by K."""
+    rng = np.random.default_rng(K)
+    grid, prox = GridParams.direct((0.0,) * 3, (4.0,) * 3, (19,) * 3), ProxParams.make(K, 4.0)
+    st = W.make_state(rng.uniform(0, 76, (RADIX, 3)).astype(np.float32), *W.directions_and_speeds(rng, RADIX))
+    assert ctx.step_shape_for(prox, RADIX, grid.num_cells) == (True, True, 1)
+    o = oracle_grid_outputs(orc, grid, prox, st)
+    assert first_mismatch(gpu_lists(ctx, grid, prox, o), o["lists"]) is None
+    fl, host = Flock(ctx, grid, prox, W.plain_steer(), st), orc.HostFlock(grid, prox, st)
+    fl.step(0.05, 0)
+    host.step(W.plain_steer(), 0.05, 0)
+    assert first_mismatch(fl.grid_outputs()["lists"].view(np.uint32), host.lists) is None
+    for k, x in fl.state().items():
+        assert first_mismatch(x.view(np.uint32), host.state()[k].view(np.uint32)) is None, k
