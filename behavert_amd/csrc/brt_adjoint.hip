@@ -30,6 +30,7 @@
 #include "brt_device.hpp"
 #include "brt_internal.hpp"
 #include "brt_steer_common.hpp"
+#include "brt_wave.hpp"
 
 namespace brt {
 
@@ -136,15 +137,7 @@ __device__ __forceinline__ V3 pair_terms(const brt_steer_params& sp, uint32_t fl
 template <int NL>
 __device__ __forceinline__ float quad_get(float v, int k) {
     if (NL == 1) return v;
-    const int x = __float_as_int(v);
-    int r;
-    switch (k) {
-        case 0: r = __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, true); break;
-        case 1: r = __builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, true); break;
-        case 2: r = __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, true); break;
-        default: r = __builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, true); break;
-    }
-    return __int_as_float(r);
+    return k == 0 ? quad_lane<0>(v) : k == 1 ? quad_lane<1>(v) : k == 2 ? quad_lane<2>(v) : quad_lane<3>(v);
 }
 
 // s + v of the quad's lanes in order: entry by entry as one lane would add them.

@@ -472,11 +472,11 @@ __global__ void __launch_bounds__(256) k_bc_similarities_steer(
             for (int g = 0; g < G; ++g) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const int x = (int)jj[g0 + g];
-                    const uint32_t j = (uint32_t)(k == 0   ? __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, true)
-                                                  : k == 1 ? __builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, true)
-                                                  : k == 2 ? __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, true)
-                                                           : __builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, true));
+                    const uint32_t x = jj[g0 + g];
+                    const uint32_t j = k == 0   ? quad_lane<0>(x)
+                                       : k == 1 ? quad_lane<1>(x)
+                                       : k == 2 ? quad_lane<2>(x)
+                                                : quad_lane<3>(x);
                     const vfloat4* const src = reinterpret_cast<const vfloat4*>(rec) + (size_t)j * RP + l;
 #pragma unroll
                     for (int r = 0; r < NR; ++r) in[g][r][k] = src[4 * r];

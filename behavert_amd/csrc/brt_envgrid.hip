@@ -19,6 +19,7 @@
 // < cells, so the higher digits are all zero and cannot change a stable order.
 #include "brt_device.hpp"
 #include "brt_internal.hpp"
+#include "brt_wave.hpp"
 
 namespace brt {
 
@@ -419,12 +420,6 @@ __global__ void __launch_bounds__(256) k_batch_hash_keys(BatchView b, const floa
     keys[i] = fd.cell_base + calcGridHash(calcGridPos(p.x, p.y, p.z, fd.g), fd.g);
 }
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Exclusive scan of one value per thread over the workgroup; total to all.
 __device__ __forceinline__ uint32_t cell_group_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -502,7 +497,7 @@ __device__ __forceinline__ void cell_group_sort(uint32_t* s_list, uint32_t* s_ra
             if (j > 64u || j == 1u)
                 __syncthreads();
             else
-                wave_sync();
+                wave_lds_sync();
         }
     }
 }

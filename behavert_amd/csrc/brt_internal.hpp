@@ -146,8 +146,8 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
                         float4* force_out, uint32_t xcd_remap, hipStream_t s, float feature_rate = 0.0f,
                         const float4* features_in = nullptr, float4* features_out = nullptr,
                         const float4* sorted_features = nullptr, float4* records = nullptr);
-// records (optional, 4 float4 per agent, with features_in only where sorted_features
-// are there): scratch through which the new state goes to the arrays; ssa != NULL.
+// features_in only with sorted_features.  records (optional, 4 float4 per agent):
+// scratch through which the new state goes to the arrays; ssa != NULL.
 // launch_pack: up to four float4 arrays (NULL: left out) into such records.
 hipError_t launch_pack(uint32_t n, const float4* a, const float4* b, const float4* c, const float4* d, float4* rec,
                        hipStream_t s);

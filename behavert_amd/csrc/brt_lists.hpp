@@ -6,16 +6,11 @@
 
 #include <cstdint>
 
+#include "brt_wave.hpp"
+
 namespace brt {
 
 typedef uint32_t vuint4 __attribute__((ext_vector_type(4)));
-
-// What every lane of the wave wrote to LDS is seen by the others.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Bit k set for the valid entries e = 4q + k of an octet (1 <= e <= count and
 // a sorted index below n); invalid lanes of jj are set to i.  Word entry 0 of

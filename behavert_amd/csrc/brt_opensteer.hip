@@ -24,10 +24,6 @@ namespace brt {
 
 namespace {
 
-// One lane per sorted agent: walk the list in order (8 entries per round, their
-// gathers issued together), accumulate the behaviour sums, then assemble the
-// force and integrate (APPLY), or only store the behaviour force in sorted
-// order (the steer-force accumulator of the decomposed sequence).
 // The feature update of the agent at sorted index i (ID id):
 // f + (mean of the listed neighbours' features - f) * rate, the mean over the
 // list's count; the entries are visited eight at a time with their ID and
@@ -79,19 +75,23 @@ __global__ void __launch_bounds__(256) k_features(uint32_t W, float rate, uint32
     if (id < n) fout[id] = f;
 }
 
+// One lane per sorted agent: walk the list in order (8 entries per round, their
+// gathers issued together), accumulate the behaviour sums, then assemble the
+// force and integrate (APPLY), or only store the behaviour force in sorted
+// order (the steer-force accumulator of the decomposed sequence).
 // FEAT: the same pass also writes the agent's feature update (the result of
 // feature_update), summing the neighbours' features in the same list walk as
 // the steering sums; with all steering weights zero it calls feature_update.
-// SFEAT: the neighbours' features are read from sfeat, the features in sorted
-// order (sfeat[j] = fin[hash[j].y], gathered with the state), so the walk reads
-// them next to their positions instead of at random agent IDs.
+// The neighbours' features are read from sfeat, the features in sorted order
+// (sfeat[j] = fin[hash[j].y], gathered with the state), so the walk reads them
+// next to their positions instead of at random agent IDs.
 // REC: the new state (and feature) goes to one 64-byte record by ID instead of
 // to the arrays: a write to a random ID costs the same whatever its size (about
 // 45 G a second), and k_unpack moves the records to the arrays in order.
 // With FEAT each lane reads its own row.
-template <bool APPLY, ListRows ROWS, bool FEAT = false, bool SFEAT = false, bool REC = false>
-__global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4) k_steer(brt_grid_params g, uint32_t W, brt_steer_params sp, SteerCuts cuts,
-                                               float dt,
+template <bool APPLY, ListRows ROWS, bool FEAT = false, bool REC = false>
+__global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4)
+    k_steer(brt_grid_params g, uint32_t W, brt_steer_params sp, SteerCuts cuts, float dt,
                                                uint32_t step, uint32_t n, const float4* __restrict__ spos,
                                                const float4* __restrict__ sfwd, const float4* __restrict__ ssa,
                                                const uint2* __restrict__ hash,
@@ -129,13 +129,11 @@ __global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4) k_steer(brt_gri
         // next words after them (K 64: 3 % faster than ahead)
         auto visit = [&](uint32_t, const uint32_t(&jj)[8], uint32_t mask) {
             float4 qp[8], qf[8], fq[8];
-            uint32_t jid[8];
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
                 qp[t] = spos[jj[t]];
                 qf[t] = sfwd[jj[t]];
-                if (FEAT && SFEAT) fq[t] = sfeat[jj[t]];
-                if (FEAT && !SFEAT) jid[t] = hash[jj[t]].y;
+                if (FEAT) fq[t] = sfeat[jj[t]];
             }
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
@@ -145,13 +143,9 @@ __global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4) k_steer(brt_gri
                 }
             }
             if (FEAT) {
-                if (!SFEAT) {
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) fq[t] = fin[jid[t] < n ? jid[t] : id];
-                }
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
-                    if (((mask >> t) & 1u) == 0u || (!SFEAT && jid[t] >= n)) continue;
+                    if (((mask >> t) & 1u) == 0u) continue;
                     fsum.x = fsum.x + fq[t].x;
                     fsum.y = fsum.y + fq[t].y;
                     fsum.z = fsum.z + fq[t].z;
@@ -170,7 +164,7 @@ __global__ void __launch_bounds__(256, ROWS == kRowsOwn ? 1 : 4) k_steer(brt_gri
             feature = feature_update(feature_rate, n, hash, fin, id,
                                       [&](auto&& fn) { return for_list_octets(lists, W, W - 1u, i, n, fn); });
         } else {
-            const float4 f = SFEAT ? sfeat[i] : fin[id];
+            const float4 f = sfeat[i];
             float4 r = f;
             if (count != 0) {
                 const float inv = 1.0f / (float)count;  // cutil float4 / float
@@ -286,7 +280,10 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
                         float4* records) {
     AgentOut o{pos_out, fwd_out, sa_out, force_out, wander};
     const SteerCuts cuts = steer_cuts(sp);
-    const ListRows rows = list_rows(list_stride(K), n);  // records: from 2^19 agents, never kRowsOwn
+    const uint32_t W = list_stride(K);
+    const dim3 grid((n + 255) / 256);
+    const ListRows rows = list_rows(W, n);  // records: from 2^19 agents, never kRowsOwn
+    if (features_in && !sorted_features) return hipErrorInvalidValue;
     if (K > 32u && n >= kXcdRunMin && xcd_remap) xcd_remap = 2u;  // as the list pass before it
     if (records) {
         o.rec = records;
@@ -294,33 +291,28 @@ hipError_t launch_steer(const brt_grid_params& g, uint32_t K, const brt_steer_pa
         const hipEvent_t stop = launch_mark().stop;
         launch_mark().stop = nullptr;
         if (features_in)
-            BRT_LAUNCH((k_steer<true, kRowsOwn, true, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K),
-                       sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
-                       features_out, sorted_features);
+            BRT_LAUNCH((k_steer<true, kRowsOwn, true, true>), grid, dim3(256), 0, s, g, W, sp, cuts, dt, step, n, spos,
+                       sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in, features_out, sorted_features);
         else
-            BRT_LAUNCH((rows == kRowsWhole ? k_steer<true, kRowsWhole, false, false, true>
-                                           : k_steer<true, kRowsBlocks, false, false, true>),
-                       dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr,
-                       nullptr);
+            BRT_LAUNCH((rows == kRowsWhole ? k_steer<true, kRowsWhole, false, true>
+                                           : k_steer<true, kRowsBlocks, false, true>),
+                       grid, dim3(256), 0, s, g, W, sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap,
+                       0.0f, nullptr, nullptr, nullptr);
         o.wander = sp.wander_weight != 0.0f ? wander : nullptr;
         launch_mark().stop = stop;
         BRT_LAUNCH(k_unpack, dim3((unsigned)(((size_t)n * 4u + 255u) / 256u)), dim3(256), 0, s, n, records, o,
                    features_in ? features_out : nullptr);
         return hipGetLastError();
     }
-    if (features_in && sorted_features)
-        BRT_LAUNCH((k_steer<true, kRowsOwn, true, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp,
-                           cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
-                           features_out, sorted_features);
-    else if (features_in)
-        BRT_LAUNCH((k_steer<true, kRowsOwn, true>), dim3((n + 255) / 256), dim3(256), 0, s, g, list_stride(K), sp, cuts, dt,
-                           step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, feature_rate, features_in,
-                           features_out, nullptr);
+    if (features_in)
+        BRT_LAUNCH((k_steer<true, kRowsOwn, true>), grid, dim3(256), 0, s, g, W, sp, cuts, dt, step, n, spos, sfwd, ssa,
+                   hash, lists, o, xcd_remap, feature_rate, features_in, features_out, sorted_features);
     else
         BRT_LAUNCH((rows == kRowsOwn     ? k_steer<true, kRowsOwn>
                     : rows == kRowsWhole ? k_steer<true, kRowsWhole>
-                                         : k_steer<true, kRowsBlocks>), dim3((n + 255) / 256), dim3(256),
-                   0, s, g, list_stride(K), sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f, nullptr, nullptr, nullptr);
+                                         : k_steer<true, kRowsBlocks>),
+                   grid, dim3(256), 0, s, g, W, sp, cuts, dt, step, n, spos, sfwd, ssa, hash, lists, o, xcd_remap, 0.0f,
+                   nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 

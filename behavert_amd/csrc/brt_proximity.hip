@@ -40,6 +40,7 @@
 #include "brt_device.hpp"
 #include "brt_internal.hpp"
 #include "brt_steer_common.hpp"
+#include "brt_wave.hpp"
 
 // Candidates tested per round of the scan loops (their loads are in flight
 // together): per-lane (vector) rounds of dense waves with LDS lists, of sparse
@@ -1240,29 +1241,8 @@ __global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) 
 //     lanes' terms in list order, the same bits as one lane's; one wave of the
 //     workgroup then integrates its 64 agents.
 
-// The quad's lane k's value; every lane of the quad is active.
-template <int K>
-__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, K * 0x55, 0xF, 0xF, true);
-}
-template <int K>
-__device__ __forceinline__ float quad_lane(float v) {
-    return __uint_as_float(quad_lane<K>(__float_as_uint(v)));
-}
-
-// s + the quad's terms, lane 0's first
-__device__ __forceinline__ float quad_add(float s, float v) {
-    return (((s + quad_lane<0>(v)) + quad_lane<1>(v)) + quad_lane<2>(v)) + quad_lane<3>(v);
-}
 __device__ __forceinline__ V3 quad_add(V3 s, V3 v) {
-    return v3(quad_add(s.x, v.x), quad_add(s.y, v.y), quad_add(s.z, v.z));
-}
-
-// what every lane of the wave wrote to LDS is seen by the others
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return v3(brt::quad_add(s.x, v.x), brt::quad_add(s.y, v.y), brt::quad_add(s.z, v.z));
 }
 
 // The row scan of a wave of quads (lane l = 0..3 of each); false: some run is
