@@ -151,6 +151,7 @@ struct ProxArgs {
     uint32_t uniform_max_cells;
     uint32_t xcd_remap;
     uint32_t log_rounds;  // LDS lists through the round log (n < 2^24)
+    uint32_t together;    // the lanes of a quad visit their cells together (kTogetherK)
     uint32_t cells;       // cells of the launch for the row scan's bounded loads; 0: no row scan
     // agents of its own row beyond which an agent would rather not have its rows
     // scanned, by one lane and by four (row_limit)
@@ -746,8 +747,7 @@ __device__ __forceinline__ void flat_fetch(const ProxArgs& a, const Seg& sg, I3 
 // in the round j_self = own_start + G * floor((i - own_start) / G), in slot
 // (i - own_start) mod G, and in no round of another cell.
 template <int G, bool PACKED>
-__device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, uint32_t own_start,
-                                          bool together) {
+__device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane& L, I3 gp, uint32_t own_start) {
     static_assert((G & (G - 1)) == 0, "the self round is found with a mask");
     const brt_grid_params& g = sg.g;
     const uint32_t maxBodies = g.max_bodies_per_cell;
@@ -757,7 +757,7 @@ __device__ __forceinline__ void scan_flat(const ProxArgs& a, const Seg& sg, Lane
     const uint32_t jself = L.i - ds;
     const uint32_t smask = ~(1u << ((uint32_t)G - 1u - ds));
     uint32_t todo = visit_mask(sg, L, gp, a.Tskip);
-    if (together) todo = visit_together(todo, gp);
+    if (a.together) todo = visit_together(todo, gp);
     // the fetched (next) cell: ordinal nc (27: none left) and its range
     uint32_t nc = 27u, ns = BRT_EMPTY_CELL, ne = 0u;
     flat_fetch(a, sg, gp, todo, nc, ns, ne);
@@ -1132,20 +1132,19 @@ __global__ void __launch_bounds__(256, FUSE || LDSL ? 1 : 5) k_prox(ProxArgs a) 
         }
         // with the packed positions a round's loads are 3G/4 instead of G
         const bool packed = a.pxyz != nullptr;
-        const bool together = a.K >= kTogetherK && (!FUSE || a.K <= kTogetherFusedMax);
         if (LDSL && BRT_PROX_FLAT && dense && a.log_rounds) {
             if (alive) {
                 if (packed)
-                    scan_flat<kGroupL, true>(a, sg, L, gp, own_start, together);
+                    scan_flat<kGroupL, true>(a, sg, L, gp, own_start);
                 else
-                    scan_flat<kGroupL, false>(a, sg, L, gp, own_start, together);
+                    scan_flat<kGroupL, false>(a, sg, L, gp, own_start);
             }
         } else if (LDSL && BRT_PROX_FLAT_SPARSE && a.log_rounds) {
             if (alive) {
                 if (packed)
-                    scan_flat<kGroupR, true>(a, sg, L, gp, own_start, together);
+                    scan_flat<kGroupR, true>(a, sg, L, gp, own_start);
                 else
-                    scan_flat<kGroupR, false>(a, sg, L, gp, own_start, together);
+                    scan_flat<kGroupR, false>(a, sg, L, gp, own_start);
             }
         } else if (alive) {
             if (dense) {
@@ -1493,7 +1492,9 @@ __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
     }
     const bool can = a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED && sg.g.grid_size[0] >= 3u;
     const bool packed = a.pxyz != nullptr;
-    if (!FUSE && can && a.n > kQuadRowsMax && a.K <= kQuadRowsMaxK && one_lane_rows(a, sg, base, lane, wid, s_list)) return;
+    if (!FUSE && can && a.n > kQuadRowsMax && a.K <= kQuadRowsMaxK &&
+        one_lane_rows(a, sg, base, lane, wid, s_list))
+        return;
     const bool rows = can && (packed ? quad_rows<true>(a, sg, L, gp, alive, l)
                                      : quad_rows<false>(a, sg, L, gp, alive, l));
     if (!rows) {
@@ -1871,7 +1872,7 @@ bool launch_quad(ProxArgs a, const brt_prox_params& p, hipStream_t s) {
 
 ProxArgs make_args(const brt_grid_params& g, const brt_prox_params& p, float threshold, const float4* spos,
                    const uint2* hash, const uint32_t* cell_start, const uint32_t* cell_end, uint32_t n,
-                   uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t cells) {
+                   uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t cells, bool fused) {
     ProxArgs a{};
     a.cells = cells < (1u << 30) ? cells : 0u;  // 32-bit byte offsets
     a.row_occ = row_limit(p, false);
@@ -1889,6 +1890,7 @@ ProxArgs make_args(const brt_grid_params& g, const brt_prox_params& p, float thr
     a.uniform_max_cells = uniform_max_cells;
     a.xcd_remap = xcd_remap;
     a.log_rounds = n < (1u << 24) ? BRT_PROX_LOG : 0u;
+    a.together = p.max_neighbors >= kTogetherK && (!fused || p.max_neighbors <= kTogetherFusedMax) ? 1u : 0u;
     a.spos = spos;
     a.hash = hash;
     a.cell_start = cell_start;
@@ -1905,7 +1907,7 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
                             uint32_t xcd_remap, uint32_t lds_lists, bool quads, hipStream_t s, const float* pxyz) {
     const uint32_t K = p.max_neighbors;
     ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
-                           g.num_cells);
+                           g.num_cells, false);
     if (p.use_knn) {
         // one wave per workgroup, fewer lanes of it where the lists need the LDS
         uint32_t B = 64;
@@ -1933,7 +1935,7 @@ hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_param
                                   uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t lds_lists, bool quads,
                                   hipStream_t s, const float* pxyz) {
     ProxArgs a = make_args(g, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
-                           g.num_cells);
+                           g.num_cells, true);
     a.pxyz = pxyz;
     a.sfwd = sfwd;
     a.ssa = ssa;
@@ -1959,7 +1961,7 @@ hipError_t launch_batch_neighbors_steer(const BatchView& b, uint32_t n, const br
                                         uint32_t xcd_remap, uint32_t lds_lists, hipStream_t s, const float* pxyz) {
     brt_grid_params g0{};
     ProxArgs a = make_args(g0, p, threshold, spos, hash, cell_start, cell_end, n, lists, uniform_max_cells, xcd_remap,
-                           b.cells);
+                           b.cells, true);
     a.pxyz = pxyz;
     a.sfwd = sfwd;
     a.ssa = ssa;
