@@ -699,13 +699,14 @@ __device__ __forceinline__ uint32_t visit_mask(const Seg& sg, const Lane& L, I3 
 
 // The cells that a lane or, where they lie in its own cell, its quad's other lanes
 // visit.  The lanes of a quad then stay in step, until each has its list, and read
-// the same candidates in one access: the flat scan is bound by the L1's accesses
-// (about one a clock per CU: 0.89 of the fused kernel's time on 1M blobs) as much
-// as by its arithmetic (0.72), of which the added cells cost some.  With shorter
+// the same candidates in one access, which takes the load off the memory path
+// (address unit busy 75 -> 62 % of the fused kernel's time on 1M blobs, 400 -> 393 us)
+// for more arithmetic (10.9 -> 12.4 k instructions per wave).  With shorter
 // lists the lanes stop too early to gain: a step of 1M agents at 10 / 32 per cell
-// and in blobs gains 4 / 3 / 3 % at K 32, 5 / 3 / 3 % at K 28, 3 / 1 / 0 % at K 24
-// and -0 / -1 / -1 % at K 16; of 500,009 agents 7 / 5 / 2 % at K 32, of 300,007
-// (one wave more than the chip holds at once) 0 / 1 / 0 %.
+// and in blobs gains 7 / 2 / 1 % at K 32, 5 / 1 / 0 % at K 28 and loses up to 1 % at K
+// 16; of 500,009 agents 7 / 4 / 2 % at K 32, of 300,007 (one wave more than the chip
+// holds at once) it loses 1 / 1 / 2 %.  The list pass alone of 1M agents gains 24 / 11 /
+// 6 % at K 32.
 // Fused steps of long lists lose by it where the cells hold many (the waves in flight
 // are fewer then): 1M agents at 10 / 32 per cell and in blobs +8 / -1 / -3 % at K 48,
 // +3 / -6 / -5 % at K 64 and +2 / -6 / -5 % at K 80; the list pass alone gains or stays:

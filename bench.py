@@ -69,9 +69,15 @@ def algorithmic_bytes_per_agent(w, packed=False, sorted_sa=False) -> dict:
 
 
 PHASE_KERNELS = {"neighbors": "k_prox<false,false,*>", "steer_integrate": "k_steer",
-                 "steer_features": "k_steer<true,true> (steering + feature update)",
-                 "hash_sort": "k_prepare+k_hash_hist+k_onesweep", "reorder_ranges": "k_reorder_ranges",
+                 "steer_features": "k_steer<true,*,true> (steering + feature update)",
+                 "hash_sort": "k_hash_hist+k_onesweep", "reorder_ranges": "k_reorder_ranges",
                  "features": "k_features", "neighbors_steer": "k_prox<true,false,*>"}
+
+
+# two-pass steps with features that move the state by ID as 64-byte records
+RECORD_KERNELS = {"reorder_ranges": "k_pack+k_reorder_records",
+                  "steer_features": "k_steer<true,*,true,true>+k_unpack (steering + feature update)"}
+RECORD_AGENTS = 1 << 19
 
 
 def committed_metric(name: str, phase: str, workload: str):
@@ -120,6 +126,7 @@ def phase_table(ctx, w, abytes, fused):
     ms, nsteps = ctx.phase_times()
     out = {}
     merged = not fused and "steer_features" in abytes
+    names = {**PHASE_KERNELS, **(RECORD_KERNELS if merged and w.n >= RECORD_AGENTS else {})}
     for k, v in ms.items():
         name = "neighbors_steer" if (fused and k == "neighbors") else k
         if fused and k == "steer_integrate":
@@ -135,7 +142,7 @@ def phase_table(ctx, w, abytes, fused):
         gbs = (abytes[bkey] * w.n / 1e9) / (avg / 1e3) if avg > 0 and abytes[bkey] > 0 else 0.0
         out[name] = with_traffic({"ms": round(avg, 5), "bytes_per_agent": round(abytes[bkey], 2),
                                   "GB/s": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4),
-                                  "kernel": PHASE_KERNELS[name]}, name, w.name, w.n)
+                                  "kernel": names[name]}, name, w.name, w.n)
     return out
 
 
@@ -262,7 +269,7 @@ def adjoint_ratio(steps=None, every=None) -> dict:
             "step_ratio": round((step_ms + adj_ms) / step_ms, 3),
             "forward_rollout_ms": round(fwd_ms, 3), "backward_rollout_ms": round(bwd_ms, 3),
             "rollout_ratio": round((fwd_ms + bwd_ms) / fwd_ms, 3),
-            "roofline": {"bound": "hbm", "scope": "adjoint step (k_adjoint_own + k_adjoint_gather)",
+            "roofline": {"bound": "hbm", "scope": "adjoint step (k_adjoint_own_quad + k_adjoint_gather)",
                          "achieved": round(adj_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(adj_gbs / HBM_PEAK_GBS, 4), "bytes_per_agent": adj_bpa,
                          "traffic": committed_traffic("adjoint", "differentiable_65k")}}
@@ -354,7 +361,7 @@ def clustering(reps=20, features=8, lp_iterations=10) -> dict:
         "similarities_steer": (lambda: ctx.bc_similarities_steer(w.prox, sp, bc, fl.hash, fl.lists, feats, stats,
                                                                  stats2, sims, *sargs, f0, f1),
                                8 + 4 * Wd + 4 * features + 4 * (K + 1) + 32 + 32 + 32,
-                               "k_bc_sort_features+k_bc_similarities<true,true>"),
+                               "k_bc_records+k_bc_similarities_steer<true>"),
         "apply": (lambda: ctx.apply_steering_force(w.grid, sp, w.dt, *sargs, fl.sorted_smooth_accel, fl.hash, f1,
                                                    *outs, force_out=fo), 8 + 48 + 16 + 48 + 16, "k_apply"),
         # T iterations: list + own label per iteration, then by-ID float3 in/out,
@@ -363,7 +370,7 @@ def clustering(reps=20, features=8, lp_iterations=10) -> dict:
                                                       memb2, conn),
                        lp_iterations * (4 * Wd + 8) + 8 + 24 + 16 + 32, f"k_lp_iterate x{lp_iterations}"),
         "hit_rate": (lambda: ctx.cluster_hit_rate(w.prox, 1.5, fl.hash, fl.lists, fl.sorted_pos, memb2, memb),
-                     8 + 4 * Wd + 16 + 12 + 12, "k_hit_rate"),
+                     8 + 4 * Wd + 16 + 12 + 12, "k_gather_labels+k_hit_rate"),
     }
     res = {}
     for name, (fn, bpa, kern) in passes.items():

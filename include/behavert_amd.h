@@ -469,7 +469,12 @@ typedef struct brt_step_buffers {
 /* One plain step in the reference's order (Samples/OpensteerDemo/plugins/
  * BehaveRT_Flocking.cpp:177-196): hash+sort, reorder+ranges, neighbours,
  * fused steering+integration, then the feature update when features != NULL
- * and feature_rate != 0. */
+ * and feature_rate != 0.
+ * Scratch of the context: 16 bytes per agent and the sort's metadata, which a first
+ * call allocates (before a capture, then).  The packed positions (12 bytes per agent)
+ * and, from 2^19 agents in two passes with features, wander or the sorted smoothed
+ * acceleration, records of the state (64 or 80) are optional: a call that cannot have
+ * them (the stream is being captured, no memory) does without, with the same results. */
 int brt_step(brt_context* ctx, const brt_grid_params* grid,
              const brt_prox_params* prox, const brt_steer_params* steer,
              float feature_rate, float dt, uint32_t step,
