@@ -122,3 +122,30 @@ def test_captured_without_room_for_records(orc):
         torch.cuda.synchronize()
         assert same(sims, rs) and same(st, rst) and same(out, rf)
     own.close()
+
+
+@pytest.mark.parametrize("n,steer", [(SOON + 63, False), (SOON - 1, True), (1000, False)])
+def test_captured_after_a_pass_from_records(orc, n, steer):
+    """A warm-up from records, then the similarities alone, or a flock too small for
+    records, captured: the call has the scratch it needs."""
+    K, F = 32, 8
+    own = Context(0)
+    prox, bc, sp, args, state, _ = inputs(orc, SOON + 63, K, F, True)
+    own.bc_similarities_steer(prox, sp, bc, *args, empty_f32(SOON + 63, 4), torch.empty((SOON + 63, K + 1), device="cuda"),
+                              *state, empty_f32(SOON + 63, 4))
+    prox, bc, sp, args, state, (rs, rst, rf) = inputs(orc, n, K, F, True)
+    sims, st, out = torch.empty((n, K + 1), device="cuda"), empty_f32(n, 4), empty_f32(n, 4)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        if steer:
+            own.bc_similarities_steer(prox, sp, bc, *args, st, sims, *state, out)
+        else:
+            own.bc_similarities(prox, bc, *args, st, sims)
+    for _ in range(3):
+        for t in (sims, st, out):
+            t.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert same(sims, rs) and same(st, rst) and (not steer or same(out, rf))
+    own.close()
