@@ -160,7 +160,9 @@ struct ClusterAccum {
 // words, else only the similarities; and, with the cluster steering, the tile that
 // the records' parts change lanes in.
 constexpr uint32_t kTileChunks = 4u * 65u;  // float4; the 65: no bank conflicts
-inline __host__ __device__ uint32_t similarity_row_words(uint32_t K, uint32_t W) { return W <= kStageWords ? W : K + 1u; }
+inline __host__ __device__ uint32_t similarity_row_words(uint32_t K, uint32_t W) {
+    return W <= kStageWords ? W : K + 1u;
+}
 inline uint32_t similarity_wave_bytes(uint32_t K, uint32_t W) {
     return ((64u * similarity_row_words(K, W) * 4u + 15u) / 16u + kTileChunks) * 16u;
 }
@@ -724,8 +726,8 @@ hipError_t launch_cluster_membership(uint32_t K, uint32_t n, uint32_t iterations
                                      const uint32_t* lists, const float4* spos, const float* m_in, float* m_out,
                                      float4* conn, float* lbl_a, float* lbl_b, uint32_t xcd_remap, hipStream_t s) {
     if (iterations == 0) {
-        hipLaunchKernelGGL((k_lp_iterate<true, true, kRowsOwn, false>), dim3((n + 255) / 256), dim3(256), 0, s, K, list_stride(K), n,
-                           hash, lists, nullptr, nullptr, m_in, m_out, spos, conn, xcd_remap);
+        hipLaunchKernelGGL((k_lp_iterate<true, true, kRowsOwn, false>), dim3((n + 255) / 256), dim3(256), 0, s, K,
+                           list_stride(K), n, hash, lists, nullptr, nullptr, m_in, m_out, spos, conn, xcd_remap);
         return hipGetLastError();
     }
     const ListRows rows = list_rows(list_stride(K), n);
