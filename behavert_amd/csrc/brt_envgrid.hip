@@ -380,7 +380,7 @@ __global__ void __launch_bounds__(kSortThreads) k_onesweep(const uint2* __restri
 // pairs alone: 251 / 1170 / 192 us by the ranges' own workgroups, 61 / 72 / 80 us so
 // (the radix sort: 40); the whole step 539 / 3200 / 315 -> 99 / 1172 / 155 us, with
 // the radix sort and its separate passes 84 / 4828 / 151.  The sample costs up to
-// 0.4 us at 130,200 evenly spread agents (17.9 -> 18.2).
+// 0.5 us at 130,200 evenly spread agents (17.9 -> 18.4).
 // The kernel keeps no array in scratch (see emit): with 20 bytes per lane there some
 // builds of it took 13 us more at every size.
 constexpr uint32_t kCellThreads = 1024;
@@ -391,7 +391,11 @@ constexpr uint32_t kCellCap = 4096;     // agents a workgroup sorts at a time
 constexpr uint32_t kCellRankMax = 512;  // agents ranked by counting up to here, else bitonic
 constexpr uint32_t kNoKey = 0x7FFFFFFFu;  // beside every key (below 2^20)
 constexpr uint32_t kCellDense = 64;     // agents of a cell ranked within it up to here
-constexpr uint32_t kCellAlone = 2048;   // agents that a workgroup sorts by itself, if some cell holds more than those
+// Agents that a workgroup sorts by itself if some cell holds more than kCellDense; in
+// larger flocks all that it holds, since every chunk reads the keys again.  One sort of
+// the range -> chunks, pairs alone: ranges of 2,214 in 16,384 agents 39 -> 36 us, 3,000
+// in 3,000 40 -> 29; 2,423 in 33,194 42 -> 72, 2,877 in 65,536 44 -> 50.
+__device__ __forceinline__ uint32_t cell_alone(uint32_t n) { return n <= 16384u ? 2048u : kCellCap; }
 // IDs of a block; a chunk ends with the block in which it reaches as many agents
 constexpr uint32_t kCellBlock = 1024;
 constexpr uint32_t kCellBlocks = (1u << kCellIdBits) / kCellBlock;
@@ -557,8 +561,9 @@ __device__ __forceinline__ uint32_t wave_place(uint32_t* next, bool hit) {
 }
 
 // Who helps with the crowded ranges.  s_cnt[g] of the kCellSample sampled keys lie in
-// range g; a range that seems to hold more than kCellAlone agents wants one helper per
-// kCellBlock (16 samples or more, where even spreading gives 4 or fewer).
+// range g; a range that seems to hold more than half of cell_alone(n) wants one helper
+// per kCellBlock agents (17 samples or more, where even spreading gives 4 or fewer; so
+// that few crowded ranges are left to their own workgroup by chance).
 // The ranges that want none are light; the h-th light range's workgroup is the h-th
 // helper, if there are so many.  One wave (lane l has the ranges 4 l .. 4 l + 3); the
 // same in every workgroup.
@@ -572,7 +577,7 @@ struct CellShare {
 #pragma unroll
         for (uint32_t g = 0; g < kOwn; ++g) {
             const uint32_t agents = (uint32_t)((uint64_t)s_cnt[kOwn * lane + g] * n / kCellSample);
-            wants[g] = agents > kCellAlone ? agents / kCellBlock : 0u;
+            wants[g] = agents > cell_alone(n) / 2u ? agents / kCellBlock : 0u;
             sum += wants[g] << 16 | (wants[g] == 0u && kOwn * lane + g < groups ? 1u : 0u);
         }
         uint32_t x = sum;
@@ -670,7 +675,8 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
     __shared__ uint32_t s_cnt[kCellGroups], s_block[kCellBlocks];
     __shared__ uint32_t s_count, s_agents, s_below, s_most, s_wanted, s_group, s_slice, s_slices, s_lo, s_hi;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const bool spread = n > kCellAlone;  // some range may be crowded
+    const uint32_t alone = cell_alone(n);
+    const bool spread = n > alone;  // some range may be crowded
     // this thread's key of the sample: in short runs, since IDs may be in order of place
     const uint32_t sampled = spread ? keys[tid / kCellRun * (n / (kCellSample / kCellRun)) + tid % kCellRun] : 0u;
     static_assert(kCellSample == kCellThreads, "one sampled key per thread");
@@ -777,7 +783,7 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
 
     // the quads' agents into s_slot, as cell | ID, and their number per cell
     const uint32_t quads = s_count;
-    if (spread && tid < kCellGroups && s_cnt[tid] > kCellAlone * kCellSample / n) s_wanted = 1u;
+    if (spread && tid < kCellGroups && s_cnt[tid] > alone / 2u * kCellSample / n) s_wanted = 1u;
     if (quads <= kCellCap) {
         for (uint32_t t = tid; t < quads; t += kCellThreads) {
             const uint32_t i = 4u * s_list[t];
@@ -814,7 +820,7 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
                 for (uint32_t j = from; j < to; ++j) r += s_list[j] < v ? 1u : 0u;
                 emit(base + r, rel, v & ((1u << kCellIdBits) - 1u));
             }
-        } else if (m <= kCellAlone) {
+        } else if (m <= alone) {
             cell_group_sort(s_slot, s_rank, m);
             for (uint32_t i = tid; i < m; i += kCellThreads) {
                 const uint32_t v = s_slot[i];
@@ -880,7 +886,7 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_sort(const uint32_t* __re
         if (most > kCellDense) s_most = 1u;
         __syncthreads();
         // (the range's own workgroup has sorted it)
-        if (m <= kCellAlone || (m <= kCellCap && s_most == 0u)) return;  // a helper: own ranges are crowded
+        if (m <= alone || (m <= kCellCap && s_most == 0u)) return;  // a helper: own ranges are crowded
 
         // chunks of consecutive IDs, each of at most 2 kCellBlock - 1 agents, in turn by
         // the workgroups that share the range

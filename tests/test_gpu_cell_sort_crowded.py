@@ -85,6 +85,21 @@ def test_ranges_on_either_side_of_the_sample(ctx, orc, n, side, blobs, seed):
     check_sort(ctx, orc, W.cube_grid(side), flock_state(n, np.clip(xyz, 0.0, np.nextafter(np.float32(side), 0))))
 
 
+@pytest.mark.parametrize("n,m", [(16384, 2048), (16384, 2049), (16385, 2049), (16385, 4096), (16385, 4097), (60000, 4097),
+                                 (60000, 3100)])
+def test_one_range_around_the_limits(ctx, orc, n, m):
+    """A range of m agents in three cells, the others anywhere: whether it is crowded
+    depends on m and on the flock's size."""
+    rng = np.random.default_rng(n + m)
+    grid = GridParams.direct((0.0,) * 3, (4.0,) * 3, (64, 64, 16))  # 256 cells, four rows, per workgroup
+    xyz = rng.uniform(0, 1, (n - m, 3)) * (256.0, 256.0, 64.0)
+    inside = (xyz[:, 1] // 16 == 6) & (xyz[:, 2] // 4 == 5)
+    xyz[inside, 2] += 4.0
+    own = np.c_[rng.integers(9, 12, m) * 4.0, np.full(m, 100.0), np.full(m, 20.0)] + rng.uniform(0, 3.9, (m, 3))
+    xyz = np.concatenate([own, xyz])
+    check_sort(ctx, orc, grid, flock_state(n, xyz[rng.permutation(n)]))
+
+
 def test_two_crowded_cells_and_their_neighbours(ctx, orc):
     """Whole steps, with the gathers of the sorted state and the lists."""
     rng = np.random.default_rng(5)
