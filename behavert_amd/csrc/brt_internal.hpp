@@ -217,13 +217,13 @@ constexpr uint32_t kQuadSumWords = 11u;
 inline uint32_t prox_quad_lds(uint32_t K, bool fused) {
     return 64u * (list_stride(K) + (fused ? kQuadSumWords : 0u)) * 4u;
 }
-// Lists alone with K up to 32, which fill early or scan rows, stop at fewer agents:
-// one lane -> four at 1 / 3 / 6 / 20 per cell / in blobs, us: K 8, 30,000 agents 14 / 19 /
-// 23 / 28 / 186 -> 9 / 16 / 18 / 19 / 82, 65,000 13 / 19 / 25 / 26 / 127 -> 15 / 25 / 24 /
-// 24 / 62; K 24, 80,000 17 / 23 / 41 / 43 / 200 -> 17 / 23 / 40 / 33 / 89, 98,304 17 / 24 /
-// 43 / 43 / 137 -> 19 / 27 / 49 / 46 / 80 (worst of all: K 16 at six per cell, 36 -> 48).
+// Lists alone with K up to 32, which fill early or scan rows, stop at fewer agents, where
+// the two are even over flocks of all densities: one lane -> four at 1 / 3 / 6 / 20 per
+// cell / in blobs, us: K 8, 49,000 agents 14 / 20 / 24 / 29 / 184 -> 11 / 19 / 21 / 21 / 67,
+// 65,000 14 / 20 / 23 / 27 / 157 -> 14 / 25 / 24 / 24 / 62; K 16, 100,003 17 / 24 / 34 / 37 /
+// 167 -> 19 / 26 / 41 / 42 / 74, 131,072 17 / 25 / 36 / 37 / 104 -> 21 / 28 / 50 / 47 / 84.
 inline bool prox_quad_fits(uint32_t K, uint32_t n, bool fused) {
-    const uint32_t most = fused || K > 32u ? kProxQuadMax : (K < 16u ? 32768u : 90112u);
+    const uint32_t most = fused || K > 32u ? kProxQuadMax : (K < 16u ? 49152u : 106496u);
     return n <= most && prox_quad_lds(K, fused) <= 64u * 1024u;
 }
 // Row stride of the LDS list tile of the neighbour kernels: the list stride,

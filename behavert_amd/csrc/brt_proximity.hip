@@ -1456,7 +1456,9 @@ __device__ __forceinline__ bool one_lane_rows(const ProxArgs& a, Seg sg, uint32_
 }
 
 // five waves per SIMD: 100,003 agents 46.3 -> 45.3 us a step, 131,072 in blobs 155 -> 146
-template <bool FUSE>
+// ONE: lists alone above kQuadRowsMax agents (apart, since it takes the sixth wave from
+// the others: 12,883 agents, K 64, in a blob 55.2 -> 56.7 us).
+template <bool FUSE, bool ONE = false>
 __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
     alignas(16) extern __shared__ uint32_t s_list[];  // 64 rows of W words, then (fused) 64 of kQuadSumWords
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l = tid & 3u;
@@ -1493,9 +1495,7 @@ __global__ void __launch_bounds__(256, 5) k_prox_quad(ProxArgs a) {
     }
     const bool can = a.cells != 0u && sg.g.max_bodies_per_cell == BRT_UNLIMITED && sg.g.grid_size[0] >= 3u;
     const bool packed = a.pxyz != nullptr;
-    if (!FUSE && can && a.n > kQuadRowsMax && a.K <= kQuadRowsMaxK &&
-        one_lane_rows(a, sg, base, lane, wid, s_list))
-        return;
+    if (ONE && can && one_lane_rows(a, sg, base, lane, wid, s_list)) return;
     const bool rows = can && (packed ? quad_rows<true>(a, sg, L, gp, alive, l)
                                      : quad_rows<false>(a, sg, L, gp, alive, l));
     if (!rows) {
@@ -1853,21 +1853,28 @@ uint32_t prox_block(uint32_t W, uint32_t n) {
 // which the two cost the same: 1.6 K with one lane per agent, 2 K but no fewer than
 // 14 with four.  One lane, 131,072 agents at 1 / 3 / 6 per cell, cell by cell -> row
 // scan, us: K 4 20 -> 16 / 20 -> 23 / 20 -> 32, K 8 22 -> 16 / 24 -> 23 / 26 -> 32, K
-// 16 23 -> 17 / 30 -> 24 / 36 -> 34; four lanes, a step: K 4 68 -> 48 / 65 -> 59 / 57
-// -> 71, K 8 57 -> 49 / 74 -> 60 / 63 -> 72.  KNN lists, whose row scan holds K + 24
-// accepted candidates: about half of that.
-uint32_t row_limit(const brt_prox_params& p, bool quads) {
-    const uint32_t K = p.max_neighbors;
-    if (quads) return 2u * K > 14u ? 2u * K : 14u;
-    const uint32_t k = p.use_knn ? (K + kKnnLog) / 2u : K * 8u / 5u;
+// 16 23 -> 17 / 30 -> 24 / 36 -> 34.  KNN lists, whose row scan holds K + 24 accepted
+// candidates: about half of that.
+uint32_t row_limit(const brt_prox_params& p) {
+    const uint32_t K = p.max_neighbors, k = p.use_knn ? (K + kKnnLog) / 2u : K * 8u / 5u;
     return k < BRT_PROX_ROW_OCC ? k : BRT_PROX_ROW_OCC;
+}
+// With four lanes no limit in flocks of up to four per cell on average or 16,384
+// agents, whose slowest wave sets the time: there the few waves over the limit take
+// longer than the others save.  A step, no limit -> limit, us: 12,883 agents, K 8, at 3 /
+// 6 per cell 23 -> 29 / 27 -> 29; 100,003 agents 52 -> 56 / 62 -> 57, K 4 51 -> 53 / 61 -> 52.
+uint32_t quad_row_limit(uint32_t K, uint32_t n, uint32_t cells) {
+    if (n <= 16384u || n / 4u <= cells) return 0xFFFFFFFFu;
+    return 2u * K > 14u ? 2u * K : 14u;
 }
 
 template <bool FUSE>
-bool launch_quad(ProxArgs a, const brt_prox_params& p, hipStream_t s) {
+bool launch_quad(ProxArgs a, uint32_t cells, hipStream_t s) {
     if (!prox_quad_fits(a.K, a.n, FUSE)) return false;
-    a.row_occ_quad = row_limit(p, true);
-    BRT_LAUNCH((k_prox_quad<FUSE>), dim3((a.n + 63u) / 64u), dim3(256), prox_quad_lds(a.K, FUSE), s, a);
+    a.row_occ_quad = quad_row_limit(a.K, a.n, cells);
+    const auto kernel =
+        !FUSE && a.n > kQuadRowsMax && a.K <= kQuadRowsMaxK ? k_prox_quad<false, true> : k_prox_quad<FUSE, false>;
+    BRT_LAUNCH(kernel, dim3((a.n + 63u) / 64u), dim3(256), prox_quad_lds(a.K, FUSE), s, a);
     return true;
 }
 
@@ -1876,7 +1883,7 @@ ProxArgs make_args(const brt_grid_params& g, const brt_prox_params& p, float thr
                    uint32_t* lists, uint32_t uniform_max_cells, uint32_t xcd_remap, uint32_t cells, bool fused) {
     ProxArgs a{};
     a.cells = cells < (1u << 30) ? cells : 0u;  // 32-bit byte offsets
-    a.row_occ = row_limit(p, false);
+    a.row_occ = row_limit(p);
     a.g = g;
     a.K = p.max_neighbors;
     a.W = list_stride(p.max_neighbors);
@@ -1918,7 +1925,7 @@ hipError_t launch_neighbors(const brt_grid_params& g, const brt_prox_params& p, 
     }
     a.pxyz = pxyz;
     const uint32_t B = prox_block(a.Ws, n);
-    if (quads && launch_quad<false>(a, p, s)) return hipGetLastError();
+    if (quads && launch_quad<false>(a, g.num_cells, s)) return hipGetLastError();
     if (lds_lists)
         BRT_LAUNCH((k_prox<false, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else {
@@ -1946,7 +1953,7 @@ hipError_t launch_neighbors_steer(const brt_grid_params& g, const brt_prox_param
     a.step = step;
     a.o = AgentOut{pos_out, fwd_out, sa_out, nullptr, wander};
     const uint32_t B = prox_block(a.Ws, n);
-    if (quads && launch_quad<true>(a, p, s)) return hipGetLastError();
+    if (quads && launch_quad<true>(a, g.num_cells, s)) return hipGetLastError();
     if (lds_lists)
         BRT_LAUNCH((k_prox<true, false, true>), dim3((n + B - 1) / B), dim3(B), (size_t)B * a.Ws * 4u, s, a);
     else

@@ -33,3 +33,13 @@ def test_lists(ctx, orc, K, n, max_bodies, sparse):
     ctx.neighbors(grid, prox, dev(o["sorted_pos"]), *[dev(o[k].view(np.int32)) for k in
                                                       ("hash", "cell_start", "cell_end")], lists)
     assert first_mismatch(u32(lists), o["lists"]) is None
+
+
+@pytest.mark.parametrize("n,K", [(106496, 16), (106497, 16), (106496, 32), (49152, 15), (49153, 15), (16384, 8),
+                                 (16385, 8), (16385, 4)])
+def test_lists_at_the_lines_by_size(ctx, orc, n, K):
+    """Crowded and sparse flocks at the sizes where the quads, or their limit of the
+    row scan (more than four per cell on average), begin or end."""
+    test_lists(ctx, orc, K, n, 0xFFFFFFFF, True)
+    test_lists(ctx, orc, K, n, 0xFFFFFFFF, False)
+    test_lists(ctx, orc, K, n - n % 64 + 1, 0xFFFFFFFF, False)
